@@ -1037,18 +1037,37 @@ bool decode_fused_supported(size_t d, size_t ffn) {
 }
 
 
+// The layer kernel's instantiations for one (d, ffn): by prefetch depth of the attention tasks, in steps of 32 keys.
+typedef void (*LayerKernel)(LayerArgs);
+struct LayerKernels {
+    LayerKernel by_depth[5];
+};
+constexpr int LAYER_DEPTHS[5] = {4, 5, 6, 8, 10};
+template <int CH_D, int CH_F> constexpr LayerKernels layer_kernels_of() {
+    return {{decode_layer_kernel<CH_D, CH_F, 1, 4>, decode_layer_kernel<CH_D, CH_F, 1, 5>, decode_layer_kernel<CH_D, CH_F, 1, 6>,
+             decode_layer_kernel<CH_D, CH_F, 1, 8>, decode_layer_kernel<CH_D, CH_F, 1, 10>}};
+}
+// 1024 / 4096 beside 2048 / 8192: one launch takes 13.3 us where the three of mode 2 take 9.8 + 6.5 + 6.6 and two gaps
+// between them (0.401 against 0.601 ms per token of the 24-layer decoder behind a short prompt).  25 MB per launch: the chain LayerNorm -> qkv rows (3.5 us)
+// -> head's rows seen (5.6) -> attention (9.3) -> merge seen (12.2) -> written (12.6) bounds it, not the stream.
+static const LayerKernels *layer_kernels(size_t d, size_t ffn) {
+    static const LayerKernels wide = layer_kernels_of<4, 16>(), narrow = layer_kernels_of<2, 8>();
+    return pieces(d) == 4 && pieces(ffn) == 16 ? &wide : pieces(d) == 2 && pieces(ffn) == 8 ? &narrow : nullptr;
+}
+// Workgroups of a launch.  The narrow layer has 12,288 rows of work: two workgroups per unit (19.53 ms for 48 tokens, 19.70 and
+// 19.94 with three and four: more rows a wavefront, fewer workgroups to start and to queue in front of the chain).
+int decode_layer_grid(moon_ctx *ctx, size_t d) { return (pieces(d) == 4 ? LN_GEMV_GROUPS_PER_CU : 2) * (ctx->cu_count > 0 ? ctx->cu_count : 256); }
+
 // Can a whole layer run as one launch of decode_layer_kernel on this device?
 bool decode_layer_supported(moon_ctx *ctx, size_t d, size_t ffn, size_t H, size_t D) {
-    if (D != 64 || pieces(d) != 4 || pieces(ffn) != 16 || H * D != d || d % 512 || ffn % 512) return false; // (whole 1 KiB pieces)
-    const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
-    const int grid = LN_GEMV_GROUPS_PER_CU * cus;
+    const LayerKernels *set = layer_kernels(d, ffn);
+    if (D != 64 || !set || H * D != d || d % 512 || ffn % 512) return false; // (whole 1 KiB pieces)
+    const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256, grid = decode_layer_grid(ctx, d);
     const int waiting = (int)(H * DEC_SPLITS + (d + 3) / 4); // attention and output workgroups
     if (waiting >= grid || 3 * d > size_t(16) * grid) return false;
     int per_cu = 0;
-    const void *kernels[5] = {reinterpret_cast<const void *>(decode_layer_kernel<4, 16, 1, 4>), reinterpret_cast<const void *>(decode_layer_kernel<4, 16, 1, 5>),
-                              reinterpret_cast<const void *>(decode_layer_kernel<4, 16, 1, 6>), reinterpret_cast<const void *>(decode_layer_kernel<4, 16, 1, 8>),
-                              reinterpret_cast<const void *>(decode_layer_kernel<4, 16, 1, 10>)};
-    for (const void *k : kernels) {
+    for (const LayerKernel kern : set->by_depth) {
+        const void *k = reinterpret_cast<const void *>(kern);
         if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)((d + ffn) * sizeof(half_t))) != hipSuccess) return false;
         int n = 0;
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k, 256, (d + ffn) * sizeof(half_t)) != hipSuccess) return false;
@@ -1069,8 +1088,9 @@ int launch_decode_layer(moon_ctx *ctx, const half_t *x, const uint32_t *token, c
         return moon_fail(ctx, MOON_ESEQ_TOO_LONG, "decode attention: pos %zu >= max_seq %zu (limit 2048)", pos, max_seq);
     LayerArgs a;
     a.trace = trace;
+    const long long grid_wgs = decode_layer_grid(ctx, d);
     {
-        const long long n_attn = (long long)(H * DEC_SPLITS), n_out = (long long)((d + 3) / 4), grid_wgs = (long long)LN_GEMV_GROUPS_PER_CU * (ctx->cu_count > 0 ? ctx->cu_count : 256);
+        const long long n_attn = (long long)(H * DEC_SPLITS), n_out = (long long)((d + 3) / 4);
         const long long w_out = n_out * 4, w_fc1 = (grid_wgs - n_attn - n_out) * 4;
         static long long qkv_wgs = -1, r_o = -1;
         if (qkv_wgs < 0) {
@@ -1112,18 +1132,16 @@ int launch_decode_layer(moon_ctx *ctx, const half_t *x, const uint32_t *token, c
     a.pos = (int)pos;
     a.ffn = (int)ffn;
     a.pos_dev = pos_dev;
-    const unsigned grid = (unsigned)(LN_GEMV_GROUPS_PER_CU * (ctx->cu_count > 0 ? ctx->cu_count : 256));
+    const unsigned grid = (unsigned)grid_wgs;
     // The instantiation whose attention tasks request all their K and V rows before the wait for q: the pos cached keys go to
     // DEC_SPLITS - 1 splits, 32 keys per prefetch step (a step too few costs a dependent round trip per 32 keys inside the
     // attention chain: 0.628 instead of 0.598 ms per token at 900-1030 cached keys; steps too many cost 1-2 % at short
     // contexts).  pos is the host's count; a loop that has stopped at an end-of-sequence token only over-provides.
     const size_t per_split = (pos + DEC_SPLITS - 2) / (DEC_SPLITS - 1), steps = (per_split + 31) / 32;
     const size_t lds = (d + ffn) * sizeof(half_t);
-    if (steps <= 4) hipLaunchKernelGGL((decode_layer_kernel<4, 16, 1, 4>), dim3(grid), dim3(256), lds, ctx->stream, a);
-    else if (steps <= 5) hipLaunchKernelGGL((decode_layer_kernel<4, 16, 1, 5>), dim3(grid), dim3(256), lds, ctx->stream, a);
-    else if (steps <= 6) hipLaunchKernelGGL((decode_layer_kernel<4, 16, 1, 6>), dim3(grid), dim3(256), lds, ctx->stream, a);
-    else if (steps <= 8) hipLaunchKernelGGL((decode_layer_kernel<4, 16, 1, 8>), dim3(grid), dim3(256), lds, ctx->stream, a);
-    else hipLaunchKernelGGL((decode_layer_kernel<4, 16, 1, 10>), dim3(grid), dim3(256), lds, ctx->stream, a);
+    int depth = 0;
+    while (depth < 4 && steps > (size_t)LAYER_DEPTHS[depth]) depth++;
+    hipLaunchKernelGGL(layer_kernels(d, ffn)->by_depth[depth], dim3(grid), dim3(256), lds, ctx->stream, a);
     MOON_HIP(ctx, hipGetLastError());
     return MOON_OK;
 }

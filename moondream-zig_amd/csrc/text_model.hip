@@ -37,6 +37,7 @@ bool decode_lm_head_top_k_supported(moon_ctx *ctx, size_t top_k, size_t V);
 bool decode_front_supported(moon_ctx *ctx, size_t d, size_t H, size_t D);
 bool decode_layer_supported(moon_ctx *ctx, size_t d, size_t ffn, size_t H, size_t D);
 size_t decode_layer_sync_words(size_t H);
+int decode_layer_grid(moon_ctx *ctx, size_t d); // workgroups of a launch
 int launch_decode_layer(moon_ctx *ctx, const half_t *x, const uint32_t *token, const half_t *gamma, const half_t *beta, float eps, size_t d,
                         const half_t *Wqkv, const half_t *bqkv, half_t *qkv, const half_t *W1, const half_t *b1, half_t *fc1, size_t ffn,
                         const half_t *Wo, const half_t *bo, const half_t *W2, const half_t *b2, half_t *hidden, const half_t *hidden_src,
@@ -804,8 +805,7 @@ extern "C" int moon_text_hidden_f32(moon_text_model *m, float *hidden, size_t n_
 // the first workgroup started; mean and latest over the role's workgroups)
 static void print_layer_trace(moon_text_model *m) {
     const Sizes z = sizes(m->cfg);
-    const int cus = m->ctx->cu_count > 0 ? m->ctx->cu_count : 256;
-    const size_t grid = size_t(4) * cus, n_attn = z.H * 8, n_out = (z.d + 3) / 4;
+    const size_t grid = (size_t)decode_layer_grid(m->ctx, z.d), n_attn = z.H * 8, n_out = (z.d + 3) / 4;
     if (grid > 4096) return;
     std::vector<long long> t(grid * 8);
     if (hipMemcpy(t.data(), m->layer_trace, t.size() * sizeof(long long), hipMemcpyDeviceToHost) != hipSuccess) return;

@@ -237,6 +237,21 @@ def test_decode_modes_agree_full_size(moon, O, ctx):
     dev.close()
 
 
+@pytest.mark.parametrize("cached", [1, 2, 224, 225, 897, 1121, 1345, 1793, 2040])
+def test_decode_modes_agree_on_the_narrow_layer(moon, O, ctx, cached):
+    """Width 1024 runs a layer in one launch too: same bits as its three launches, at the edges of every prefetch depth."""
+    cfg = moon.text_model.make_config(vocab=3000, dim=1024, hidden_dim=4096, n_layers=2, n_heads=16)
+    dev = moon.text_model.TextModel(cfg, seed=7, std=0.02, ctx=ctx)
+    ids = O.fill_uniform_u32(cached, 0, 50, 3000)
+    dev.forward(ids)
+    assert dev.greedy_profile(1)[1]["attention"][1] == 0  # (the attention is no launch of its own)
+    (t1, l1, _), *others = _all_modes(dev, ids, 7)
+    for t, l, _ in others:
+        assert t == t1
+        assert np.array_equal(l.view(np.uint16), l1.view(np.uint16))
+    dev.close()
+
+
 def test_prefill_with_out_proj_and_fc2_in_one_launch(moon, O, ctx, monkeypatch):
     """At 192 rows and more the prefill runs a block's out_proj and fc2 as ONE launch (their partial sums are finished
     together); MOON_GEMM_NO_PAIR keeps them apart.  Same arithmetic but other splits of K.  Three layers of the real width
