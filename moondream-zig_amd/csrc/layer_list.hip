@@ -23,7 +23,7 @@ struct LayerList {
     int *ids = nullptr, *slot = nullptr, *tile_group = nullptr, *tile_row = nullptr, *tile_end = nullptr, *n_tiles = nullptr;
     uint32_t *grouped_rows = nullptr, *counter = nullptr, *want = nullptr;
     uint32_t *want_pinned = nullptr;
-    size_t mix_partial_floats = 0;
+    size_t mix_partial_floats = 0, partial_rows = 0;
     float *x1 = nullptr, *y3 = nullptr;                    // one token: the other copy of x, the parts of a joined layer's second product
     float *dt = nullptr, *delta_o = nullptr, *scratch = nullptr; // delta rule's rows: decays, outputs, chunks
     void *dgate = nullptr;
@@ -398,7 +398,10 @@ int create(LayerList *l, const Design *design, const SafeTensors *file, uint64_t
     MOON_TRY(alloc_n(l, R * nr, &l->router));
     MOON_TRY(alloc_t(l, R * k0, &l->a2));
     MOON_TRY(alloc_n(l, n16, &l->proj));
-    MOON_TRY(alloc_n(l, std::max(parts * R, std::min(SEG_MAX_SPLITS * R, 128 * cus / tiles_n)) * l->dp, &l->partial)); // (see seg_gemm_splits, joined_splits)
+    // the second products' slabs (seg_gemm_splits, joined_splits): two of a whole call's rows, more of short calls
+    l->partial_rows = std::max(parts * R, std::min(SEG_MAX_SPLITS * R, std::max(2 * R, 128 * cus / tiles_n)));
+    MOON_HIP(ctx, hipMalloc((void **)&l->partial, l->partial_rows * l->dp * sizeof(float))); // (written whole before it is read)
+    l->allocs.push_back(l->partial);
     if (parts > 1) {
         MOON_TRY(alloc_n(l, l->dp, &l->x1));
         MOON_TRY(alloc_n(l, 3 * l->dp, &l->y3));
@@ -726,10 +729,11 @@ int layer_list_forward(LayerList *l, const uint32_t *ids_dev, size_t n_rows, siz
         o.N = o.n32 = dp;
         o.K = d.k0;
         o.c32 = l->partial;
+        o.c32_rows = (int)l->partial_rows;
         o.ld32 = dp;
         f.out_l = d.out_l;
         f.out_r = d.out_r;
-        o.splits = d.out_l ? joined_splits(ctx, d, n, dp, &o, &f.splits_l, &f.splits_r) : seg_gemm_splits(ctx, n, dp, d.k0);
+        o.splits = d.out_l ? joined_splits(ctx, d, n, dp, &o, &f.splits_l, &f.splits_r) : seg_gemm_splits(ctx, n, dp, d.k0, l->partial_rows);
         MOON_TRY(launch_seg_gemm(ctx, dt, o));
         f.partial = l->partial;
         f.splits = o.splits;

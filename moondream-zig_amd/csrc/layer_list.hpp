@@ -114,12 +114,13 @@ struct SegGemm {
     int splits;               // splits > 1: n16 = 0, n32 = N, slab s of c32 (M x ld32 apart) gets k-range s
     int kb[SEG_MAX_SPLITS + 1]; // k-range s is [kb[s], kb[s + 1]), multiples of 64; all zero: even ranges
     int last_first;           // the last k-range's tiles start first, on every die (where the last ranges are the long ones)
+    int c32_rows;             // splits > 1: rows that c32 has room for, all slabs together
     float softcap;            // > 0: on the f32 segment
 };
 constexpr int SEG_TILE_ROWS = 128; // rows of a tile (both element types walk tile lists of this height)
 int launch_seg_gemm(moon_ctx *ctx, int dtype, SegGemm p);
-// k splits worth taking for an all-f32 product of this shape
-int seg_gemm_splits(moon_ctx *ctx, size_t M, size_t N, size_t K);
+// k splits worth taking for an all-f32 product of this shape; together their slabs have at most max_rows rows
+int seg_gemm_splits(moon_ctx *ctx, size_t M, size_t N, size_t K, size_t max_rows);
 
 // ---- row kernels (layer_rows.hip)
 // x[n] = embed[ids[n]] * scale (embed != null), or x += the k splits of a product + the chosen experts' weighted rows; then the

@@ -1,148 +1,176 @@
 // Products of the layer-list decoders: C[M, N] = A . W^T with the columns in segments (16-bit, f32, gated pairs), rows gathered
-// and grouped where a router asks for it.  bf16 runs on the matrix cores through the wavefront-specialised tile product of
-// gemm_dma.hpp; f32 is computed with f32 multiply-adds (no reduced-precision mode).
-#include "gemm_dma.hpp"
+// and grouped where a router asks for it.  bf16 runs on the matrix cores through the stream of tiles of gemm_stream.hpp; f32 is computed with f32 multiply-adds (no reduced-precision mode).
+#include "gemm_stream.hpp"
 #include "layer_list.hpp"
 #include "lm_types.hpp"
 
 #include <algorithm>
 #include <atomic>
+#include <map>
 
 namespace {
 
 struct TilePos {
     int m0, m_end, n0, group, split;
 };
-// Tile of this workgroup: consecutive workgroups land on different XCDs, so each XCD gets a contiguous run of tiles, walked m
-// first (tiles that share weight columns meet in one L2).  false: nothing to do.
-__device__ __forceinline__ bool seg_tile(const SegGemm &p, int tile_m, int tile_n, TilePos &t) {
+// Tile number `at` of a launch, in the order workgroups 0, 1, .. would take them: neighbours land on different XCDs, so each XCD gets a
+// contiguous run of tiles.  1: a tile, 0: nothing to do, -1: no number from here on has one on this XCD.
+// A run is walked in blocks of 2 x SEG_BAND tiles: the 32 tiles that an XCD works on at once then share 512 to 1,024 rows of either
+// operand, where whole columns of tiles (m first) read all of A again for every few columns: 117 against 123 us at 1920 x 16192 x
+// 2048 in 256-row tiles, 130 against 152 in 128-row tiles, weights from HBM.
+constexpr int SEG_BAND = 8;
+__device__ __forceinline__ int seg_tile(const SegGemm &p, int at, int tile_m, int tile_n, TilePos &t) {
     const int tiles_n = (p.N + tile_n - 1) / tile_n;
     const int tiles_m = p.tile_group ? p.max_tiles : (p.M + tile_m - 1) / tile_m;
     const int tiles = tiles_m * tiles_n, total = tiles * p.splits, per_xcd = (total + 7) / 8;
-    int wg = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
+    int wg = (at % 8) * per_xcd + at / 8;
     if (p.last_first) { // each XCD: its run of tiles of the last range, then of the one before, ..
-        const int run = (tiles + 7) / 8, j = blockIdx.x / 8, tile = (blockIdx.x % 8) * run + j % run;
-        if (j >= run * p.splits || tile >= tiles) return false;
+        const int run = (tiles + 7) / 8, j = at / 8, tile = (at % 8) * run + j % run;
+        if (j >= run * p.splits) return -1;
+        if (tile >= tiles) return 0;
         wg = (p.splits - 1 - j / run) * tiles + tile;
-    } else if ((int)(blockIdx.x / 8) >= per_xcd || wg >= total) return false;
+    } else if (at / 8 >= per_xcd || wg >= total) return -1;
     t.split = wg / tiles;
-    const int tile = wg % tiles, tn = tile / tiles_m, tm = tile % tiles_m;
+    const int tile = wg % tiles;
+    int tn = tile / tiles_m, tm = tile % tiles_m;
+    if (!p.tile_group) { // bands of SEG_BAND columns of tiles, walked two rows of tiles at a time
+        const int band = tile / (tiles_m * SEG_BAND), in = tile % (tiles_m * SEG_BAND), wide = min(SEG_BAND, tiles_n - band * SEG_BAND);
+        const int pair = in / (2 * wide), rest = in % (2 * wide), high = min(2, tiles_m - 2 * pair);
+        tm = 2 * pair + rest % high;
+        tn = band * SEG_BAND + rest / high;
+    }
     t.n0 = tn * tile_n;
-    if (p.tile_group) {
-        if (tm >= p.n_tiles[0]) return false;
-        t.group = p.tile_group[tm];
-        t.m0 = p.tile_row[tm];
-        t.m_end = min(t.m0 + tile_m, p.tile_end[tm]);
+    if (p.tile_group) { // (scalar loads: a launch does not write its own list, and a vector load would wait for the copies in flight)
+        typedef const __attribute__((address_space(4))) int *list_t;
+        auto entry = [&](const int *list, int i) { return ((list_t)list)[i]; };
+        if (tm >= entry(p.n_tiles, 0)) return 0;
+        t.group = entry(p.tile_group, tm);
+        t.m0 = entry(p.tile_row, tm);
+        t.m_end = min(t.m0 + tile_m, entry(p.tile_end, tm));
     } else {
         t.group = 0;
         t.m0 = tm * tile_m;
         t.m_end = min(t.m0 + tile_m, p.M);
     }
-    return true;
+    return 1;
 }
 
-// A wavefront's 64 x 64 accumulators -> its segment, through LDS so that the stores are whole lines.  scratch: 64 * 68 halfs.
-constexpr int SEG_PITCH16 = 72, SEG_PITCHG = 40, SEG_PITCH32 = 68;
-constexpr int SEG_SCRATCH_BYTES = 64 * SEG_PITCH16 * 2; // >= 64 * SEG_PITCHG * 2 and 32 * SEG_PITCH32 * 4
-static_assert(SEG_SCRATCH_BYTES >= 32 * SEG_PITCH32 * 4, "scratch");
+// A multiplier wavefront's accumulators -> their segment, 32 rows at a time through its 4 KiB of LDS so that the stores are whole
+// lines: rows of 128 (gated pairs: 64) bytes, the 16-byte granules XOR-swizzled by row.
 typedef bf16_t bf16x4_t __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ void seg_store(const SegGemm &p, const float16_t (&acc)[2][2], const TilePos &t, int wm, int wn, int lane, void *scratch) {
+template <int MI>
+__device__ __forceinline__ void seg_store(const SegGemm &p, const float16_t (&acc)[2][MI], const TilePos &t, int wm, int wn, int lane, char *scratch) {
     const int n = t.n0 + wn * 64, col = lane & 31, g = lane >> 5;
     if (n >= p.N) return;
+    const int m_wave = t.m0 + wm * 32 * MI, row8 = lane >> 3, g8 = lane & 7;
+    // the wavefront reads back what its own lanes wrote; its next writes come behind those reads, LDS serves it in order
+    auto written = [] { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); };
+    auto fence = [] { asm volatile("" ::: "memory"); };
     if (n < p.n16) {
-        bf16_t *s = reinterpret_cast<bf16_t *>(scratch);
 #pragma unroll
-        for (int ni = 0; ni < 2; ni++)
+        for (int mi = 0; mi < MI; mi++) {
 #pragma unroll
-            for (int mi = 0; mi < 2; mi++)
+            for (int ni = 0; ni < 2; ni++)
 #pragma unroll
                 for (int q = 0; q < 4; q++) {
                     bf16x4_t o;
 #pragma unroll
                     for (int e = 0; e < 4; e++) o[e] = (bf16_t)acc[ni][mi][4 * q + e];
-                    *reinterpret_cast<bf16x4_t *>(s + (mi * 32 + col) * SEG_PITCH16 + ni * 32 + 8 * q + 4 * g) = o;
+                    *reinterpret_cast<bf16x4_t *>(scratch + col * 128 + ((ni * 4 + q) ^ (col & 7)) * 16 + g * 8) = o;
                 }
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // the wavefront reads back what its own lanes wrote
+            written();
 #pragma unroll
-        for (int r = 0; r < 8; r++) {
-            const int ml = r * 8 + (lane >> 3), m = t.m0 + wm * 64 + ml;
-            if (m >= t.m_end) continue;
-            *reinterpret_cast<lm_u32x4 *>(reinterpret_cast<bf16_t *>(p.c16) + size_t(m) * p.ld16 + n + (lane & 7) * 8) =
-                *reinterpret_cast<const lm_u32x4 *>(s + ml * SEG_PITCH16 + (lane & 7) * 8);
+            for (int r = 0; r < 4; r++) {
+                const int ml = r * 8 + row8, m = m_wave + mi * 32 + ml;
+                const lm_u32x4 v = *reinterpret_cast<const lm_u32x4 *>(scratch + ml * 128 + (g8 ^ (ml & 7)) * 16);
+                if (m < t.m_end) *reinterpret_cast<lm_u32x4 *>(reinterpret_cast<bf16_t *>(p.c16) + size_t(m) * p.ld16 + n + g8 * 8) = v;
+            }
+            fence();
         }
     } else if (n < p.n32) {
-        float *s = reinterpret_cast<float *>(scratch);
-        float *dst = p.c32 + size_t(t.split) * p.M * p.ld32;
+        float *dst = p.c32 + size_t(t.split) * p.M * p.ld32 + (n - p.n16) + g8 * 4;
 #pragma unroll
-        for (int mi = 0; mi < 2; mi++) {
+        for (int mi = 0; mi < MI; mi++)
 #pragma unroll
-            for (int ni = 0; ni < 2; ni++)
+            for (int ni = 0; ni < 2; ni++) {
 #pragma unroll
                 for (int q = 0; q < 4; q++) {
-                    float4 o = {acc[ni][mi][4 * q], acc[ni][mi][4 * q + 1], acc[ni][mi][4 * q + 2], acc[ni][mi][4 * q + 3]};
-                    if (p.softcap > 0.0f) o = {lm_softcap(o.x, p.softcap), lm_softcap(o.y, p.softcap), lm_softcap(o.z, p.softcap), lm_softcap(o.w, p.softcap)};
-                    *reinterpret_cast<float4 *>(s + col * SEG_PITCH32 + ni * 32 + 8 * q + 4 * g) = o;
+                    float4_t o = {acc[ni][mi][4 * q], acc[ni][mi][4 * q + 1], acc[ni][mi][4 * q + 2], acc[ni][mi][4 * q + 3]};
+                    if (p.softcap > 0.0f) o = float4_t{lm_softcap(o[0], p.softcap), lm_softcap(o[1], p.softcap), lm_softcap(o[2], p.softcap), lm_softcap(o[3], p.softcap)};
+                    *reinterpret_cast<float4_t *>(scratch + col * 128 + ((2 * q + g) ^ (col & 7)) * 16) = o;
                 }
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                written();
 #pragma unroll
-            for (int r = 0; r < 8; r++) {
-                const int ml = r * 4 + (lane >> 4), m = t.m0 + wm * 64 + mi * 32 + ml;
-                if (m >= t.m_end) continue;
-                *reinterpret_cast<float4 *>(dst + size_t(m) * p.ld32 + (n - p.n16) + (lane & 15) * 4) =
-                    *reinterpret_cast<const float4 *>(s + ml * SEG_PITCH32 + (lane & 15) * 4);
+                for (int r = 0; r < 4; r++) {
+                    const int ml = r * 8 + row8, m = m_wave + mi * 32 + ml;
+                    const float4_t v = *reinterpret_cast<const float4_t *>(scratch + ml * 128 + (g8 ^ (ml & 7)) * 16);
+                    if (m < t.m_end) *reinterpret_cast<float4_t *>(dst + size_t(m) * p.ld32 + ni * 32) = v;
+                }
+                fence();
             }
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // the reads are done before the other half overwrites the rows
-        }
     } else {
-        bf16_t *s = reinterpret_cast<bf16_t *>(scratch);
+        const int row4 = lane >> 2, g4 = lane & 3;
 #pragma unroll
-        for (int mi = 0; mi < 2; mi++)
+        for (int mi = 0; mi < MI; mi++) {
 #pragma unroll
             for (int q = 0; q < 4; q++) {
                 bf16x4_t o;
 #pragma unroll
                 for (int e = 0; e < 4; e++) o[e] = (bf16_t)(lm_silu(acc[0][mi][4 * q + e]) * acc[1][mi][4 * q + e]);
-                *reinterpret_cast<bf16x4_t *>(s + (mi * 32 + col) * SEG_PITCHG + 8 * q + 4 * g) = o;
+                *reinterpret_cast<bf16x4_t *>(scratch + col * 64 + (q ^ ((col >> 1) & 3)) * 16 + g * 8) = o;
             }
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            written();
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const int ml = r * 16 + (lane >> 2), m = t.m0 + wm * 64 + ml;
-            if (m >= t.m_end) continue;
-            *reinterpret_cast<lm_u32x4 *>(reinterpret_cast<bf16_t *>(p.glu) + size_t(m) * p.ldg + (n - p.n32) / 2 + (lane & 3) * 8) =
-                *reinterpret_cast<const lm_u32x4 *>(s + ml * SEG_PITCHG + (lane & 3) * 8);
+            for (int r = 0; r < 2; r++) {
+                const int ml = r * 16 + row4, m = m_wave + mi * 32 + ml;
+                const lm_u32x4 v = *reinterpret_cast<const lm_u32x4 *>(scratch + ml * 64 + (g4 ^ ((ml >> 1) & 3)) * 16);
+                if (m < t.m_end) *reinterpret_cast<lm_u32x4 *>(reinterpret_cast<bf16_t *>(p.glu) + size_t(m) * p.ldg + (n - p.n32) / 2 + g4 * 8) = v;
+            }
+            fence();
         }
     }
 }
 
+template <int MI>
 __global__ __launch_bounds__(DMA_THREADS) void seg_gemm_bf16_kernel(SegGemm p) {
-    extern __shared__ __attribute__((aligned(16))) half_t lds_dma[]; // (the tile product addresses LDS from 0: nothing static beside it)
-    TilePos t;
-    if (!seg_tile(p, BM, BN, t)) return;
-    const int k_begin = p.kb[t.split], k_end = p.kb[t.split + 1], n_ktiles = (k_end - k_begin + BK - 1) / BK;
-    if (n_ktiles <= 0) return;
-    const int lane = threadIdx.x & 63, role_wave = (threadIdx.x >> 6) & 3;
-    if (threadIdx.x >= 256) {
-        DmaSource s;
-        s.a = p.A;
-        s.w = reinterpret_cast<const bf16_t *>(p.W) + size_t(t.group) * p.w_group;
-        s.a_bytes = p.a_rows * p.lda * 2; // (the launcher has checked that both fit)
-        s.w_bytes = p.N * p.K * 2;
-        s.w_k_bytes = 2;
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int r = dma_row(role_wave, j, lane), g8 = swz(r, lane & 7) * 8;
-            const int m = min(t.m0 + r, t.m_end - 1);
-            s.off_a[j] = ((p.rows ? (int)p.rows[m] : m) * p.lda + g8) * 2;
-            s.off_w[j] = (min(t.n0 + r, p.N - 1) * p.K + g8) * 2;
+    extern __shared__ __attribute__((aligned(16))) half_t lds_stream[]; // (the tile product addresses LDS from 0: nothing static beside it)
+    using S = Stream<MI>;
+    const int lane = threadIdx.x & 63, role_wave = __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) & 3);
+    int at = blockIdx.x;
+    auto next = [&](TilePos &t) { // (both roles walk the same tiles)
+        for (;; at += gridDim.x) {
+            const int r = seg_tile(p, at, S::ROWS, BN, t);
+            if (r < 0) return false;
+            if (r > 0) break;
         }
-        dma_load_tiles(s, lds_dma, k_begin, n_ktiles, role_wave);
+        at += gridDim.x;
+        return true;
+    };
+    if (threadIdx.x >= 256) {
+        stream_load<MI, TilePos>(lds_stream, role_wave, next, [&](const TilePos &t, StreamSource<MI> &s) {
+            // (the launcher has checked that both operands fit a descriptor)
+            const bf16_t *w = reinterpret_cast<const bf16_t *>(p.W) + size_t(t.group) * p.w_group;
+            s.a = __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p.A), 0, p.a_rows * p.lda * 2, 0x00020000);
+            s.w = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t *>(w), 0, p.N * p.K * 2, 0x00020000);
+#pragma unroll
+            for (int j = 0; j < 2 * MI; j++) {
+                const int r = stream_row_a(MI, role_wave, j, lane), m = min(t.m0 + r, t.m_end - 1);
+                s.off_a[j] = ((p.rows ? (int)p.rows[m] : m) * p.lda + swz(r, lane & 7) * 8) * 2;
+            }
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int r = 32 * role_wave + 8 * j + (lane >> 3);
+                s.off_w[j] = (min(t.n0 + r, p.N - 1) * p.K + swz(r, lane & 7) * 8) * 2;
+            }
+            s.k = p.kb[t.split] * 2;
+            s.n_ktiles = (p.kb[t.split + 1] - p.kb[t.split]) / BK;
+        });
         return;
     }
     const int wm = role_wave & 1, wn = role_wave >> 1;
-    float16_t acc[2][2];
-    dma_multiply_tiles<MfmaBf16, false>(acc, k_begin, k_end, n_ktiles, wm, wn, lane);
-    seg_store(p, acc, t, wm, wn, lane, reinterpret_cast<char *>(dma_free_stages(lds_dma, n_ktiles)) + size_t(role_wave) * SEG_SCRATCH_BYTES);
+    char *scratch = reinterpret_cast<char *>(lds_stream) + S::STAGES * S::STAGE_BYTES + role_wave * STREAM_SCRATCH_BYTES;
+    stream_multiply<MfmaBf16, MI, TilePos>(wm, wn, lane, next, [&](const TilePos &t) { return (p.kb[t.split + 1] - p.kb[t.split]) / BK; },
+                                           [&](const TilePos &t, const float16_t (&acc)[2][MI]) { seg_store<MI>(p, acc, t, wm, wn, lane, scratch); });
 }
 
 // f32: 64 x 64 tile, a thread owns rows ty, ty + 16, .. and columns tx, tx + 16, tx + 32, tx + 48 (so a gate column and its up
@@ -151,7 +179,7 @@ constexpr int F32_K = 16;
 __global__ __launch_bounds__(256) void seg_gemm_f32_kernel(SegGemm p) {
     __shared__ float sa[F32_K][64 + 4], sw[F32_K][64 + 4];
     TilePos t;
-    if (!seg_tile(p, SEG_TILE_ROWS, 64, t)) return;
+    if (seg_tile(p, blockIdx.x, SEG_TILE_ROWS, 64, t) <= 0) return;
     const int k_begin = p.kb[t.split], k_end = p.kb[t.split + 1];
     const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4, lr = tid >> 2, lk = (tid & 3) * 4;
     const float *A = reinterpret_cast<const float *>(p.A), *W = reinterpret_cast<const float *>(p.W) + size_t(t.group) * p.w_group;
@@ -190,10 +218,67 @@ __global__ __launch_bounds__(256) void seg_gemm_f32_kernel(SegGemm p) {
 
 } // namespace
 
-int seg_gemm_splits(moon_ctx *ctx, size_t M, size_t N, size_t K) {
-    const size_t cus = ctx->cu_count > 0 ? ctx->cu_count : 256, tiles = (M + BM - 1) / BM * ((N + BN - 1) / BN);
-    size_t s = std::min<size_t>(std::min<size_t>(cus / std::max<size_t>(tiles, 1), K / 512), 8);
-    return (int)std::max<size_t>(s, 1);
+// What a k-tile and the rest of a tile take with every compute unit busy and weights from HBM, us, by tile height.  The higher tiles
+// move fewer bytes per product, and a product's tiles seldom fill the last round, so the height is chosen by the rounds: 1920 rows x
+// 16192 x 2048 take 126 us in 256-row tiles (4 rounds), 132 in 192, 140 in 128 (a workgroup per 128-row tile: 171); 1920 x 2048 x
+// 7552 takes 77 us in 128-row tiles, 57 in 256-row tiles of two k ranges, whose second slab costs 3 us in row_finish.
+struct SegTime {
+    double k_tile, rest;
+};
+static SegTime seg_time(int mi) {
+    static const SegTime by_height[3] = {{0.58, 1.5}, {0.78, 2.0}, {0.95, 2.5}};
+    return by_height[mi - 2];
+}
+// us of tiles of that height: the workgroups take the ranges' tiles one after the other, the first free one the next.
+static double seg_estimate(int cus, int mi, int M, int N, const int *kb, int splits, bool last_first) {
+    const int tiles = (M + 64 * mi - 1) / (64 * mi) * ((N + BN - 1) / BN);
+    std::map<double, int> free{{0.0, cus}}; // workgroups by when they are done
+    for (int s = 0; s < splits; s++) {
+        const int r = last_first ? splits - 1 - s : s;
+        const double w = (kb[r + 1] - kb[r]) / BK * seg_time(mi).k_tile + seg_time(mi).rest;
+        for (int left = tiles; left > 0;) {
+            const auto first = free.begin();
+            const int n = std::min(left, first->second);
+            free[first->first + w] += n;
+            left -= n;
+            if ((first->second -= n) == 0) free.erase(first);
+        }
+    }
+    return free.rbegin()->first;
+}
+// the tile height (in 64 rows) for a product whose ranges are set
+static int seg_choose(moon_ctx *ctx, const SegGemm &p) {
+    const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
+    int best = 2;
+    double t = 1e30;
+    for (int mi = 2; mi <= 4; mi++)
+        if (const double e = seg_estimate(cus, mi, p.M, p.N, p.kb, p.splits, p.last_first); e < t) {
+            t = e;
+            best = mi;
+        }
+    return best;
+}
+
+static void even_ranges(int K, int splits, int *kb) {
+    for (int s = 0, per = (int)pad_to((K + splits - 1) / splits, BK); s <= splits; s++) kb[s] = std::min(K, s * per);
+}
+
+int seg_gemm_splits(moon_ctx *ctx, size_t M, size_t N, size_t K, size_t max_rows) {
+    const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
+    const double slab = (double)M * N * 8 / 4.5e6; // another range's sums, written and read, us at 4.5 TB/s
+    int best = 1;
+    double t = 1e30;
+    for (int splits = 1; splits <= SEG_MAX_SPLITS && (splits == 1 || (K / splits >= 512 && splits * M <= max_rows)); splits++) {
+        int kb[SEG_MAX_SPLITS + 1];
+        even_ranges((int)K, splits, kb);
+        if (kb[splits - 1] >= kb[splits]) continue;
+        for (int mi = 2; mi <= 4; mi++)
+            if (const double e = seg_estimate(cus, mi, (int)M, (int)N, kb, splits, false) + (splits - 1) * slab; e < t) {
+                t = e;
+                best = splits;
+            }
+    }
+    return best;
 }
 
 int launch_seg_gemm(moon_ctx *ctx, int dtype, SegGemm p) {
@@ -202,29 +287,41 @@ int launch_seg_gemm(moon_ctx *ctx, int dtype, SegGemm p) {
         return moon_fail(ctx, MOON_EINVAL_DIM, "segmented product: sizes must be padded to 64 (N %d, K %d, segments %d %d)", p.N, p.K, p.n16, p.n32);
     if (p.splits < 1) p.splits = 1;
     if (p.splits > 1 && (p.n16 || p.n32 != p.N || p.tile_group)) return moon_fail(ctx, MOON_EINVAL, "segmented product: only a plain f32 result splits k");
+    if (p.splits > 1 && (long long)p.splits * p.M > p.c32_rows) return moon_fail(ctx, MOON_EINVAL, "segmented product: %d slabs of %d rows, room for %d", p.splits, p.M, p.c32_rows);
     if (p.splits > SEG_MAX_SPLITS) return moon_fail(ctx, MOON_EINVAL, "segmented product: %d k splits", p.splits);
-    if (!p.kb[p.splits])
-        for (int s = 0, per = (int)pad_to((p.K + p.splits - 1) / p.splits, BK); s <= p.splits; s++) p.kb[s] = std::min(p.K, s * per);
+    if (!p.kb[p.splits]) even_ranges(p.K, p.splits, p.kb);
     for (int s = 0; s < p.splits; s++)
         if (p.kb[0] || p.kb[s] >= p.kb[s + 1] || p.kb[s + 1] % BK || p.kb[p.splits] != p.K)
             return moon_fail(ctx, MOON_EINVAL, "segmented product: %d k splits leave one empty", p.splits);
-    const int tile_n = dtype == MOON_DTYPE_BF16 ? BN : 64;
-    const size_t tiles = size_t(p.tile_group ? p.max_tiles : (p.M + SEG_TILE_ROWS - 1) / SEG_TILE_ROWS) * ((p.N + tile_n - 1) / tile_n) * p.splits;
-    const dim3 grid((unsigned)(p.last_first ? (tiles / p.splits + 7) / 8 * 8 * p.splits : (tiles + 7) / 8 * 8));
+    int rows = 64;
     if (dtype == MOON_DTYPE_BF16) {
         const size_t lim = (size_t(1) << 31) - 4096;
         if (size_t(p.a_rows) * p.lda * 2 >= lim || size_t(p.N) * p.K * 2 >= lim)
             return moon_fail(ctx, MOON_EINVAL_DIM, "segmented product: an operand of 2 GiB or more");
-        static std::atomic<bool> attr_set[64];
-        const int dev = ctx->device >= 0 && ctx->device < 64 ? ctx->device : -1;
-        if (dev < 0 || !attr_set[dev].load()) {
-            MOON_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void *>(seg_gemm_bf16_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)DMA_LDS_BYTES));
-            if (dev >= 0) attr_set[dev].store(true);
-        }
-        hipLaunchKernelGGL(seg_gemm_bf16_kernel, grid, dim3(DMA_THREADS), DMA_LDS_BYTES, ctx->stream, p);
-    } else
+        const int mi = p.tile_group ? 2 : seg_choose(ctx, p);
+        rows = 64 * mi;
+        auto go = [&](auto kern, size_t lds, std::atomic<bool> (&attr_set)[64]) -> int {
+            const int dev = ctx->device >= 0 && ctx->device < 64 ? ctx->device : -1;
+            if (dev < 0 || !attr_set[dev].load()) {
+                MOON_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+                if (dev >= 0) attr_set[dev].store(true);
+            }
+            const int cus = std::max(8, (ctx->cu_count > 0 ? ctx->cu_count : 256) / 8 * 8);
+            const size_t per_range = size_t(p.tile_group ? p.max_tiles : (p.M + rows - 1) / rows) * ((p.N + BN - 1) / BN);
+            const size_t places = p.last_first ? (per_range + 7) / 8 * 8 * p.splits : (per_range * p.splits + 7) / 8 * 8;
+            hipLaunchKernelGGL(kern, dim3((unsigned)std::min<size_t>(places, cus)), dim3(DMA_THREADS), lds, ctx->stream, p);
+            return MOON_OK;
+        };
+        static std::atomic<bool> set2[64], set3[64], set4[64];
+        if (mi == 4) MOON_TRY(go(seg_gemm_bf16_kernel<4>, Stream<4>::LDS_BYTES, set4));
+        else if (mi == 3) MOON_TRY(go(seg_gemm_bf16_kernel<3>, Stream<3>::LDS_BYTES, set3));
+        else MOON_TRY(go(seg_gemm_bf16_kernel<2>, Stream<2>::LDS_BYTES, set2));
+    } else {
+        const size_t tiles = size_t(p.tile_group ? p.max_tiles : (p.M + SEG_TILE_ROWS - 1) / SEG_TILE_ROWS) * (p.N / 64);
+        const dim3 grid((unsigned)(p.last_first ? (tiles + 7) / 8 * 8 * p.splits : (tiles * p.splits + 7) / 8 * 8));
         hipLaunchKernelGGL(seg_gemm_f32_kernel, grid, dim3(256), 0, ctx->stream, p);
+    }
     MOON_HIP(ctx, hipGetLastError());
-    MOON_NOTE_KERNEL(ctx, "%s %d workgroups, k split %d", dtype == MOON_DTYPE_BF16 ? "seg_gemm_bf16_kernel" : "seg_gemm_f32_kernel", (int)tiles, p.splits);
+    MOON_NOTE_KERNEL(ctx, "%s %d rows a tile, k split %d", dtype == MOON_DTYPE_BF16 ? "seg_gemm_bf16_kernel" : "seg_gemm_f32_kernel", rows, p.splits);
     return MOON_OK;
 }

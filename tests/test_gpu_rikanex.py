@@ -385,3 +385,19 @@ def test_trace_program(moon, ctx, folders, tmp_path):
     for i, rows in ((0, [0, 29]), (2, [32]), (3, [1])):
         got = np.fromfile(tmp_path / f"{i}.f32", "<f4").reshape(len(rows), cfg["vocab"])
         assert_close(got, want[rows], "float32")
+
+
+@pytest.mark.parametrize("rows", [130, 256, 257, 385, 640, 1025, 1301, 1537, 2000])
+@pytest.mark.parametrize("ff", [64, 3264])
+def test_tile_heights_of_the_products(moon, ctx, tmp_path, rows, ff):
+    """Prompts of a few hundred rows and more take tiles of 128, 192 or 256 rows and split k in other ways; the f32 session's plain
+    product takes none of these.  One layer of width 1024, all rows of the residual stream; limit: bf16 as everywhere in this file."""
+    cfg = config(130, 1024, [layer(attention(8, 2, 64, 64, 100, 0.125), dense(ff))], embed_scale=2.0)
+    path, ids = write_folder(tmp_path / "m", cfg, weights(cfg)), tokens(rows, 130)
+    streams = {}
+    for dtype in DTYPES:
+        m = opened(moon, ctx, path, dtype, max_seq=2048)
+        m.forward(ids)
+        streams[dtype] = m.hidden_f32(rows)
+        m.close()
+    assert_close(streams["bfloat16"], streams["float32"], "bfloat16")
