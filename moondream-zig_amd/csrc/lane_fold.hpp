@@ -2,6 +2,19 @@
 #pragma once
 #include "epilogue.hpp"
 
+constexpr int DPP_ROW_ROR8 = 0x128; // the lane 8 away within a row of 16
+
+// Sum over aligned groups of n lanes (a power of two, the same in every lane); every lane of a group returns it.
+__device__ __forceinline__ float group_sum(float v, int n) {
+    if (n >= 2) v += dpp_move<DPP_QUAD_XOR1>(v);
+    if (n >= 4) v += dpp_move<DPP_QUAD_XOR2>(v);
+    if (n >= 8) v += dpp_move<DPP_ROW_HALF_MIRROR>(v);
+    if (n >= 16) v += dpp_move<DPP_ROW_MIRROR>(v);
+    if (n >= 32) v += __shfl_xor(v, 16);
+    if (n >= 64) v += __shfl_xor(v, 32);
+    return v;
+}
+
 // Sums of N values over the lanes that differ in the bits of OFF and below down to `stop` (a power of two, the same in every lane).
 // At every step a lane hands one half of its values to its partner and keeps the other, so N / 2 + N / 4 + .. exchanges do; done(i, sum)
 // is called for the values that end up in this lane (by several lanes where there are fewer values than lanes).
@@ -15,6 +28,19 @@ __device__ __forceinline__ void fold_lanes(float (&v)[N], int lane, int stop, in
     const bool upper = lane & OFF;
     if constexpr (N > 1) {
         float half[N / 2];
+        if constexpr (OFF == 32 || OFF == 16) {
+            // one instruction swaps the upper rows of one value with the lower rows of the other (no trip through LDS)
+#pragma unroll
+            for (int i = 0; i < N / 2; i++) {
+                const unsigned a = __builtin_bit_cast(unsigned, v[i]), b = __builtin_bit_cast(unsigned, v[i + N / 2]);
+                const auto r = OFF == 32 ? __builtin_amdgcn_permlane32_swap(a, b, false, false) : __builtin_amdgcn_permlane16_swap(a, b, false, false);
+                const unsigned r0 = r[0], r1 = r[1];
+                half[i] = __builtin_bit_cast(float, r0) + __builtin_bit_cast(float, r1);
+            }
+        } else if constexpr (OFF == 8) {
+#pragma unroll
+            for (int i = 0; i < N / 2; i++) half[i] = (upper ? v[i + N / 2] : v[i]) + dpp_move<DPP_ROW_ROR8>(upper ? v[i] : v[i + N / 2]);
+        } else
 #pragma unroll
         for (int i = 0; i < N / 2; i++) half[i] = (upper ? v[i + N / 2] : v[i]) + __shfl_xor(upper ? v[i] : v[i + N / 2], OFF);
         if constexpr (OFF > 1) fold_lanes<N / 2, OFF / 2>(half, lane, stop, base + (upper ? N / 2 : 0), done);

@@ -4,9 +4,16 @@
 //                 the LM head.
 //   decode_mix    the token's attention over the cache (norm of q and k, rotation, value mixing, cache update, sink, output gate), keys
 //                 split over workgroups, the one that finishes last merging; beside it, in workgroups of their own, the router's choice
-//                 and the chosen experts' silu(gate) * up, or one token of the gated delta rule, a head per workgroup.
+//                 and the chosen experts' silu(gate) * up, or one token of the gated delta rule, a head per workgroup; and the dense
+//                 activation's part of the second product, which needs nothing of the attention.
 //   decode_out    x += W2 . (heads | dense activation) + the chosen experts' weighted down products, or the parts of W2 . (..) that
-//                 the next decode_proj joins.
+//                 the next decode_proj joins; without what decode_mix has left.
+// The attention is a chain of dependent steps that keeps a few units busy for 8 to 9 us, whatever it reads, while the stream of the dense
+// columns (22.5 of the second product's 30.9 MB at width 2048, feed-forward 5504) takes about as long: together 0.844 instead of
+// 0.908 ms per token behind 768 cached keys, 0.802 instead of 0.847 behind 60.  In the chain itself the projections are requested ahead of the
+// cache rows (loads return in order), lanes are summed with cross-lane moves instead of trips through LDS, the newest key is a piece like
+// the others and rows are found without divisions: 0.771 and 0.747 ms.  One split for a short context, which would save the merge, is slower
+// (0.785 against 0.747 at 60 to 90 keys): a step of 32 keys costs more than the hop.
 // All are bound by HBM: weights are read once with 128-bit non-temporal loads.  No workgroup waits for another.
 #include "delta_math.hpp"
 #include "lane_fold.hpp"
@@ -231,6 +238,7 @@ __global__ __launch_bounds__(256) void decode_proj_kernel(DecodeProj p) {
     }
 }
 
+constexpr int MIX_DOWN_ROWS = 4;   // rows of the dense activation's product per workgroup
 constexpr int MIX_HEADS = 8;       // query heads one workgroup serves
 constexpr int MIX_KEYS = 1024;     // keys of one split at most
 constexpr int MIX_TARGET = 32;     // keys of one split at least
@@ -245,8 +253,10 @@ __host__ __device__ __forceinline__ size_t mix_lds_floats(int nh, int dimp, int 
 }
 
 // Attention of one token: kv head g, query heads h0 .. h0 + nh - 1, split `split` of S.  Keys are numbered: the blocks that lie before
-// the window, then the window's tokens.  WHOLE: the mechanisms of the last part of DecodeMix.
-template <class T, int NH, bool WHOLE>
+// the window, then the window's tokens.  WHOLE: the mechanisms of the last part of DecodeMix.  LONG: head sizes of more than 64 pieces.
+// Every phase runs once or twice per launch, so what bounds it is latency, instruction fetches among it: nothing here is unrolled that
+// need not be, and cache rows are found without divisions.
+template <class T, int NH, bool WHOLE, bool LONG>
 __device__ __forceinline__ void mix_attention(const DecodeMix &p, int g, int hb, int split, int S, int keys_max, float *lds) {
     const int per = p.H / p.G, n_hb = mix_head_blocks(per), h0 = g * per + hb * MIX_HEADS, nh = min(MIX_HEADS, per - hb * MIX_HEADS);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -256,6 +266,7 @@ __device__ __forceinline__ void mix_attention(const DecodeMix &p, int g, int hb,
     const bool own = !(WHOLE && p.borrowed);    // the token's key and value are not in the cache yet
     const int newest = own ? n_keys - 1 : -1;   // their number
     float *s_q = lds, *s_k = s_q + NH * p.dimp, *s_v = s_k + p.dimp, *s_s = s_v + p.vdimp, *s_r = s_s + NH * keys_max, *s_ml = s_r + 4 * NH * p.vdimp;
+    T *t_k = reinterpret_cast<T *>(s_k), *t_v = reinterpret_cast<T *>(s_v); // the token's key and value as the cache holds them
     T *ck = reinterpret_cast<T *>(p.ck) + size_t(g) * p.cap * p.dimp, *cv = reinterpret_cast<T *>(p.cv) + size_t(g) * p.cap * p.vdimp;
     const T *pk_rows = reinterpret_cast<const T *>(p.pk) + size_t(g) * p.blocks * p.dimp, *pv_rows = reinterpret_cast<const T *>(p.pv) + size_t(g) * p.blocks * p.vdimp;
     const bool has_new = own && cnt > 0 && j1 == n_keys;
@@ -264,14 +275,51 @@ __device__ __forceinline__ void mix_attention(const DecodeMix &p, int g, int hb,
     constexpr int PE = Piece<T>::N, PF = 4;
     const int kp = p.dimp / PE, lpk = min(64, next_pow2(kp)), kpw = 64 / lpk, sub = lane / lpk, c0 = lane % lpk;
     const int vp = p.vdimp / PE, lpv = min(64, next_pow2(vp)), vpw = 64 / lpv, vsub = lane / lpv, vc0 = lane % lpv;
+    const int base_row = lo % p.cap; // (a window's tokens are at most cap)
+    auto token_row = [&](int j) { return base_row + j >= p.cap ? base_row + j - p.cap : base_row + j; };
+    const int new_row = token_row(pos - lo);
     auto k_piece = [&](int key, int c) {
-        const T *row = WHOLE && key < blocks ? pk_rows + size_t(key) * p.dimp : ck + size_t((key - blocks + lo) % p.cap) * p.dimp;
+        const T *row = WHOLE && key < blocks ? pk_rows + size_t(key) * p.dimp : ck + size_t(token_row(key - blocks)) * p.dimp;
         return *reinterpret_cast<const lm_u32x4 *>(row + c * PE);
     };
     auto v_piece = [&](int key, int c) {
-        const T *row = WHOLE && key < blocks ? pv_rows + size_t(key) * p.vdimp : cv + size_t((key - blocks + lo) % p.cap) * p.vdimp;
+        const T *row = WHOLE && key < blocks ? pv_rows + size_t(key) * p.vdimp : cv + size_t(token_row(key - blocks)) * p.vdimp;
         return *reinterpret_cast<const lm_u32x4 *>(row + c * PE);
     };
+    // The token's own projections first: a wavefront's loads return in order, and the cache rows come from further away.  This lane's
+    // first element of the wavefront's tasks (query heads, the new key, the new value).
+    constexpr int TASKS = (NH + 2 + 3) / 4;
+    const int n_tasks = nh + (has_new ? 2 : 0);
+    auto task_src = [&](int task) { return p.proj + (task == nh + 1 ? p.ov + g * p.vdimp : task < nh ? (h0 + task) * p.dimp : p.ok + g * p.dimp); };
+    float first[TASKS];
+#pragma unroll
+    for (int i = 0; i < TASKS; i++) {
+        const int task = wave + 4 * i;
+        first[i] = task < n_tasks && lane < (task == nh + 1 ? p.vdimp : p.dimp) ? task_src(task)[lane] : 0.0f;
+    }
+    auto task_half = [&](int task) { return WHOLE ? task == nh + 1 ? (p.rotv ? p.vdim / 2 : 0) : p.rot ? p.rot_dims / 2 : 0 : 0; }; // pairs that turn
+    float first_w[WHOLE ? TASKS : 1];
+    float2 first_cs[WHOLE ? TASKS : 1];
+    if (WHOLE) {
+#pragma unroll
+        for (int i = 0; i < TASKS; i++) {
+            const int task = wave + 4 * i, half = task_half(task);
+            first_w[i] = 1.0f;
+            first_cs[i] = float2{1.0f, 0.0f};
+            if (task >= n_tasks) continue;
+            if (p.whole && task <= nh && lane < p.dimp) first_w[i] = task < nh ? p.qn[(h0 + task) * p.dimp + lane] : p.kn[g * p.dimp + lane];
+            if (lane < 2 * half) first_cs[i] = (task == nh + 1 ? p.rotv : p.rot)[size_t(pos) * half + lane % half];
+        }
+    }
+    // (all of q and k are normed together: every workgroup adds their squares up)
+    constexpr int SQ = 2; // 4,096 bytes of q at a time
+    const int nq = WHOLE && p.whole ? p.H * p.dimp : 0, nk = WHOLE && p.whole && has_new ? p.G * p.dimp : 0;
+    float4_t sq_q[WHOLE ? SQ : 1], sq_k = {0, 0, 0, 0};
+    if (WHOLE) {
+#pragma unroll
+        for (int i = 0; i < SQ; i++) sq_q[i] = tid * 4 + 1024 * i < nq ? *reinterpret_cast<const float4_t *>(p.proj + tid * 4 + 1024 * i) : float4_t{0, 0, 0, 0};
+        if (tid * 4 < nk) sq_k = *reinterpret_cast<const float4_t *>(p.proj + p.ok + tid * 4);
+    }
     lm_u32x4 pk[PF], pv[PF];
 #pragma unroll
     for (int i = 0; i < PF; i++) {
@@ -301,23 +349,26 @@ __device__ __forceinline__ void mix_attention(const DecodeMix &p, int g, int hb,
     if constexpr (WHOLE) {
         // q and k are normed as a whole: the heads go to LDS turned and weighted, the norms' factors come last
         float ss[2] = {0.0f, 0.0f};
-        const int nq = p.H * p.dimp, nk = has_new ? p.G * p.dimp : 0;
-        if (p.whole) {
-            for (int i = tid * 4; i < nq; i += 1024) {
-                const float4_t v = *reinterpret_cast<const float4_t *>(p.proj + i);
-                ss[0] += (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]);
-            }
-            for (int i = tid * 4; i < nk; i += 1024) {
-                const float4_t v = *reinterpret_cast<const float4_t *>(p.proj + p.ok + i);
-                ss[1] += (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]);
-            }
-        }
-        for (int task = wave; task < nh + (has_new ? 2 : 0); task += 4) {
+        auto squares = [](const float4_t &v) { return (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]); };
+#pragma unroll
+        for (int i = 0; i < SQ; i++) ss[0] += squares(sq_q[i]);
+        ss[1] = squares(sq_k);
+        for (int i = tid * 4 + 1024 * SQ; i < nq; i += 1024) ss[0] += squares(*reinterpret_cast<const float4_t *>(p.proj + i));
+        for (int i = tid * 4 + 1024; i < nk; i += 1024) ss[1] += squares(*reinterpret_cast<const float4_t *>(p.proj + p.ok + i));
+#pragma unroll
+        for (int i = 0; i < TASKS; i++) {
+            const int task = wave + 4 * i, half = task_half(task);
+            if (task >= n_tasks) continue;
             const bool is_v = task == nh + 1, is_q = task < nh;
-            const float *src = p.proj + (is_v ? p.ov + g * p.vdimp : is_q ? (h0 + task) * p.dimp : p.ok + g * p.dimp);
-            const float *w = is_v || !p.whole ? nullptr : is_q ? p.qn + (h0 + task) * p.dimp : p.kn + g * p.dimp;
-            for (int d = lane; d < (is_v ? p.vdimp : p.dimp); d += 64)
-                (is_v ? s_v : is_q ? s_q + task * p.dimp : s_k)[d] = turned(src, w, d, is_v ? p.rotv : p.rot, (is_v ? p.vdim : p.rot_dims) / 2);
+            const int size = is_v ? p.vdimp : p.dimp;
+            float *dst = is_v ? s_v : is_q ? s_q + task * p.dimp : s_k;
+            if (size <= 64) { // the other element of a pair is another lane's
+                const float y = first[i] * first_w[i], z = __shfl(y, lane < half ? lane + half : lane - half);
+                if (lane < size) dst[lane] = lane >= 2 * half ? y : lane < half ? y * first_cs[i].x - z * first_cs[i].y : y * first_cs[i].x + z * first_cs[i].y;
+                continue;
+            }
+            const float *src = task_src(task), *w = is_v || !p.whole ? nullptr : is_q ? p.qn + (h0 + task) * p.dimp : p.kn + g * p.dimp;
+            for (int d = lane; d < size; d += 64) dst[d] = turned(src, w, d, is_v ? p.rotv : p.rot, half);
         }
         ss[0] = wave_sum(ss[0]);
         ss[1] = wave_sum(ss[1]);
@@ -330,36 +381,42 @@ __device__ __forceinline__ void mix_attention(const DecodeMix &p, int g, int hb,
         const float f_k = p.whole ? 1.0f / sqrtf(((s_r[1] + s_r[3]) + (s_r[5] + s_r[7])) / (float)(p.G * p.dim) + p.eps) : 1.0f;
         for (int i = tid; i < nh * p.dimp; i += 256) s_q[i] = (float)(T)(s_q[i] * f_q);
         if (has_new)
-            for (int i = tid; i < p.dimp + p.vdimp; i += 256) {
-                const bool is_v = i >= p.dimp;
+            for (int i0 = 0; i0 < p.dimp + p.vdimp; i0 += 256) { // (in rounds: the rounded values lie over the others)
+                const int i = i0 + tid;
+                const bool is_v = i >= p.dimp, live = i < p.dimp + p.vdimp;
                 const int d = is_v ? i - p.dimp : i;
-                const T c = (T)(is_v ? s_v[d] : s_k[d] * f_k);
-                (is_v ? s_v : s_k)[d] = (float)c;
-                if (hb == 0) (is_v ? cv + size_t(pos % p.cap) * p.vdimp : ck + size_t(pos % p.cap) * p.dimp)[d] = c;
+                const T c = (T)(live ? is_v ? s_v[d] : s_k[d] * f_k : 0.0f);
+                lds_barrier();
+                if (!live) continue;
+                (is_v ? t_v : t_k)[d] = c;
+                if (hb == 0) (is_v ? cv + size_t(new_row) * p.vdimp : ck + size_t(new_row) * p.dimp)[d] = c;
             }
     } else
-    for (int task = wave; task < nh + (has_new ? 2 : 0); task += 4) {
+#pragma unroll
+    for (int i = 0; i < TASKS; i++) {
+        const int task = wave + 4 * i;
+        if (task >= n_tasks) continue;
+        const float *src = task_src(task);
         if (task == nh + 1) { // the new value
-            const T *first = p.mixes ? reinterpret_cast<const T *>(p.v_first) + (size_t(g) * p.cap_first + pos % p.cap_first) * p.vdimp : nullptr;
+            const T *v1 = p.mixes ? reinterpret_cast<const T *>(p.v_first) + (size_t(g) * p.cap_first + pos % p.cap_first) * p.vdimp : nullptr;
             for (int d = lane; d < p.vdimp; d += 64) {
-                float v = (float)(T)p.proj[p.ov + g * p.vdimp + d];
-                if (first) v = (1.0f - p.lambda) * v + p.lambda * (float)first[d];
+                float v = (float)(T)(d == lane ? first[i] : src[d]);
+                if (v1) v = (1.0f - p.lambda) * v + p.lambda * (float)v1[d];
                 const T c = (T)v;
-                s_v[d] = (float)c;
-                if (hb == 0) cv[size_t(pos % p.cap) * p.vdimp + d] = c;
+                t_v[d] = c;
+                if (hb == 0) cv[size_t(new_row) * p.vdimp + d] = c;
             }
         } else { // a query head or the new key
             const bool is_q = task < nh;
-            const float *src = p.proj + (is_q ? (h0 + task) * p.dimp : p.ok + g * p.dimp);
-            float ss = 0.0f;
-            for (int d = lane; d < p.dimp; d += 64) ss = fmaf(src[d], src[d], ss);
+            float ss = first[i] * first[i];
+            for (int d = lane + 64; d < p.dimp; d += 64) ss = fmaf(src[d], src[d], ss);
             const float f = p.qk_rms ? 1.0f / sqrtf(wave_sum(ss) / (float)p.dim + p.eps) : 1.0f;
             for (int d = lane; d < p.dimp; d += 64) {
-                const T c = (T)(src[d] * f);
+                const T c = (T)((d == lane ? first[i] : src[d]) * f);
                 if (is_q) s_q[task * p.dimp + d] = (float)c;
                 else {
-                    s_k[d] = (float)c;
-                    if (hb == 0) ck[size_t(pos % p.cap) * p.dimp + d] = c;
+                    t_k[d] = c;
+                    if (hb == 0) ck[size_t(new_row) * p.dimp + d] = c;
                 }
             }
         }
@@ -374,7 +431,7 @@ __device__ __forceinline__ void mix_attention(const DecodeMix &p, int g, int hb,
             float sum = 0.0f;
 #pragma unroll 4
             for (int j = b * p.pool; j < pos; j++) sum += (float)rows[size_t(j % p.cap) * size + d];
-            sum += is_v ? s_v[d] : s_k[d];
+            sum += (float)(is_v ? t_v : t_k)[d];
             reinterpret_cast<T *>(is_v ? p.pv : p.pk)[(size_t(g) * p.blocks + b) * size + d] = (T)(sum / (float)p.pool);
         }
     }
@@ -385,28 +442,27 @@ __device__ __forceinline__ void mix_attention(const DecodeMix &p, int g, int hb,
         float acc[NH];
 #pragma unroll
         for (int h = 0; h < NH; h++) acc[h] = 0.0f;
-        if (key < j1)
-            for (int c = c0; c < kp; c += lpk) {
-                float kf[PE];
-                if (key == newest) {
+        for (int c = c0; c < kp; c += LONG ? lpk : kp) {
+            float kf[PE];
+            lm_u32x4 piece = first;
+            if (LONG && c != c0 && key < j1 && key != newest) piece = k_piece(key, c);
+            if (key == newest) piece = *reinterpret_cast<const lm_u32x4 *>(t_k + c * PE);
+            Piece<T>::unpack(piece, kf);
 #pragma unroll
-                    for (int e = 0; e < PE; e++) kf[e] = s_k[c * PE + e];
-                } else Piece<T>::unpack(c == c0 ? first : k_piece(key, c), kf);
+            for (int h = 0; h < NH; h++) // (heads past nh: whatever LDS holds, never stored)
 #pragma unroll
-                for (int h = 0; h < NH; h++)
-                    if (h < nh)
-#pragma unroll
-                        for (int e = 0; e < PE; e++) acc[h] = fmaf(kf[e], s_q[h * p.dimp + c * PE + e], acc[h]);
-            }
+                for (int e = 0; e < PE; e++) acc[h] = fmaf(kf[e], s_q[h * p.dimp + c * PE + e], acc[h]);
+        }
 #pragma unroll
         for (int h = 0; h < NH; h++) {
-            for (int off = lpk >> 1; off >= 1; off >>= 1) acc[h] += __shfl_xor(acc[h], off);
+            acc[h] = group_sum(acc[h], lpk);
             if (key < j1 && c0 == 0 && h < nh) s_s[h * keys_max + key - j0] = acc[h] * scale[h];
         }
     };
 #pragma unroll
     for (int i = 0; i < PF; i++)
         if (j0 + (i * 4 + wave) * kpw < j1) score_step(j0 + (i * 4 + wave) * kpw + sub, pk[i]);
+#pragma unroll 1
     for (int j = j0 + (PF * 4 + wave) * kpw; j < j1; j += 4 * kpw) {
         const int key = j + sub;
         lm_u32x4 first = {0, 0, 0, 0};
@@ -431,32 +487,30 @@ __device__ __forceinline__ void mix_attention(const DecodeMix &p, int g, int hb,
         }
     }
     lds_barrier();
-    for (int c = vc0; c < (vp + lpv - 1) / lpv * lpv; c += lpv) {
+    for (int c = vc0; c < (LONG ? (vp + lpv - 1) / lpv * lpv : lpv); c += lpv) {
         float acc[NH][PE];
 #pragma unroll
         for (int h = 0; h < NH; h++)
 #pragma unroll
             for (int e = 0; e < PE; e++) acc[h][e] = 0.0f;
-        auto value_step = [&](int key, const lm_u32x4 &piece) {
+        auto value_step = [&](int key, lm_u32x4 piece) {
             float vf[PE];
-            if (key == newest) {
+            if (key == newest) piece = *reinterpret_cast<const lm_u32x4 *>(t_v + c * PE);
+            Piece<T>::unpack(piece, vf);
 #pragma unroll
-                for (int e = 0; e < PE; e++) vf[e] = s_v[c * PE + e];
-            } else Piece<T>::unpack(piece, vf);
+            for (int h = 0; h < NH; h++) { // (heads past nh as above)
+                const float w = s_s[h * keys_max + key - j0];
 #pragma unroll
-            for (int h = 0; h < NH; h++)
-                if (h < nh) {
-                    const float w = s_s[h * keys_max + key - j0];
-#pragma unroll
-                    for (int e = 0; e < PE; e++) acc[h][e] = fmaf(w, vf[e], acc[h][e]);
-                }
+                for (int e = 0; e < PE; e++) acc[h][e] = fmaf(w, vf[e], acc[h][e]);
+            }
         };
         if (c < vp) {
 #pragma unroll
             for (int i = 0; i < PF; i++) {
                 const int key = j0 + (i * 4 + wave) * vpw + vsub;
-                if (key < j1) value_step(key, c == vc0 || key == newest ? pv[i] : v_piece(key, c));
+                if (key < j1) value_step(key, LONG && c != vc0 && key != newest ? v_piece(key, c) : pv[i]);
             }
+#pragma unroll 1
             for (int key = j0 + (PF * 4 + wave) * vpw + vsub; key < j1; key += 4 * vpw) value_step(key, key == newest ? pv[0] : v_piece(key, c));
         }
         float flat[NH * PE];
@@ -724,28 +778,15 @@ __device__ __forceinline__ void mix_experts(const DecodeMix &p, int wg, int n_wg
     }
 }
 
-template <class T, int NH, int U, bool WHOLE>
-__global__ __launch_bounds__(256) void decode_mix_kernel(DecodeMix p, int S, int keys_max, int n_attn, int n_expert) {
-    extern __shared__ __attribute__((aligned(16))) char s_mix[];
-    // attention first: it is a chain of dependent steps, the experts' part is one long stream
-    const int i = blockIdx.x, n_hb = mix_head_blocks(p.H / p.G);
-    if (WHOLE && i >= n_attn + n_expert) {
-        const int h = i - n_attn - n_expert;
-        if (p.ddimp <= DELTA_ROWS * (256 / (p.dvdimp / 4))) mix_delta<T, true>(p, h, reinterpret_cast<float *>(s_mix));
-        else mix_delta<T, false>(p, h, reinterpret_cast<float *>(s_mix));
-    } else if (i < n_attn) mix_attention<T, NH, WHOLE>(p, i / S / n_hb, i / S % n_hb, i % S, S, keys_max, reinterpret_cast<float *>(s_mix));
-    else mix_experts<T, U>(p, i - n_attn, n_expert, s_mix);
-}
-
-// x[n] += sum over the pieces of row n of W2 against a, and of the chosen experts' rows against their activations.  A workgroup
-// owns RW rows; its four wavefronts share each row's pieces, so a lane reads its part of the vectors once for all rows.
-// PARTS = 3: the sums over three stretches of the columns are kept apart.
-template <class T, int RW, int U, int PARTS>
-__global__ __launch_bounds__(256) void decode_out_kernel(DecodeOut p) {
-    __shared__ float s_part[4][PARTS][RW];
+// Rows [row0, row0 + RW) of W2 against columns [c0, c1) of a (16-byte pieces), and of the chosen experts' down matrices against their
+// activations.  A workgroup owns the rows; its four wavefronts share each row's pieces, so a lane reads its part of the vectors once
+// for all rows.  PARTS = 3: the sums over three stretches of the columns are kept apart.  done(k, r, sum) is called by one thread per
+// sum.
+template <class T, int RW, int U, int PARTS, class Done>
+__device__ __forceinline__ void out_rows(const DecodeOut &p, int row0, int c0, int c1, float (&s_part)[4][3][4], Done done) {
     constexpr int PE = Piece<T>::N;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, row0 = blockIdx.x * RW;
-    const int pa = p.k0 / PE, pf = p.top ? p.ffp / PE : 1, total = pa + p.top * pf;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int pa = c1 - c0, pf = p.top ? p.ffp / PE : 1, total = pa + p.top * pf;
     int begin, end;
     share(total, 4, wave, begin, end);
     float acc[PARTS][RW];
@@ -767,8 +808,8 @@ __global__ __launch_bounds__(256) void decode_out_kernel(DecodeOut p) {
                 const T *m;
                 size_t pitch;
                 if (i < pa) {
-                    x[u] = reinterpret_cast<const lm_u32x4 *>(p.a)[i];
-                    m = reinterpret_cast<const T *>(p.w2) + size_t(row0) * p.k0 + size_t(i) * PE;
+                    x[u] = reinterpret_cast<const lm_u32x4 *>(p.a)[c0 + i];
+                    m = reinterpret_cast<const T *>(p.w2) + size_t(row0) * p.k0 + size_t(c0 + i) * PE;
                     pitch = p.k0;
                 } else {
                     const int k = (i - pa) / pf, c = (i - pa) % pf;
@@ -787,7 +828,7 @@ __global__ __launch_bounds__(256) void decode_out_kernel(DecodeOut p) {
 #pragma unroll
             for (int r = 0; r < RW; r++) {
                 const float d = dot_piece<T>(w[u][r], x[u], 0.0f);
-                const int i = base + u * 64 + lane;
+                const int i = c0 + base + u * 64 + lane;
                 if (PARTS == 1) acc[0][r] = fmaf(d, scale[u], acc[0][r]);
                 else
 #pragma unroll
@@ -804,21 +845,52 @@ __global__ __launch_bounds__(256) void decode_out_kernel(DecodeOut p) {
     lds_barrier();
     const int k = tid / RW, r = tid % RW;
     if (k >= PARTS || row0 + r >= p.width) return;
-    const float s = (s_part[0][k][r] + s_part[1][k][r]) + (s_part[2][k][r] + s_part[3][k][r]);
-    if (PARTS == 1) p.x[row0 + r] += s;
-    else p.y[k * p.dp + row0 + r] = s;
+    done(k, row0 + r, (s_part[0][k][r] + s_part[1][k][r]) + (s_part[2][k][r] + s_part[3][k][r]));
 }
 
-template <class T, int NH, bool WHOLE> int mix_launch_as(moon_ctx *ctx, const DecodeMix &p, int S, int keys_max, int n_attn, int n_expert, size_t lds) {
-    auto kern = p.dp / Piece<T>::N > 64 ? decode_mix_kernel<T, NH, 4, WHOLE> : decode_mix_kernel<T, NH, 1, WHOLE>;
-    if (lds > 64 * 1024) MOON_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL(kern, dim3(n_attn + n_expert + (WHOLE ? p.dH : 0)), dim3(256), lds, ctx->stream, p, S, keys_max, n_attn, n_expert);
+// x += W2 . a, but for what decode_mix has left in p.down already.
+template <class T, int RW, int U, int PARTS>
+__global__ __launch_bounds__(256) void decode_out_kernel(DecodeOut p) {
+    __shared__ float s_part[4][3][4];
+    const int row = blockIdx.x * RW + threadIdx.x % RW;
+    float down = 0.0f;
+    if (PARTS == 1 && p.down && threadIdx.x < RW && row < p.width) down = p.down[row]; // (requested before the weights)
+    out_rows<T, RW, U, PARTS>(p, blockIdx.x * RW, 0, (p.down ? p.k2 : p.k0) / Piece<T>::N, s_part, [&](int k, int n, float s) {
+        if (PARTS == 1) p.x[n] += s + down;
+        else if (k < 2 || !p.down) p.y[k * p.dp + n] = s;
+    });
+}
+
+template <class T, int NH, int U, bool WHOLE, bool LONG>
+__global__ __launch_bounds__(256) void decode_mix_kernel(DecodeMix p, DecodeOut o, int S, int keys_max, int n_attn, int n_expert) {
+    extern __shared__ __attribute__((aligned(16))) char s_mix[];
+    __shared__ float s_part[4][3][4];
+    // attention first: it is a chain of dependent steps, the experts' part and the dense activation's product are long streams
+    const int i = blockIdx.x, n_hb = mix_head_blocks(p.H / p.G), n_delta = WHOLE ? p.dH : 0;
+    if (i < n_attn) mix_attention<T, NH, WHOLE, LONG>(p, i / S / n_hb, i / S % n_hb, i % S, S, keys_max, reinterpret_cast<float *>(s_mix));
+    else if (WHOLE && i < n_attn + n_delta) {
+        const int h = i - n_attn;
+        if (p.ddimp <= DELTA_ROWS * (256 / (p.dvdimp / 4))) mix_delta<T, true>(p, h, reinterpret_cast<float *>(s_mix));
+        else mix_delta<T, false>(p, h, reinterpret_cast<float *>(s_mix));
+    } else if (i < n_attn + n_delta + n_expert) mix_experts<T, U>(p, i - n_attn - n_delta, n_expert, s_mix);
+    else
+        out_rows<T, MIX_DOWN_ROWS, 4, 1>(o, (i - n_attn - n_delta - n_expert) * MIX_DOWN_ROWS, o.k2 / Piece<T>::N, o.k0 / Piece<T>::N, s_part,
+                                         [&](int, int n, float s) { o.down[n] = s; });
+}
+
+template <class T, int NH, bool WHOLE> int mix_launch_as(moon_ctx *ctx, const DecodeMix &p, const DecodeOut &o, int S, int keys_max, int n_attn, int n_expert, size_t lds) {
+    const bool longer = std::max(p.dimp, p.vdimp) > 64 * Piece<T>::N;
+    auto kern = longer ? decode_mix_kernel<T, NH, 4, WHOLE, true> : p.dp / Piece<T>::N > 64 ? decode_mix_kernel<T, NH, 4, WHOLE, false> : decode_mix_kernel<T, NH, 1, WHOLE, false>;
+    if (lds > 60 * 1024) MOON_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    const int n_down = o.down ? (o.width + MIX_DOWN_ROWS - 1) / MIX_DOWN_ROWS : 0;
+    hipLaunchKernelGGL(kern, dim3(n_attn + n_expert + (WHOLE ? p.dH : 0) + n_down), dim3(256), lds, ctx->stream, p, o, S, keys_max, n_attn, n_expert);
     MOON_HIP(ctx, hipGetLastError());
     return MOON_OK;
 }
 bool mix_whole(const DecodeMix &p) { return p.whole || p.rot || p.rotv || p.pool || p.temp || p.borrowed || p.dH; }
-template <class T, int NH> int mix_launch(moon_ctx *ctx, const DecodeMix &p, int S, int keys_max, int n_attn, int n_expert, size_t lds) {
-    return mix_whole(p) ? mix_launch_as<T, NH, true>(ctx, p, S, keys_max, n_attn, n_expert, lds) : mix_launch_as<T, NH, false>(ctx, p, S, keys_max, n_attn, n_expert, lds);
+template <class T, int NH> int mix_launch(moon_ctx *ctx, const DecodeMix &p, const DecodeOut &o, int S, int keys_max, int n_attn, int n_expert, size_t lds) {
+    return mix_whole(p) ? mix_launch_as<T, NH, true>(ctx, p, o, S, keys_max, n_attn, n_expert, lds)
+                        : mix_launch_as<T, NH, false>(ctx, p, o, S, keys_max, n_attn, n_expert, lds);
 }
 
 template <class T> int proj_launch(moon_ctx *ctx, const DecodeProj &p) {
@@ -848,6 +920,7 @@ template <class T> int out_launch(moon_ctx *ctx, const DecodeOut &p) {
         else if (p.width >= 2 * 2 * cus) hipLaunchKernelGGL((decode_out_kernel<T, 2, 6, N>), dim3((p.width + 1) / 2), dim3(256), 0, ctx->stream, p);
         else hipLaunchKernelGGL((decode_out_kernel<T, 1, 8, N>), dim3(p.width), dim3(256), 0, ctx->stream, p);
     };
+    if (p.down && (p.top || p.k2 % 64 || p.k2 >= p.k0)) return moon_fail(ctx, MOON_EINVAL, "decode: no dense columns behind %d of %d", p.k2, p.k0);
     if (p.y && (p.top || p.k1 % 64 || p.k2 % 64 || p.k1 > p.k2 || p.k2 > p.k0)) return moon_fail(ctx, MOON_EINVAL, "decode: columns in parts %d %d %d", p.k1, p.k2, p.k0);
     if (p.y) go(std::integral_constant<int, 3>{});
     else go(std::integral_constant<int, 1>{});
@@ -871,7 +944,7 @@ size_t decode_mix_partial_floats(moon_ctx *ctx, size_t heads, size_t kv_heads, s
     return std::max(std::max(wgs, cus), wgs * ((max_keys + MIX_KEYS - 1) / MIX_KEYS)) * MIX_HEADS * (vdimp + 2);
 }
 
-int launch_decode_mix(moon_ctx *ctx, int dtype, const DecodeMix &p) {
+int launch_decode_mix(moon_ctx *ctx, int dtype, const DecodeMix &p, const DecodeOut &o) {
     const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256, per = p.H / p.G, wgs = p.G * mix_head_blocks(per);
     const int n_win = (int)(p.window ? std::min(p.pos + 1, (size_t)p.window) : p.pos + 1), n_keys = n_win + (p.pool ? (int)(p.pos + 1 - n_win) / p.pool : 0);
     if (p.pool && ((p.pos + 1) / p.pool > (size_t)p.blocks || (p.pos + 1 >= (size_t)p.pool && p.pool > p.cap))) return moon_fail(ctx, MOON_EINVAL_DIM, "decode attention: %d pooled blocks kept", p.blocks);
@@ -895,10 +968,10 @@ int launch_decode_mix(moon_ctx *ctx, int dtype, const DecodeMix &p) {
     auto go = [&](auto tag) -> int {
         using T = decltype(tag);
         switch (NH) {
-        case 1: return mix_launch<T, 1>(ctx, p, S, keys_max, wgs * S, n_expert, lds);
-        case 2: return mix_launch<T, 2>(ctx, p, S, keys_max, wgs * S, n_expert, lds);
-        case 4: return mix_launch<T, 4>(ctx, p, S, keys_max, wgs * S, n_expert, lds);
-        default: return mix_launch<T, 8>(ctx, p, S, keys_max, wgs * S, n_expert, lds);
+        case 1: return mix_launch<T, 1>(ctx, p, o, S, keys_max, wgs * S, n_expert, lds);
+        case 2: return mix_launch<T, 2>(ctx, p, o, S, keys_max, wgs * S, n_expert, lds);
+        case 4: return mix_launch<T, 4>(ctx, p, o, S, keys_max, wgs * S, n_expert, lds);
+        default: return mix_launch<T, 8>(ctx, p, o, S, keys_max, wgs * S, n_expert, lds);
         }
     };
     return dtype == MOON_DTYPE_BF16 ? go(bf16_t{}) : go(float{});

@@ -18,7 +18,7 @@ struct LayerList {
     int first_mix = -1;
     void *embed = nullptr, *head = nullptr;
     float *fgamma = nullptr, *fbeta = nullptr;
-    float *x = nullptr, *router = nullptr, *partial = nullptr, *proj = nullptr, *logits = nullptr, *mix_partial = nullptr, *weight = nullptr;
+    float *x = nullptr, *down = nullptr, *router = nullptr, *partial = nullptr, *proj = nullptr, *logits = nullptr, *mix_partial = nullptr, *weight = nullptr;
     void *h = nullptr, *c1 = nullptr, *a2 = nullptr, *act = nullptr, *y = nullptr;
     int *ids = nullptr, *slot = nullptr, *tile_group = nullptr, *tile_row = nullptr, *tile_end = nullptr, *n_tiles = nullptr;
     uint32_t *grouped_rows = nullptr, *counter = nullptr, *want = nullptr;
@@ -398,6 +398,7 @@ int create(LayerList *l, const Design *design, const SafeTensors *file, uint64_t
     MOON_TRY(alloc_n(l, R * nr, &l->router));
     MOON_TRY(alloc_t(l, R * k0, &l->a2));
     MOON_TRY(alloc_n(l, n16, &l->proj));
+    MOON_TRY(alloc_n(l, l->dp, &l->down));
     // the second products' slabs (seg_gemm_splits, joined_splits): two of a whole call's rows, more of short calls
     l->partial_rows = std::max(parts * R, std::min(SEG_MAX_SPLITS * R, std::max(2 * R, 128 * cus / tiles_n)));
     MOON_HIP(ctx, hipMalloc((void **)&l->partial, l->partial_rows * l->dp * sizeof(float))); // (written whole before it is read)
@@ -878,7 +879,6 @@ int layer_list_step(LayerList *l, const uint32_t *token_dev, size_t pos, const u
             o.weight = l->weight;
         }
         x.dp = dp;
-        MOON_TRY(launch_decode_mix(ctx, dt, x));
         o.x = x_now;
         o.y = joined ? l->y3 : nullptr;
         o.k1 = d.ka;
@@ -888,6 +888,8 @@ int layer_list_step(LayerList *l, const uint32_t *token_dev, size_t pos, const u
         o.k0 = d.k0;
         o.w2 = d.w2;
         o.a = l->a2;
+        o.down = o.k2 < o.k0 ? (joined ? l->y3 + 2 * dp : l->down) : nullptr;
+        MOON_TRY(launch_decode_mix(ctx, dt, x, o));
         MOON_TRY(launch_decode_out(ctx, dt, o));
     }
     if (!joined) return MOON_OK;

@@ -297,14 +297,11 @@ struct DecodeMix {            // attention of the token (and its cache update) b
     void *ring;
     void *dout;               // T [dH][dvdimp]
 };
-size_t decode_mix_partial_floats(moon_ctx *ctx, size_t heads, size_t kv_heads, size_t vdimp, size_t max_keys);
-size_t decode_mix_counters(size_t heads, size_t kv_heads);
-int launch_decode_mix(moon_ctx *ctx, int dtype, const DecodeMix &p);
-
 struct DecodeOut {            // x += W2 . a + the chosen experts' weighted second product
     float *x;
     float *y;                 // set: x stays as it is, and the products over a's columns [0, k1), [k1, k2), [k2, k0) go to y [3][dp]
     int k1, k2;
+    float *down;              // set: decode_mix leaves W2's columns [k2, k0) (the dense activation's) times a here, [width]; with y that is y's last part
     int width, dp, k0;
     const void *w2, *a;
     int top, ffp;
@@ -312,6 +309,11 @@ struct DecodeOut {            // x += W2 . a + the chosen experts' weighted seco
     const int *ids;
     const float *weight;
 };
+size_t decode_mix_partial_floats(moon_ctx *ctx, size_t heads, size_t kv_heads, size_t vdimp, size_t max_keys);
+size_t decode_mix_counters(size_t heads, size_t kv_heads);
+// o: what decode_out will be called with; its part that needs no attention (DecodeOut::down) runs beside the attention
+int launch_decode_mix(moon_ctx *ctx, int dtype, const DecodeMix &p, const DecodeOut &o);
+
 int launch_decode_out(moon_ctx *ctx, int dtype, const DecodeOut &p);
 
 // ---- the engine (layer_list.hip): weights, caches and buffers of one sequence's session, prompt rows and single tokens

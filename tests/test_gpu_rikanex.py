@@ -401,3 +401,12 @@ def test_tile_heights_of_the_products(moon, ctx, tmp_path, rows, ff):
         streams[dtype] = m.hidden_f32(rows)
         m.close()
     assert_close(streams["bfloat16"], streams["float32"], "bfloat16")
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("dim,vdim", [(512, 512), (520, 64), (64, 528), (1016, 1024)])
+def test_head_sizes_around_a_wavefront_of_pieces(moon, ctx, tmp_path, dim, vdim, dtype):
+    """One token: heads of up to 64 16-byte pieces are a lane's piece each, larger ones are walked."""
+    cfg = config(90, 64, [layer(attention(3, 1, dim, vdim, 9, dim**-0.5), dense(72)), layer(attention(2, 2, dim, vdim, 30, dim**-0.5, True), dense(8))])
+    w, ids = weights(cfg, 3), tokens(40, 90)
+    assert_close(run(moon, ctx, tmp_path, cfg, w, ids, dtype, [3] + [1] * 37), R.forward(cfg, w, ids)[0], dtype)
