@@ -512,20 +512,11 @@ __device__ __forceinline__ void gemm_nt_dma2_body(const GemmArgs &p, int wg_arg 
 #pragma unroll
             for (int v = 0; v < 16; v++) acc[i][j][v] = 0.0f;
 
-    unsigned off_a[BK / 16][MI], off_w[BK / 16][2]; // LDS byte offsets (within a stage) of this lane's operand slices
+    // (blocks of 32 rows are 4 KiB apart whatever the lane and enter as the reads' offset: gemm_dma.hpp)
+    unsigned lane_off[BK / 16];
 #pragma unroll
-    for (int s = 0; s < BK / 16; s++) {
-#pragma unroll
-        for (int i = 0; i < MI; i++) {
-            const int rm = wm * 32 * MI + i * 32 + frag_row;
-            off_a[s][i] = (rm * BK + swz(rm, 2 * s + frag_g) * 8) * 2;
-        }
-#pragma unroll
-        for (int i = 0; i < 2; i++) {
-            const int rn = wn * 64 + i * 32 + frag_row;
-            off_w[s][i] = (BM2 * BK + rn * BK + swz(rn, 2 * s + frag_g) * 8) * 2;
-        }
-    }
+    for (int s = 0; s < BK / 16; s++) lane_off[s] = (frag_row * BK + swz(frag_row, 2 * s + frag_g) * 8) * 2;
+    const unsigned block_a = wm * MI * 4096, block_w = (BM2 * BK + wn * 64 * BK) * 2;
     unsigned off_wk[2]; // BKN: see gemm_nt_dma_kernel
 #pragma unroll
     for (int ni = 0; ni < 2; ni++) {
@@ -539,18 +530,21 @@ __device__ __forceinline__ void gemm_nt_dma2_body(const GemmArgs &p, int wg_arg 
         half8_t fa[MI], fw[2];
         half4_t wk[2][2]; // BKN: fw[ni] arrives as two 8-byte halves
     };
-    auto read_frags = [&](int kt, int s, Frag &f) {
-        const unsigned sb = unsigned(kt % DMA2_STAGES) * STAGE_BYTES;
+    unsigned sb = 0; // the k-tile's stage
+    auto read_frags = [&](int s, Frag &f) {
+        const unsigned at_a = lane_off[s] + (sb + block_a);
 #pragma unroll
-        for (int i = 0; i < MI; i++) asm volatile("ds_read_b128 %0, %1" : "=v"(f.fa[i]) : "v"(sb + off_a[s][i]));
+        for (int i = 0; i < MI; i++) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(f.fa[i]) : "v"(at_a), "n"(i * 4096));
+        if (!BKN) {
+            const unsigned at_w = lane_off[s] + (sb + block_w);
 #pragma unroll
-        for (int i = 0; i < 2; i++) {
-            if (!BKN) asm volatile("ds_read_b128 %0, %1" : "=v"(f.fw[i]) : "v"(sb + off_w[s][i]));
-            else {
+            for (int i = 0; i < 2; i++) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(f.fw[i]) : "v"(at_w), "n"(i * 4096));
+        } else {
+#pragma unroll
+            for (int i = 0; i < 2; i++)
 #pragma unroll
                 for (int q = 0; q < 2; q++)
-                    asm volatile("ds_read_b64_tr_b16 %0, %1" : "=v"(f.wk[i][q]) : "v"(sb + off_wk[i] + unsigned(16 * s + 4 * q) * (BN * 2)));
-            }
+                    asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(f.wk[i][q]) : "v"(sb + off_wk[i]), "n"((16 * s + 4 * q) * (BN * 2)));
         }
     };
     // (all but the newest group of reads have landed: MI + 2 reads a group, MI + 4 with BKN)
@@ -592,30 +586,31 @@ __device__ __forceinline__ void gemm_nt_dma2_body(const GemmArgs &p, int wg_arg 
 
     Frag fr[2];
     lds_barrier(); // tile 0 is visible
-    read_frags(0, 0, fr[0]);
-    auto first_three = [&](int kt) {
-        read_frags(kt, 1, fr[1]);
+    read_frags(0, fr[0]);
+    auto first_three = [&] {
+        read_frags(1, fr[1]);
         wait_older(fr[0]);
         multiply(fr[0]);
         __builtin_amdgcn_sched_barrier(0);
-        read_frags(kt, 2, fr[0]);
+        read_frags(2, fr[0]);
         wait_older(fr[1]);
         multiply(fr[1]);
         __builtin_amdgcn_sched_barrier(0);
-        read_frags(kt, 3, fr[1]);
+        read_frags(3, fr[1]);
         wait_older(fr[0]);
         multiply(fr[0]);
         __builtin_amdgcn_sched_barrier(0);
     };
-    for (int kt = 0; kt + 1 < n_ktiles; kt++) { // (every k-tile is a full one)
-        first_three(kt);
+    for (int left = n_ktiles - 1; left > 0; left--) { // (every k-tile is a full one)
+        first_three();
         wait_all(fr[1]);
         __builtin_amdgcn_s_barrier();
-        read_frags(kt + 1, 0, fr[0]);
+        sb = sb + STAGE_BYTES == DMA2_STAGES * STAGE_BYTES ? 0 : sb + STAGE_BYTES;
+        read_frags(0, fr[0]);
         multiply(fr[1]);
         __builtin_amdgcn_sched_barrier(0);
     }
-    first_three(n_ktiles - 1);
+    first_three();
     wait_all(fr[1]);
     multiply(fr[1]);
     if constexpr (SHARED_EPILOGUE) {

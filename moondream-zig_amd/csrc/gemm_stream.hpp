@@ -73,8 +73,8 @@ template <class Op, int MI, class Tile, class Next, class KTiles, class Store>
 __device__ __forceinline__ void stream_multiply(int wm, int wn, int lane, Next next, KTiles ktiles, Store store) {
     using S = Stream<MI>;
     const int frag_row = lane & 31, frag_g = lane >> 5;
-    // Where this lane's part of a 32-row block's 16-wide slice s lies: the swizzle repeats every 32 rows, so blocks are 4 KiB apart
-    // whatever the lane and enter as the instruction's offset.
+    // Where this lane's part of a 32-row block's 16-wide slice s lies: blocks are 4 KiB apart whatever the lane and enter as the
+    // read's offset (gemm_dma.hpp).
     unsigned lane_off[BK / 16];
 #pragma unroll
     for (int s = 0; s < BK / 16; s++) lane_off[s] = (frag_row * BK + swz(frag_row, 2 * s + frag_g) * 8) * 2;
