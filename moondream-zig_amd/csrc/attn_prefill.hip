@@ -2,7 +2,7 @@
 // attention.multiMaskedSDPA with the mask of createAttentionMask, attention.zig:256-281, 416-541) and the
 // non-causal 729-token vision attention (16 heads x 72, attention.multiMasklessSDPA, attention.zig:125-234).
 //
-// One 256-thread workgroup owns 32 query rows of one head.  Its four wavefronts split the key range in tiles
+// One 256-thread workgroup owns 32 query rows of one head (64 in flash_attn64_kernel, for large calls).  Its four wavefronts split the key range in tiles
 // of 64 keys (wave w takes tiles w, w+4, ...), each running an online-softmax pass of its own over private LDS
 // staging, so the main loop has no workgroup barrier; the four partial results (m, l, O) are merged through
 // LDS at the end.  Per tile a wave computes, with v_mfma_f32_32x32x16_f16 and f32 accumulation,
@@ -20,6 +20,7 @@ namespace {
 
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
+typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 
 constexpr int FA_Q = 32;     // query rows per workgroup
 constexpr int FA_KT = 64;    // keys per tile
@@ -365,19 +366,349 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
     }
 }
 
+// Sixty-four query rows per workgroup, for calls with enough of them.  The kernel above spends as long on bringing a tile from the L2
+// into LDS and out of it as on the matrix instructions; here a fragment of K or V read from LDS serves both blocks of 32 rows,
+// which halves that, and the copies go to LDS directly, whose rows need no padding (no staging registers, for which 64 rows have
+// no room); the matrix core adds up the probabilities where O^T has a row to spare.  What bounds it now: the exponentials and
+// what goes with them, whose time in the vector unit two wavefronts per SIMD hardly overlap with the matrix core's (32 heads x
+// 4096 x 4096 of 72, counted: 52 % vector, 41 % matrix, no bank conflicts).  16 heads of 72, 1458 rows: 31.7 -> 26.2 us; 32 heads
+// of 64, 768 causal rows: 15.1 -> 13.8 us.  Tried and slower: the exponentials of one block between the matrix instructions of
+// the other, in program order (5 to 8 %).
+template <int D>
+struct FbCfg {
+    static constexpr int QS = 2;                  // blocks of 32 query rows per workgroup
+    static constexpr int Q = 32 * QS;             // query rows per workgroup
+    static constexpr int DK = (D + 15) / 16 * 16; // contraction length of K.Q^T, zero padded
+    static constexpr int KSTEPS = DK / 16;
+    static constexpr int DT = (D + 31) / 32;      // 32-row tiles of O^T, rows >= D are zero
+    // The denominator is the sum of the probabilities as the matrix core takes them, rounded.  Where O^T has rows past D, one of
+    // them collects it: V is 1 there.
+    static constexpr bool SUM_ROW = D % 32 != 0;
+    static constexpr int G = D / 8;               // 16-byte granules per row
+    static constexpr int TILE = FA_KT * D;        // halfs of a K or V tile
+    static constexpr int COPIES = FA_KT * G / 64; // copies of 64 granules that bring a tile
+    static_assert((FA_KT * G) % 64 == 0 && (D == 64 || D == 72), "whole copies, and a bank layout of its own for each row length");
+    // merge of the four wavefronts: O as [wave][q][SD] floats over the tiles (row stride D + 4: the 16-byte accesses of 16
+    // consecutive q fall on distinct banks), the maxima and sums [wave][q] behind them in an area of their own
+    static constexpr int SD = D + 4;
+    static constexpr size_t MERGE_BYTES = size_t(FA_WAVES) * Q * SD * sizeof(float);
+    static constexpr size_t TILE_BYTES = size_t(FA_WAVES) * 2 * TILE * sizeof(half_t);
+    static constexpr size_t ML_OFFSET = TILE_BYTES > MERGE_BYTES ? TILE_BYTES : MERGE_BYTES;
+    static constexpr size_t LDS_BYTES = ML_OFFSET + 2 * FA_WAVES * Q * sizeof(float);
+    static_assert(2 * LDS_BYTES <= 160 * 1024, "two workgroups per compute unit");
+};
+
+// Where a tile's granules lie in LDS.  The copies fill it in order, 64 granules of 16 bytes at a time, so rows are unpadded and
+// the choice is which key a slot holds (D = 72) or which granule of its row (D = 64).  A K read takes one granule of each of
+// 16 consecutive keys, a transposing V read 4 granules of each of 4 consecutive keys; 16 granules are all 64 banks.
+//   D = 72: slot s starts at granule 9 s.  Slots 4 apart start 4 granules apart mod 16, so keys 4 a + b of a group of 16 sit in slot
+//           4 b + a (its own inverse): four consecutive keys fill the banks, and so do 16 with one granule each.
+//   D = 64: slot s is key s and starts at granule 8 s.  Granule c sits at c ^ f(s): of two rows with the same parity that follow
+//           each other f differs in bit 2, and over 16 rows each half of the banks sees all eight values.
+template <int D> __device__ __forceinline__ int fb_slot(int key) { return D == 72 ? (key & ~15) | (key & 3) << 2 | (key >> 2 & 3) : key; }
+template <int D> __device__ __forceinline__ int fb_swizzle(int key) { return D == 72 ? 0 : (key >> 1 & 1) << 2 | (key >> 2 & 3); }
+
+// The tile whose first row lies at `rows` into the LDS at byte lds: left bytes are what the head's rows still hold from there, what
+// lies past them reads as zero.  Written as instructions because the compiler, which cannot tell which of its LDS reads a copy
+// in flight touches, would wait for every copy before each of them; fb_landed says what has arrived.  The LDS reads before it
+// have returned when the first copy starts.
+template <int COPIES>
+__device__ __forceinline__ void fb_copy(const half_t *rows, int left, unsigned lds, const int (&off)[COPIES]) {
+    const unsigned long at = reinterpret_cast<unsigned long>(rows);
+    u32x4 rs = {(unsigned)__builtin_amdgcn_readfirstlane((int)at), (unsigned)__builtin_amdgcn_readfirstlane((int)(at >> 32) & 0xffff),
+                (unsigned)__builtin_amdgcn_readfirstlane(left), 0x00020000u};
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < COPIES; i++)
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" // (5 wait states: scalars that the vector unit wrote)
+                     ::"s"(lds + i * 1024), "v"(off[i]), "s"(rs) : "memory");
+}
+template <int NEWER> __device__ __forceinline__ void fb_landed() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NEWER) : "memory"); }
+
+template <int D>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void flash_attn64_kernel(FaArgs p) {
+    using C = FbCfg<D>;
+    constexpr int QS = C::QS;
+    extern __shared__ __attribute__((aligned(16))) half_t smem[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6); // (wave: a scalar)
+    const int col = lane & 31, hf = lane >> 5;
+    const bool causal = p.causal_pos >= 0;
+    // which head and rows: as in flash_attn_kernel
+    int item = (int)(blockIdx.y * gridDim.x + blockIdx.x);
+    const int n_items = (int)(gridDim.x * gridDim.y);
+    if (n_items % 8 == 0) item = (item % 8) * (n_items / 8) + item / 8;
+    int h = item / (int)gridDim.x, bx = item % (int)gridDim.x;
+    if (causal && n_items % 8 == 0 && (n_items / 8) % (int)gridDim.x == 0) {
+        const int per_die = n_items / 8, heads_per_die = per_die / (int)gridDim.x, j = item % per_die;
+        h = (item / per_die) * heads_per_die + j % heads_per_die;
+        bx = j / heads_per_die;
+    }
+    const int qb = causal ? (int)gridDim.x - 1 - bx : bx;
+    const int q0 = qb * C::Q;
+    const half_t *Ks = smem + wave * 2 * C::TILE, *Vs = Ks + C::TILE;
+    const unsigned k_lds = __builtin_amdgcn_readfirstlane((unsigned)reinterpret_cast<unsigned long>((__attribute__((address_space(3))) const half_t *)Ks));
+    const unsigned v_lds = k_lds + C::TILE * sizeof(half_t);
+    // where this lane points the transposing loads of O^T row tile dt (see fa_read_tr): keys 4 hf + (lane % 16) / 4 of the 8 keys
+    // of a contraction half-step (and, second, 8 keys on), d-columns 32 dt + 16 ((lane / 16) % 2) + 4 (lane % 4) .. + 3.  Rows of
+    // O^T at or past D take no V, so the lanes that would name columns past the row name its last four instead.
+    int voff[2][C::DT];
+#pragma unroll
+    for (int j = 0; j < 2; j++)
+#pragma unroll
+        for (int dt = 0; dt < C::DT; dt++) {
+            const int key = (D == 72 ? 0 : 8 * j) + 4 * hf + ((lane & 15) >> 2), c = min(32 * dt + 16 * ((lane >> 4) & 1) + 4 * (lane & 3), D - 4);
+            voff[j][dt] = fb_slot<D>(key) * D + ((c >> 3 ^ fb_swizzle<D>(key)) << 3 | (c & 7)) + (D == 72 ? j * fb_slot<D>(8) * D : 0);
+        }
+    // this head's rows: (Lkv - 1) row strides and one row of D halfs
+    const int row_bytes = (int)p.kv_row_stride * 2, head_bytes = (p.Lkv - 1) * row_bytes + D * 2;
+    const half_t *kh = p.k + size_t(h) * p.kv_head_stride, *vh = p.v + size_t(h) * p.kv_head_stride;
+    int off[C::COPIES]; // this lane's granules of a tile, from its first row (K and V lie alike)
+#pragma unroll
+    for (int i = 0; i < C::COPIES; i++) {
+        const int x = i * 64 + lane, key = fb_slot<D>(x / C::G); // (the slot of a slot's number is its key)
+        off[i] = key * row_bytes + (x % C::G ^ fb_swizzle<D>(key)) * 16;
+        asm volatile("" : "+v"(off[i])); // (one register each: the compiler would keep the 64-bit products)
+    }
+
+    // keys any row of this block can see
+    long kv_end = p.Lkv;
+    if (causal && p.causal_pos + q0 + C::Q < kv_end) kv_end = p.causal_pos + q0 + C::Q;
+    const int n_tiles = (int)((kv_end + FA_KT - 1) / FA_KT);
+    const size_t tile_stride = size_t(FA_KT) * p.kv_row_stride;
+
+    if (wave < n_tiles) {
+        fb_copy(kh + wave * tile_stride, head_bytes - wave * FA_KT * row_bytes, k_lds, off);
+        fb_copy(vh + wave * tile_stride, head_bytes - wave * FA_KT * row_bytes, v_lds, off);
+    }
+    // this lane's query rows as the MFMA "B" operand: Q[q0 + 32 u + col][16*s + 8*hf .. +7]
+    half8_t qf[QS][C::KSTEPS];
+#pragma unroll
+    for (int u = 0; u < QS; u++) {
+        const int qrow = min(q0 + 32 * u + col, p.Lq - 1);
+        const half_t *qp = p.q + size_t(h) * p.q_head_stride + size_t(qrow) * p.q_row_stride;
+#pragma unroll
+        for (int s = 0; s < C::KSTEPS; s++) {
+            const int d = 16 * s + 8 * hf;
+#pragma unroll
+            for (int e = 0; e < 8; e++) qf[u][s][e] = (half_t)0.0f;
+            if (d < D) qf[u][s] = *reinterpret_cast<const half8_t *>(qp + d);
+        }
+    }
+    // Tell the compiler that the query rows have arrived: it would wait for them at their first use, in every round of the loop,
+    // by counting to zero, and with them for the tile that is on its way.  (One round trip brings all three.)
+    __builtin_amdgcn_s_waitcnt(0xf70); // vmcnt(0), the other counters at their maxima
+
+    float16_t o[QS][C::DT];
+    float m_run[QS], l_run[QS]; // l_run: this lane's half of the row sum (where O^T has no row for it)
+#pragma unroll
+    for (int u = 0; u < QS; u++) {
+        m_run[u] = -INFINITY;
+        l_run[u] = 0.0f;
+#pragma unroll
+        for (int dt = 0; dt < C::DT; dt++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) o[u][dt][v] = 0.0f;
+    }
+    const float c2 = p.scale * 1.4426950408889634f; // > 0: the maximum of the scaled scores is the scaled maximum
+
+    for (int t = wave; t < n_tiles; t += FA_WAVES) {
+        const int key0 = t * FA_KT;
+        const bool more = t + FA_WAVES < n_tiles;
+        const half_t *k_next = kh + (t + FA_WAVES) * tile_stride, *v_next = vh + (t + FA_WAVES) * tile_stride;
+        const int left = head_bytes - (t + FA_WAVES) * FA_KT * row_bytes;
+        fb_landed<C::COPIES>(); // the K tile (the V tile's copies are newer)
+
+        float16_t s[QS][2];
+#pragma unroll
+        for (int kt = 0; kt < 2; kt++) {
+#pragma unroll
+            for (int u = 0; u < QS; u++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) s[u][kt][v] = 0.0f;
+            const half_t *row = Ks + fb_slot<D>(32 * kt + col) * D;
+#pragma unroll
+            for (int st = 0; st < C::KSTEPS; st++) {
+                const bool past = 16 * st + 8 >= D; // the second half of the wavefront has no granule here: zeros
+                const int g = past ? 2 * st : (2 * st + hf) ^ fb_swizzle<D>(col);
+                u32x4 a = *reinterpret_cast<const u32x4 *>(row + g * 8);
+                if (past && hf) a = u32x4{0, 0, 0, 0};
+#pragma unroll
+                for (int u = 0; u < QS; u++) s[u][kt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8_t, a), qf[u][st], s[u][kt], 0, 0, 0);
+            }
+        }
+        if (more) fb_copy(k_next, left, k_lds, off);
+#pragma unroll
+        for (int u = 0; u < QS; u++) {
+            // s[u][kt][v] = score of key key0 + 32*kt + 8*(v/4) + 4*hf + v%4 against query q0 + 32 u + col
+            const bool edge = (key0 + FA_KT > p.Lkv) || (causal && (long)(key0 + FA_KT - 1) > p.causal_pos + q0 + 32 * u);
+            float mx = -INFINITY;
+            // Scores stay unscaled in s; the scale (times log2 e) enters in the one fma that feeds exp2.  m_run is kept in those
+            // units (scaled, base 2).
+            if (edge) { // (a tile that needs no masking takes the other path: no compare, no branch per score)
+                const int first = causal ? (int)min((long)p.Lkv, p.causal_pos + q0 + 32 * u) : p.Lkv; // the last key that row 32 u sees
+                const int seen = min(p.Lkv - 1, first + col) - key0 - 4 * hf;                         // keys past this one of the tile are masked
+#pragma unroll
+                for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+                    for (int v = 0; v < 16; v++) {
+                        const float x = 32 * kt + 8 * (v >> 2) + (v & 3) > seen ? -INFINITY : s[u][kt][v];
+                        s[u][kt][v] = x;
+                        mx = fmaxf(mx, x);
+                    }
+            } else {
+#pragma unroll
+                for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+                    for (int v = 0; v < 16; v++) mx = fmaxf(mx, s[u][kt][v]);
+            }
+            mx = fmaxf(mx, __shfl_xor(mx, 32));
+            // (A reference that may lag behind the maximum, by less than f16 minds, would spare most of the rescaling, but the largest
+            // probability would no longer be exactly 1: error against 64 bits 5 to 11 % larger at 729 and 1458 rows.)
+            const float m_new = fmaxf(m_run[u], mx * c2);
+            if (__any(m_new != m_run[u])) {
+                const float alpha = __builtin_amdgcn_exp2f(m_run[u] - (m_new == -INFINITY ? 0.0f : m_new));
+                m_run[u] = m_new;
+                l_run[u] *= alpha;
+                // (in the last row tile only the registers of rows below D, and of the row of sums, are rescaled)
+#pragma unroll
+                for (int dt = 0; dt < C::DT; dt++)
+#pragma unroll
+                    for (int v = 0; v < 16; v++)
+                        if (32 * dt + 8 * (v >> 2) < D || (32 * dt + 8 * (v >> 2) == D && v % 4 == 0)) o[u][dt][v] *= alpha;
+            }
+            const float m_use = m_run[u] == -INFINITY ? 0.0f : m_run[u]; // a row that has seen no key yet
+#pragma unroll
+            for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) s[u][kt][v] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[u][kt][v], c2, -m_use));
+        }
+
+        if (more) fb_landed<C::COPIES>(); // the V tile
+        else fb_landed<0>();
+        float psum[QS] = {};
+        // O^T += V^T . P^T : contraction step (kt, sp) uses the keys a lane already holds in s[u][kt][8*sp .. 8*sp+7],
+        // i.e. key0 + 32*kt + 16*sp + {4*hf + 0..3, 8 + 4*hf + 0..3}
+#pragma unroll
+        for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+            for (int sp = 0; sp < 2; sp++) {
+                half8_t pb[QS];
+#pragma unroll
+                for (int u = 0; u < QS; u++)
+#pragma unroll
+                    for (int e = 0; e < 8; e += 2) {
+                        const half2_t two = {(half_t)s[u][kt][8 * sp + e], (half_t)s[u][kt][8 * sp + e + 1]}, one = {(half_t)1.0f, (half_t)1.0f};
+                        pb[u][e] = two[0];
+                        pb[u][e + 1] = two[1];
+                        if (!C::SUM_ROW) psum[u] = __builtin_amdgcn_fdot2(two, one, psum[u], false); // (exact products, denormals too)
+                    }
+#pragma unroll
+                for (int dt = 0; dt < C::DT; dt++) {
+                    const half4_t lo = fa_read_tr(Vs + voff[0][dt] + (32 * kt + 16 * sp) * D);
+                    const half4_t hi = fa_read_tr(Vs + voff[1][dt] + (32 * kt + 16 * sp) * D);
+                    half8_t a = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+                    if (C::SUM_ROW && dt == C::DT - 1) {
+                        const unsigned ones = 0x3c003c00u; // two halfs of 1
+                        if (col >= D % 32) a = __builtin_bit_cast(half8_t, u32x4{ones, ones, ones, ones});
+                    }
+#pragma unroll
+                    for (int u = 0; u < QS; u++) o[u][dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, pb[u], o[u][dt], 0, 0, 0);
+                }
+            }
+#pragma unroll
+        for (int u = 0; u < QS; u++) l_run[u] += psum[u];
+        if (more) fb_copy(v_next, left, v_lds, off);
+    }
+
+    // merge the four waves' partial results
+    float *so = reinterpret_cast<float *>(smem);                                                        // [wave][q][SD]
+    float *sm = reinterpret_cast<float *>(reinterpret_cast<char *>(smem) + C::ML_OFFSET);               // [wave][q]
+    float *sl = sm + FA_WAVES * C::Q;                                                                   // [wave][q]
+#pragma unroll
+    for (int u = 0; u < QS; u++) {
+        const float l_wave = C::SUM_ROW ? o[u][C::DT - 1][D % 32 / 2] : l_run[u] + __shfl_xor(l_run[u], 32);
+        if (hf == 0) {
+            sm[wave * C::Q + 32 * u + col] = m_run[u];
+            sl[wave * C::Q + 32 * u + col] = l_wave;
+        }
+    }
+    __syncthreads(); // every wave is done with its staging area, which O takes over, and has published its maximum
+#pragma unroll
+    for (int u = 0; u < QS; u++) {
+        float m_all = -INFINITY;
+#pragma unroll
+        for (int w = 0; w < FA_WAVES; w++) m_all = fmaxf(m_all, sm[w * C::Q + 32 * u + col]);
+        const float f = (m_run[u] == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(m_run[u] - m_all); // (maxima are in base-2 units)
+#pragma unroll
+        for (int dt = 0; dt < C::DT; dt++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int d = 32 * dt + 8 * j + 4 * hf; // o[u][dt][4*j .. 4*j+3] are rows d .. d+3 of O^T
+                if (32 * dt + 8 * j < D) {
+                    float4 r;
+                    r.x = o[u][dt][4 * j] * f;
+                    r.y = o[u][dt][4 * j + 1] * f;
+                    r.z = o[u][dt][4 * j + 2] * f;
+                    r.w = o[u][dt][4 * j + 3] * f;
+                    *reinterpret_cast<float4 *>(so + (wave * C::Q + 32 * u + col) * C::SD + d) = r;
+                }
+            }
+    }
+    __syncthreads();
+    {
+        const int q = tid % C::Q;
+        float m_all = -INFINITY, l_all = 0.0f;
+#pragma unroll
+        for (int w = 0; w < FA_WAVES; w++) m_all = fmaxf(m_all, sm[w * C::Q + q]);
+#pragma unroll
+        for (int w = 0; w < FA_WAVES; w++) {
+            const float mw = sm[w * C::Q + q];
+            if (mw != -INFINITY) l_all += __builtin_amdgcn_exp2f(mw - m_all) * sl[w * C::Q + q];
+        }
+        const float inv = 1.0f / l_all;
+        const int row = q0 + q;
+        if (row < p.Lq) {
+            for (int dg = tid / C::Q; dg < C::G; dg += 256 / C::Q) {
+                float acc[8];
+#pragma unroll
+                for (int e = 0; e < 8; e++) acc[e] = 0.0f;
+#pragma unroll
+                for (int w = 0; w < FA_WAVES; w++) {
+                    const float4 a = *reinterpret_cast<const float4 *>(so + (w * C::Q + q) * C::SD + dg * 8);
+                    const float4 b = *reinterpret_cast<const float4 *>(so + (w * C::Q + q) * C::SD + dg * 8 + 4);
+                    acc[0] += a.x; acc[1] += a.y; acc[2] += a.z; acc[3] += a.w;
+                    acc[4] += b.x; acc[5] += b.y; acc[6] += b.z; acc[7] += b.w;
+                }
+                half8_t r;
+#pragma unroll
+                for (int e = 0; e < 8; e++) r[e] = (half_t)(acc[e] * inv);
+                const size_t oi = p.out_merged ? (size_t(row) * p.H + h) * D + dg * 8 : (size_t(h) * p.Lq + row) * D + dg * 8;
+                *reinterpret_cast<half8_t *>(p.out + oi) = r;
+            }
+        }
+    }
+}
+
 template <int D>
 int launch_flash(moon_ctx *ctx, const FaArgs &p) {
-    using C = FaCfg<D>;
-    static std::atomic<bool> attr_set[64]; // the opt-in to this much dynamic LDS is per device (and per instantiation)
+    // Sixty-four rows where they give every compute unit a workgroup, or three to two units where a row sees only the keys before it:
+    // 16 heads of 72, 1024 rows 14.0 us (32 rows: 14.6), 1458 rows 24.1 (27.4); 32 heads of 64, causal, 768 rows 13.8 (15.1),
+    // 1024 rows 14.6 (16.0).  Below that the chip is better filled with 32: 512 rows of 16 heads 7.2 us (9.0), 450 causal rows of
+    // 32 heads 7.6 (9.4).
+    const size_t blocks64 = (size_t)((p.Lq + 63) / 64) * p.H;
+    const bool two = 2 * blocks64 >= (p.causal_pos >= 0 ? 3 : 2) * (size_t)ctx->cu_count;
+    const auto kernel = two ? flash_attn64_kernel<D> : flash_attn_kernel<D>;
+    const size_t lds = two ? FbCfg<D>::LDS_BYTES : FaCfg<D>::LDS_BYTES;
+    const unsigned blocks = two ? (unsigned)((p.Lq + 63) / 64) : (unsigned)((p.Lq + FA_Q - 1) / FA_Q);
+    static std::atomic<bool> attr_set[2][64]; // the opt-in to this much dynamic LDS is per device (and per kernel)
     const int dev = ctx->device >= 0 && ctx->device < 64 ? ctx->device : -1;
-    if (dev < 0 || !attr_set[dev].load()) {
-        MOON_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void *>(flash_attn_kernel<D>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                          (int)C::LDS_BYTES));
-        if (dev >= 0) attr_set[dev].store(true);
+    if (dev < 0 || !attr_set[two][dev].load()) {
+        MOON_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        if (dev >= 0) attr_set[two][dev].store(true);
     }
-    hipLaunchKernelGGL(flash_attn_kernel<D>, dim3((unsigned)((p.Lq + FA_Q - 1) / FA_Q), (unsigned)p.H), dim3(256), C::LDS_BYTES, ctx->stream, p);
+    hipLaunchKernelGGL(kernel, dim3(blocks, (unsigned)p.H), dim3(256), lds, ctx->stream, p);
     MOON_HIP(ctx, hipGetLastError());
-    MOON_NOTE_KERNEL(ctx, "flash_attn_kernel<%d> %d workgroups", D, (int)((p.Lq + FA_Q - 1) / FA_Q) * (int)p.H);
+    MOON_NOTE_KERNEL(ctx, "flash_attn%s_kernel<%d> %d workgroups", two ? "64" : "", D, (int)blocks * p.H);
     return MOON_OK;
 }
 

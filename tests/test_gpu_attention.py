@@ -162,6 +162,23 @@ def test_matrix_core_attention_over_seeded_random_shapes(moon, O, ctx):
     print(f"\nworst rel-Frobenius over 48 shapes: {worst:.2e}")
 
 
+# 64 rows per workgroup from 256 of them on, causal from 384 (32 heads: from 449 and 705 rows), 32 below; the last block of 64 with 1,
+# 32, 33 and 64 rows
+@pytest.mark.parametrize("S,D,pos", [(448, 72, None), (449, 72, None), (480, 64, None), (481, 72, None), (512, 64, None), (704, 64, 62), (705, 64, 0),
+                                     (736, 64, 1), (737, 64, 62)])
+def test_both_row_blocks_of_the_matrix_core_attention(moon, O, ctx, S, D, pos):
+    """Scores that grow along the keys, from far below one to tens: every tile raises the maximum of its rows."""
+    H, L = 32, S + (pos or 0)
+    q, k, v = _qkv(O, H, S, L, D)
+    k = (k.astype(np.float32) * np.linspace(0.02, 5.0, L, dtype=np.float32)[:, None]).astype(np.float16)
+    if pos is None:
+        out, want = moon.attention.multi_maskless_sdpa(H, D, q, k, v, ctx=ctx), O.sdpa_multi(q, k, v, None)
+    else:
+        mask = moon.attention.create_attention_mask(pos, S)
+        out, want = moon.attention.multi_masked_sdpa(q, k, v, mask, H, D, ctx=ctx), O.sdpa_multi(q, k, v, mask)
+    assert O.rel_frobenius(out, want) <= TOL
+
+
 def test_decode_attention_after_cleanup_starts_from_fresh_counters(moon, O, ctx):
     """moon_cleanup frees the workspace that holds the per-head counters of the one-launch decode attention
     (cleanupThreadPool, attention.zig:814).  The next call gets new memory, whatever it holds, at whatever address, and must
