@@ -1,5 +1,5 @@
-// The wavefront-specialised 128 x 128 x 64 tile product, shared by the f16 kernel of gemm.hip and the segmented kernels of
-// seg_gemm.hip.  A 512-thread workgroup holds four LOADER wavefronts and four
+// The wavefront-specialised 128 x 128 x 64 tile product of the f16 kernel of gemm.hip (the segmented kernels of
+// seg_gemm.hip stream their tiles: gemm_stream.hpp).  A 512-thread workgroup holds four LOADER wavefronts and four
 // MULTIPLIER wavefronts, one of each per SIMD, so the hardware interleaves their instruction streams:
 //   * loaders copy the operand tiles global -> LDS with buffer_load_dwordx4 ... lds (every lane names a 16-byte source,
 //     the 64 destinations are consecutive in LDS; no registers are spent on staging).  DMA_STAGES - 1 k-tiles (96 KiB) are
