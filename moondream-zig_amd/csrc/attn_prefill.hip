@@ -691,12 +691,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
 
 template <int D>
 int launch_flash(moon_ctx *ctx, const FaArgs &p) {
-    // Sixty-four rows where they give every compute unit a workgroup, or three to two units where a row sees only the keys before it:
-    // 16 heads of 72, 1024 rows 14.0 us (32 rows: 14.6), 1458 rows 24.1 (27.4); 32 heads of 64, causal, 768 rows 13.8 (15.1),
-    // 1024 rows 14.6 (16.0).  Below that the chip is better filled with 32: 512 rows of 16 heads 7.2 us (9.0), 450 causal rows of
-    // 32 heads 7.6 (9.4).
-    const size_t blocks64 = (size_t)((p.Lq + 63) / 64) * p.H;
-    const bool two = 2 * blocks64 >= (p.causal_pos >= 0 ? 3 : 2) * (size_t)ctx->cu_count;
+    // Sixty-four rows where all heads together have that many for every compute unit, or half as many again where a row sees only the
+    // keys before it.  Times of a call, 64 rows (32 rows): 16 heads of 72, 1000 rows 12.5 us (13.2), 1200 rows 18.9 (21.2); 32 heads of
+    // 72, 500 rows 8.9 (8.8); 32 heads of 64, causal, 705 rows 10.9 (10.8), 768 rows 11.0 (11.3), 1024 rows 13.6 (15.1), 1458 rows 24.0
+    // (24.8).  Well below the line the chip is better filled with 32: 16 heads of 72, 512 rows 7.2 us against 9.0.
+    const bool two = (size_t)p.Lq * p.H >= (p.causal_pos >= 0 ? 96 : 64) * (size_t)ctx->cu_count;
     const auto kernel = two ? flash_attn64_kernel<D> : flash_attn_kernel<D>;
     const size_t lds = two ? FbCfg<D>::LDS_BYTES : FaCfg<D>::LDS_BYTES;
     const unsigned blocks = two ? (unsigned)((p.Lq + 63) / 64) : (unsigned)((p.Lq + FA_Q - 1) / FA_Q);

@@ -162,10 +162,10 @@ def test_matrix_core_attention_over_seeded_random_shapes(moon, O, ctx):
     print(f"\nworst rel-Frobenius over 48 shapes: {worst:.2e}")
 
 
-# 64 rows per workgroup from 256 of them on, causal from 384 (32 heads: from 449 and 705 rows), 32 below; the last block of 64 with 1,
-# 32, 33 and 64 rows
-@pytest.mark.parametrize("S,D,pos", [(448, 72, None), (449, 72, None), (480, 64, None), (481, 72, None), (512, 64, None), (704, 64, 62), (705, 64, 0),
-                                     (736, 64, 1), (737, 64, 62)])
+# 64 rows per workgroup from 64 rows of all heads together for each of 256 compute units on, causal from 96 (32 heads: from 512 and
+# 768 rows), 32 below; the last block of 64 with 1, 32, 33 and 64 rows
+@pytest.mark.parametrize("S,D,pos", [(511, 72, None), (512, 72, None), (513, 72, None), (544, 64, None), (545, 72, None), (767, 64, 62), (768, 64, 0),
+                                     (769, 64, 62), (800, 64, 1), (801, 64, 62)])
 def test_both_row_blocks_of_the_matrix_core_attention(moon, O, ctx, S, D, pos):
     """Scores that grow along the keys, from far below one to tens: every tile raises the maximum of its rows."""
     H, L = 32, S + (pos or 0)
