@@ -20,7 +20,6 @@ namespace {
 
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
-typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 
 constexpr int FA_Q = 32;     // query rows per workgroup
 constexpr int FA_KT = 64;    // keys per tile
@@ -369,11 +368,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
 // Sixty-four query rows per workgroup, for calls with enough of them.  The kernel above spends as long on bringing a tile from the L2
 // into LDS and out of it as on the matrix instructions; here a fragment of K or V read from LDS serves both blocks of 32 rows,
 // which halves that, and the copies go to LDS directly, whose rows need no padding (no staging registers, for which 64 rows have
-// no room); the matrix core adds up the probabilities where O^T has a row to spare.  What bounds it now: the exponentials and
-// what goes with them, whose time in the vector unit two wavefronts per SIMD hardly overlap with the matrix core's (32 heads x
-// 4096 x 4096 of 72, counted: 52 % vector, 41 % matrix, no bank conflicts).  16 heads of 72, 1458 rows: 31.7 -> 26.2 us; 32 heads
-// of 64, 768 causal rows: 15.1 -> 13.8 us.  Tried and slower: the exponentials of one block between the matrix instructions of
-// the other, in program order (5 to 8 %).
+// no room).  What bounds it now: the exponentials and what goes with them, whose time in the vector unit two wavefronts per SIMD
+// hardly overlap with the matrix core's (32 heads x 4096 x 4096 of 72, counted: vector instructions issued in 63 % of the cycles,
+// matrix core busy in 42 %, no bank conflicts; of 64: 68 and 35 %).  Calls back to back, 32 rows -> 64: 16 heads of 72, 1458 rows
+// 25.6 -> 23.8 us; 32 heads of 64, 1024 causal rows 15.2 -> 13.9, 2000 rows 38.9 -> 33.8.  Tried and slower: the exponentials of one
+// block between the matrix instructions of the other, in program order (5 to 8 %).  The denominator is summed in f32, as above: taken
+// from the matrix core it is a sum of rounded probabilities, 5 % faster for heads of 72, and loses the faint keys of a long call.
 template <int D>
 struct FbCfg {
     static constexpr int QS = 2;                  // blocks of 32 query rows per workgroup
@@ -381,9 +381,6 @@ struct FbCfg {
     static constexpr int DK = (D + 15) / 16 * 16; // contraction length of K.Q^T, zero padded
     static constexpr int KSTEPS = DK / 16;
     static constexpr int DT = (D + 31) / 32;      // 32-row tiles of O^T, rows >= D are zero
-    // The denominator is the sum of the probabilities as the matrix core takes them, rounded.  Where O^T has rows past D, one of
-    // them collects it: V is 1 there.
-    static constexpr bool SUM_ROW = D % 32 != 0;
     static constexpr int G = D / 8;               // 16-byte granules per row
     static constexpr int TILE = FA_KT * D;        // halfs of a K or V tile
     static constexpr int COPIES = FA_KT * G / 64; // copies of 64 granules that bring a tile
@@ -499,7 +496,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
     __builtin_amdgcn_s_waitcnt(0xf70); // vmcnt(0), the other counters at their maxima
 
     float16_t o[QS][C::DT];
-    float m_run[QS], l_run[QS]; // l_run: this lane's half of the row sum (where O^T has no row for it)
+    float m_run[QS], l_run[QS]; // l_run: this lane's half of the row sum
 #pragma unroll
     for (int u = 0; u < QS; u++) {
         m_run[u] = -INFINITY;
@@ -569,23 +566,29 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
                 const float alpha = __builtin_amdgcn_exp2f(m_run[u] - (m_new == -INFINITY ? 0.0f : m_new));
                 m_run[u] = m_new;
                 l_run[u] *= alpha;
-                // (in the last row tile only the registers of rows below D, and of the row of sums, are rescaled)
+                // (in the last row tile only the registers of rows below D are rescaled)
 #pragma unroll
                 for (int dt = 0; dt < C::DT; dt++)
 #pragma unroll
                     for (int v = 0; v < 16; v++)
-                        if (32 * dt + 8 * (v >> 2) < D || (32 * dt + 8 * (v >> 2) == D && v % 4 == 0)) o[u][dt][v] *= alpha;
+                        if (32 * dt + 8 * (v >> 2) < D) o[u][dt][v] *= alpha;
             }
             const float m_use = m_run[u] == -INFINITY ? 0.0f : m_run[u]; // a row that has seen no key yet
+            // (the denominator is the sum of the probabilities before they are rounded for the matrix core)
+            float psum = 0.0f;
 #pragma unroll
             for (int kt = 0; kt < 2; kt++)
 #pragma unroll
-                for (int v = 0; v < 16; v++) s[u][kt][v] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[u][kt][v], c2, -m_use));
+                for (int v = 0; v < 16; v++) {
+                    const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(s[u][kt][v], c2, -m_use));
+                    s[u][kt][v] = e;
+                    psum += e;
+                }
+            l_run[u] += psum;
         }
 
         if (more) fb_landed<C::COPIES>(); // the V tile
         else fb_landed<0>();
-        float psum[QS] = {};
         // O^T += V^T . P^T : contraction step (kt, sp) uses the keys a lane already holds in s[u][kt][8*sp .. 8*sp+7],
         // i.e. key0 + 32*kt + 16*sp + {4*hf + 0..3, 8 + 4*hf + 0..3}
 #pragma unroll
@@ -596,27 +599,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
 #pragma unroll
                 for (int u = 0; u < QS; u++)
 #pragma unroll
-                    for (int e = 0; e < 8; e += 2) {
-                        const half2_t two = {(half_t)s[u][kt][8 * sp + e], (half_t)s[u][kt][8 * sp + e + 1]}, one = {(half_t)1.0f, (half_t)1.0f};
-                        pb[u][e] = two[0];
-                        pb[u][e + 1] = two[1];
-                        if (!C::SUM_ROW) psum[u] = __builtin_amdgcn_fdot2(two, one, psum[u], false); // (exact products, denormals too)
-                    }
+                    for (int e = 0; e < 8; e++) pb[u][e] = (half_t)s[u][kt][8 * sp + e];
 #pragma unroll
                 for (int dt = 0; dt < C::DT; dt++) {
                     const half4_t lo = fa_read_tr(Vs + voff[0][dt] + (32 * kt + 16 * sp) * D);
                     const half4_t hi = fa_read_tr(Vs + voff[1][dt] + (32 * kt + 16 * sp) * D);
-                    half8_t a = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-                    if (C::SUM_ROW && dt == C::DT - 1) {
-                        const unsigned ones = 0x3c003c00u; // two halfs of 1
-                        if (col >= D % 32) a = __builtin_bit_cast(half8_t, u32x4{ones, ones, ones, ones});
-                    }
+                    const half8_t a = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
 #pragma unroll
                     for (int u = 0; u < QS; u++) o[u][dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, pb[u], o[u][dt], 0, 0, 0);
                 }
             }
-#pragma unroll
-        for (int u = 0; u < QS; u++) l_run[u] += psum[u];
         if (more) fb_copy(v_next, left, v_lds, off);
     }
 
@@ -626,7 +618,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
     float *sl = sm + FA_WAVES * C::Q;                                                                   // [wave][q]
 #pragma unroll
     for (int u = 0; u < QS; u++) {
-        const float l_wave = C::SUM_ROW ? o[u][C::DT - 1][D % 32 / 2] : l_run[u] + __shfl_xor(l_run[u], 32);
+        const float l_wave = l_run[u] + __shfl_xor(l_run[u], 32);
         if (hf == 0) {
             sm[wave * C::Q + 32 * u + col] = m_run[u];
             sl[wave * C::Q + 32 * u + col] = l_wave;

@@ -179,6 +179,25 @@ def test_both_row_blocks_of_the_matrix_core_attention(moon, O, ctx, S, D, pos):
     assert O.rel_frobenius(out, want) <= TOL
 
 
+@pytest.mark.parametrize("D", [64, 72])
+@pytest.mark.parametrize("rows", [64, 16384])  # 32 rows per workgroup, 64
+@pytest.mark.parametrize("units", [1.45, 0.49])  # a probability, in steps of f16 below its normal range: rounded, it would count as one of them or none
+def test_matrix_core_attention_sums_probabilities_in_f32(moon, ctx, rows, D, units):
+    """One key whose value is 1 and many faint ones of value 0: the result is the reciprocal of the softmax denominator, 1 + keys x p.
+    Limit: half a step of the f16 result (2^-12 below 1) and 1 % of the faint keys' share for the exponent's f32 rounding."""
+    keys = 1 << 15
+    faint = np.float16(np.log(units * 2.0**-24) * D**0.5)
+    p = np.exp(float(faint) * D**-0.5)
+    assert abs(p * 2**24 / units - 1) < 0.02  # (the score is a step of f16 away at most)
+    q, k, v = [np.zeros((1, n, D), np.float16) for n in (rows, keys, keys)]
+    q[..., 0] = 1.0
+    k[:, 1:, 0] = faint
+    v[:, 0] = 1.0
+    out = moon.attention.multi_maskless_sdpa(1, D, q, k, v, ctx=ctx)
+    want = 1.0 / (1.0 + (keys - 1) * p)
+    assert np.abs(out.astype(np.float64) - want).max() <= 2.0**-12 + 0.01 * (1.0 - want)
+
+
 def test_decode_attention_after_cleanup_starts_from_fresh_counters(moon, O, ctx):
     """moon_cleanup frees the workspace that holds the per-head counters of the one-launch decode attention
     (cleanupThreadPool, attention.zig:814).  The next call gets new memory, whatever it holds, at whatever address, and must
