@@ -418,7 +418,7 @@ __device__ __forceinline__ void fb_copy(const half_t *rows, int left, unsigned l
 #pragma unroll
     for (int i = 0; i < COPIES; i++)
         asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" // (5 wait states: scalars that the vector unit wrote)
-                     ::"s"(lds + i * 1024), "v"(off[i]), "s"(rs) : "memory");
+                     ::"s"(lds + i * 1024), "v"(off[i]), "s"(rs) : "memory", "m0");
 }
 template <int NEWER> __device__ __forceinline__ void fb_landed() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NEWER) : "memory"); }
 
