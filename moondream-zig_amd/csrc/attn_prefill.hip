@@ -409,6 +409,10 @@ template <int D> __device__ __forceinline__ int fb_swizzle(int key) { return D =
 // lies past them reads as zero.  Written as instructions because the compiler, which cannot tell which of its LDS reads a copy
 // in flight touches, would wait for every copy before each of them; fb_landed says what has arrived.  The LDS reads before it
 // have returned when the first copy starts.
+// (M0 is a register that the compiler keeps for itself and sets anew for each of its own uses: naming it makes it do so behind a copy,
+// and clang says that it is not preserved, which is the point)
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 template <int COPIES>
 __device__ __forceinline__ void fb_copy(const half_t *rows, int left, unsigned lds, const int (&off)[COPIES]) {
     const unsigned long at = reinterpret_cast<unsigned long>(rows);
@@ -420,6 +424,7 @@ __device__ __forceinline__ void fb_copy(const half_t *rows, int left, unsigned l
         asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" // (5 wait states: scalars that the vector unit wrote)
                      ::"s"(lds + i * 1024), "v"(off[i]), "s"(rs) : "memory", "m0");
 }
+#pragma clang diagnostic pop
 template <int NEWER> __device__ __forceinline__ void fb_landed() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NEWER) : "memory"); }
 
 template <int D>
