@@ -688,11 +688,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
 
 template <int D>
 int launch_flash(moon_ctx *ctx, const FaArgs &p) {
-    // Sixty-four rows where all heads together have that many for every compute unit, or half as many again where a row sees only the
-    // keys before it.  Times of a call, 64 rows (32 rows): 16 heads of 72, 1000 rows 12.5 us (13.2), 1200 rows 18.9 (21.2); 32 heads of
-    // 72, 500 rows 8.9 (8.8); 32 heads of 64, causal, 705 rows 10.9 (10.8), 768 rows 11.0 (11.3), 1024 rows 13.6 (15.1), 1458 rows 24.0
-    // (24.8).  Well below the line the chip is better filled with 32: 16 heads of 72, 512 rows 7.2 us against 9.0.
-    const bool two = (size_t)p.Lq * p.H >= (p.causal_pos >= 0 ? 96 : 64) * (size_t)ctx->cu_count;
+    // Two workgroups fit a compute unit.  Sixty-four rows from where 32 rows would take a second round (rows of all heads > 64 per unit),
+    // for heads of 64, whose tiles cost less to bring, from the third half round (96), and where a row sees only the keys before it, so
+    // that the light blocks fill up the first round, from 112.  Times of a call, 32 rows -> 64, on 256 units:
+    //   heads of 72           16 x 1024 (64 per unit) 14.1 -> 14.3 us, 16 x 1100 21.6 -> 20.9, 32 x 512 (64) 9.4 -> 9.7, 32 x 550 15.3 -> 14.6
+    //   heads of 64           32 x 600 13.4 -> 13.9, 32 x 768 (96) 14.2 -> 14.3, 32 x 832 19.0 -> 16.1, 16 x 1664 29.8 -> 24.4
+    //   heads of 64, causal   32 x 768 (96) 12.0 -> 11.5, 32 x 800 12.4 -> 12.7, 32 x 832 12.8 -> 13.0, 16 x 1600 17.4 -> 18.3, 8 x 3328 (104) 28.8 -> 29.4;
+    //                         32 x 896 (112) 13.6 -> 13.4, 16 x 1792 (112) 20.0 -> 18.9, 8 x 3584 (112) 31.9 -> 31.5, 32 x 1024 15.4 -> 13.9
+    // Well below the line the chip is better filled with 32: 16 heads of 72, 512 rows 7.6 us against 9.5.
+    const size_t rows = (size_t)p.Lq * p.H, cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
+    const bool two = p.causal_pos >= 0 ? rows >= 112 * cus : rows > (D == 64 ? 96 : 64) * cus;
     const auto kernel = two ? flash_attn64_kernel<D> : flash_attn_kernel<D>;
     const size_t lds = two ? FbCfg<D>::LDS_BYTES : FaCfg<D>::LDS_BYTES;
     const unsigned blocks = two ? (unsigned)((p.Lq + 63) / 64) : (unsigned)((p.Lq + FA_Q - 1) / FA_Q);

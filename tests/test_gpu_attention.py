@@ -3,6 +3,7 @@ import ctypes as C
 
 import numpy as np
 import pytest
+import torch
 
 from conftest import TOL
 
@@ -162,10 +163,11 @@ def test_matrix_core_attention_over_seeded_random_shapes(moon, O, ctx):
     print(f"\nworst rel-Frobenius over 48 shapes: {worst:.2e}")
 
 
-# 64 rows per workgroup from 64 rows of all heads together for each of 256 compute units on, causal from 96 (32 heads: from 512 and
-# 768 rows), 32 below; the last block of 64 with 1, 32, 33 and 64 rows
+# 64 rows per workgroup where all heads together have more than 64 rows for each compute unit (heads of 64: 96; causal: at least 112),
+# 32 below (on 256 units 32 heads cross the line behind 512, 768 and 895 rows); the last block of 64 with 1, 32, 33 and 64 rows
 @pytest.mark.parametrize("S,D,pos", [(511, 72, None), (512, 72, None), (513, 72, None), (544, 64, None), (545, 72, None), (767, 64, 62), (768, 64, 0),
-                                     (769, 64, 62), (800, 64, 1), (801, 64, 62)])
+                                     (769, 64, 62), (800, 64, 1), (801, 64, 62), (544, 72, None), (576, 72, None), (768, 64, None), (769, 64, None), (800, 64, None),
+                                     (832, 64, None), (895, 64, 62), (896, 64, 0), (897, 64, 62), (928, 64, 1), (929, 64, 62), (960, 64, 0)])
 def test_both_row_blocks_of_the_matrix_core_attention(moon, O, ctx, S, D, pos):
     """Scores that grow along the keys, from far below one to tens: every tile raises the maximum of its rows."""
     H, L = 32, S + (pos or 0)
@@ -177,6 +179,48 @@ def test_both_row_blocks_of_the_matrix_core_attention(moon, O, ctx, S, D, pos):
         mask = moon.attention.create_attention_mask(pos, S)
         out, want = moon.attention.multi_masked_sdpa(q, k, v, mask, H, D, ctx=ctx), O.sdpa_multi(q, k, v, mask)
     assert O.rel_frobenius(out, want) <= TOL
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    sixty_four = H * S >= 112 * cus if pos is not None else H * S > (96 if D == 64 else 64) * cus
+    assert ctx.last_kernel().startswith("flash_attn64_kernel" if sixty_four else "flash_attn_kernel")
+
+
+@pytest.mark.parametrize("D,causal", [(64, False), (64, True), (72, False)])
+def test_values_that_are_not_finite_meet_the_same_rows_in_both_row_blocks(moon, O, ctx, D, causal):
+    """Infinities and NaN among queries, keys and values: calls of 64 rows (32 per workgroup) against one of all rows (64)."""
+    H, L = 32, 1030
+    q, k, v = _qkv(O, H, L, L, D)
+    q[:, 17], q[:, 77, 5], k[:, 300, 0] = np.nan, np.inf, np.inf
+    v[:8, 200, 3], v[:8, 700, 5], v[8:16, 1029, 1] = np.inf, np.nan, -np.inf
+
+    def rows(lo, hi):
+        if not causal:
+            return moon.attention.multi_maskless_sdpa(H, D, np.ascontiguousarray(q[:, lo:hi]), k, v, ctx=ctx)
+        cut = [np.ascontiguousarray(a) for a in (q[:, lo:hi], k[:, :hi], v[:, :hi])]
+        return moon.attention.multi_masked_sdpa(*cut, moon.attention.create_attention_mask(lo, hi - lo), H, D, ctx=ctx)
+
+    whole = rows(0, L)
+    assert "flash_attn64" in ctx.last_kernel()
+    parts = []
+    for lo in range(0, L, 64):
+        parts.append(rows(lo, min(lo + 64, L)))
+        assert "flash_attn64" not in ctx.last_kernel()
+    parts = np.concatenate(parts, axis=1)
+    assert np.array_equal(np.isnan(whole), np.isnan(parts)) and np.array_equal(np.isinf(whole), np.isinf(parts))
+    fine = np.isfinite(whole)
+    assert 0.2 < fine.mean() < 0.999
+    assert O.rel_frobenius(whole[fine], parts[fine]) <= TOL
+
+
+@pytest.mark.parametrize("D", [64, 72])
+def test_the_last_tile_reads_nothing_that_an_earlier_call_left(moon, O, ctx, D):
+    """The 64-row kernel's last tile is cut off in memory; what lies behind the keys in LDS has weight 0 and must be a number."""
+    H, L = 32, 1030
+    q, k, v = _qkv(O, H, L, L, D)
+    bad = np.full_like(v, np.nan)
+    moon.attention.multi_maskless_sdpa(H, D, q, bad, bad, ctx=ctx)
+    out = moon.attention.multi_maskless_sdpa(H, D, q, k, v, ctx=ctx)
+    assert "flash_attn64" in ctx.last_kernel()
+    assert O.rel_frobenius(out, O.sdpa_multi(q, k, v, None)) <= TOL
 
 
 @pytest.mark.parametrize("D", [64, 72])
