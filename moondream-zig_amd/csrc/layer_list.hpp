@@ -113,7 +113,7 @@ struct SegGemm {
     int max_tiles;
     int splits;               // splits > 1: n16 = 0, n32 = N, slab s of c32 (M x ld32 apart) gets k-range s
     int kb[SEG_MAX_SPLITS + 1]; // k-range s is [kb[s], kb[s + 1]), multiples of 64; all zero: even ranges
-    int last_first;           // the last k-range's tiles start first, on every die (where the last ranges are the long ones)
+    int longest_first;        // the tiles of the longest k-range start first, on every die (where the ranges differ); otherwise no range may be longer than the first
     int c32_rows;             // splits > 1: rows that c32 has room for, all slabs together
     float softcap;            // > 0: on the f32 segment
 };

@@ -3,43 +3,22 @@
 #include "gemm_stream.hpp"
 #include "layer_list.hpp"
 #include "lm_types.hpp"
+#include "seg_schedule.hpp"
 
 #include <algorithm>
 #include <atomic>
-#include <map>
 
 namespace {
+
+static_assert(SEG_K_TILE == BK && SEG_TILE_COLUMNS == BN && SEG_MAX_SPLITS <= SEG_DIES, "what the schedule's estimate takes for granted");
 
 struct TilePos {
     int m0, m_end, n0, group, split;
 };
-// Tile number `at` of a launch, in the order workgroups 0, 1, .. would take them: neighbours land on different XCDs, so each XCD gets a
-// contiguous run of tiles.  1: a tile, 0: nothing to do, -1: no number from here on has one on this XCD.
-// A run is walked in blocks of 2 x SEG_BAND tiles: the 32 tiles that an XCD works on at once then share 512 to 1,024 rows of either
-// operand, where whole columns of tiles (m first) read all of A again for every few columns: 117 against 123 us at 1920 x 16192 x
-// 2048 in 256-row tiles, 130 against 152 in 128-row tiles, weights from HBM.
-constexpr int SEG_BAND = 8;
-__device__ __forceinline__ int seg_tile(const SegGemm &p, int at, int tile_m, int tile_n, TilePos &t) {
-    const int tiles_n = (p.N + tile_n - 1) / tile_n;
-    const int tiles_m = p.tile_group ? p.max_tiles : (p.M + tile_m - 1) / tile_m;
-    const int tiles = tiles_m * tiles_n, total = tiles * p.splits, per_xcd = (total + 7) / 8;
-    int wg = (at % 8) * per_xcd + at / 8;
-    if (p.last_first) { // each XCD: its run of tiles of the last range, then of the one before, ..
-        const int run = (tiles + 7) / 8, j = at / 8, tile = (at % 8) * run + j % run;
-        if (j >= run * p.splits) return -1;
-        if (tile >= tiles) return 0;
-        wg = (p.splits - 1 - j / run) * tiles + tile;
-    } else if (at / 8 >= per_xcd || wg >= total) return -1;
-    t.split = wg / tiles;
-    const int tile = wg % tiles;
-    int tn = tile / tiles_m, tm = tile % tiles_m;
-    if (!p.tile_group) { // bands of SEG_BAND columns of tiles, walked two rows of tiles at a time
-        const int band = tile / (tiles_m * SEG_BAND), in = tile % (tiles_m * SEG_BAND), wide = min(SEG_BAND, tiles_n - band * SEG_BAND);
-        const int pair = in / (2 * wide), rest = in % (2 * wide), high = min(2, tiles_m - 2 * pair);
-        tm = 2 * pair + rest % high;
-        tn = band * SEG_BAND + rest / high;
-    }
-    t.n0 = tn * tile_n;
+// A die's slot (seg_schedule.hpp) -> its tile; returns what seg_find does, and 0 for a place behind the end of a tile list.
+__device__ __forceinline__ int seg_tile(const SegGemm &p, const SegWalk &w, int die, int slot, int tile_m, int tile_n, TilePos &t) {
+    int tm, tn;
+    if (const int r = seg_find(w, die, slot, tm, tn, t.split); r <= 0) return r;
     if (p.tile_group) { // (scalar loads: a launch does not write its own list, and a vector load would wait for the copies in flight)
         typedef const __attribute__((address_space(4))) int *list_t;
         auto entry = [&](const int *list, int i) { return ((list_t)list)[i]; };
@@ -52,6 +31,7 @@ __device__ __forceinline__ int seg_tile(const SegGemm &p, int at, int tile_m, in
         t.m0 = tm * tile_m;
         t.m_end = min(t.m0 + tile_m, p.M);
     }
+    t.n0 = tn * tile_n;
     return 1;
 }
 
@@ -60,6 +40,7 @@ __device__ __forceinline__ int seg_tile(const SegGemm &p, int at, int tile_m, in
 typedef bf16_t bf16x4_t __attribute__((ext_vector_type(4)));
 template <int MI>
 __device__ __forceinline__ void seg_store(const SegGemm &p, const float16_t (&acc)[2][MI], const TilePos &t, int wm, int wn, int lane, char *scratch) {
+    asm volatile("" : "+v"(lane)); // (per tile: kept over the products, a lane's addresses would not fit the registers, and scratch loads held up each tile by 1 us)
     const int n = t.n0 + wn * 64, col = lane & 31, g = lane >> 5;
     if (n >= p.N) return;
     const int m_wave = t.m0 + wm * 32 * MI, row8 = lane >> 3, g8 = lane & 7;
@@ -132,26 +113,23 @@ __device__ __forceinline__ void seg_store(const SegGemm &p, const float16_t (&ac
 }
 
 template <int MI>
-__global__ __launch_bounds__(DMA_THREADS) void seg_gemm_bf16_kernel(SegGemm p) {
+__global__ __launch_bounds__(DMA_THREADS) void seg_gemm_bf16_kernel(SegGemm p, SegWalk w) {
     extern __shared__ __attribute__((aligned(16))) half_t lds_stream[]; // (the tile product addresses LDS from 0: nothing static beside it)
     using S = Stream<MI>;
     const int lane = threadIdx.x & 63, role_wave = __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) & 3);
-    int at = blockIdx.x;
+    int round = 0;
     auto next = [&](TilePos &t) { // (both roles walk the same tiles)
-        for (;; at += gridDim.x) {
-            const int r = seg_tile(p, at, S::ROWS, BN, t);
-            if (r < 0) return false;
-            if (r > 0) break;
+        for (;;) {
+            const int r = seg_tile(p, w, blockIdx.x % SEG_DIES, seg_slot(w.longest_first, blockIdx.x / SEG_DIES, gridDim.x / SEG_DIES, round++), S::ROWS, BN, t);
+            if (r != 0) return r > 0;
         }
-        at += gridDim.x;
-        return true;
     };
     if (threadIdx.x >= 256) {
         stream_load<MI, TilePos>(lds_stream, role_wave, next, [&](const TilePos &t, StreamSource<MI> &s) {
             // (the launcher has checked that both operands fit a descriptor)
-            const bf16_t *w = reinterpret_cast<const bf16_t *>(p.W) + size_t(t.group) * p.w_group;
+            const bf16_t *weights = reinterpret_cast<const bf16_t *>(p.W) + size_t(t.group) * p.w_group;
             s.a = __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p.A), 0, p.a_rows * p.lda * 2, 0x00020000);
-            s.w = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t *>(w), 0, p.N * p.K * 2, 0x00020000);
+            s.w = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t *>(weights), 0, p.N * p.K * 2, 0x00020000);
 #pragma unroll
             for (int j = 0; j < 2 * MI; j++) {
                 const int r = stream_row_a(MI, role_wave, j, lane), m = min(t.m0 + r, t.m_end - 1);
@@ -176,10 +154,10 @@ __global__ __launch_bounds__(DMA_THREADS) void seg_gemm_bf16_kernel(SegGemm p) {
 // f32: 64 x 64 tile, a thread owns rows ty, ty + 16, .. and columns tx, tx + 16, tx + 32, tx + 48 (so a gate column and its up
 // column are in one thread).  Tile lists are 128 rows high: two passes over m.
 constexpr int F32_K = 16;
-__global__ __launch_bounds__(256) void seg_gemm_f32_kernel(SegGemm p) {
+__global__ __launch_bounds__(256) void seg_gemm_f32_kernel(SegGemm p, SegWalk w) {
     __shared__ float sa[F32_K][64 + 4], sw[F32_K][64 + 4];
     TilePos t;
-    if (seg_tile(p, blockIdx.x, SEG_TILE_ROWS, 64, t) <= 0) return;
+    if (seg_tile(p, w, blockIdx.x % SEG_DIES, blockIdx.x / SEG_DIES, SEG_TILE_ROWS, 64, t) <= 0) return;
     const int k_begin = p.kb[t.split], k_end = p.kb[t.split + 1];
     const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4, lr = tid >> 2, lk = (tid & 3) * 4;
     const float *A = reinterpret_cast<const float *>(p.A), *W = reinterpret_cast<const float *>(p.W) + size_t(t.group) * p.w_group;
@@ -188,10 +166,10 @@ __global__ __launch_bounds__(256) void seg_gemm_f32_kernel(SegGemm p) {
         const int m_src = min(mb + lr, t.m_end - 1);
         const float *arow = A + size_t(p.rows ? (int)p.rows[m_src] : m_src) * p.lda, *wrow = W + size_t(t.n0 + lr) * p.K;
         for (int k = k_begin; k < k_end; k += F32_K) {
-            const float4 a = *reinterpret_cast<const float4 *>(arow + k + lk), w = *reinterpret_cast<const float4 *>(wrow + k + lk);
+            const float4 a = *reinterpret_cast<const float4 *>(arow + k + lk), b = *reinterpret_cast<const float4 *>(wrow + k + lk);
             __syncthreads();
             sa[lk][lr] = a.x; sa[lk + 1][lr] = a.y; sa[lk + 2][lr] = a.z; sa[lk + 3][lr] = a.w;
-            sw[lk][lr] = w.x; sw[lk + 1][lr] = w.y; sw[lk + 2][lr] = w.z; sw[lk + 3][lr] = w.w;
+            sw[lk][lr] = b.x; sw[lk + 1][lr] = b.y; sw[lk + 2][lr] = b.z; sw[lk + 3][lr] = b.w;
             __syncthreads();
 #pragma unroll
             for (int kk = 0; kk < F32_K; kk++)
@@ -218,41 +196,13 @@ __global__ __launch_bounds__(256) void seg_gemm_f32_kernel(SegGemm p) {
 
 } // namespace
 
-// What a k-tile and the rest of a tile take with every compute unit busy and weights from HBM, us, by tile height.  The higher tiles
-// move fewer bytes per product, and a product's tiles seldom fill the last round, so the height is chosen by the rounds: 1920 rows x
-// 16192 x 2048 take 126 us in 256-row tiles (4 rounds), 132 in 192, 140 in 128 (a workgroup per 128-row tile: 171); 1920 x 2048 x
-// 7552 takes 77 us in 128-row tiles, 57 in 256-row tiles of two k ranges, whose second slab costs 3 us in row_finish.
-struct SegTime {
-    double k_tile, rest;
-};
-static SegTime seg_time(int mi) {
-    static const SegTime by_height[3] = {{0.58, 1.5}, {0.78, 2.0}, {0.95, 2.5}};
-    return by_height[mi - 2];
-}
-// us of tiles of that height: the workgroups take the ranges' tiles one after the other, the first free one the next.
-static double seg_estimate(int cus, int mi, int M, int N, const int *kb, int splits, bool last_first) {
-    const int tiles = (M + 64 * mi - 1) / (64 * mi) * ((N + BN - 1) / BN);
-    std::map<double, int> free{{0.0, cus}}; // workgroups by when they are done
-    for (int s = 0; s < splits; s++) {
-        const int r = last_first ? splits - 1 - s : s;
-        const double w = (kb[r + 1] - kb[r]) / BK * seg_time(mi).k_tile + seg_time(mi).rest;
-        for (int left = tiles; left > 0;) {
-            const auto first = free.begin();
-            const int n = std::min(left, first->second);
-            free[first->first + w] += n;
-            left -= n;
-            if ((first->second -= n) == 0) free.erase(first);
-        }
-    }
-    return free.rbegin()->first;
-}
 // the tile height (in 64 rows) for a product whose ranges are set
 static int seg_choose(moon_ctx *ctx, const SegGemm &p) {
     const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
     int best = 2;
     double t = 1e30;
     for (int mi = 2; mi <= 4; mi++)
-        if (const double e = seg_estimate(cus, mi, p.M, p.N, p.kb, p.splits, p.last_first); e < t) {
+        if (const double e = seg_estimate(cus, mi, p.M, p.N, p.kb, p.splits, p.longest_first); e < t) {
             t = e;
             best = mi;
         }
@@ -306,10 +256,9 @@ int launch_seg_gemm(moon_ctx *ctx, int dtype, SegGemm p) {
                 MOON_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
                 if (dev >= 0) attr_set[dev].store(true);
             }
-            const int cus = std::max(8, (ctx->cu_count > 0 ? ctx->cu_count : 256) / 8 * 8);
-            const size_t per_range = size_t(p.tile_group ? p.max_tiles : (p.M + rows - 1) / rows) * ((p.N + BN - 1) / BN);
-            const size_t places = p.last_first ? (per_range + 7) / 8 * 8 * p.splits : (per_range * p.splits + 7) / 8 * 8;
-            hipLaunchKernelGGL(kern, dim3((unsigned)std::min<size_t>(places, cus)), dim3(DMA_THREADS), lds, ctx->stream, p);
+            const int cus = std::max(SEG_DIES, (ctx->cu_count > 0 ? ctx->cu_count : 256) / SEG_DIES * SEG_DIES);
+            const SegWalk w = seg_walk(p.tile_group ? p.max_tiles : (p.M + rows - 1) / rows, (p.N + BN - 1) / BN, p.tile_group, p.kb, p.splits, p.longest_first);
+            hipLaunchKernelGGL(kern, dim3((unsigned)seg_workgroups(w, cus)), dim3(DMA_THREADS), lds, ctx->stream, p, w);
             return MOON_OK;
         };
         static std::atomic<bool> set2[64], set3[64], set4[64];
@@ -317,9 +266,8 @@ int launch_seg_gemm(moon_ctx *ctx, int dtype, SegGemm p) {
         else if (mi == 3) MOON_TRY(go(seg_gemm_bf16_kernel<3>, Stream<3>::LDS_BYTES, set3));
         else MOON_TRY(go(seg_gemm_bf16_kernel<2>, Stream<2>::LDS_BYTES, set2));
     } else {
-        const size_t tiles = size_t(p.tile_group ? p.max_tiles : (p.M + SEG_TILE_ROWS - 1) / SEG_TILE_ROWS) * (p.N / 64);
-        const dim3 grid((unsigned)(p.last_first ? (tiles + 7) / 8 * 8 * p.splits : (tiles * p.splits + 7) / 8 * 8));
-        hipLaunchKernelGGL(seg_gemm_f32_kernel, grid, dim3(256), 0, ctx->stream, p);
+        const SegWalk w = seg_walk(p.tile_group ? p.max_tiles : (p.M + SEG_TILE_ROWS - 1) / SEG_TILE_ROWS, p.N / 64, p.tile_group, p.kb, p.splits, p.longest_first);
+        hipLaunchKernelGGL(seg_gemm_f32_kernel, dim3((unsigned)(SEG_DIES * w.slots)), dim3(256), 0, ctx->stream, p, w);
     }
     MOON_HIP(ctx, hipGetLastError());
     MOON_NOTE_KERNEL(ctx, "%s %d rows a tile, k split %d", dtype == MOON_DTYPE_BF16 ? "seg_gemm_bf16_kernel" : "seg_gemm_f32_kernel", rows, p.splits);

@@ -1,0 +1,130 @@
+// Which tiles of a segmented product (seg_gemm.hip) a workgroup takes, and how long that takes: kept free of device-only calls so that
+// a host program can walk the same schedule (tests/cxx/seg_schedule_check.cpp).
+//
+// Neighbouring workgroups land on different dies, so each die gets a contiguous run of the product's tiles, numbered as its slots, and
+// its workgroups take the slots in rounds.  Where ranges of k differ in length the longest comes first and every other round goes
+// backwards: whoever took the first, longest tile of a round takes the last of the next, and two rounds end as early as if the first
+// free workgroup took the next slot (second product of a joined layer, 768 rows x 2048 x (2048 + 2048 + 3712): 54.5 us in rounds that
+// all go the same way, 42 so).  Tiles of one length are better taken the same way every round (1920 rows x 16192 x 2048 and 64 experts'
+// tiles: 1 and 3 % of a prompt).
+#pragma once
+
+#include <cstdint>
+
+#if defined(__HIPCC__)
+#define SEG_FN __host__ __device__ __forceinline__
+#else
+#define SEG_FN inline
+#endif
+
+namespace {
+
+constexpr int SEG_DIES = 8;
+
+// A die's run is walked in blocks of 2 x SEG_BAND tiles: the 32 tiles that a die works on at once then share 512 to 1,024 rows of either
+// operand, where whole columns of tiles (m first) read all of A again for every few columns: 117 against 123 us at 1920 x 16192 x
+// 2048 in 256-row tiles, 130 against 152 in 128-row tiles, weights from HBM.  A list
+// of row tiles (grouped rows), each with weights of its own, is walked m first.
+constexpr int SEG_BAND = 8;
+
+struct SegWalk {
+    int tiles_m, tiles_n, columns; // columns: m first
+    int tiles, all;    // of one range of k, of all of them
+    int slots;         // of a die, at most
+    int per_die;       // longest_first: tiles of one range, otherwise of all of them
+    int longest_first; // 1: every die takes its tiles of the longest range, then of the next, ..
+    int by_run;   // longest_first: per_die, otherwise tiles
+    int by_block; // columns: tiles_m, otherwise the tiles of a band
+    int by_last;  // two rows of tiles of the last band
+    int order[8];      // the ranges, longest first
+};
+inline void seg_order(const int *kb, int splits, int (&order)[8]) { // (of ranges of one length the last first)
+    for (int s = 0; s < splits; s++) {
+        int at = s;
+        for (; at > 0 && kb[order[at - 1] + 1] - kb[order[at - 1]] <= kb[s + 1] - kb[s]; at--) order[at] = order[at - 1];
+        order[at] = s;
+    }
+}
+inline SegWalk seg_walk(int tiles_m, int tiles_n, bool list, const int *kb, int splits, int longest_first) {
+    SegWalk w{};
+    w.tiles_m = tiles_m;
+    w.tiles_n = tiles_n;
+    w.columns = list;
+    w.tiles = tiles_m * tiles_n;
+    w.all = w.tiles * splits;
+    w.longest_first = longest_first;
+    w.per_die = ((longest_first ? w.tiles : w.all) + SEG_DIES - 1) / SEG_DIES;
+    w.slots = longest_first ? w.per_die * splits : w.per_die;
+    w.by_run = longest_first ? w.per_die : w.tiles;
+    w.by_block = tiles_m * (w.columns ? 1 : SEG_BAND);
+    w.by_last = 2 * (tiles_n - (tiles_n - 1) / SEG_BAND * SEG_BAND);
+    seg_order(kb, splits, w.order);
+    return w;
+}
+// workgroups that have something to do, when there are `most` (a multiple of SEG_DIES)
+inline int seg_workgroups(const SegWalk &w, int most) { return SEG_DIES * w.slots < most ? SEG_DIES * w.slots : most; }
+// the slot that workgroup i of a die's n takes in round r
+SEG_FN int seg_slot(int longest_first, int i, int n, int r) { return r * n + (longest_first & r & 1 ? n - 1 - i : i); }
+
+// A die's slot -> its tile's row and column of tiles and its range.  1: a tile, 0: nothing to do, -1: no slot from here on has one on
+// this die.
+SEG_FN int seg_find(const SegWalk &w, int die, int slot, int &tm, int &tn, int &range) {
+    if (slot >= w.slots) return -1;
+    int tile;
+    if (w.longest_first) {
+        const int before = slot / w.by_run;
+        tile = die * w.per_die + slot - before * w.per_die;
+        if (tile >= w.tiles) return 0;
+        range = w.order[before];
+    } else {
+        const int at = die * w.per_die + slot;
+        if (at >= w.all) return -1;
+        range = at / w.by_run;
+        tile = at - range * w.tiles;
+    }
+    const int block = tile / w.by_block;
+    if (w.columns) {
+        tn = block;
+        tm = tile - block * w.tiles_m;
+        return 1;
+    }
+    const int in = tile - block * w.tiles_m * SEG_BAND, wide = w.tiles_n - block * SEG_BAND < SEG_BAND ? w.tiles_n - block * SEG_BAND : SEG_BAND;
+    const int pair = wide == SEG_BAND ? in / (2 * SEG_BAND) : in / w.by_last, rest = in - pair * 2 * wide;
+    const int two = w.tiles_m - 2 * pair >= 2; // rows of tiles in this pair, less one
+    tm = 2 * pair + (rest & two);
+    tn = block * SEG_BAND + (rest >> two);
+    return 1;
+}
+
+// What a k-tile (64) and the rest of a tile take with every compute unit busy and weights from HBM, us, by tile height in 64 rows.  The
+// higher tiles move fewer bytes per product, and a product's tiles seldom fill the last round, so the height is chosen by the
+// rounds: 1920 rows x 16192 x 2048 take 126 us in 256-row tiles (4 rounds), 132 in 192, 140 in 128 (a workgroup per 128-row tile:
+// 171); 1920 x 2048 x 7552 takes 77 us in 128-row tiles, 57 in 256-row tiles of two k ranges, whose second slab costs 3 us in row_finish.
+constexpr int SEG_K_TILE = 64, SEG_TILE_COLUMNS = 128;
+struct SegTime {
+    double k_tile, rest;
+};
+inline SegTime seg_time(int mi) {
+    constexpr SegTime by_height[3] = {{0.58, 1.5}, {0.78, 2.0}, {0.95, 2.5}};
+    return by_height[mi - 2];
+}
+// us until the last workgroup is done with tiles of that height, range s being [kb[s], kb[s + 1])
+inline double seg_estimate(int cus, int mi, int M, int N, const int *kb, int splits, bool longest_first) {
+    const int tiles = (M + 64 * mi - 1) / (64 * mi) * ((N + SEG_TILE_COLUMNS - 1) / SEG_TILE_COLUMNS);
+    const int per_die = ((longest_first ? tiles : tiles * splits) + SEG_DIES - 1) / SEG_DIES, slots = longest_first ? per_die * splits : per_die;
+    const int n = cus / SEG_DIES < 1 ? 1 : cus / SEG_DIES;
+    auto cost = [&](int s) { return (kb[s + 1] - kb[s]) / SEG_K_TILE * seg_time(mi).k_tile + seg_time(mi).rest; };
+    // the first die has the longest walk; of even ranges (at most eight) it takes tiles of the first alone, the longest
+    if (!longest_first) return (slots + n - 1) / n * cost(0);
+    double longest = 0;
+    int order[8];
+    seg_order(kb, splits, order);
+    for (int i = 0; i < n && i < slots; i++) {
+        double t = 0;
+        for (int r = 0, slot; (slot = seg_slot(1, i, n, r)) < slots; r++) t += cost(order[slot / per_die]);
+        if (t > longest) longest = t;
+    }
+    return longest;
+}
+
+} // namespace
