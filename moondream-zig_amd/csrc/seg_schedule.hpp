@@ -21,6 +21,23 @@ namespace {
 
 constexpr int SEG_DIES = 8;
 
+// n / d by a multiplication, for all 32-bit n (Granlund and Montgomery, "Division by invariant integers using multiplication", 1994,
+// figure 4.1).  The scalar unit has no division: the half dozen that find a tile held up every workgroup's first copy and last
+// store (products of 2 rows and width 1024, one tile per workgroup: 12.1 and 8.0 us with them, 11.2 and 7.4 without).
+struct FastDiv {
+    uint32_t mul;
+    int first, second; // shifts
+};
+inline FastDiv fast_div(uint32_t d) {
+    int l = 0;
+    while (l < 32 && (uint64_t(1) << l) < d) l++;
+    return {(uint32_t)((((uint64_t(1) << l) - d) << 32) / d + 1), l < 1 ? l : 1, l < 1 ? 0 : l - 1};
+}
+SEG_FN uint32_t seg_div(uint32_t n, const FastDiv &f) {
+    const uint32_t t = (uint32_t)((uint64_t(n) * f.mul) >> 32);
+    return (t + ((n - t) >> f.first)) >> f.second;
+}
+
 // A die's run is walked in blocks of 2 x SEG_BAND tiles: the 32 tiles that a die works on at once then share 512 to 1,024 rows of either
 // operand, where whole columns of tiles (m first) read all of A again for every few columns: 117 against 123 us at 1920 x 16192 x
 // 2048 in 256-row tiles, 130 against 152 in 128-row tiles, weights from HBM.  A list
@@ -33,9 +50,9 @@ struct SegWalk {
     int slots;         // of a die, at most
     int per_die;       // longest_first: tiles of one range, otherwise of all of them
     int longest_first; // 1: every die takes its tiles of the longest range, then of the next, ..
-    int by_run;   // longest_first: per_die, otherwise tiles
-    int by_block; // columns: tiles_m, otherwise the tiles of a band
-    int by_last;  // two rows of tiles of the last band
+    FastDiv by_run;    // longest_first: per_die, otherwise tiles
+    FastDiv by_block;  // columns: tiles_m, otherwise the tiles of a band
+    FastDiv by_last;   // two rows of tiles of the last band
     int order[8];      // the ranges, longest first
 };
 inline void seg_order(const int *kb, int splits, int (&order)[8]) { // (of ranges of one length the last first)
@@ -55,9 +72,9 @@ inline SegWalk seg_walk(int tiles_m, int tiles_n, bool list, const int *kb, int 
     w.longest_first = longest_first;
     w.per_die = ((longest_first ? w.tiles : w.all) + SEG_DIES - 1) / SEG_DIES;
     w.slots = longest_first ? w.per_die * splits : w.per_die;
-    w.by_run = longest_first ? w.per_die : w.tiles;
-    w.by_block = tiles_m * (w.columns ? 1 : SEG_BAND);
-    w.by_last = 2 * (tiles_n - (tiles_n - 1) / SEG_BAND * SEG_BAND);
+    w.by_run = fast_div((uint32_t)(longest_first ? w.per_die : w.tiles));
+    w.by_block = fast_div((uint32_t)tiles_m * (w.columns ? 1 : SEG_BAND));
+    w.by_last = fast_div(2u * (uint32_t)(tiles_n - (tiles_n - 1) / SEG_BAND * SEG_BAND));
     seg_order(kb, splits, w.order);
     return w;
 }
@@ -72,24 +89,24 @@ SEG_FN int seg_find(const SegWalk &w, int die, int slot, int &tm, int &tn, int &
     if (slot >= w.slots) return -1;
     int tile;
     if (w.longest_first) {
-        const int before = slot / w.by_run;
+        const int before = (int)seg_div((uint32_t)slot, w.by_run);
         tile = die * w.per_die + slot - before * w.per_die;
         if (tile >= w.tiles) return 0;
         range = w.order[before];
     } else {
         const int at = die * w.per_die + slot;
         if (at >= w.all) return -1;
-        range = at / w.by_run;
+        range = (int)seg_div((uint32_t)at, w.by_run);
         tile = at - range * w.tiles;
     }
-    const int block = tile / w.by_block;
+    const int block = (int)seg_div((uint32_t)tile, w.by_block);
     if (w.columns) {
         tn = block;
         tm = tile - block * w.tiles_m;
         return 1;
     }
     const int in = tile - block * w.tiles_m * SEG_BAND, wide = w.tiles_n - block * SEG_BAND < SEG_BAND ? w.tiles_n - block * SEG_BAND : SEG_BAND;
-    const int pair = wide == SEG_BAND ? in / (2 * SEG_BAND) : in / w.by_last, rest = in - pair * 2 * wide;
+    const int pair = wide == SEG_BAND ? in / (2 * SEG_BAND) : (int)seg_div((uint32_t)in, w.by_last), rest = in - pair * 2 * wide;
     const int two = w.tiles_m - 2 * pair >= 2; // rows of tiles in this pair, less one
     tm = 2 * pair + (rest & two);
     tn = block * SEG_BAND + (rest >> two);

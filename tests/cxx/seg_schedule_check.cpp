@@ -1,4 +1,5 @@
-// Host check of the schedule of the segmented products (moondream-zig_amd/csrc/seg_schedule.hpp): every tile of every range taken exactly once whatever the shape and the number of workgroups, the estimate against the
+// Host check of the schedule of the segmented products (moondream-zig_amd/csrc/seg_schedule.hpp): division by multiplication against
+// the division, every tile of every range taken exactly once whatever the shape and the number of workgroups, the estimate against the
 // sums along every workgroup's walk, and the walk against a first-free-takes-the-next one where the ranges of k differ in length.
 #include "seg_schedule.hpp"
 
@@ -52,6 +53,14 @@ static double first_free(int workgroups, int tiles, int mi, const int *kb, int s
 int main() {
     std::mt19937_64 rng(1);
     auto in = [&](uint64_t lo, uint64_t hi) { return lo + rng() % (hi - lo + 1); };
+
+    for (int i = 0; i < 2000000; i++) {
+        const uint32_t d = (uint32_t)(i < 1000 ? i + 1 : i % 3 ? in(1, uint64_t(1) << in(1, 31)) : 0xffffffffu - in(0, 1000)); // (the compiler's own '/' is the truth)
+        const uint32_t n = i % 5 == 0 ? 0xffffffffu - (uint32_t)in(0, 3) : i % 5 == 1 ? (uint32_t)(d * in(0, 0xffffffffu / d)) : (uint32_t)(rng() >> in(32, 62));
+        const FastDiv f = fast_div(d);
+        expect(seg_div(n, f) == n / d, "division", (int)n, (int)d, 0, 0);
+        if (n) expect(seg_div(n - 1, f) == (n - 1) / d, "division", (int)(n - 1), (int)d, 0, 0);
+    }
 
     for (int i = 0; i < 4000; i++) {
         const int mi = (int)in(2, 4), M = (int)in(1, i % 2 ? 300 : 2100), N = 64 * (int)in(1, i % 3 ? 40 : 300), splits = (int)in(1, 8), longest_first = (int)in(0, 1);
