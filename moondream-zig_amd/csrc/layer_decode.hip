@@ -778,12 +778,13 @@ __device__ __forceinline__ void mix_experts(const DecodeMix &p, int wg, int n_wg
     }
 }
 
+typedef float OutSums[4][3][4]; // [wavefront][part][row]
 // Rows [row0, row0 + RW) of W2 against columns [c0, c1) of a (16-byte pieces), and of the chosen experts' down matrices against their
 // activations.  A workgroup owns the rows; its four wavefronts share each row's pieces, so a lane reads its part of the vectors once
 // for all rows.  PARTS = 3: the sums over three stretches of the columns are kept apart.  done(k, r, sum) is called by one thread per
 // sum.
 template <class T, int RW, int U, int PARTS, class Done>
-__device__ __forceinline__ void out_rows(const DecodeOut &p, int row0, int c0, int c1, float (&s_part)[4][3][4], Done done) {
+__device__ __forceinline__ void out_rows(const DecodeOut &p, int row0, int c0, int c1, OutSums &s_part, Done done) {
     constexpr int PE = Piece<T>::N;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int pa = c1 - c0, pf = p.top ? p.ffp / PE : 1, total = pa + p.top * pf;
@@ -851,7 +852,7 @@ __device__ __forceinline__ void out_rows(const DecodeOut &p, int row0, int c0, i
 // x += W2 . a, but for what decode_mix has left in p.down already.
 template <class T, int RW, int U, int PARTS>
 __global__ __launch_bounds__(256) void decode_out_kernel(DecodeOut p) {
-    __shared__ float s_part[4][3][4];
+    __shared__ OutSums s_part;
     const int row = blockIdx.x * RW + threadIdx.x % RW;
     float down = 0.0f;
     if (PARTS == 1 && p.down && threadIdx.x < RW && row < p.width) down = p.down[row]; // (requested before the weights)
@@ -863,8 +864,7 @@ __global__ __launch_bounds__(256) void decode_out_kernel(DecodeOut p) {
 
 template <class T, int NH, int U, bool WHOLE, bool LONG>
 __global__ __launch_bounds__(256) void decode_mix_kernel(DecodeMix p, DecodeOut o, int S, int keys_max, int n_attn, int n_expert) {
-    extern __shared__ __attribute__((aligned(16))) char s_mix[];
-    __shared__ float s_part[4][3][4];
+    extern __shared__ __attribute__((aligned(16))) char s_mix[]; // (all there is: heads may fill a compute unit's)
     // attention first: it is a chain of dependent steps, the experts' part and the dense activation's product are long streams
     const int i = blockIdx.x, n_hb = mix_head_blocks(p.H / p.G), n_delta = WHOLE ? p.dH : 0;
     if (i < n_attn) mix_attention<T, NH, WHOLE, LONG>(p, i / S / n_hb, i / S % n_hb, i % S, S, keys_max, reinterpret_cast<float *>(s_mix));
@@ -874,14 +874,15 @@ __global__ __launch_bounds__(256) void decode_mix_kernel(DecodeMix p, DecodeOut 
         else mix_delta<T, false>(p, h, reinterpret_cast<float *>(s_mix));
     } else if (i < n_attn + n_delta + n_expert) mix_experts<T, U>(p, i - n_attn - n_delta, n_expert, s_mix);
     else
-        out_rows<T, MIX_DOWN_ROWS, 4, 1>(o, (i - n_attn - n_delta - n_expert) * MIX_DOWN_ROWS, o.k2 / Piece<T>::N, o.k0 / Piece<T>::N, s_part,
+        out_rows<T, MIX_DOWN_ROWS, 4, 1>(o, (i - n_attn - n_delta - n_expert) * MIX_DOWN_ROWS, o.k2 / Piece<T>::N, o.k0 / Piece<T>::N,
+                                         *reinterpret_cast<OutSums *>(s_mix),
                                          [&](int, int n, float s) { o.down[n] = s; });
 }
 
 template <class T, int NH, bool WHOLE> int mix_launch_as(moon_ctx *ctx, const DecodeMix &p, const DecodeOut &o, int S, int keys_max, int n_attn, int n_expert, size_t lds) {
     const bool longer = std::max(p.dimp, p.vdimp) > 64 * Piece<T>::N;
     auto kern = longer ? decode_mix_kernel<T, NH, 4, WHOLE, true> : p.dp / Piece<T>::N > 64 ? decode_mix_kernel<T, NH, 4, WHOLE, false> : decode_mix_kernel<T, NH, 1, WHOLE, false>;
-    if (lds > 60 * 1024) MOON_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    if (lds > 64 * 1024) MOON_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     const int n_down = o.down ? (o.width + MIX_DOWN_ROWS - 1) / MIX_DOWN_ROWS : 0;
     hipLaunchKernelGGL(kern, dim3(n_attn + n_expert + (WHOLE ? p.dH : 0) + n_down), dim3(256), lds, ctx->stream, p, o, S, keys_max, n_attn, n_expert);
     MOON_HIP(ctx, hipGetLastError());
@@ -963,6 +964,7 @@ int launch_decode_mix(moon_ctx *ctx, int dtype, const DecodeMix &p, const Decode
     const size_t lds = std::max(std::max(mix_lds_floats(NH, p.dimp, p.vdimp, keys_max) * sizeof(float),
                                          p.E ? size_t(p.dp) * el + (size_t(2) * p.E + 2 * p.top) * sizeof(float) : 0),
                                 p.dH ? delta_lds_floats(p.ddimp, p.dvdimp, p.kd) * sizeof(float) : 0);
+    static_assert(sizeof(OutSums) <= (8 + 8 + 8 + 1 + 4 * 8 + 4 + 8) * sizeof(float), "the smallest heads leave room for the down product's sums");
     if (size_t(NH) * S > mix_lds_floats(NH, p.dimp, p.vdimp, keys_max) - 4 * NH - 8) return moon_fail(ctx, MOON_ESEQ_TOO_LONG, "decode attention: %d splits", S);
     if (lds > 160 * 1024) return moon_fail(ctx, MOON_EINVAL_DIM, "decode attention: heads of %d and %d", p.dimp, p.vdimp);
     auto go = [&](auto tag) -> int {

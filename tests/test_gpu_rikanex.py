@@ -410,3 +410,11 @@ def test_head_sizes_around_a_wavefront_of_pieces(moon, ctx, tmp_path, dim, vdim,
     cfg = config(90, 64, [layer(attention(3, 1, dim, vdim, 9, dim**-0.5), dense(72)), layer(attention(2, 2, dim, vdim, 30, dim**-0.5, True), dense(8))])
     w, ids = weights(cfg, 3), tokens(40, 90)
     assert_close(run(moon, ctx, tmp_path, cfg, w, ids, dtype, [3] + [1] * 37), R.forward(cfg, w, ids)[0], dtype)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_heads_that_fill_a_compute_units_memory(moon, ctx, tmp_path, dtype):
+    """One token: eight query heads of 776 and 1,024 on one key head need 160 KiB of LDS at 18 keys, all that a workgroup can have."""
+    cfg = config(90, 64, [layer(attention(8, 1, 776, 1024, 18, 0.03), dense(72))])
+    w, ids = weights(cfg, 4), tokens(30, 90)
+    assert_close(run(moon, ctx, tmp_path, cfg, w, ids, dtype, [1]), R.forward(cfg, w, ids)[0], dtype)
