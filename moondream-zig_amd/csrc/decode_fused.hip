@@ -9,6 +9,7 @@
 #include "attn_decode.hpp"
 #include "norm.hpp"
 #include "sample_quick.hpp"
+#include "wait_places.hpp"
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
@@ -1059,7 +1060,8 @@ static const LayerKernels *layer_kernels(size_t d, size_t ffn) {
 int decode_layer_grid(moon_ctx *ctx, size_t d) { return (pieces(d) == 4 ? LN_GEMV_GROUPS_PER_CU : 2) * (ctx->cu_count > 0 ? ctx->cu_count : 256); }
 
 // Can a whole layer run as one launch of decode_layer_kernel on this device?
-bool decode_layer_supported(moon_ctx *ctx, size_t d, size_t ffn, size_t H, size_t D) {
+// wait: its workgroups that wait, and the places there are for them, per die (wait_places.hpp).
+bool decode_layer_supported(moon_ctx *ctx, size_t d, size_t ffn, size_t H, size_t D, WaitNeed *wait) {
     const LayerKernels *set = layer_kernels(d, ffn);
     if (D != 64 || !set || H * D != d || d % 512 || ffn % 512) return false; // (whole 1 KiB pieces)
     const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256, grid = decode_layer_grid(ctx, d);
@@ -1073,6 +1075,7 @@ bool decode_layer_supported(moon_ctx *ctx, size_t d, size_t ffn, size_t H, size_
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k, 256, (d + ffn) * sizeof(half_t)) != hipSuccess) return false;
         per_cu = per_cu == 0 ? n : std::min(per_cu, n);
     }
+    *wait = {(waiting + 7) / 8, per_cu * cus / 8};
     return per_cu * cus > waiting; // producers always find a slot
 }
 size_t decode_layer_sync_words(size_t H) { return (size_t)layer_sync_words(H); }
@@ -1148,7 +1151,7 @@ int launch_decode_layer(moon_ctx *ctx, const half_t *x, const uint32_t *token, c
 
 // Can the layer's front kernel (LayerNorm + qkv + fc1 + attention) run on this device?  It needs head_dim 64 and room
 // for well more workgroups than there are attention tasks (the only ones that wait).
-bool decode_front_supported(moon_ctx *ctx, size_t d, size_t H, size_t D) {
+bool decode_front_supported(moon_ctx *ctx, size_t d, size_t H, size_t D, WaitNeed *wait) {
     if (D != 64 || pieces(d) != 4 || H * D != d) return false;
     const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
     const int grid = LN_GEMV_GROUPS_PER_CU * cus;
@@ -1157,6 +1160,7 @@ bool decode_front_supported(moon_ctx *ctx, size_t d, size_t H, size_t D) {
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void *>(decode_front_kernel<4, 10>), 256, d * sizeof(half_t)) !=
         hipSuccess)
         return false;
+    *wait = {(int)(H * DEC_SPLITS + 7) / 8, per_cu * cus / 8};
     return per_cu * cus >= 2 * (int)(H * DEC_SPLITS);
 }
 

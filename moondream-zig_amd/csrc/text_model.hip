@@ -11,10 +11,12 @@
 
 #include "layer_list.hpp"
 #include "model_folder.hpp"
+#include "wait_places.hpp"
 
 #include <cstdlib>
 #include <cstring>
 #include <algorithm>
+#include <optional>
 #include <vector>
 
 // fused decode kernels (decode_fused.hip)
@@ -34,8 +36,8 @@ int launch_decode_lm_head(moon_ctx *ctx, const half_t *x, const half_t *gamma, c
                           uint32_t *out_ids, uint32_t bump, const moon_sampling_config *top_k_cfg = nullptr, const float *u_dev = nullptr,
                           uint32_t *decided = nullptr);
 bool decode_lm_head_top_k_supported(moon_ctx *ctx, size_t top_k, size_t V);
-bool decode_front_supported(moon_ctx *ctx, size_t d, size_t H, size_t D);
-bool decode_layer_supported(moon_ctx *ctx, size_t d, size_t ffn, size_t H, size_t D);
+bool decode_front_supported(moon_ctx *ctx, size_t d, size_t H, size_t D, WaitNeed *wait);
+bool decode_layer_supported(moon_ctx *ctx, size_t d, size_t ffn, size_t H, size_t D, WaitNeed *wait);
 size_t decode_layer_sync_words(size_t H);
 int decode_layer_grid(moon_ctx *ctx, size_t d); // workgroups of a launch
 int launch_decode_layer(moon_ctx *ctx, const half_t *x, const uint32_t *token, const half_t *gamma, const half_t *beta, float eps, size_t d,
@@ -83,6 +85,8 @@ struct moon_text_model {
     size_t cur_len = 0, last_n = 0;
     bool cache_invalid = false;    // a fused decode kernel gave up on a wait: positions may be missing from the cache until moon_text_reset
     int decode_mode = 0;           // 0: one kernel per layer where the device holds it (default); 2: three kernels per layer; 3: two
+    int call_mode = 0;             // the same for the call that runs (DecodeCall)
+    WaitNeed layer_wait, front_wait; // places that a call's whole-layer or front launches take
     float *attn_partial = nullptr; // [H][8][66]
     // fused per-layer decode kernels
     bool fused = false;              // shape supported by decode_fused.hip
@@ -216,11 +220,11 @@ int alloc_all(moon_text_model *m) {
     MOON_TRY(dalloc_t(m, z.L * z.H, &m->head_count));
     MOON_TRY(launch_fill_uniform_u32(m->ctx, m->head_count, z.L * z.H, 0, 0, 1)); // zeros
     m->attn_launches.assign(z.L, 0);
-    m->front = m->fused && decode_front_supported(m->ctx, z.d, z.H, z.D);
+    m->front = m->fused && decode_front_supported(m->ctx, z.d, z.H, z.D, &m->front_wait);
     MOON_TRY(dalloc_t(m, z.L * z.H * 32 + 1, &m->front_sync));
     MOON_TRY(launch_fill_uniform_u32(m->ctx, m->front_sync, z.L * z.H * 32 + 1, 0, 0, 1)); // zeros
     m->front_launches.assign(z.L, 0);
-    m->whole_layer = m->fused && decode_layer_supported(m->ctx, z.d, z.ffn, z.H, z.D);
+    m->whole_layer = m->fused && decode_layer_supported(m->ctx, z.d, z.ffn, z.H, z.D, &m->layer_wait);
     m->layer_sync_words = decode_layer_sync_words(z.H);
     MOON_TRY(dalloc_t(m, z.L * m->layer_sync_words + 1, &m->layer_sync));
     MOON_TRY(launch_fill_uniform_u32(m->ctx, m->layer_sync, z.L * m->layer_sync_words + 1, 0, 0, 1)); // zeros
@@ -291,6 +295,35 @@ struct ProfScope {
     }
 };
 
+// A call that decodes tokens one by one: the mode it runs in.  Where workgroups would wait inside launches, it holds their places on the
+// device until the stream has drained; where other contexts' calls have them, it runs in mode 2, which waits for nothing (the
+// same bits).
+struct DecodeCall {
+    moon_text_model *m;
+    const WaitNeed *need = nullptr;
+    bool drained = false;
+    static WaitPlaces &places(int device) {
+        static WaitPlaces of[64];
+        return of[device & 63];
+    }
+    explicit DecodeCall(moon_text_model *model) : m(model) {
+        m->call_mode = m->decode_mode;
+        if (!m->fused) return;
+        if (m->whole_layer && m->call_mode == 0) need = &m->layer_wait;
+        else if (m->front && m->call_mode != 2) need = &m->front_wait;
+        if (need && !places(m->ctx->device).take(*need)) {
+            need = nullptr;
+            m->call_mode = 2;
+        }
+    }
+    ~DecodeCall() {
+        if (!need) return;
+        if (!drained) (void)hipStreamSynchronize(m->ctx->stream); // (an error on the way: launches may still be queued)
+        places(m->ctx->device).give(*need);
+    }
+    DecodeCall(const DecodeCall &) = delete;
+};
+
 // one decoder layer on n rows of m->hidden appended at position pos (text_model.zig:150-172)
 // token_dev: (decode only) the layer input is row token_dev[0] of the embedding table instead of m->hidden
 // chain_ln (rows of a prompt only): the LayerNorm of this layer's input is already in m->ln_in unless this is the first layer,
@@ -312,7 +345,7 @@ int layer_forward(moon_text_model *m, size_t layer, size_t n, size_t pos, bool p
     if (n == 1 && m->fused) {
         // three kernels: LN + qkv + fc1;  rope + append + attention (+ merge);  out_proj + fc2 + both residual adds
         const half_t *x = token_dev ? m->wte : m->hidden;
-        const int mode = m->decode_mode;
+        const int mode = m->call_mode;
         if (m->whole_layer && mode == 0) {
             // one kernel for the layer
             const uint32_t head_target = ++m->attn_launches[layer] * 8u;
@@ -619,6 +652,8 @@ extern "C" size_t moon_text_position(const moon_text_model *m) { return m ? m->c
 // n rows already in m->hidden: the layers, the bookkeeping and, for a single row, the fused kernels' error words
 static int forward_rows_locked(moon_text_model *m, size_t n_ids) {
     moon_ctx *ctx = m->ctx;
+    std::optional<DecodeCall> call;
+    if (n_ids == 1) call.emplace(m);
     for (size_t l = 0; l < m->cfg.n_layers; l++) MOON_TRY(layer_forward(m, l, n_ids, m->cur_len, false, nullptr, n_ids > 1));
     m->cur_len += n_ids;
     m->last_n = n_ids;
@@ -634,6 +669,7 @@ static int forward_rows_locked(moon_text_model *m, size_t n_ids) {
                                      ctx->stream));
     }
     MOON_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    if (call) call->drained = true;
     if (wait_error[0] || wait_error[1]) { // as in the generation loop: the token's cache row may be missing
         m->cur_len -= n_ids;
         m->cache_invalid = true;
@@ -851,7 +887,8 @@ static int greedy_locked(moon_text_model *m, size_t n_steps, uint32_t *out_ids, 
     hipLaunchKernelGGL(start_loop_kernel, dim3(1), dim3(1), 0, ctx->stream, state, (uint32_t)m->cur_len, eos_plus1);
     MOON_HIP(ctx, hipGetLastError());
     if (n_out) *n_out = 0;
-    const int mode = m->decode_mode;
+    DecodeCall call(m);
+    const int mode = m->call_mode;
     const bool use_layer = m->whole_layer && mode == 0;
     if (use_layer) { // counters count up for the life of the model: clear them long before 32 bits are used up (192 per launch)
         const Sizes z = sizes(m->cfg);
@@ -944,6 +981,7 @@ static int greedy_locked(moon_text_model *m, size_t n_steps, uint32_t *out_ids, 
     if (use_front)
         MOON_HIP(ctx, hipMemcpyAsync(m->host_words + 24, m->front_sync + m->cfg.n_layers * m->cfg.n_heads * 32, sizeof(uint32_t), hipMemcpyDeviceToHost, ctx->stream));
     MOON_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    call.drained = true;
     if (ids_staged) memcpy(out_ids, m->stage_down, n_steps * sizeof(uint32_t));
     const uint32_t front_error = words[24];
     const uint32_t final_state[4] = {words[20], words[21], words[22], words[23]};

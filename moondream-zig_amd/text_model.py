@@ -92,7 +92,8 @@ class TextModel:
         self.ctx.check(self.ctx.lib.moon_text_reset(self.handle))
 
     def set_decode_mode(self, mode: int):
-        """0 (default): one fused kernel per layer; 2: three kernels per layer (no waits inside kernels); 3: two per layer."""
+        """0 (default): one fused kernel per layer; 2: three kernels per layer (no waits inside kernels); 3: two per layer.
+        Calls of several contexts at once run as 2 where the device cannot hold all that wait; several processes: ask for 2."""
         self.ctx.check(self.ctx.lib.moon_text_set_decode_mode(self.handle, mode))
 
     @property

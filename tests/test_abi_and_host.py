@@ -109,3 +109,8 @@ def test_schedule_of_the_segmented_products():
     """csrc/seg_schedule.hpp on the host: every tile taken once, the estimate that picks the tile height is that of the walk the kernel
     makes, and ranges of different length end together."""
     _host_check("seg_schedule")
+
+
+def test_places_of_waiting_workgroups():
+    """csrc/wait_places.hpp on the host: the decode calls that may be in flight on a device at once, from several contexts and threads."""
+    _host_check("wait_places")

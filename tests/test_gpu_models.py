@@ -237,6 +237,46 @@ def test_decode_modes_agree_full_size(moon, O, ctx):
     dev.close()
 
 
+def test_sessions_of_several_contexts_decode_at_once(moon, O):
+    """A context per thread, three decoders of width 1024 and one of 2048: their whole-layer launches would have more workgroups waiting
+    than the chip holds, so some calls run in launches that wait for nothing.  The same tokens and logits as alone."""
+    import threading
+    shapes = [(1024, 4096, 16)] * 3 + [(2048, 8192, 32)]
+    ctxs = [moon.Context(0) for _ in shapes]
+    devs = [moon.text_model.TextModel(moon.text_model.make_config(vocab=3000, dim=d, hidden_dim=f, n_layers=4, n_heads=h), seed=i, std=0.02, ctx=c)
+            for i, ((d, f, h), c) in enumerate(zip(shapes, ctxs))]
+    prompts = [O.fill_uniform_u32(40 + 9 * i, i, 50, 3000) for i in range(len(devs))]
+
+    def reply(i):
+        devs[i].reset()
+        devs[i].forward(prompts[i])
+        tokens = devs[i].greedy(48).tolist()
+        devs[i].forward(prompts[i][:1])
+        return tokens, devs[i].logits().view(np.uint16).tolist()
+
+    alone, together, errors = [reply(i) for i in range(len(devs))], {}, []
+    start = threading.Barrier(len(devs))
+
+    def work(i):
+        try:
+            start.wait()
+            together[i] = [reply(i) for _ in range(8)]
+        except Exception as e:
+            errors.append((i, e))
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(len(devs))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors
+    for i, want in enumerate(alone):
+        assert all(got == want for got in together[i])
+    for d, c in zip(devs, ctxs):
+        d.close()
+        c.close()
+
+
 @pytest.mark.parametrize("cached", [1, 2, 224, 225, 897, 1121, 1345, 1793, 2040])
 def test_decode_modes_agree_on_the_narrow_layer(moon, O, ctx, cached):
     """Width 1024 runs a layer in one launch too: same bits as its three launches, at the edges of every prefetch depth."""
