@@ -1,3 +1,4 @@
+import glob
 import importlib
 import os
 import sys
@@ -35,3 +36,15 @@ def ctx(moon):
 
 # parity bar: relative Frobenius error against the oracle's f32-accumulated, f16-rounded result
 TOL = 1e-3
+
+
+def compute_units():
+    """Of the machine's GPUs, as the kernel driver lists them."""
+    units = set()
+    for path in glob.glob("/sys/class/kfd/kfd/topology/nodes/*/properties"):
+        with open(path) as f:
+            node = dict(line.split() for line in f)
+        if int(node["simd_count"]):
+            units.add(int(node["simd_count"]) // int(node["simd_per_cu"]))
+    assert len(units) == 1, units
+    return units.pop()

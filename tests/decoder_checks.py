@@ -1,5 +1,6 @@
 """What the tests of the decoders opened from a model folder share: running them and comparing rows of logits."""
 import numpy as np
+from conftest import compute_units
 from rikanex_models import write_folder
 
 
@@ -36,3 +37,17 @@ def run(moon, ctx, tmp_path, cfg, w, ids, dtype, portions=None, max_seq=512):
     got = feed(m, ids, portions or [len(ids)])
     m.close()
     return got
+
+
+def streams_of_both_types(moon, ctx, cfg, ids, note=None):
+    """The residual stream behind one prompt, bf16 and f32, random weights; note: what the bf16 session's last product must have been, as
+    dispatched on 256 compute units (the last product's note is its tile height and its ranges of k)."""
+    out = []
+    for dtype in ("bfloat16", "float32"):
+        m = moon.text_model.TextModel.open_synthetic(cfg, dtype, 2048, seed=5, std=0.02, ctx=ctx)
+        m.forward(ids)
+        if note and dtype == "bfloat16" and compute_units() == 256:
+            assert ctx.last_kernel() == note
+        out.append(m.hidden_f32(len(ids)))
+        m.close()
+    return out

@@ -3,9 +3,8 @@ import ctypes as C
 
 import numpy as np
 import pytest
-import torch
 
-from conftest import TOL
+from conftest import TOL, compute_units
 
 pytestmark = pytest.mark.gpu
 
@@ -179,7 +178,7 @@ def test_both_row_blocks_of_the_matrix_core_attention(moon, O, ctx, S, D, pos):
         mask = moon.attention.create_attention_mask(pos, S)
         out, want = moon.attention.multi_masked_sdpa(q, k, v, mask, H, D, ctx=ctx), O.sdpa_multi(q, k, v, mask)
     assert O.rel_frobenius(out, want) <= TOL
-    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    cus = compute_units()
     sixty_four = H * S >= 112 * cus if pos is not None else H * S > (96 if D == 64 else 64) * cus
     assert ctx.last_kernel().startswith("flash_attn64_kernel" if sixty_four else "flash_attn_kernel")
 

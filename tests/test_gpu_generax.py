@@ -8,7 +8,7 @@ import sys
 import generax_oracle as G
 import numpy as np
 import pytest
-from decoder_checks import feed, opened, row_errors, rows_close, run
+from decoder_checks import feed, opened, row_errors, rows_close, run, streams_of_both_types
 from generax_models import MODELS, ODD, attention, beacon_weights, config, delta, parallel, plain, rotation, softmax_mixer, weights
 from rikanex_models import tokens, write_folder
 
@@ -484,3 +484,13 @@ def test_trace_program(moon, ctx, folders, tmp_path):
     for i, rows in ((0, [0, 29]), (2, [32]), (3, [1])):
         got = np.fromfile(tmp_path / f"{i}.f32", "<f4").reshape(len(rows), cfg["vocab"])
         assert_close(got, want[rows], "float32")
+
+
+@pytest.mark.parametrize("rows,ff,height", [(768, 3712, 128), (1301, 3712, 192), (1600, 3712, 256), (1530, 1024, 256)])
+def test_tile_heights_of_a_joined_layer(moon, ctx, rows, ff, height):
+    """The second product of a joined layer has ranges of k of two lengths, the feed-forward's the longer or the shorter one; each die's
+    workgroups take them longest first, most of them two or three."""
+    part = softmax_mixer(32, 8, 64, 64, 512, 0.125, 16)
+    cfg = config(128, 2048, [parallel(part, delta(32, 32, 64, 64, 4), ff)], softcap=30.0)
+    got, want = streams_of_both_types(moon, ctx, cfg, tokens(rows, 128), f"seg_gemm_bf16_kernel {height} rows a tile, k split 3")
+    assert_close(got, want, "bfloat16")

@@ -6,7 +6,7 @@ import sys
 import numpy as np
 import pytest
 import rikanex_oracle as R
-from decoder_checks import feed, opened, row_errors, rows_close, run
+from decoder_checks import feed, opened, row_errors, rows_close, run, streams_of_both_types
 from rikanex_models import (MODELS, ODD, TALL, WIDE, attention, config, dense, beacon_weights, layer, moe, tokens, weights, write_folder)
 
 pytestmark = pytest.mark.gpu
@@ -390,8 +390,9 @@ def test_trace_program(moon, ctx, folders, tmp_path):
 @pytest.mark.parametrize("rows", [130, 256, 257, 385, 640, 1025, 1301, 1537, 2000])
 @pytest.mark.parametrize("ff", [64, 3264])
 def test_tile_heights_of_the_products(moon, ctx, tmp_path, rows, ff):
-    """Prompts of a few hundred rows and more take tiles of 128, 192 or 256 rows and split k in other ways; the f32 session's plain
-    product takes none of these.  One layer of width 1024, all rows of the residual stream; limit: bf16 as everywhere in this file."""
+    """Prompts of a few hundred rows and more take tiles of 128, 192 or 256 rows in the first product (16-bit and gated columns) and split k
+    of the second in other ways; the f32 session's plain product takes none of these.  One layer of width 1024, all rows of the
+    residual stream; limit: bf16 as everywhere in this file."""
     cfg = config(130, 1024, [layer(attention(8, 2, 64, 64, 100, 0.125), dense(ff))], embed_scale=2.0)
     path, ids = write_folder(tmp_path / "m", cfg, weights(cfg)), tokens(rows, 130)
     streams = {}
@@ -401,6 +402,23 @@ def test_tile_heights_of_the_products(moon, ctx, tmp_path, rows, ff):
         streams[dtype] = m.hidden_f32(rows)
         m.close()
     assert_close(streams["bfloat16"], streams["float32"], "bfloat16")
+
+
+@pytest.mark.parametrize("rows,ff,height,splits", [(385, 3264, 128, 4), (768, 3264, 192, 4), (768, 5504, 192, 4), (1025, 3264, 256, 3), (1301, 3264, 192, 2), (1537, 5504, 256, 2),
+                                                   (1920, 5504, 256, 2), (2000, 3264, 128, 1)])
+def test_tile_heights_of_the_second_product(moon, ctx, rows, ff, height, splits):
+    """The same at width 2048, where the f32 result too takes every height, in one and in several ranges of k."""
+    cfg = config(128, 2048, [layer(attention(32, 8, 64, 64, 100, 0.125), dense(ff))], embed_scale=2.0)
+    got, want = streams_of_both_types(moon, ctx, cfg, tokens(rows, 128), f"seg_gemm_bf16_kernel {height} rows a tile, k split {splits}")
+    assert_close(got, want, "bfloat16")
+
+
+@pytest.mark.parametrize("rows", [300, 1025])
+def test_more_grouped_tiles_than_compute_units(moon, ctx, rows):
+    """Routed experts: up to 82 and 128 row tiles by 11 columns, a workgroup walks several of them, some of them places without a tile."""
+    cfg = config(128, 512, [layer(attention(8, 2, 64, 64, 100, 0.125), moe(64, 8, 704))], embed_scale=512.0)
+    got, want = streams_of_both_types(moon, ctx, cfg, tokens(rows, 128))
+    assert_close(got, want, "bfloat16")
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
