@@ -374,6 +374,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
 // 25.6 -> 23.8 us; 32 heads of 64, 1024 causal rows 15.2 -> 13.9, 2000 rows 38.9 -> 33.8.  Tried and slower: the exponentials of one
 // block between the matrix instructions of the other, in program order (5 to 8 %).  The denominator is summed in f32, as above: taken
 // from the matrix core it is a sum of rounded probabilities, 5 % faster for heads of 72, and loses the faint keys of a long call.
+// Each row goes through the same operations in the same order as above: the same bits (tested).
 template <int D>
 struct FbCfg {
     static constexpr int QS = 2;                  // blocks of 32 query rows per workgroup
@@ -567,10 +568,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
             // (A reference that may lag behind the maximum, by less than f16 minds, would spare most of the rescaling, but the largest
             // probability would no longer be exactly 1: error against 64 bits 5 to 11 % larger at 729 and 1458 rows.)
             const float m_new = fmaxf(m_run[u], mx * c2);
+            float alpha = 1.0f;
             if (__any(m_new != m_run[u])) {
-                const float alpha = __builtin_amdgcn_exp2f(m_run[u] - (m_new == -INFINITY ? 0.0f : m_new));
+                alpha = __builtin_amdgcn_exp2f(m_run[u] - (m_new == -INFINITY ? 0.0f : m_new));
                 m_run[u] = m_new;
-                l_run[u] *= alpha;
                 // (in the last row tile only the registers of rows below D are rescaled)
 #pragma unroll
                 for (int dt = 0; dt < C::DT; dt++)
@@ -589,7 +590,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
                     s[u][kt][v] = e;
                     psum += e;
                 }
-            l_run[u] += psum;
+            l_run[u] = l_run[u] * alpha + psum;
         }
 
         if (more) fb_landed<C::COPIES>(); // the V tile

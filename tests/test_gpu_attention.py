@@ -185,11 +185,11 @@ def test_both_row_blocks_of_the_matrix_core_attention(moon, O, ctx, S, D, pos):
 
 @pytest.mark.parametrize("D,causal", [(64, False), (64, True), (72, False)])
 def test_values_that_are_not_finite_meet_the_same_rows_in_both_row_blocks(moon, O, ctx, D, causal):
-    """Infinities and NaN among queries, keys and values: calls of 64 rows (32 per workgroup) against one of all rows (64)."""
-    H, L = 32, 1030
+    """Infinities and NaN among queries, keys and values: calls of 64 rows (32 per workgroup) against one of all rows (64), bit for bit."""
+    H, L = 32, 1041  # (the last part has 17 rows, enough for the matrix-core kernels)
     q, k, v = _qkv(O, H, L, L, D)
     q[:, 17], q[:, 77, 5], k[:, 300, 0] = np.nan, np.inf, np.inf
-    v[:8, 200, 3], v[:8, 700, 5], v[8:16, 1029, 1] = np.inf, np.nan, -np.inf
+    v[:8, 200, 3], v[:8, 700, 5], v[8:16, 1040, 1] = np.inf, np.nan, -np.inf
 
     def rows(lo, hi):
         if not causal:
@@ -202,12 +202,10 @@ def test_values_that_are_not_finite_meet_the_same_rows_in_both_row_blocks(moon, 
     parts = []
     for lo in range(0, L, 64):
         parts.append(rows(lo, min(lo + 64, L)))
-        assert "flash_attn64" not in ctx.last_kernel()
+        assert ctx.last_kernel().startswith("flash_attn_kernel")
     parts = np.concatenate(parts, axis=1)
-    assert np.array_equal(np.isnan(whole), np.isnan(parts)) and np.array_equal(np.isinf(whole), np.isinf(parts))
-    fine = np.isfinite(whole)
-    assert 0.2 < fine.mean() < 0.999
-    assert O.rel_frobenius(whole[fine], parts[fine]) <= TOL
+    assert 0.2 < np.isfinite(whole).mean() < 0.999
+    assert np.array_equal(whole, parts, equal_nan=True)
 
 
 @pytest.mark.parametrize("D", [64, 72])
