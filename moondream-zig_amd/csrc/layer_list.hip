@@ -734,7 +734,7 @@ int layer_list_forward(LayerList *l, const uint32_t *ids_dev, size_t n_rows, siz
         o.ld32 = dp;
         f.out_l = d.out_l;
         f.out_r = d.out_r;
-        o.splits = d.out_l ? joined_splits(ctx, d, n, dp, &o, &f.splits_l, &f.splits_r) : seg_gemm_splits(ctx, n, dp, d.k0, l->partial_rows);
+        o.splits = d.out_l ? joined_splits(ctx, d, n, dp, &o, &f.splits_l, &f.splits_r) : seg_gemm_splits(ctx, dt, n, dp, d.k0, l->partial_rows);
         MOON_TRY(launch_seg_gemm(ctx, dt, o));
         f.partial = l->partial;
         f.splits = o.splits;

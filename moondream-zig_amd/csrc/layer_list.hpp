@@ -120,7 +120,7 @@ struct SegGemm {
 constexpr int SEG_TILE_ROWS = 128; // rows of a tile (both element types walk tile lists of this height)
 int launch_seg_gemm(moon_ctx *ctx, int dtype, SegGemm p);
 // k splits worth taking for an all-f32 product of this shape; together their slabs have at most max_rows rows
-int seg_gemm_splits(moon_ctx *ctx, size_t M, size_t N, size_t K, size_t max_rows);
+int seg_gemm_splits(moon_ctx *ctx, int dtype, size_t M, size_t N, size_t K, size_t max_rows);
 
 // ---- row kernels (layer_rows.hip)
 // x[n] = embed[ids[n]] * scale (embed != null), or x += the k splits of a product + the chosen experts' weighted rows; then the

@@ -213,7 +213,10 @@ static void even_ranges(int K, int splits, int *kb) {
     for (int s = 0, per = (int)pad_to((K + splits - 1) / splits, BK); s <= splits; s++) kb[s] = std::min(K, s * per);
 }
 
-int seg_gemm_splits(moon_ctx *ctx, size_t M, size_t N, size_t K, size_t max_rows) {
+// f32: its multiply-adds take ten times as long as a range's slab, and ranges even out what the units get, so as many as there is room
+// for.  Two layers of a prompt, us, with the bf16 kernel's estimate -> so: width 1024, feed-forward 2752, 500 rows 928 -> 904, 640 rows
+// 1238 -> 1192; 2048, 5504: 640 rows 3170 -> 3060, 1301 rows 7800 -> 7760.
+int seg_gemm_splits(moon_ctx *ctx, int dtype, size_t M, size_t N, size_t K, size_t max_rows) {
     const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
     const double slab = (double)M * N * 8 / 4.5e6; // another range's sums, written and read, us at 4.5 TB/s
     int best = 1;
@@ -222,6 +225,10 @@ int seg_gemm_splits(moon_ctx *ctx, size_t M, size_t N, size_t K, size_t max_rows
         int kb[SEG_MAX_SPLITS + 1];
         even_ranges((int)K, splits, kb);
         if (kb[splits - 1] >= kb[splits]) continue;
+        if (dtype != MOON_DTYPE_BF16) {
+            best = splits;
+            continue;
+        }
         for (int mi = 2; mi <= 4; mi++)
             if (const double e = seg_estimate(cus, mi, (int)M, (int)N, kb, splits, false) + (splits - 1) * slab; e < t) {
                 t = e;

@@ -6,6 +6,7 @@ import sys
 import numpy as np
 import pytest
 import rikanex_oracle as R
+from conftest import compute_units
 from decoder_checks import feed, opened, row_errors, rows_close, run, streams_of_both_types
 from rikanex_models import (MODELS, ODD, TALL, WIDE, attention, config, dense, beacon_weights, layer, moe, tokens, weights, write_folder)
 
@@ -411,6 +412,24 @@ def test_tile_heights_of_the_second_product(moon, ctx, rows, ff, height, splits)
     cfg = config(128, 2048, [layer(attention(32, 8, 64, 64, 100, 0.125), dense(ff))], embed_scale=2.0)
     got, want = streams_of_both_types(moon, ctx, cfg, tokens(rows, 128), f"seg_gemm_bf16_kernel {height} rows a tile, k split {splits}")
     assert_close(got, want, "bfloat16")
+
+
+@pytest.mark.parametrize("width,rows,ff,splits", [(1024, 500, 2752, 7), (1024, 640, 2752, 6), (1024, 900, 2752, 4), (2048, 768, 5504, 5), (2048, 1301, 5504, 3), (2048, 2000, 5504, 2)])
+def test_ranges_of_the_second_product_in_f32(moon, ctx, width, rows, ff, splits):
+    """An f32 session takes as many ranges of k as its buffer has slabs for.  The last rows again as a call of their own, whose ranges are
+    others: sums of up to 7,552 products in another order; limit 1e-5 of a row's norm."""
+    cfg = config(128, width, [layer(attention(width // 64, 4, 64, 64, 100, 0.125), dense(ff))], embed_scale=2.0)
+    m, ids, last = moon.text_model.TextModel.open_synthetic(cfg, "float32", 2048, seed=5, std=0.02, ctx=ctx), tokens(rows, 128), 37
+    m.forward(ids)
+    if compute_units() == 256:
+        assert ctx.last_kernel() == f"seg_gemm_f32_kernel 64 rows a tile, k split {splits}"
+    whole = m.hidden_f32(rows)[-last:]
+    m.reset()
+    m.forward(ids[:-last])
+    m.forward(ids[-last:])
+    apart = m.hidden_f32(last)
+    m.close()
+    assert np.linalg.norm(whole - apart, axis=1).max() <= 1e-5 * np.linalg.norm(whole, axis=1).min()
 
 
 @pytest.mark.parametrize("rows", [300, 1025])
