@@ -273,7 +273,7 @@ int launch_seg_gemm(moon_ctx *ctx, int dtype, SegGemm p) {
         else if (mi == 3) MOON_TRY(go(seg_gemm_bf16_kernel<3>, Stream<3>::LDS_BYTES, set3));
         else MOON_TRY(go(seg_gemm_bf16_kernel<2>, Stream<2>::LDS_BYTES, set2));
     } else {
-        const SegWalk w = seg_walk(p.tile_group ? p.max_tiles : (p.M + SEG_TILE_ROWS - 1) / SEG_TILE_ROWS, p.N / 64, p.tile_group, p.kb, p.splits, p.longest_first);
+        const SegWalk w = seg_walk(p.tile_group ? p.max_tiles : (p.M + SEG_TILE_ROWS - 1) / SEG_TILE_ROWS, p.N / 64, true, p.kb, p.splits, p.longest_first);
         hipLaunchKernelGGL(seg_gemm_f32_kernel, dim3((unsigned)(SEG_DIES * w.slots)), dim3(256), 0, ctx->stream, p, w);
     }
     MOON_HIP(ctx, hipGetLastError());
