@@ -696,6 +696,8 @@ int launch_flash(moon_ctx *ctx, const FaArgs &p) {
     //   heads of 64           32 x 600 13.4 -> 13.9, 32 x 768 (96) 14.2 -> 14.3, 32 x 832 19.0 -> 16.1, 16 x 1664 29.8 -> 24.4
     //   heads of 64, causal   32 x 768 (96) 12.0 -> 11.5, 32 x 800 12.4 -> 12.7, 32 x 832 12.8 -> 13.0, 16 x 1600 17.4 -> 18.3, 8 x 3328 (104) 28.8 -> 29.4;
     //                         32 x 896 (112) 13.6 -> 13.4, 16 x 1792 (112) 20.0 -> 18.9, 8 x 3584 (112) 31.9 -> 31.5, 32 x 1024 15.4 -> 13.9
+    // Past the line the two kernels' rounds end at different sizes, so a few sizes lose up to 2 % (32 heads of 64: 1360 causal rows 22.6 ->
+    // 23.0, 1056 rows 26.5 -> 27.1); from there on up to 25 % are gained (32 x 2048: 65.7 -> 52.6; of 72: 79.6 -> 61.7).
     // Well below the line the chip is better filled with 32: 16 heads of 72, 512 rows 7.6 us against 9.5.
     const size_t rows = (size_t)p.Lq * p.H, cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
     const bool two = p.causal_pos >= 0 ? rows >= 112 * cus : rows > (D == 64 ? 96 : 64) * cus;

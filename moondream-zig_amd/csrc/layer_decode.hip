@@ -14,6 +14,9 @@
 // cache rows (loads return in order), lanes are summed with cross-lane moves instead of trips through LDS, the newest key is a piece like
 // the others and rows are found without divisions: 0.771 and 0.747 ms.  One split for a short context, which would save the merge, is slower
 // (0.785 against 0.747 at 60 to 90 keys): a step of 32 keys costs more than the hop.
+// Every role of decode_mix has the attention's LDS and the experts' registers.  It pays all the same: with heads of 512, which leave a unit one
+// workgroup, eight layers (8 heads on one key head) went from 819 to 631 us per token behind 60 keys and from 1,907 to 1,200 behind 1,900; a
+// kernel without the experts' part, which lets three or four workgroups of the down product share a unit, is 1.4 to 2 % slower (heads of 64).
 // All are bound by HBM: weights are read once with 128-bit non-temporal loads.  No workgroup waits for another.
 #include "delta_math.hpp"
 #include "lane_fold.hpp"
