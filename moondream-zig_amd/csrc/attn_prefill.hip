@@ -13,12 +13,13 @@
 // The scale 1/sqrt(D) multiplies the f32 product (attention.zig:192-194, 487-489), masked scores are -inf, the
 // result is divided by the f32 row sum and rounded once to f16.
 #include "epilogue.hpp"
+#include "tile_copy.hpp"
 
 #include <atomic>
 
 namespace {
 
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+typedef tile_u32x4 u32x4;
 typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
 
 constexpr int FA_Q = 32;     // query rows per workgroup
@@ -401,32 +402,9 @@ struct FbCfg {
 // 16 consecutive keys, a transposing V read 4 granules of each of 4 consecutive keys; 16 granules are all 64 banks.
 //   D = 72: slot s starts at granule 9 s.  Slots 4 apart start 4 granules apart mod 16, so keys 4 a + b of a group of 16 sit in slot
 //           4 b + a (its own inverse): four consecutive keys fill the banks, and so do 16 with one granule each.
-//   D = 64: slot s is key s and starts at granule 8 s.  Granule c sits at c ^ f(s): of two rows with the same parity that follow
-//           each other f differs in bit 2, and over 16 rows each half of the banks sees all eight values.
+//   D = 64: slot s is key s and starts at granule 8 s.  Granule c sits at c ^ row64_swizzle(s).
 template <int D> __device__ __forceinline__ int fb_slot(int key) { return D == 72 ? (key & ~15) | (key & 3) << 2 | (key >> 2 & 3) : key; }
-template <int D> __device__ __forceinline__ int fb_swizzle(int key) { return D == 72 ? 0 : (key >> 1 & 1) << 2 | (key >> 2 & 3); }
-
-// The tile whose first row lies at `rows` into the LDS at byte lds: left bytes are what the head's rows still hold from there, what
-// lies past them reads as zero.  Written as instructions because the compiler, which cannot tell which of its LDS reads a copy
-// in flight touches, would wait for every copy before each of them; fb_landed says what has arrived.  The LDS reads before it
-// have returned when the first copy starts.
-// (M0 is a register that the compiler keeps for itself and sets anew for each of its own uses: naming it makes it do so behind a copy,
-// and clang says that it is not preserved, which is the point)
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-template <int COPIES>
-__device__ __forceinline__ void fb_copy(const half_t *rows, int left, unsigned lds, const int (&off)[COPIES]) {
-    const unsigned long at = reinterpret_cast<unsigned long>(rows);
-    u32x4 rs = {(unsigned)__builtin_amdgcn_readfirstlane((int)at), (unsigned)__builtin_amdgcn_readfirstlane((int)(at >> 32) & 0xffff),
-                (unsigned)__builtin_amdgcn_readfirstlane(left), 0x00020000u};
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-#pragma unroll
-    for (int i = 0; i < COPIES; i++)
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" // (5 wait states: scalars that the vector unit wrote)
-                     ::"s"(lds + i * 1024), "v"(off[i]), "s"(rs) : "memory", "m0");
-}
-#pragma clang diagnostic pop
-template <int NEWER> __device__ __forceinline__ void fb_landed() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NEWER) : "memory"); }
+template <int D> __device__ __forceinline__ int fb_swizzle(int key) { return D == 72 ? 0 : row64_swizzle(key); }
 
 template <int D>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void flash_attn64_kernel(FaArgs p) {
@@ -480,8 +458,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
     const size_t tile_stride = size_t(FA_KT) * p.kv_row_stride;
 
     if (wave < n_tiles) {
-        fb_copy(kh + wave * tile_stride, head_bytes - wave * FA_KT * row_bytes, k_lds, off);
-        fb_copy(vh + wave * tile_stride, head_bytes - wave * FA_KT * row_bytes, v_lds, off);
+        tile_copy(kh + wave * tile_stride, head_bytes - wave * FA_KT * row_bytes, k_lds, off);
+        tile_copy(vh + wave * tile_stride, head_bytes - wave * FA_KT * row_bytes, v_lds, off);
     }
     // this lane's query rows as the MFMA "B" operand: Q[q0 + 32 u + col][16*s + 8*hf .. +7]
     half8_t qf[QS][C::KSTEPS];
@@ -519,7 +497,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
         const bool more = t + FA_WAVES < n_tiles;
         const half_t *k_next = kh + (t + FA_WAVES) * tile_stride, *v_next = vh + (t + FA_WAVES) * tile_stride;
         const int left = head_bytes - (t + FA_WAVES) * FA_KT * row_bytes;
-        fb_landed<C::COPIES>(); // the K tile (the V tile's copies are newer)
+        tile_landed<C::COPIES>(); // the K tile (the V tile's copies are newer)
 
         float16_t s[QS][2];
 #pragma unroll
@@ -539,7 +517,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
                 for (int u = 0; u < QS; u++) s[u][kt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8_t, a), qf[u][st], s[u][kt], 0, 0, 0);
             }
         }
-        if (more) fb_copy(k_next, left, k_lds, off);
+        if (more) tile_copy(k_next, left, k_lds, off);
 #pragma unroll
         for (int u = 0; u < QS; u++) {
             // s[u][kt][v] = score of key key0 + 32*kt + 8*(v/4) + 4*hf + v%4 against query q0 + 32 u + col
@@ -593,8 +571,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
             l_run[u] = l_run[u] * alpha + psum;
         }
 
-        if (more) fb_landed<C::COPIES>(); // the V tile
-        else fb_landed<0>();
+        if (more) tile_landed<C::COPIES>(); // the V tile
+        else tile_landed<0>();
         // O^T += V^T . P^T : contraction step (kt, sp) uses the keys a lane already holds in s[u][kt][8*sp .. 8*sp+7],
         // i.e. key0 + 32*kt + 16*sp + {4*hf + 0..3, 8 + 4*hf + 0..3}
 #pragma unroll
@@ -615,7 +593,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
                     for (int u = 0; u < QS; u++) o[u][dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, pb[u], o[u][dt], 0, 0, 0);
                 }
             }
-        if (more) fb_copy(v_next, left, v_lds, off);
+        if (more) tile_copy(v_next, left, v_lds, off);
     }
 
     // merge the four waves' partial results

@@ -10,10 +10,13 @@
 //     S^T[key][q] = K . Q^T     (a lane holds 32 scores of ONE query)
 //     O^T[d][q]  += V^T . P^T   (V row-major in LDS, transposed by the LDS load)
 // Scores and weights are f32.  A weight enters the second product as two bf16 terms, its rounding and the remainder, so the
-// product sees 16 bits of it.
+// product sees 16 bits of it.  Heads of 64 in calls with enough rows share their tiles between four wavefronts instead
+// (window_attn_shared_kernel).
 // f32, and head sizes above 256, take one wavefront per (row, head) with plain multiply-adds.
+#include "lane_fold.hpp"
 #include "layer_list.hpp"
 #include "lm_types.hpp"
+#include "tile_copy.hpp"
 
 #include <algorithm>
 #include <atomic>
@@ -45,6 +48,13 @@ template <int P> struct WaCfg { // P: head sizes up to P (a multiple of 32), row
 
 __device__ __forceinline__ wa_short4_t wa_read_tr(const bf16_t *p) {
     return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) wa_short4_t *)(p));
+}
+
+// Two weights as two bf16 terms each: a packed conversion, its two halves back as f32, the remainders
+__device__ __forceinline__ uint2 split_pair(float w0, float w1) {
+    const unsigned hi = __builtin_bit_cast(unsigned, __builtin_convertvector(float2_t{w0, w1}, bf16x2_t));
+    const float2_t rest = {w0 - __builtin_bit_cast(float, hi << 16), w1 - __builtin_bit_cast(float, hi & 0xffff0000u)};
+    return uint2{hi, __builtin_bit_cast(unsigned, __builtin_convertvector(rest, bf16x2_t))};
 }
 
 // POOL: the tiles of the blocks' keys come first, in the same softmax
@@ -228,14 +238,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(P <= 64 ? 2
         for (int kt = 0; kt < 2; kt++)
 #pragma unroll
             for (int sp = 0; sp < 2; sp++) {
-                lm_u32x4 hi_bits, lo_bits; // two at a time: a packed conversion, its two halves back as f32, the remainders
+                lm_u32x4 hi_bits, lo_bits;
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
-                    const float2_t w = {s[kt][8 * sp + 2 * e], s[kt][8 * sp + 2 * e + 1]};
-                    hi_bits[e] = __builtin_bit_cast(unsigned, __builtin_convertvector(w, bf16x2_t));
-                    const unsigned pair = hi_bits[e];
-                    const float2_t rest = {w[0] - __builtin_bit_cast(float, pair << 16), w[1] - __builtin_bit_cast(float, pair & 0xffff0000u)};
-                    lo_bits[e] = __builtin_bit_cast(unsigned, __builtin_convertvector(rest, bf16x2_t));
+                    const uint2 pair = split_pair(s[kt][8 * sp + 2 * e], s[kt][8 * sp + 2 * e + 1]);
+                    hi_bits[e] = pair.x;
+                    lo_bits[e] = pair.y;
                 }
                 const bf16x8_t hi = __builtin_bit_cast(bf16x8_t, hi_bits), lo = __builtin_bit_cast(bf16x8_t, lo_bits);
 #pragma unroll
@@ -249,11 +257,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(P <= 64 ? 2
             }
     }
 
-    // this thread's gate values for the merged result, requested before the merge
+    // this thread's gate values (and angles) for the merged result, requested before the merge
     const int q = tid & 31, row = row0 + q, d0 = (tid >> 5) * 8;
     const bf16_t *gate = p.gate ? reinterpret_cast<const bf16_t *>(p.gate) + size_t(min(row, p.n - 1)) * p.ldq + h * p.vdimp : nullptr;
     bf16x8_t gz = {};
     if (gate && d0 < p.vdimp) gz = *reinterpret_cast<const bf16x8_t *>(gate + d0);
+    const bool pairs = P == 64 && p.rotv && p.vdim == 64; // (eight pairs lie in two granules: 37.1 -> 33 us at 1301 rows of 32 rotated heads)
+    float4_t turn[4] = {}; // and its angles: cos, sin, cos, sin
+    if (P == 64 && pairs)
+#pragma unroll
+        for (int e = 0; e < 4; e++) turn[e] = reinterpret_cast<const float4_t *>(p.rotv + size_t(p.pos0 + min(row, p.n - 1)) * 32 + (d0 & 31))[e];
     // merge the wavefronts' results; the sink is one more term of the denominator
     const float l_wave = l_run + __shfl_xor(l_run, 32);
     float *so = reinterpret_cast<float *>(wa_lds), *sm = reinterpret_cast<float *>(reinterpret_cast<char *>(wa_lds) + C::ML_OFFSET), *sl = sm + WA_WAVES * WA_Q;
@@ -291,7 +304,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(P <= 64 ? 2
             for (int e = 0; e < 8; e++) acc[e] += so[(w * WA_Q + q) * C::SD + d + e];
 #pragma unroll
         for (int e = 0; e < 8; e++) acc[e] *= inv;
-        if (p.rotv) { // each element with the other one of its pair
+        if (P == 64 && pairs) { // the other ones of eight pairs lie 32 elements away
+            float other[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int w = 0; w < WA_WAVES; w++)
+#pragma unroll
+                for (int e = 0; e < 8; e++) other[e] += so[(w * WA_Q + q) * C::SD + (d ^ 32) + e];
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const float c = turn[e / 2][2 * (e & 1)], sn = turn[e / 2][2 * (e & 1) + 1], z = other[e] * inv;
+                acc[e] = d & 32 ? acc[e] * c - z * sn : acc[e] * c + z * sn;
+            }
+        } else if (p.rotv) { // each element with the other one of its pair
             const int half = p.vdim / 2;
 #pragma unroll
             for (int e = 0; e < 8; e++)
@@ -312,6 +336,271 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(P <= 64 ? 2
         for (int e = 0; e < 8; e++) r[e] = (bf16_t)(acc[e] * (gate ? lm_sigmoid((float)gz[e]) : 1.0f));
         *reinterpret_cast<bf16x8_t *>(out + d) = r;
     }
+}
+
+constexpr int WS_PAIRED = 64; // workgroups of a die that are there at once: two per unit
+
+// Heads of 64 in calls with many rows.  A workgroup takes four units of 32 query rows, heads that read the same keys where a group has
+// them, else the next rows; a unit's wavefront walks all of its keys, so the four share every tile and nothing is merged over rows.  Two
+// such groups of wavefronts take every other tile, merged once at the end: with one, the wavefronts of a call that puts one workgroup on a
+// unit are alone on their SIMDs and spend 1.5 us a tile, mostly waiting; with two, 1.9 us for two.  Tiles are copied straight to LDS
+// (tile_copy.hpp), the next one while one is worked on, with a barrier per tile.
+// A window of 1024 is 17 tiles: the kernel above gives a wavefront four of them, and its first loads, scores' masks and merge cost as much
+// as the tiles.  What bounds this one is the vector unit (of about 1,370 cycles a tile and wavefront, exponentials 510, the weights' second
+// term 380) and, in calls of one workgroup per unit, latency: start and end take 7 us.
+// Times, above -> here: 32 heads, window 1024, 1920 rows 49.7 -> 36.9 us, 1301 rows 34.0 -> 27.8, with blocks 33.1 -> 26.3, rotated 36.1 -> 26.7.
+// Measured and not kept: 64 rows per wavefront in the arrangement above (43.5 us at 1920 rows; better, by 15 %, only around 768); two
+// wavefronts instead of four there (46.9); remainders of the weights by two-element dot products (1 to 3 us slower); wave priorities.
+struct WsCfg {
+    static constexpr int D = 64, KSTEPS = D / 16, DT = D / 32, G = D / 8, STAGES = 2, GROUPS = 2;
+    static constexpr int TILE = WA_KT * D, COPIES = WA_KT * G / 64 / WA_WAVES; // elements of a K or V tile, copies of each per wavefront
+    static constexpr size_t LDS_BYTES = size_t(GROUPS) * STAGES * 2 * TILE * 2;
+};
+__host__ __device__ __forceinline__ int ws_heads(int per_group) { return per_group % 4 == 0 ? 4 : per_group % 2 == 0 ? 2 : 1; } // heads per workgroup
+__host__ __device__ __forceinline__ int ws_rows(int per_group) { return WA_Q * WA_WAVES / ws_heads(per_group); }                 // rows per workgroup
+
+template <bool POOL>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void window_attn_shared_kernel(WindowAttn p) {
+    using C = WsCfg;
+    constexpr int D = C::D, ROW = D * 2; // ROW: bytes of a cache row
+    extern __shared__ __attribute__((aligned(16))) bf16_t wa_lds[];
+    const int tid = threadIdx.x, lane = tid & 63, kg = __builtin_amdgcn_readfirstlane(tid >> 8), wave = __builtin_amdgcn_readfirstlane(tid >> 6 & 3), col = lane & 31, hf = lane >> 5;
+    const int per = p.H / p.G, nh = ws_heads(per), rows = ws_rows(per), n_qb = (p.n + rows - 1) / rows, n_hb = p.H / nh;
+    // which heads and rows: a die takes whole stretches of the (heads, block) list, late blocks first
+    int item = blockIdx.x;
+    const int n_items = n_qb * n_hb;
+    int hb = item / n_qb, qb = item % n_qb;
+    if (n_items % 8 == 0 && (n_items / 8) % n_qb == 0) { // whole heads per die: their blocks walk together
+        const int per_die = n_items / 8, heads = per_die / n_qb;
+        int j = item / 8;
+        if (per_die <= WS_PAIRED && j >= WS_PAIRED / 2) j = per_die - 1 - (j - WS_PAIRED / 2); // two per unit: the lightest beside the heaviest
+        hb = item % 8 * heads + j % heads;
+        qb = j / heads;
+    }
+    qb = n_qb - 1 - qb;
+    const int h = hb * nh + wave % nh, g = h / per, wg_row0 = qb * rows, row0 = wg_row0 + wave / nh * WA_Q;
+    const int wg_first = p.pos0 + wg_row0, last_pos = p.pos0 + min(wg_row0 + rows, p.n) - 1; // positions of the workgroup's first and last row
+    const int first_pos = p.pos0 + row0, pos = first_pos + col;                               // of the wavefront's first row and this lane's
+    const int lo_key = p.window ? max(0, wg_first - p.window + 1) : 0;
+    const int seen = POOL ? blocks_seen(last_pos, p.window, p.pool) : 0, t_blocks = (seen + WA_KT - 1) / WA_KT;
+    const int t_begin = POOL ? lo_key / WA_KT - t_blocks : lo_key / WA_KT, t_end = last_pos / WA_KT + 1;
+    const int t_window = POOL ? lo_key / WA_KT : 0;
+    const size_t head_rows = size_t(g) * p.cap * ROW, head_blocks = POOL ? size_t(g) * p.blocks * ROW : 0;
+    const char *ck = reinterpret_cast<const char *>(p.ck) + head_rows, *cv = reinterpret_cast<const char *>(p.cv) + head_rows;
+    const char *pk = reinterpret_cast<const char *>(p.pk) + head_blocks, *pv = reinterpret_cast<const char *>(p.pv) + head_blocks;
+    const unsigned lds0 = __builtin_amdgcn_readfirstlane((unsigned)reinterpret_cast<unsigned long>((__attribute__((address_space(3))) const bf16_t *)wa_lds));
+    int off[C::COPIES]; // this lane's granules of a tile, from its first row (K and V lie alike)
+#pragma unroll
+    for (int i = 0; i < C::COPIES; i++) {
+        const int row = (wave * C::COPIES + i) * 8 + (lane >> 3);
+        off[i] = row * ROW + ((lane & 7) ^ row64_swizzle(row)) * 16;
+    }
+    // This wavefront's part of tile t to stage t % STAGES; rows that must not be read are offsets past the end, which bring zeros.
+    constexpr int NOWHERE = 0x7fffffff;
+    auto copy = [&](int t, int stage) {
+        const unsigned k_lds = lds0 + (kg * C::STAGES + stage) * 2 * C::TILE * 2 + wave * C::COPIES * 1024, v_lds = k_lds + C::TILE * 2;
+        const bool blocks = POOL && t < t_window;
+        const int key0 = blocks ? (t - t_begin) * WA_KT : t * WA_KT, lo = blocks ? 0 : lo_key, hi = blocks ? seen - 1 : last_pos, rows = blocks ? p.blocks : p.cap;
+        const int slot0 = key0 < rows ? key0 : key0 % rows;
+        const bool whole = key0 >= lo && key0 + WA_KT - 1 <= hi && slot0 + WA_KT <= rows; // in one piece
+        int offs[C::COPIES];
+#pragma unroll
+        for (int i = 0; i < C::COPIES; i++) {
+            const int row = (wave * C::COPIES + i) * 8 + (lane >> 3), key = key0 + row;
+            offs[i] = off[i] + slot0 * ROW;
+            if (whole) continue;
+            if (slot0 + row >= rows) offs[i] -= rows * ROW; // (a cache that wraps has more rows than a tile)
+            if (key < lo || key > hi) offs[i] = NOWHERE;
+        }
+        tile_copy(blocks ? pk : ck, rows * ROW, k_lds, offs);
+        tile_copy(blocks ? pv : cv, rows * ROW, v_lds, offs);
+    };
+    int t = t_begin + kg;
+    if (t < t_end) copy(t, 0);
+    const float scale = p.temp ? p.scale * p.temp[h] : p.scale;
+    bf16x8_t qf[C::KSTEPS]; // the MFMA "B" operand: Q[row0 + col][16 s + 8 hf .. + 7]
+    {
+        const bf16_t *q = reinterpret_cast<const bf16_t *>(p.q) + size_t(min(row0 + col, p.n - 1)) * p.ldq + h * D;
+#pragma unroll
+        for (int s = 0; s < C::KSTEPS; s++) {
+            lm_u32x4 v = *reinterpret_cast<const lm_u32x4 *>(q + 16 * s + 8 * hf);
+            if (scale < 0.0f) v ^= 0x80008000u; // (as in window_attn_kernel)
+            qf[s] = __builtin_bit_cast(bf16x8_t, v);
+        }
+    }
+    int voff[2][C::DT]; // where this lane points the transposing loads: keys 4 hf + (lane % 16) / 4 (+ 8), columns 32 dt + 16 ((lane / 16) % 2) + 4 (lane % 4)
+#pragma unroll
+    for (int j = 0; j < 2; j++)
+#pragma unroll
+        for (int dt = 0; dt < C::DT; dt++) {
+            const int key = 8 * j + 4 * hf + ((lane & 15) >> 2), c = 32 * dt + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+            voff[j][dt] = key * D + ((c >> 3 ^ row64_swizzle(key)) << 3 | (c & 7));
+        }
+    __builtin_amdgcn_s_waitcnt(0xf70); // vmcnt(0): the query rows have arrived (else the compiler waits for them, and every copy, in each round)
+
+    float16_t o[C::DT];
+    float m_run = -INFINITY, l_run = 0.0f;
+#pragma unroll
+    for (int dt = 0; dt < C::DT; dt++)
+#pragma unroll
+        for (int v = 0; v < 16; v++) o[dt][v] = 0.0f;
+    const int mine0 = POOL ? blocks_seen(pos, p.window, p.pool) - 1 - 4 * hf : 0; // the last block that this lane's row sees, from its first one
+    constexpr float LOG2E = 1.4426950408889634f;
+    const float c2 = fmaxf(fabsf(scale) * LOG2E, 1e-37f);
+    const float sink = p.sink ? p.sink[h] * LOG2E : -INFINITY;
+
+    for (int left = (t_end - t_begin + C::GROUPS - 1) / C::GROUPS, stage = 0; left > 0; left--, t += C::GROUPS, stage ^= 1) {
+        const int key0 = t * WA_KT;
+        tile_landed<0>(); // this wavefront's part of the tile; behind the barrier everybody's, and the tile before has been read by all
+        asm volatile("s_barrier" ::: "memory");
+        if (t + C::GROUPS < t_end) copy(t + C::GROUPS, stage ^ 1);
+        if (t >= t_end) continue;
+        const bool blocks = POOL && t < t_window;
+        if (!blocks && (key0 > first_pos + WA_Q - 1 || (p.window && key0 + WA_KT <= first_pos - p.window + 1))) continue; // no row sees any of it
+        const bf16_t *Ks = wa_lds + (kg * C::STAGES + stage) * 2 * C::TILE, *Vs = Ks + C::TILE;
+        float16_t s[2];
+        bf16x8_t a[2][C::KSTEPS];
+#pragma unroll
+        for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+            for (int st = 0; st < C::KSTEPS; st++) a[kt][st] = *reinterpret_cast<const bf16x8_t *>(Ks + (32 * kt + col) * D + ((2 * st + hf) ^ row64_swizzle(col)) * 8);
+#pragma unroll
+        for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) s[kt][v] = 0.0f;
+#pragma unroll
+        for (int st = 0; st < C::KSTEPS; st++)
+#pragma unroll
+            for (int kt = 0; kt < 2; kt++) s[kt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[kt][st], qf[st], s[kt], 0, 0, 0);
+        // s[kt][v]: key key0 + 32 kt + 8 (v / 4) + 4 hf + v % 4 against this lane's query
+        if (blocks || key0 + WA_KT - 1 > first_pos || (p.window && key0 <= first_pos + WA_Q - 1 - p.window)) { // some row does not see the whole tile
+            const int age0 = blocks ? mine0 - (t - t_begin) * WA_KT : pos - key0 - 4 * hf; // how far back this lane's first key (block) is
+            const unsigned ages = !blocks && p.window ? (unsigned)p.window : 0x7fffffffu;
+#pragma unroll
+            for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) // (a key ahead of the query wraps to a large age)
+                    s[kt][v] = (unsigned)(age0 - (32 * kt + 8 * (v >> 2) + (v & 3))) < ages ? s[kt][v] : -INFINITY;
+        }
+        asm volatile("" : "+v"(s[0]), "+v"(s[1])); // (in these registers on both paths: left alone, the scores are copied on each)
+        float mx = -INFINITY;
+#pragma unroll
+        for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) mx = fmaxf(mx, s[kt][v]);
+        mx = half_max(mx);
+        const float m_new = fmaxf(m_run, mx * c2), m_use = m_new == -INFINITY ? 0.0f : m_new;
+        float alpha = 1.0f;
+        if (__any(m_new != m_run)) {
+            alpha = __builtin_amdgcn_exp2f(m_run - m_use);
+            m_run = m_new;
+#pragma unroll
+            for (int dt = 0; dt < C::DT; dt++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) o[dt][v] *= alpha;
+        }
+        float psum = 0.0f;
+#pragma unroll
+        for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) {
+                const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(s[kt][v], c2, -m_use));
+                s[kt][v] = e;
+                psum += e;
+            }
+        l_run = l_run * alpha + psum;
+        // contraction step (kt, sp) uses the keys a lane holds in s[kt][8 sp .. 8 sp + 7], as in window_attn_kernel
+#pragma unroll
+        for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+            for (int sp = 0; sp < 2; sp++) {
+                lm_u32x4 hi_bits, lo_bits;
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const uint2 pair = split_pair(s[kt][8 * sp + 2 * e], s[kt][8 * sp + 2 * e + 1]);
+                    hi_bits[e] = pair.x;
+                    lo_bits[e] = pair.y;
+                }
+                const bf16x8_t hi = __builtin_bit_cast(bf16x8_t, hi_bits), lo = __builtin_bit_cast(bf16x8_t, lo_bits);
+                bf16x8_t v[C::DT];
+#pragma unroll
+                for (int dt = 0; dt < C::DT; dt++) {
+                    const wa_short4_t a0 = wa_read_tr(Vs + voff[0][dt] + (32 * kt + 16 * sp) * D), a1 = wa_read_tr(Vs + voff[1][dt] + (32 * kt + 16 * sp) * D);
+                    v[dt] = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7));
+                }
+#pragma unroll
+                for (int dt = 0; dt < C::DT; dt++) o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v[dt], lo, o[dt], 0, 0, 0);
+#pragma unroll
+                for (int dt = 0; dt < C::DT; dt++) o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v[dt], hi, o[dt], 0, 0, 0);
+            }
+    }
+
+    // o[dt][4 j + e] is element 32 dt + 8 j + 4 hf + e of this lane's row.  The second group hands its result over, [wave][register][lane].
+    float *so = reinterpret_cast<float *>(wa_lds) + wave * (C::DT * 16 + 2) * 64 + lane;
+    l_run += __shfl_xor(l_run, 32);
+    // what the results still need, requested before the merge: this lane's gate granules 4 dt + 2 i + hf, cos and sin of two pairs each
+    const int row = row0 + col, at_row = min(row, p.n - 1);
+    const bf16_t *gate = p.gate ? reinterpret_cast<const bf16_t *>(p.gate) + size_t(at_row) * p.ldq + h * D : nullptr;
+    bf16x8_t gz[C::DT][2] = {};
+    if (kg == 0 && gate)
+#pragma unroll
+        for (int dt = 0; dt < C::DT; dt++)
+#pragma unroll
+            for (int i = 0; i < 2; i++) gz[dt][i] = *reinterpret_cast<const bf16x8_t *>(gate + (4 * dt + 2 * i + hf) * 8);
+    float4_t turn[4][2];
+    if (kg == 0 && p.rotv) // (over all of the head: the other one of a pair is 32 elements away)
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+#pragma unroll
+            for (int e = 0; e < 2; e++) turn[j][e] = reinterpret_cast<const float4_t *>(p.rotv + size_t(p.pos0 + at_row) * (D / 2))[4 * j + 2 * hf + e];
+    __syncthreads(); // every wavefront is done with the tiles
+    if (kg == 1) {
+#pragma unroll
+        for (int dt = 0; dt < C::DT; dt++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) so[(16 * dt + v) * 64] = o[dt][v];
+        so[C::DT * 16 * 64] = m_run;
+        so[(C::DT * 16 + 1) * 64] = l_run;
+    }
+    __syncthreads();
+    if (kg == 1) return;
+    // (the sink is one more term of the denominator)
+    const float m_other = so[C::DT * 16 * 64], m_all = fmaxf(fmaxf(sink, m_run), m_other);
+    const float f = m_run == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_run - m_all), f_other = m_other == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_other - m_all);
+    const float inv = 1.0f / (l_run * f + so[(C::DT * 16 + 1) * 64] * f_other + (p.sink ? __builtin_amdgcn_exp2f(sink - m_all) : 0.0f));
+#pragma unroll
+    for (int dt = 0; dt < C::DT; dt++)
+#pragma unroll
+        for (int v = 0; v < 16; v++) o[dt][v] = (o[dt][v] * f + so[(16 * dt + v) * 64] * f_other) * inv;
+    if (p.rotv) {
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+#pragma unroll
+            for (int e = 0; e < 4; e += 2) {
+                const float4_t cs = turn[j][e / 2];
+#pragma unroll
+                for (int k = 0; k < 2; k++) {
+                    const float x = o[0][4 * j + e + k], y = o[1][4 * j + e + k];
+                    o[0][4 * j + e + k] = x * cs[2 * k] + y * cs[2 * k + 1];
+                    o[1][4 * j + e + k] = y * cs[2 * k] - x * cs[2 * k + 1];
+                }
+            }
+    }
+    bf16_t *out = reinterpret_cast<bf16_t *>(p.out) + size_t(at_row) * p.ldo + h * D;
+#pragma unroll
+    for (int dt = 0; dt < C::DT; dt++)
+#pragma unroll
+        for (int i = 0; i < 2; i++) { // halves of two granules against whole ones: the lower lanes take granule 4 dt + 2 i, the upper the next
+            bf16x8_t r;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const auto x = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, (float)o[dt][8 * i + e]), __builtin_bit_cast(unsigned, (float)o[dt][8 * i + 4 + e]), false, false);
+                const unsigned x0 = x[0], x1 = x[1];
+                r[e] = (bf16_t)(__builtin_bit_cast(float, x0) * (gate ? lm_sigmoid((float)gz[dt][i][e]) : 1.0f));
+                r[4 + e] = (bf16_t)(__builtin_bit_cast(float, x1) * (gate ? lm_sigmoid((float)gz[dt][i][4 + e]) : 1.0f));
+            }
+            if (row < p.n) *reinterpret_cast<bf16x8_t *>(out + (4 * dt + 2 * i + hf) * 8) = r;
+        }
 }
 
 // One wavefront per (row, head): 64 keys at a time, one per lane for the scores, one element per lane for the values.
@@ -379,20 +668,43 @@ __global__ __launch_bounds__(256) void window_attn_rows_kernel(WindowAttn p) {
     }
 }
 
-template <int P, bool POOL> int launch_mfma_as(moon_ctx *ctx, const WindowAttn &p) {
-    using C = WaCfg<P>;
-    static std::atomic<bool> attr_set[64]; // the opt-in to this much dynamic LDS is per device (and per instantiation)
-    const int dev = ctx->device >= 0 && ctx->device < 64 ? ctx->device : -1;
+// Where the shared tiles pay.  The kernel with merged wavefronts spreads any call over the device, its time goes with the rows times their
+// tiles; the other's goes with the longest walk, T tiles, and a start and an end.  On 256 units, merged -> shared (us): 32 heads, window 1024,
+// 600 rows (75 per unit, T = 10) 16.7 -> 17.0, 768 (96, 12) 19.2 -> 19.3 (with blocks 18.9 -> 17.4, rotated 18.7 -> 17.4), 960 (120, 15) 22.9 -> 22.9
+// (21.9 -> 20.8, 22.4 -> 21.5), 1100 (138, 18) 28.4 -> 26.4, 1920 (240, 18) 49.7 -> 36.8; 16 heads, window 512 (T = 10), 960 rows (60) 12.5 -> 16.7,
+// 1200 (75) 17.6 -> 17.2, 1920 (120) 23.2 -> 19.3; window 1000 (T = 17), 1500 (94) 25.0 -> 26.0, 1920 (120) 28.1 -> 27.4.
+bool shares_tiles(moon_ctx *ctx, const WindowAttn &p) {
+    const int last = p.pos0 + p.n - 1, lo = p.window ? std::max(0, last - (WA_Q - 1) - p.window + 1) : 0, seen = p.pool ? std::max(0, last - p.window + 1) / p.pool : 0;
+    const size_t tiles = last / WA_KT - lo / WA_KT + 1 + (seen + WA_KT - 1) / WA_KT, cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
+    return p.dimp == WsCfg::D && p.vdimp == WsCfg::D && (!p.rotv || p.vdim == WsCfg::D) && size_t(p.n) * p.H >= (7 * tiles + 10) * cus;
+}
+
+template <class Kernel> int launch_as(moon_ctx *ctx, const WindowAttn &p, Kernel kernel, std::atomic<bool> (&attr_set)[64], size_t lds, int workgroups, int threads) {
+    const int dev = ctx->device >= 0 && ctx->device < 64 ? ctx->device : -1; // the opt-in to this much dynamic LDS is per device (and per kernel)
     if (dev < 0 || !attr_set[dev].load()) {
-        MOON_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void *>(window_attn_kernel<P, POOL>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)C::LDS_BYTES));
+        MOON_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
         if (dev >= 0) attr_set[dev].store(true);
     }
-    hipLaunchKernelGGL((window_attn_kernel<P, POOL>), dim3((unsigned)((p.n + WA_Q - 1) / WA_Q * p.H)), dim3(256), C::LDS_BYTES, ctx->stream, p);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)workgroups), dim3(threads), lds, ctx->stream, p);
     MOON_HIP(ctx, hipGetLastError());
+    return MOON_OK;
+}
+template <int P, bool POOL> int launch_mfma_as(moon_ctx *ctx, const WindowAttn &p) {
+    if constexpr (P == 64)
+        if (shares_tiles(ctx, p)) {
+            static std::atomic<bool> attr_set[64];
+            const int per = p.H / p.G, rows = ws_rows(per);
+            MOON_TRY(launch_as(ctx, p, window_attn_shared_kernel<POOL>, attr_set, WsCfg::LDS_BYTES, (p.n + rows - 1) / rows * (p.H / ws_heads(per)), 512));
+            MOON_NOTE_KERNEL(ctx, "window_attn_shared_kernel %d rows of %d heads", rows, ws_heads(per));
+            return MOON_OK;
+        }
+    static std::atomic<bool> attr_set[64];
+    MOON_TRY(launch_as(ctx, p, window_attn_kernel<P, POOL>, attr_set, WaCfg<P>::LDS_BYTES, (p.n + WA_Q - 1) / WA_Q * p.H, 256));
     MOON_NOTE_KERNEL(ctx, "window_attn_kernel<%d>", P);
     return MOON_OK;
 }
-template <int P> int launch_mfma(moon_ctx *ctx, const WindowAttn &p) { return p.pool ? launch_mfma_as<P, true>(ctx, p) : launch_mfma_as<P, false>(ctx, p); }
+// (a call before whose window no block lies yet takes the kernel without them)
+template <int P> int launch_mfma(moon_ctx *ctx, const WindowAttn &p) { return p.pool && p.pos0 + p.n - p.window >= p.pool ? launch_mfma_as<P, true>(ctx, p) : launch_mfma_as<P, false>(ctx, p); }
 
 } // namespace
 

@@ -4,6 +4,14 @@
 
 constexpr int DPP_ROW_ROR8 = 0x128; // the lane 8 away within a row of 16
 
+// Maximum of a lane's value and the one 32 lanes away (no trip through LDS)
+__device__ __forceinline__ float half_max(float v) {
+    const unsigned b = __builtin_bit_cast(unsigned, v);
+    const auto r = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+    const unsigned r0 = r[0], r1 = r[1];
+    return fmaxf(__builtin_bit_cast(float, r0), __builtin_bit_cast(float, r1));
+}
+
 // Sum over aligned groups of n lanes (a power of two, the same in every lane); every lane of a group returns it.
 __device__ __forceinline__ float group_sum(float v, int n) {
     if (n >= 2) v += dpp_move<DPP_QUAD_XOR1>(v);

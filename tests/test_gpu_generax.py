@@ -494,3 +494,22 @@ def test_tile_heights_of_a_joined_layer(moon, ctx, rows, ff, height):
     cfg = config(128, 2048, [parallel(part, delta(32, 32, 64, 64, 4), ff)], softcap=30.0)
     got, want = streams_of_both_types(moon, ctx, cfg, tokens(rows, 128), f"seg_gemm_bf16_kernel {height} rows a tile, k split 3")
     assert_close(got, want, "bfloat16")
+
+
+@pytest.mark.parametrize("kv_heads", [16, 32, 64])
+@pytest.mark.parametrize("window,pool,calls", [(1000, 16, [256]), (64, 5, [333]), (65, 64, [321]), (100, 1, [300, 257]), (30, 16, [2048, 500]), (1, 3, [190])], ids=str)
+def test_attention_over_shared_tiles(moon, ctx, kv_heads, window, pool, calls):
+    """64 heads in groups of four, two and one, whose calls of some hundred rows share key tiles: blocks ahead of the window (up to 300 of them,
+    none in the first case), and heads that turn back.  bf16 against f32, whose attention is a plain loop per row."""
+    mixer = attention(64, kv_heads, 64, 64, window, 0.25, rotation(64, 1e4))
+    cfg = config(128, 64, [parallel(softmax_mixer(64, kv_heads, 64, 64, window, 0.25, pool), delta(1, 1, 64, 64, 2)), plain(mixer), plain(dict(mixer, kv_from=1))], softcap=30.0)
+    ids, got = tokens(sum(calls), 128), {}
+    for dtype in DTYPES:
+        m = moon.text_model.TextModel.open_synthetic(cfg, dtype, sum(calls) + 5, seed=5, std=0.05, ctx=ctx)
+        at = 0
+        for n in calls:
+            m.forward(ids[at:at + n])
+            at += n
+        got[dtype] = m.hidden_f32(calls[-1])
+        m.close()
+    assert_close(got["bfloat16"], got["float32"], "bfloat16")

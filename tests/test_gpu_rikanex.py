@@ -455,3 +455,26 @@ def test_heads_that_fill_a_compute_units_memory(moon, ctx, tmp_path, dtype):
     cfg = config(90, 64, [layer(attention(8, 1, 776, 1024, 18, 0.03), dense(72))])
     w, ids = weights(cfg, 4), tokens(30, 90)
     assert_close(run(moon, ctx, tmp_path, cfg, w, ids, dtype, [1]), R.forward(cfg, w, ids)[0], dtype)
+
+
+def compare_streams(moon, ctx, cfg, calls, max_seq):
+    """Residual streams of the last call's rows, bf16 against f32 (whose attention is a plain loop per row)."""
+    ids, got = tokens(sum(calls), cfg["vocab"]), {}
+    for dtype in DTYPES:
+        m = moon.text_model.TextModel.open_synthetic(cfg, dtype, max_seq, seed=5, std=0.05, ctx=ctx)
+        at = 0
+        for n in calls:
+            m.forward(ids[at:at + n])
+            at += n
+        got[dtype] = m.hidden_f32(calls[-1])
+        m.close()
+    assert_close(got["bfloat16"], got["float32"], "bfloat16")
+
+
+@pytest.mark.parametrize("kv_heads", [16, 32, 64])
+@pytest.mark.parametrize("window,calls", [(1000, [256]), (1000, [333]), (64, [161]), (65, [321]), (100, [300, 257]), (100, [2048, 500]), (1, [190])], ids=str)
+def test_attention_over_shared_tiles(moon, ctx, kv_heads, window, calls):
+    """64 heads in groups of four, two and one, whose calls of some hundred rows share key tiles: whole and ragged blocks of rows and tiles, windows
+    at their edges, rows behind others, and (2048 + 500) a cache whose rows are used again.  Scores with a spread of about 2."""
+    cfg = config(128, 64, [layer(attention(64, kv_heads, 64, 64, window, 0.25, True)), layer(attention(64, kv_heads, 64, 64, window, -0.25, True))], embed_scale=2.0)
+    compare_streams(moon, ctx, cfg, calls, sum(calls) + 5)
