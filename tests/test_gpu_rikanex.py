@@ -478,3 +478,19 @@ def test_attention_over_shared_tiles(moon, ctx, kv_heads, window, calls):
     at their edges, rows behind others, and (2048 + 500) a cache whose rows are used again.  Scores with a spread of about 2."""
     cfg = config(128, 64, [layer(attention(64, kv_heads, 64, 64, window, 0.25, True)), layer(attention(64, kv_heads, 64, 64, window, -0.25, True))], embed_scale=2.0)
     compare_streams(moon, ctx, cfg, calls, sum(calls) + 5)
+
+
+@pytest.mark.parametrize("experts,top", [(1, 1), (63, 5), (64, 8), (64, 64), (65, 8), (130, 70)])
+def test_choice_of_experts_where_scores_tie(moon, ctx, tmp_path, experts, top):
+    """Up to 64 experts are a lane's each, more are walked.  Router weights of zero: every score is 1/2, corrections that repeat decide, and the lower
+    index wins; then random scores."""
+    cfg = config(90, 64, [layer(attention(2, 1, 16, 16, 9, 0.25), moe(experts, top, 8))])
+    for tie in (True, False):
+        w, ids = weights(cfg, 3), tokens(20, 90)
+        router, correction = (next(k for k in w if k.endswith(part)) for part in ("router", "correction"))
+        if tie:
+            w[router] = np.zeros_like(w[router])
+            w[correction] = (np.arange(experts) % 3 * 0.25).astype(np.float32)
+        want, _ = R.forward(cfg, w, ids)
+        for portions in ([20], [1]):
+            assert_close(run(moon, ctx, tmp_path, cfg, w, ids, "float32", portions), want, "float32")
