@@ -15,18 +15,19 @@ static_assert(SEG_K_TILE == BK && SEG_TILE_COLUMNS == BN && SEG_MAX_SPLITS <= SE
 struct TilePos {
     int m0, m_end, n0, group, split;
 };
-// A die's slot (seg_schedule.hpp) -> its tile; returns what seg_find does, and 0 for a place behind the end of a tile list.
+// A die's slot (seg_schedule.hpp) -> its tile; returns what seg_find does.
 __device__ __forceinline__ int seg_tile(const SegGemm &p, const SegWalk &w, int die, int slot, int tile_m, int tile_n, TilePos &t) {
     int tm, tn;
-    if (const int r = seg_find(w, die, slot, tm, tn, t.split); r <= 0) return r;
     if (p.tile_group) { // (scalar loads: a launch does not write its own list, and a vector load would wait for the copies in flight)
         typedef const __attribute__((address_space(4))) int *list_t;
         auto entry = [&](const int *list, int i) { return ((list_t)list)[i]; };
-        if (tm >= entry(p.n_tiles, 0)) return 0;
+        if (const int r = seg_find_listed(w, entry(p.n_tiles, 0), die, slot, tm, tn); r <= 0) return r;
+        t.split = 0;
         t.group = entry(p.tile_group, tm);
         t.m0 = entry(p.tile_row, tm);
         t.m_end = min(t.m0 + tile_m, entry(p.tile_end, tm));
     } else {
+        if (const int r = seg_find(w, die, slot, tm, tn, t.split); r <= 0) return r;
         t.group = 0;
         t.m0 = tm * tile_m;
         t.m_end = min(t.m0 + tile_m, p.M);
@@ -264,7 +265,8 @@ int launch_seg_gemm(moon_ctx *ctx, int dtype, SegGemm p) {
                 if (dev >= 0) attr_set[dev].store(true);
             }
             const int cus = std::max(SEG_DIES, (ctx->cu_count > 0 ? ctx->cu_count : 256) / SEG_DIES * SEG_DIES);
-            const SegWalk w = seg_walk(p.tile_group ? p.max_tiles : (p.M + rows - 1) / rows, (p.N + BN - 1) / BN, p.tile_group, p.kb, p.splits, p.longest_first);
+            const int tiles_n = (p.N + BN - 1) / BN;
+            const SegWalk w = p.tile_group ? seg_walk_listed(p.max_tiles, tiles_n) : seg_walk((p.M + rows - 1) / rows, tiles_n, false, p.kb, p.splits, p.longest_first);
             hipLaunchKernelGGL(kern, dim3((unsigned)seg_workgroups(w, cus)), dim3(DMA_THREADS), lds, ctx->stream, p, w);
             return MOON_OK;
         };
@@ -273,7 +275,7 @@ int launch_seg_gemm(moon_ctx *ctx, int dtype, SegGemm p) {
         else if (mi == 3) MOON_TRY(go(seg_gemm_bf16_kernel<3>, Stream<3>::LDS_BYTES, set3));
         else MOON_TRY(go(seg_gemm_bf16_kernel<2>, Stream<2>::LDS_BYTES, set2));
     } else {
-        const SegWalk w = seg_walk(p.tile_group ? p.max_tiles : (p.M + SEG_TILE_ROWS - 1) / SEG_TILE_ROWS, p.N / 64, true, p.kb, p.splits, p.longest_first);
+        const SegWalk w = p.tile_group ? seg_walk_listed(p.max_tiles, p.N / 64) : seg_walk((p.M + SEG_TILE_ROWS - 1) / SEG_TILE_ROWS, p.N / 64, true, p.kb, p.splits, p.longest_first);
         hipLaunchKernelGGL(seg_gemm_f32_kernel, dim3((unsigned)(SEG_DIES * w.slots)), dim3(256), 0, ctx->stream, p, w);
     }
     MOON_HIP(ctx, hipGetLastError());

@@ -41,9 +41,9 @@ SEG_FN uint32_t seg_div(uint32_t n, const FastDiv &f) {
 // A die's run is walked in blocks of 2 x SEG_BAND tiles: the 32 tiles that a die works on at once then share 512 to 1,024 rows of either
 // operand, where whole columns of tiles (m first) read all of A again for every few columns: 117 against 123 us at 1920 x 16192 x
 // 2048 in 256-row tiles, 130 against 152 in 128-row tiles, weights from HBM.  A column of up to three tiles is a block by itself
-// (blocks would leave a single row of tiles behind: 1 to 2 % of a prompt of 300 rows), and a list of row tiles (grouped rows), each with
-// weights of its own, is walked m first.  So are f32 products, whose multiply-adds bound them and whose workgroups are all in flight at
-// once (width 512, two layers of 1301 rows: 1.35 ms in blocks, 1.32 m first).
+// (blocks would leave a single row of tiles behind: 1 to 2 % of a prompt of 300 rows).  f32 products are walked m first: multiply-adds
+// bound them and their workgroups are all in flight at once (width 512, two layers of 1301 rows: 1.35 ms in blocks, 1.32 m first).
+// A list of row tiles (grouped rows, each with weights of its own) is walked n first, see seg_find_listed.
 constexpr int SEG_BAND = 8, SEG_COLUMN = 3;
 
 struct SegWalk {
@@ -53,7 +53,7 @@ struct SegWalk {
     int per_die;       // longest_first: tiles of one range, otherwise of all of them
     int longest_first; // 1: every die takes its tiles of the longest range, then of the next, ..
     FastDiv by_run;    // longest_first: per_die, otherwise tiles
-    FastDiv by_block;  // columns: tiles_m, otherwise the tiles of a band
+    FastDiv by_block;  // columns: tiles_m, otherwise the tiles of a band; listed row tiles: tiles_n
     FastDiv by_last;   // two rows of tiles of the last band
     int order[8];      // the ranges, longest first
 };
@@ -78,6 +78,13 @@ inline SegWalk seg_walk(int tiles_m, int tiles_n, bool m_first, const int *kb, i
     w.by_block = fast_div((uint32_t)tiles_m * (w.columns ? 1 : SEG_BAND));
     w.by_last = fast_div(2u * (uint32_t)(tiles_n - (tiles_n - 1) / SEG_BAND * SEG_BAND));
     seg_order(kb, splits, w.order);
+    return w;
+}
+// row tiles from a list, up to tiles_m of them: how many there are is known on the device only
+inline SegWalk seg_walk_listed(int tiles_m, int tiles_n) {
+    const int kb[2] = {0, 1};
+    SegWalk w = seg_walk(tiles_m, tiles_n, true, kb, 1, 0);
+    w.by_block = fast_div((uint32_t)tiles_n);
     return w;
 }
 // workgroups that have something to do, when there are `most` (a multiple of SEG_DIES)
@@ -112,6 +119,18 @@ SEG_FN int seg_find(const SegWalk &w, int die, int slot, int &tm, int &tn, int &
     const int two = w.tiles_m - 2 * pair >= 2; // rows of tiles in this pair, less one
     tm = 2 * pair + (rest & two);
     tn = block * SEG_BAND + (rest >> two);
+    return 1;
+}
+
+// The same for a list of which `there` row tiles exist.  The dies share the tiles that exist, and a row tile's columns follow each other: its
+// rows stay in the die's L2 while the weights, read once, pass by.  Dealt as if the list were full, m first, a die's run held 16 % more
+// tiles than the average, and every column of tiles read all rows again: 64 experts of 704, 768 rows of width 2048 with 8 choices, first
+// product 101 -> 86 us, second 51 -> 45 (weights 369 and 184 MB, 72 and 36 us at a copy's rate).
+SEG_FN int seg_find_listed(const SegWalk &w, int there, int die, int slot, int &tm, int &tn) {
+    const int all = there * w.tiles_n, per_die = (all + SEG_DIES - 1) / SEG_DIES, at = die * per_die + slot;
+    if (slot >= per_die || at >= all) return -1;
+    tm = (int)seg_div((uint32_t)at, w.by_block);
+    tn = at - tm * w.tiles_n;
     return 1;
 }
 

@@ -82,6 +82,24 @@ int main() {
         expect(std::fabs(said - longest) <= 1e-9 * longest, "estimate of the walk", M, N, splits, cus);
     }
 
+    // listed row tiles: those that exist once each, and no die with more than an eighth of them, rounded up
+    for (int i = 0; i < 2000; i++) {
+        const int most_tiles = (int)in(1, 640), there = (int)in(0, most_tiles), tiles_n = (int)in(1, 90), most = (int)(i % 4 ? 256 : in(8, 320) / SEG_DIES * SEG_DIES);
+        const SegWalk w = seg_walk_listed(most_tiles, tiles_n);
+        const int grid = seg_workgroups(w, most);
+        std::vector<int> seen((size_t)most_tiles * tiles_n, 0), by_die(SEG_DIES, 0);
+        for (int b = 0; b < grid; b++)
+            for (int round = 0, tm, tn; seg_find_listed(w, there, b % SEG_DIES, seg_slot(0, b / SEG_DIES, grid / SEG_DIES, round), tm, tn) >= 0; round++) {
+                if (tm < 0 || tm >= there || tn < 0 || tn >= tiles_n) failures++;
+                else seen[(size_t)tm * tiles_n + tn]++;
+                by_die[b % SEG_DIES]++;
+            }
+        bool once = true;
+        for (size_t t = 0; t < seen.size(); t++) once = once && seen[t] == (t < (size_t)there * tiles_n);
+        expect(once, "every listed tile once", most_tiles, there, tiles_n, most);
+        expect(*std::max_element(by_die.begin(), by_die.end()) <= (there * tiles_n + SEG_DIES - 1) / SEG_DIES, "dies share the list", most_tiles, there, tiles_n, most);
+    }
+
     // A joined layer's second product: three ranges, the last one of another length.  The height with the smallest estimate does as well
     // as the best height would if the first free workgroup took the next tile, as long as a workgroup has two tiles.
     for (int width : {1024, 2048})
