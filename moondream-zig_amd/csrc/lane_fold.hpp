@@ -12,6 +12,17 @@ __device__ __forceinline__ float half_max(float v) {
     return fmaxf(__builtin_bit_cast(float, r0), __builtin_bit_cast(float, r1));
 }
 
+// Sum over this lane and those below it (no trip through LDS): within rows of 16, then the last lanes of the rows before.
+__device__ __forceinline__ int lane_prefix_sum(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false); // from 1, 2, 4 and 8 lanes below within the row, zero where there is none
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false); // lane 15 of a row to the second and fourth row
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false); // lane 31 to the upper half
+    return v;
+}
+
 // Sum over aligned groups of n lanes (a power of two, the same in every lane); every lane of a group returns it.
 __device__ __forceinline__ float group_sum(float v, int n) {
     if (n >= 2) v += dpp_move<DPP_QUAD_XOR1>(v);
