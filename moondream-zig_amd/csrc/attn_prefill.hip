@@ -13,6 +13,7 @@
 // The scale 1/sqrt(D) multiplies the f32 product (attention.zig:192-194, 487-489), masked scores are -inf, the
 // result is divided by the f32 row sum and rounded once to f16.
 #include "epilogue.hpp"
+#include "lane_fold.hpp"
 #include "tile_copy.hpp"
 
 #include <atomic>
@@ -407,7 +408,7 @@ template <int D> __device__ __forceinline__ int fb_slot(int key) { return D == 7
 template <int D> __device__ __forceinline__ int fb_swizzle(int key) { return D == 72 ? 0 : row64_swizzle(key); }
 
 template <int D>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void flash_attn64_kernel(FaArgs p) {
+__device__ __forceinline__ void flash_rows64(const FaArgs &p) {
     using C = FbCfg<D>;
     constexpr int QS = C::QS;
     extern __shared__ __attribute__((aligned(16))) half_t smem[];
@@ -665,6 +666,215 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
     }
 }
 
+// The same for calls of which 96 rows of a head per workgroup still fit one round, one workgroup to a compute unit (heads of 72): three
+// blocks of 32 rows, each walked by four wavefronts as in flash_attn_kernel, twelve in all; the three with the same tiles share them.  With 64
+// rows per workgroup such a call puts two workgroups on some units and one on others (16 heads, 1458 rows: 368 on 256), and
+// the units with two decide.  Here every SIMD has three wavefronts of six tiles each.  A tile (three wavefronts a SIMD) takes 2.9 us, about the
+// sum of what the vector unit (1.2), the matrix core (1.0) and LDS (1.0) need for it: the barrier per tile keeps the wavefronts in step, so
+// the three hardly overlap.  Calls back to back, 64 rows -> 96: 16 heads, 1100 rows 19.9 -> 15.0 us, 1250 20.6 -> 16.0, 1458 23.2 -> 19.4 (28.7 -> 24.0
+// inside the encoder); 32 heads, 600 rows 14.6 -> 11.1, 729 15.1 -> 12.1; 8 heads, 2916 rows 40.8 -> 33.3.  In two rounds it loses (16 x 2000: 33.0 against 44.4) or
+// gains little (32 x 1250: 32.6 and 30.9), and where 32 rows per workgroup fit one round they are better (16 x 1024: 12.9 and 13.3).
+// Tried and slower: three blocks per wavefront, the accumulators in both halves of the registers (42.5 us at 1458 rows).
+// Each row goes through the same operations in the same order as above: the same bits (tested).
+constexpr int FC_BLOCKS = 3, FC_THREADS = 64 * FC_BLOCKS * FA_WAVES;
+template <int D>
+struct FcCfg {
+    static constexpr int BLOCKS = FC_BLOCKS, Q = 32 * BLOCKS, STAGES = 2;
+    static constexpr int DK = (D + 15) / 16 * 16, KSTEPS = DK / 16, DT = (D + 31) / 32, G = D / 8;
+    static constexpr int TILE = FA_KT * D;                  // halfs of a K or V tile
+    static constexpr int COPIES = FA_KT * G / 64 / BLOCKS;  // copies of 64 granules that a wavefront makes of each
+    static_assert(FA_KT * G == 64 * BLOCKS * COPIES, "whole copies");
+    static constexpr int SD = D + 4;
+    static constexpr size_t MERGE_BYTES = size_t(FA_WAVES) * Q * SD * sizeof(float);
+    static constexpr size_t TILE_BYTES = size_t(FA_WAVES) * STAGES * 2 * TILE * sizeof(half_t);
+    static constexpr size_t ML_OFFSET = TILE_BYTES > MERGE_BYTES ? TILE_BYTES : MERGE_BYTES;
+    static constexpr size_t LDS_BYTES = ML_OFFSET + 2 * FA_WAVES * Q * sizeof(float);
+    static_assert(LDS_BYTES <= 160 * 1024, "LDS");
+};
+
+template <int D>
+__device__ __forceinline__ void flash_rows96(const FaArgs &p) {
+    using C = FcCfg<D>;
+    extern __shared__ __attribute__((aligned(16))) half_t smem[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), block = wave % C::BLOCKS, group = wave / C::BLOCKS;
+    const int col = lane & 31, hf = lane >> 5;
+    // which head and rows: a die takes whole stretches of the (head, block) list
+    int item = (int)(blockIdx.y * gridDim.x + blockIdx.x);
+    const int n_items = (int)(gridDim.x * gridDim.y);
+    if (n_items % 8 == 0) item = (item % 8) * (n_items / 8) + item / 8;
+    const int h = item / (int)gridDim.x, q0 = item % (int)gridDim.x * C::Q;
+    const unsigned lds0 = __builtin_amdgcn_readfirstlane((unsigned)reinterpret_cast<unsigned long>((__attribute__((address_space(3))) const half_t *)smem));
+    int voff[2][C::DT]; // where this lane points the transposing loads, as in flash_rows64
+#pragma unroll
+    for (int j = 0; j < 2; j++)
+#pragma unroll
+        for (int dt = 0; dt < C::DT; dt++) {
+            const int key = (D == 72 ? 0 : 8 * j) + 4 * hf + ((lane & 15) >> 2), c = min(32 * dt + 16 * ((lane >> 4) & 1) + 4 * (lane & 3), D - 4);
+            voff[j][dt] = fb_slot<D>(key) * D + ((c >> 3 ^ fb_swizzle<D>(key)) << 3 | (c & 7)) + (D == 72 ? j * fb_slot<D>(8) * D : 0);
+        }
+    const int row_bytes = (int)p.kv_row_stride * 2, head_bytes = (p.Lkv - 1) * row_bytes + D * 2;
+    const half_t *kh = p.k + size_t(h) * p.kv_head_stride, *vh = p.v + size_t(h) * p.kv_head_stride;
+    int off[C::COPIES]; // this lane's granules of a tile, from its first row (K and V lie alike)
+#pragma unroll
+    for (int i = 0; i < C::COPIES; i++) {
+        const int x = (block * C::COPIES + i) * 64 + lane, key = fb_slot<D>(x / C::G);
+        off[i] = key * row_bytes + (x % C::G ^ fb_swizzle<D>(key)) * 16;
+    }
+    const int n_tiles = (p.Lkv + FA_KT - 1) / FA_KT;
+    const size_t tile_stride = size_t(FA_KT) * p.kv_row_stride;
+    auto copy = [&](int t, int stage) {
+        const unsigned k_lds = lds0 + (group * C::STAGES + stage) * 2 * C::TILE * 2 + block * C::COPIES * 1024;
+        tile_copy(kh + t * tile_stride, head_bytes - t * FA_KT * row_bytes, k_lds, off);
+        tile_copy(vh + t * tile_stride, head_bytes - t * FA_KT * row_bytes, k_lds + C::TILE * 2, off);
+    };
+    int t = group;
+    if (t < n_tiles) copy(t, 0);
+    half8_t qf[C::KSTEPS]; // this lane's query row as the MFMA "B" operand: Q[q0 + 32 block + col][16*s + 8*hf .. +7]
+    {
+        const half_t *qp = p.q + size_t(h) * p.q_head_stride + size_t(min(q0 + 32 * block + col, p.Lq - 1)) * p.q_row_stride;
+#pragma unroll
+        for (int s = 0; s < C::KSTEPS; s++) {
+            const int d = 16 * s + 8 * hf;
+#pragma unroll
+            for (int e = 0; e < 8; e++) qf[s][e] = (half_t)0.0f;
+            if (d < D) qf[s] = *reinterpret_cast<const half8_t *>(qp + d);
+        }
+    }
+    float16_t o[C::DT];
+#pragma unroll
+    for (int dt = 0; dt < C::DT; dt++)
+#pragma unroll
+        for (int v = 0; v < 16; v++) o[dt][v] = 0.0f;
+    float m_run = -INFINITY, l_run = 0.0f; // l_run: this lane's half of the row sum
+    const float c2 = p.scale * 1.4426950408889634f; // > 0: the maximum of the scaled scores is the scaled maximum
+
+    for (int left = (n_tiles + FA_WAVES - 1) / FA_WAVES, stage = 0; left > 0; left--, t += FA_WAVES, stage ^= 1) {
+        tile_landed<0>(); // this wavefront's part of the tile; behind the barrier everybody's, and the tile before has been read by all
+        asm volatile("s_barrier" ::: "memory");
+        if (t + FA_WAVES < n_tiles) copy(t + FA_WAVES, stage ^ 1);
+        if (t >= n_tiles) continue;
+        const half_t *Ks = smem + (group * C::STAGES + stage) * 2 * C::TILE, *Vs = Ks + C::TILE;
+        const int key0 = t * FA_KT;
+        float16_t s[2];
+#pragma unroll
+        for (int kt = 0; kt < 2; kt++) {
+#pragma unroll
+            for (int v = 0; v < 16; v++) s[kt][v] = 0.0f;
+            const half_t *row = Ks + fb_slot<D>(32 * kt + col) * D;
+#pragma unroll
+            for (int st = 0; st < C::KSTEPS; st++) {
+                const bool past = 16 * st + 8 >= D; // the second half of the wavefront has no granule here: zeros
+                const int g = past ? 2 * st : (2 * st + hf) ^ fb_swizzle<D>(col);
+                u32x4 a = *reinterpret_cast<const u32x4 *>(row + g * 8);
+                if (past && hf) a = u32x4{0, 0, 0, 0};
+                s[kt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8_t, a), qf[st], s[kt], 0, 0, 0);
+            }
+        }
+        // s[kt][v] = score of key key0 + 32*kt + 8*(v/4) + 4*hf + v%4; from here on as in flash_rows64
+        if (key0 + FA_KT > p.Lkv) {
+            const int seen = p.Lkv - 1 - key0 - 4 * hf; // keys past this one of the tile are masked
+#pragma unroll
+            for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) s[kt][v] = 32 * kt + 8 * (v >> 2) + (v & 3) > seen ? -INFINITY : s[kt][v];
+        }
+        asm volatile("" : "+v"(s[0]), "+v"(s[1])); // (in these registers on both paths: left alone, the scores are copied on each)
+        float mx = -INFINITY;
+#pragma unroll
+        for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) mx = fmaxf(mx, s[kt][v]);
+        mx = half_max(mx);
+        const float m_new = fmaxf(m_run, mx * c2);
+        float alpha = 1.0f;
+        if (__any(m_new != m_run)) {
+            alpha = __builtin_amdgcn_exp2f(m_run - (m_new == -INFINITY ? 0.0f : m_new));
+            m_run = m_new;
+#pragma unroll
+            for (int dt = 0; dt < C::DT; dt++)
+#pragma unroll
+                for (int v = 0; v < 16; v++)
+                    if (32 * dt + 8 * (v >> 2) < D) o[dt][v] *= alpha;
+        }
+        const float m_use = m_run == -INFINITY ? 0.0f : m_run;
+        float psum = 0.0f;
+#pragma unroll
+        for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) {
+                const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(s[kt][v], c2, -m_use));
+                s[kt][v] = e;
+                psum += e;
+            }
+        l_run = l_run * alpha + psum;
+#pragma unroll
+        for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+            for (int sp = 0; sp < 2; sp++) {
+                half8_t pb;
+#pragma unroll
+                for (int e = 0; e < 8; e++) pb[e] = (half_t)s[kt][8 * sp + e];
+#pragma unroll
+                for (int dt = 0; dt < C::DT; dt++) {
+                    const half4_t lo = fa_read_tr(Vs + voff[0][dt] + (32 * kt + 16 * sp) * D);
+                    const half4_t hi = fa_read_tr(Vs + voff[1][dt] + (32 * kt + 16 * sp) * D);
+                    o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7), pb, o[dt], 0, 0, 0);
+                }
+            }
+    }
+
+    // merge the four groups' results, as in flash_rows64
+    float *so = reinterpret_cast<float *>(smem);                                          // [group][q][SD]
+    float *sm = reinterpret_cast<float *>(reinterpret_cast<char *>(smem) + C::ML_OFFSET); // [group][q]
+    float *sl = sm + FA_WAVES * C::Q;                                                     // [group][q]
+    const int mine = group * C::Q + 32 * block + col;
+    const float l_wave = l_run + __shfl_xor(l_run, 32);
+    if (hf == 0) {
+        sm[mine] = m_run;
+        sl[mine] = l_wave;
+    }
+    __syncthreads(); // every wavefront is done with the tiles, which O takes over, and has published its maximum
+    float m_all = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < FA_WAVES; w++) m_all = fmaxf(m_all, sm[w * C::Q + 32 * block + col]);
+    const float f = m_run == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_run - m_all); // (maxima are in base-2 units)
+#pragma unroll
+    for (int dt = 0; dt < C::DT; dt++)
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            if (32 * dt + 8 * j < D) // o[dt][4*j .. 4*j+3] are rows 32 dt + 8 j + 4 hf .. + 3 of O^T
+                *reinterpret_cast<float4 *>(so + mine * C::SD + 32 * dt + 8 * j + 4 * hf) = float4{o[dt][4 * j] * f, o[dt][4 * j + 1] * f, o[dt][4 * j + 2] * f, o[dt][4 * j + 3] * f};
+    __syncthreads();
+    for (int i = tid; i < C::Q * C::G; i += FC_THREADS) {
+        const int q = i % C::Q, dg = i / C::Q, row = q0 + q;
+        if (row >= p.Lq) continue;
+        float most = -INFINITY, l_all = 0.0f;
+#pragma unroll
+        for (int w = 0; w < FA_WAVES; w++) most = fmaxf(most, sm[w * C::Q + q]);
+#pragma unroll
+        for (int w = 0; w < FA_WAVES; w++) {
+            const float mw = sm[w * C::Q + q];
+            if (mw != -INFINITY) l_all += __builtin_amdgcn_exp2f(mw - most) * sl[w * C::Q + q];
+        }
+        const float inv = 1.0f / l_all;
+        float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < FA_WAVES; w++)
+#pragma unroll
+            for (int e = 0; e < 8; e++) acc[e] += so[(w * C::Q + q) * C::SD + dg * 8 + e];
+        half8_t r;
+#pragma unroll
+        for (int e = 0; e < 8; e++) r[e] = (half_t)(acc[e] * inv);
+        *reinterpret_cast<half8_t *>(p.out + (p.out_merged ? (size_t(row) * p.H + h) * D : (size_t(h) * p.Lq + row) * D) + dg * 8) = r;
+    }
+}
+
+template <int D, bool SHARED>
+__global__ __launch_bounds__(SHARED ? FC_THREADS : 256) __attribute__((amdgpu_waves_per_eu(SHARED ? 3 : 2))) void flash_attn64_kernel(FaArgs p) {
+    if constexpr (SHARED) flash_rows96<D>(p);
+    else flash_rows64<D>(p);
+}
+
 template <int D>
 int launch_flash(moon_ctx *ctx, const FaArgs &p) {
     // Two workgroups fit a compute unit.  Sixty-four rows from where 32 rows would take a second round (rows of all heads > 64 per unit),
@@ -679,19 +889,24 @@ int launch_flash(moon_ctx *ctx, const FaArgs &p) {
     // Well below the line the chip is better filled with 32: 16 heads of 72, 512 rows 7.6 us against 9.5.
     const size_t rows = (size_t)p.Lq * p.H, cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
     const bool two = p.causal_pos >= 0 ? rows >= 112 * cus : rows > (D == 64 ? 96 : 64) * cus;
-    const auto kernel = two ? flash_attn64_kernel<D> : flash_attn_kernel<D>;
-    const size_t lds = two ? FbCfg<D>::LDS_BYTES : FaCfg<D>::LDS_BYTES;
-    const unsigned blocks = two ? (unsigned)((p.Lq + 63) / 64) : (unsigned)((p.Lq + FA_Q - 1) / FA_Q);
-    static std::atomic<bool> attr_set[2][64]; // the opt-in to this much dynamic LDS is per device (and per kernel)
-    const int dev = ctx->device >= 0 && ctx->device < 64 ? ctx->device : -1;
-    if (dev < 0 || !attr_set[two][dev].load()) {
-        MOON_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        if (dev >= 0) attr_set[two][dev].store(true);
-    }
-    hipLaunchKernelGGL(kernel, dim3(blocks, (unsigned)p.H), dim3(256), lds, ctx->stream, p);
-    MOON_HIP(ctx, hipGetLastError());
-    MOON_NOTE_KERNEL(ctx, "flash_attn%s_kernel<%d> %d workgroups", two ? "64" : "", D, (int)blocks * p.H);
-    return MOON_OK;
+    auto go = [&](auto kernel, std::atomic<bool> (&attr_set)[64], int rows_wg, int threads, size_t lds, const char *name) -> int {
+        const unsigned blocks = (unsigned)((p.Lq + rows_wg - 1) / rows_wg);
+        const int dev = ctx->device >= 0 && ctx->device < 64 ? ctx->device : -1; // the opt-in to this much dynamic LDS is per device (and per kernel)
+        if (dev < 0 || !attr_set[dev].load()) {
+            MOON_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+            if (dev >= 0) attr_set[dev].store(true);
+        }
+        hipLaunchKernelGGL(kernel, dim3(blocks, (unsigned)p.H), dim3(threads), lds, ctx->stream, p);
+        MOON_HIP(ctx, hipGetLastError());
+        MOON_NOTE_KERNEL(ctx, "%s %d workgroups", name, (int)blocks * p.H);
+        return MOON_OK;
+    };
+    static std::atomic<bool> set32[64], set64[64], set96[64];
+    if constexpr (D == 72)
+        if (two && p.causal_pos < 0 && size_t(p.Lq + 95) / 96 * p.H <= cus)
+            return go(flash_attn64_kernel<D, true>, set96, FcCfg<D>::Q, FC_THREADS, FcCfg<D>::LDS_BYTES, "flash_attn64_kernel<72, shared>");
+    if (two) return go(flash_attn64_kernel<D, false>, set64, FbCfg<D>::Q, 256, FbCfg<D>::LDS_BYTES, D == 64 ? "flash_attn64_kernel<64>" : "flash_attn64_kernel<72>");
+    return go(flash_attn_kernel<D>, set32, FA_Q, 256, FaCfg<D>::LDS_BYTES, D == 64 ? "flash_attn_kernel<64>" : "flash_attn_kernel<72>");
 }
 
 } // namespace

@@ -208,6 +208,28 @@ def test_values_that_are_not_finite_meet_the_same_rows_in_both_row_blocks(moon, 
     assert np.array_equal(whole, parts, equal_nan=True)
 
 
+# 96 rows per workgroup where they fit one round and 64 are more than 32 rows fit; the last block with 1, 32, 33, 64, 65 and 96 rows
+@pytest.mark.parametrize("H,Lq,Lkv", [(16, 1025, 1025), (16, 1056, 63), (16, 1057, 64), (16, 1440, 65), (16, 1441, 300), (16, 1458, 1458), (16, 1536, 256), (32, 513, 700),
+                                      (32, 768, 1), (8, 2112, 129), (5, 3300, 100)])
+def test_row_blocks_that_share_tiles_give_the_same_bits(moon, ctx, H, Lq, Lkv):
+    """Scores that grow along the keys, some values that are not finite: one call of all rows against calls of 64 (32 per workgroup)."""
+    rng = np.random.default_rng(Lq)
+    q, k, v = (rng.standard_normal((H, n, 72), dtype=np.float32) for n in (Lq, Lkv, Lkv))
+    k *= np.linspace(0.02, 5.0, Lkv, dtype=np.float32)[:, None]
+    q, k, v = (a.astype(np.float16) for a in (q, k, v))
+    q[0, 17], v[1, Lkv // 2, 3], v[2, Lkv - 1, 5] = np.nan, np.inf, np.nan
+    whole = moon.attention.multi_maskless_sdpa(H, 72, q, k, v, ctx=ctx)
+    if compute_units() == 256:
+        assert ctx.last_kernel().startswith("flash_attn64_kernel<72, shared>")
+    parts = []
+    for lo in range(0, Lq, 64):
+        lo = min(lo, Lq - 16)  # (fewer rows take another kernel)
+        parts.append((lo, moon.attention.multi_maskless_sdpa(H, 72, np.ascontiguousarray(q[:, lo:lo + 64]), k, v, ctx=ctx)))
+        assert ctx.last_kernel().startswith("flash_attn_kernel")
+    for lo, part in parts:
+        assert np.array_equal(whole[:, lo:lo + 64], part, equal_nan=True)
+
+
 @pytest.mark.parametrize("D", [64, 72])
 def test_the_last_tile_reads_nothing_that_an_earlier_call_left(moon, O, ctx, D):
     """The 64-row kernel's last tile is cut off in memory; what lies behind the keys in LDS has weight 0 and must be a number."""
