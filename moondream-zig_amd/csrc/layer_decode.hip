@@ -19,6 +19,7 @@
 // kernel without the experts' part, which lets three or four workgroups of the down product share a unit, is 1.4 to 2 % slower (heads of 64).
 // All are bound by HBM: weights are read once with 128-bit non-temporal loads.  No workgroup waits for another.
 #include "delta_math.hpp"
+#include "kernel_args.hpp"
 #include "lane_fold.hpp"
 #include "layer_list.hpp"
 #include "lm_types.hpp"
@@ -68,7 +69,8 @@ __device__ __forceinline__ int pair_row(int i, int half) { return (i >> 5) * 64 
 // NV: 16-byte pieces of x, gamma and beta a thread holds (rows of up to 1024 NV elements, a multiple of 4); 0: any row, from memory.
 // JOIN: x is completed with a joined layer's results first.
 template <class T, int U, int NV, bool JOIN>
-__global__ __launch_bounds__(256) void decode_proj_kernel(DecodeProj p) {
+__global__ __launch_bounds__(256) void decode_proj_kernel(DecodeProj) {
+    const DecodeProj &p = fetch_arguments<DecodeProj>();
     extern __shared__ __attribute__((aligned(16))) char s_raw[]; // h: T [dp], then (NV = 0) x: float [width]
     T *s_h = reinterpret_cast<T *>(s_raw);
     float *s_x = reinterpret_cast<float *>(s_raw + size_t(p.dp) * sizeof(T));
@@ -865,8 +867,19 @@ __global__ __launch_bounds__(256) void decode_out_kernel(DecodeOut p) {
     });
 }
 
+struct MixArgs {
+    DecodeMix p;
+    DecodeOut o;
+    int S, keys_max, n_attn, n_expert;
+};
 template <class T, int NH, int U, bool WHOLE, bool LONG>
-__global__ __launch_bounds__(256) void decode_mix_kernel(DecodeMix p, DecodeOut o, int S, int keys_max, int n_attn, int n_expert) {
+__global__ __launch_bounds__(256) void decode_mix_kernel(MixArgs given) {
+    // (WHOLE has so many that addresses of the compiler's own serve it better, once the lines are there: 793 against 805 us a token at width 2048)
+    const MixArgs &fetched = fetch_arguments<MixArgs>(), &args = WHOLE ? given : fetched;
+    if (WHOLE) __builtin_amdgcn_sched_barrier(0);
+    const DecodeMix &p = args.p;
+    const DecodeOut &o = args.o;
+    const int S = args.S, keys_max = args.keys_max, n_attn = args.n_attn, n_expert = args.n_expert;
     extern __shared__ __attribute__((aligned(16))) char s_mix[]; // (all there is: heads may fill a compute unit's)
     // attention first: it is a chain of dependent steps, the experts' part and the dense activation's product are long streams
     const int i = blockIdx.x, n_hb = mix_head_blocks(p.H / p.G), n_delta = WHOLE ? p.dH : 0;
@@ -887,7 +900,7 @@ template <class T, int NH, bool WHOLE> int mix_launch_as(moon_ctx *ctx, const De
     auto kern = longer ? decode_mix_kernel<T, NH, 4, WHOLE, true> : p.dp / Piece<T>::N > 64 ? decode_mix_kernel<T, NH, 4, WHOLE, false> : decode_mix_kernel<T, NH, 1, WHOLE, false>;
     if (lds > 64 * 1024) MOON_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     const int n_down = o.down ? (o.width + MIX_DOWN_ROWS - 1) / MIX_DOWN_ROWS : 0;
-    hipLaunchKernelGGL(kern, dim3(n_attn + n_expert + (WHOLE ? p.dH : 0) + n_down), dim3(256), lds, ctx->stream, p, o, S, keys_max, n_attn, n_expert);
+    hipLaunchKernelGGL(kern, dim3(n_attn + n_expert + (WHOLE ? p.dH : 0) + n_down), dim3(256), lds, ctx->stream, MixArgs{p, o, S, keys_max, n_attn, n_expert});
     MOON_HIP(ctx, hipGetLastError());
     return MOON_OK;
 }
