@@ -494,3 +494,13 @@ def test_choice_of_experts_where_scores_tie(moon, ctx, tmp_path, experts, top):
         want, _ = R.forward(cfg, w, ids)
         for portions in ([20], [1]):
             assert_close(run(moon, ctx, tmp_path, cfg, w, ids, "float32", portions), want, "float32")
+
+
+@pytest.mark.parametrize("experts,top,rows", [(64, 8, 128), (64, 8, 129), (130, 8, 300), (512, 5, 1999), (8, 8, 2048), (70, 9, 2048)])
+def test_parts_of_the_grouping_by_expert(moon, ctx, tmp_path, experts, top, rows):
+    """One workgroup groups up to 1,024 pairs of a row and an expert, several up to 16,384 and sixteen any more, then in turns: a last part of 8 pairs,
+    16 full parts, two turns.  The oracle is the same sequence in calls of 100 rows, each a workgroup's."""
+    cfg = config(90, 64, [layer(attention(2, 1, 16, 16, 9, 0.25), moe(experts, top, 8))])
+    w, ids = weights(cfg, 3), tokens(rows, 90)
+    whole, apart = (run(moon, ctx, tmp_path / str(n), cfg, w, ids, "float32", [n], 2048) for n in (rows, 100))
+    assert_close(whole, apart, "float32")
