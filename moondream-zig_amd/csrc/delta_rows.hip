@@ -190,7 +190,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void d
 }
 
 // Four wavefronts share the key channels, NT tiles of 16 each; the fifth one finishes the outputs, a chunk behind.  AHEAD: chunks whose
-// operands are requested before they are needed.
+// operands are requested before they are needed.  A chain over the chunks: 0.5 us each (1301 rows of 32 heads of 64: 45 us, 82 chunks; 52 while
+// the first step of every AHEAD waited for all loads and stores under way, see below).  Pairs of chunks, whose second one starts from the first
+// one's U through a product made beforehand, have half the exchanges and took longer (61 us, and 6 for the products).
 constexpr int SCAN_THREADS = 320;
 template <int NT> struct ScanChunk {
     float4_t k[NT], q[NT], r[NT], g[NT], v;
@@ -212,39 +214,46 @@ __global__ __launch_bounds__(SCAN_THREADS) __attribute__((amdgpu_waves_per_eu(1,
     const size_t stride = chunk_floats(p.dimp, p.vdimp);
     const float *src = p.scratch + size_t(h) * chunks * stride;
     if (wave == 4) {
-        float4_t P[AHEAD], u_before, p_before;
+        // A buffer of the chunk's rows, none before the first chunk: rows past its end are not stored.  Without branches around the stores, and with P
+        // where it was loaded to until it is used, no wait for an operand waits for stores or for the operand requested last.
+        const unsigned row_bytes = (unsigned)(p.H * p.vdimp) * 4, ahead = (unsigned)(h * p.vdimp + v0) * 4, off_o = 4 * quad * row_bytes + col * 4;
+        float4_t P[AHEAD], u_before = {0, 0, 0, 0};
         const unsigned off_p = (49 * p.dimp + col * DC + 4 * quad) * 4;
         auto request = [&](int a, int chunk) { P[a] = scan_load(src + min(chunk, chunks - 1) * stride, off_p); };
-        auto finish = [&](int chunk, int half) { // chunk's parts lie in `half`
+        auto finish = [&](int chunk, int half, float4_t p_before) { // chunk's parts lie in `half`
             float4_t o = (s_o[half][0][lane] + s_o[half][1][lane]) + (s_o[half][2][lane] + s_o[half][3][lane]);
 #pragma unroll
             for (int j = 0; j < 4; j++) o = __builtin_amdgcn_mfma_f32_16x16x4f32(p_before[j], u_before[j], o, 0, 0, 0);
+            const auto out = __builtin_amdgcn_make_buffer_rsrc(p.o + (ptrdiff_t)chunk * DC * p.H * p.vdimp + h * p.vdimp + v0, 0,
+                                                               chunk < 0 ? 0u : (unsigned)min(DC, p.n - chunk * DC) * row_bytes - ahead, 0x00020000);
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const int row = chunk * DC + 4 * quad + e;
-                if (row < p.n) p.o[(size_t(row) * p.H + h) * p.vdimp + v0 + col] = o[e];
-            }
+            for (int e = 0; e < 4; e++)
+                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, (float)o[e]), out, off_o + e * row_bytes, 0, 0);
         };
 #pragma unroll
         for (int a = 0; a < AHEAD; a++) request(a, a);
+        __builtin_amdgcn_s_waitcnt(0x0f70); // vmcnt(0): or the first round, without stores in between, would set the number that every round waits for
         auto step = [&](int a, int chunk) {
-            const int half = chunk & 1;
+            const int half = chunk & 1, before = (a + AHEAD - 1) % AHEAD;
             lds_barrier();
             const float4_t u = (s_u[half][0][lane] + s_u[half][1][lane]) + (s_u[half][2][lane] + s_u[half][3][lane]);
-            if (chunk) finish(chunk - 1, half);
+            finish(chunk - 1, half, P[before]);
             u_before = u;
-            p_before = P[a];
-            request(a, chunk + AHEAD);
+            request(before, chunk - 1 + AHEAD);
         };
         int base = 0;
         for (; base + AHEAD <= chunks; base += AHEAD)
 #pragma unroll
             for (int a = 0; a < AHEAD; a++) step(a, base + a);
+        float4_t p_last = P[AHEAD - 1];
 #pragma unroll
         for (int a = 0; a < AHEAD; a++)
-            if (base + a < chunks) step(a, base + a);
+            if (base + a < chunks) {
+                step(a, base + a);
+                p_last = P[a];
+            }
         lds_barrier();
-        finish(chunks - 1, chunks & 1);
+        finish(chunks - 1, chunks & 1, p_last);
         return;
     }
     float *state = p.state + size_t(h) * p.dimp * p.vdimp + v0 + col;
@@ -266,6 +275,9 @@ __global__ __launch_bounds__(SCAN_THREADS) __attribute__((amdgpu_waves_per_eu(1,
         off_g[i] = (3 * DC * p.dimp + 16 * tile + 4 * quad) * 4;
     }
     const unsigned off_v = (49 * p.dimp + (DC + v0 + col) * DC + 4 * quad) * 4;
+    // V' enters with the first wavefront; the others' loads lie past the end of an empty buffer and are zero (a choice between V' and zero made
+    // in registers was moved ahead to the round's start, where it waited for the chunk requested last)
+    const auto values = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(src), 0, wave == 0 ? (unsigned)(chunks * stride * 4) : 0u, 0x00020000);
     auto request = [&](ScanChunk<NT> &b, int chunk) {
         const float *at = src + min(chunk, chunks - 1) * stride;
 #pragma unroll
@@ -275,14 +287,14 @@ __global__ __launch_bounds__(SCAN_THREADS) __attribute__((amdgpu_waves_per_eu(1,
             b.r[i] = scan_load(at, off_r[i]);
             b.g[i] = scan_load(at, off_g[i]);
         }
-        b.v = scan_load(at, off_v);
+        b.v = __builtin_bit_cast(float4_t, __builtin_amdgcn_raw_buffer_load_b128(values, off_v + (unsigned)(min(chunk, chunks - 1) * stride * 4), 0, 0));
     };
 #pragma unroll
     for (int a = 0; a < AHEAD; a++) request(ring[a], a);
     float4_t o = {0, 0, 0, 0};
     auto step = [&](ScanChunk<NT> &b, int chunk) {
         const int half = chunk & 1;
-        float4_t u = wave == 0 ? b.v : float4_t{0, 0, 0, 0};
+        float4_t u = b.v;
 #pragma unroll
         for (int i = 0; i < NT; i++) // (a tile past the end is another wavefront's, with a state of zero here)
 #pragma unroll

@@ -513,3 +513,13 @@ def test_attention_over_shared_tiles(moon, ctx, kv_heads, window, pool, calls):
         got[dtype] = m.hidden_f32(calls[-1])
         m.close()
     assert_close(got["bfloat16"], got["float32"], "bfloat16")
+
+
+@pytest.mark.parametrize("dim,rows", [(64, 1), (64, 112), (64, 113), (64, 128), (64, 129), (64, 300), (128, 63), (128, 65), (128, 144), (256, 32), (256, 33), (256, 50), (512, 16),
+                                      (512, 17), (512, 50)])
+def test_chunks_around_the_delta_rules_rounds(moon, ctx, tmp_path, dim, rows):
+    """The scan takes chunks of 16 tokens in rounds of 8, 4, 2 or 1 by head size: whole rounds, one chunk less and more, a last chunk of one token, and
+    two tokens behind them for the state that is left."""
+    cfg = config(90, 64, [parallel(softmax_mixer(2, 1, 16, 16, 9, 0.6, 4), delta(2, 1, dim, 32, 3))])
+    w, ids = weights(cfg, 3), tokens(rows + 2, 90)
+    assert_close(run(moon, ctx, tmp_path, cfg, w, ids, "float32", [rows, 1]), G.forward(cfg, w, ids)[0], "float32")
