@@ -20,6 +20,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <type_traits>
 
 namespace {
 
@@ -354,17 +355,25 @@ constexpr int WS_PAIRED = 64; // workgroups of a die that are there at once: two
 struct WsCfg {
     static constexpr int D = 64, KSTEPS = D / 16, DT = D / 32, G = D / 8, STAGES = 2, GROUPS = 2;
     static constexpr int TILE = WA_KT * D, COPIES = WA_KT * G / 64 / WA_WAVES; // elements of a K or V tile, copies of each per wavefront
-    static constexpr size_t LDS_BYTES = size_t(GROUPS) * STAGES * 2 * TILE * 2;
+    static constexpr size_t TILE_BYTES = size_t(GROUPS) * STAGES * 2 * TILE * 2, LDS_BYTES = TILE_BYTES + GROUPS * WA_WAVES * sizeof(int);
 };
 __host__ __device__ __forceinline__ int ws_heads(int per_group) { return per_group % 4 == 0 ? 4 : per_group % 2 == 0 ? 2 : 1; } // heads per workgroup
 __host__ __device__ __forceinline__ int ws_rows(int per_group) { return WA_Q * WA_WAVES / ws_heads(per_group); }                 // rows per workgroup
 
-template <bool POOL>
+// The lane's number, asked for anew: a value that the compiler does not keep in a register (or in memory) across what came before
+__device__ __forceinline__ int lane_again() {
+    int lane;
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(lane));
+    return lane;
+}
+
+// APART: wavefronts of one workgroup have different rows (fewer than four heads read the same keys)
+template <bool POOL, bool APART>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void window_attn_shared_kernel(WindowAttn p) {
     using C = WsCfg;
     constexpr int D = C::D, ROW = D * 2; // ROW: bytes of a cache row
     extern __shared__ __attribute__((aligned(16))) bf16_t wa_lds[];
-    const int tid = threadIdx.x, lane = tid & 63, kg = __builtin_amdgcn_readfirstlane(tid >> 8), wave = __builtin_amdgcn_readfirstlane(tid >> 6 & 3), col = lane & 31, hf = lane >> 5;
+    const int tid = threadIdx.x, kg = __builtin_amdgcn_readfirstlane(tid >> 8), wave = __builtin_amdgcn_readfirstlane(tid >> 6 & 3);
     const int per = p.H / p.G, nh = ws_heads(per), rows = ws_rows(per), n_qb = (p.n + rows - 1) / rows, n_hb = p.H / nh;
     // which heads and rows: a die takes whole stretches of the (heads, block) list, late blocks first
     int item = blockIdx.x;
@@ -380,160 +389,181 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void w
     qb = n_qb - 1 - qb;
     const int h = hb * nh + wave % nh, g = h / per, wg_row0 = qb * rows, row0 = wg_row0 + wave / nh * WA_Q;
     const int wg_first = p.pos0 + wg_row0, last_pos = p.pos0 + min(wg_row0 + rows, p.n) - 1; // positions of the workgroup's first and last row
-    const int first_pos = p.pos0 + row0, pos = first_pos + col;                               // of the wavefront's first row and this lane's
+    const int first_pos = p.pos0 + row0;                                                      // and of the wavefront's first row
     const int lo_key = p.window ? max(0, wg_first - p.window + 1) : 0;
     const int seen = POOL ? blocks_seen(last_pos, p.window, p.pool) : 0, t_blocks = (seen + WA_KT - 1) / WA_KT;
     const int t_begin = POOL ? lo_key / WA_KT - t_blocks : lo_key / WA_KT, t_end = last_pos / WA_KT + 1;
     const int t_window = POOL ? lo_key / WA_KT : 0;
+    const int lo_mine = p.window ? max(0, first_pos - p.window + 1) : 0, seen_mine = POOL ? blocks_seen(first_pos + WA_Q - 1, p.window, p.pool) : 0; // of the wavefront's 32 rows
     const size_t head_rows = size_t(g) * p.cap * ROW, head_blocks = POOL ? size_t(g) * p.blocks * ROW : 0;
     const char *ck = reinterpret_cast<const char *>(p.ck) + head_rows, *cv = reinterpret_cast<const char *>(p.cv) + head_rows;
     const char *pk = reinterpret_cast<const char *>(p.pk) + head_blocks, *pv = reinterpret_cast<const char *>(p.pv) + head_blocks;
     const unsigned lds0 = __builtin_amdgcn_readfirstlane((unsigned)reinterpret_cast<unsigned long>((__attribute__((address_space(3))) const bf16_t *)wa_lds));
-    int off[C::COPIES]; // this lane's granules of a tile, from its first row (K and V lie alike)
-#pragma unroll
-    for (int i = 0; i < C::COPIES; i++) {
-        const int row = (wave * C::COPIES + i) * 8 + (lane >> 3);
-        off[i] = row * ROW + ((lane & 7) ^ row64_swizzle(row)) * 16;
-    }
-    // This wavefront's part of tile t to stage t % STAGES; rows that must not be read are offsets past the end, which bring zeros.
-    constexpr int NOWHERE = 0x7fffffff;
-    auto copy = [&](int t, int stage) {
-        const unsigned k_lds = lds0 + (kg * C::STAGES + stage) * 2 * C::TILE * 2 + wave * C::COPIES * 1024, v_lds = k_lds + C::TILE * 2;
-        const bool blocks = POOL && t < t_window;
-        const int key0 = blocks ? (t - t_begin) * WA_KT : t * WA_KT, lo = blocks ? 0 : lo_key, hi = blocks ? seen - 1 : last_pos, rows = blocks ? p.blocks : p.cap;
-        const int slot0 = key0 < rows ? key0 : key0 % rows;
-        const bool whole = key0 >= lo && key0 + WA_KT - 1 <= hi && slot0 + WA_KT <= rows; // in one piece
-        int offs[C::COPIES];
-#pragma unroll
-        for (int i = 0; i < C::COPIES; i++) {
-            const int row = (wave * C::COPIES + i) * 8 + (lane >> 3), key = key0 + row;
-            offs[i] = off[i] + slot0 * ROW;
-            if (whole) continue;
-            if (slot0 + row >= rows) offs[i] -= rows * ROW; // (a cache that wraps has more rows than a tile)
-            if (key < lo || key > hi) offs[i] = NOWHERE;
-        }
-        tile_copy(blocks ? pk : ck, rows * ROW, k_lds, offs);
-        tile_copy(blocks ? pv : cv, rows * ROW, v_lds, offs);
-    };
-    int t = t_begin + kg;
-    if (t < t_end) copy(t, 0);
-    const float scale = p.temp ? p.scale * p.temp[h] : p.scale;
-    bf16x8_t qf[C::KSTEPS]; // the MFMA "B" operand: Q[row0 + col][16 s + 8 hf .. + 7]
-    {
-        const bf16_t *q = reinterpret_cast<const bf16_t *>(p.q) + size_t(min(row0 + col, p.n - 1)) * p.ldq + h * D;
-#pragma unroll
-        for (int s = 0; s < C::KSTEPS; s++) {
-            lm_u32x4 v = *reinterpret_cast<const lm_u32x4 *>(q + 16 * s + 8 * hf);
-            if (scale < 0.0f) v ^= 0x80008000u; // (as in window_attn_kernel)
-            qf[s] = __builtin_bit_cast(bf16x8_t, v);
-        }
-    }
-    int voff[2][C::DT]; // where this lane points the transposing loads: keys 4 hf + (lane % 16) / 4 (+ 8), columns 32 dt + 16 ((lane / 16) % 2) + 4 (lane % 4)
-#pragma unroll
-    for (int j = 0; j < 2; j++)
-#pragma unroll
-        for (int dt = 0; dt < C::DT; dt++) {
-            const int key = 8 * j + 4 * hf + ((lane & 15) >> 2), c = 32 * dt + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
-            voff[j][dt] = key * D + ((c >> 3 ^ row64_swizzle(key)) << 3 | (c & 7));
-        }
-    __builtin_amdgcn_s_waitcnt(0xf70); // vmcnt(0): the query rows have arrived (else the compiler waits for them, and every copy, in each round)
-
-    float16_t o[C::DT];
-    float m_run = -INFINITY, l_run = 0.0f;
-#pragma unroll
-    for (int dt = 0; dt < C::DT; dt++)
-#pragma unroll
-        for (int v = 0; v < 16; v++) o[dt][v] = 0.0f;
-    const int mine0 = POOL ? blocks_seen(pos, p.window, p.pool) - 1 - 4 * hf : 0; // the last block that this lane's row sees, from its first one
     constexpr float LOG2E = 1.4426950408889634f;
+    const float scale = p.temp ? p.scale * p.temp[h] : p.scale;
     const float c2 = fmaxf(fabsf(scale) * LOG2E, 1e-37f);
     const float sink = p.sink ? p.sink[h] * LOG2E : -INFINITY;
+    float16_t o[C::DT];
+    float m_run, l_run;
 
-    for (int left = (t_end - t_begin + C::GROUPS - 1) / C::GROUPS, stage = 0; left > 0; left--, t += C::GROUPS, stage ^= 1) {
-        const int key0 = t * WA_KT;
-        tile_landed<0>(); // this wavefront's part of the tile; behind the barrier everybody's, and the tile before has been read by all
-        asm volatile("s_barrier" ::: "memory");
-        if (t + C::GROUPS < t_end) copy(t + C::GROUPS, stage ^ 1);
-        if (t >= t_end) continue;
-        const bool blocks = POOL && t < t_window;
-        if (!blocks && (key0 > first_pos + WA_Q - 1 || (p.window && key0 + WA_KT <= first_pos - p.window + 1))) continue; // no row sees any of it
-        const bf16_t *Ks = wa_lds + (kg * C::STAGES + stage) * 2 * C::TILE, *Vs = Ks + C::TILE;
-        float16_t s[2];
-        bf16x8_t a[2][C::KSTEPS];
+    // STRICT: values that none of the wavefront's 32 rows read are zero.  A tile may have some for the workgroup's other rows, whose weights here are
+    // zero; zero times infinity is not.
+    auto walk = [&](auto strict, int lane) {
+        constexpr bool STRICT = decltype(strict)::value;
+        const int col = lane & 31, hf = lane >> 5, pos = first_pos + col; // pos: this lane's query
+        int off[C::COPIES]; // this lane's granules of a tile, from its first row (K and V lie alike)
 #pragma unroll
-        for (int kt = 0; kt < 2; kt++)
+        for (int i = 0; i < C::COPIES; i++) {
+            const int row = (wave * C::COPIES + i) * 8 + (lane >> 3);
+            off[i] = row * ROW + ((lane & 7) ^ row64_swizzle(row)) * 16;
+        }
+        // This wavefront's part of tile t to stage t % STAGES; rows that must not be read are offsets past the end, which bring zeros.
+        constexpr int NOWHERE = 0x7fffffff;
+        auto copy = [&](int t, int stage) {
+            const unsigned k_lds = lds0 + (kg * C::STAGES + stage) * 2 * C::TILE * 2 + wave * C::COPIES * 1024, v_lds = k_lds + C::TILE * 2;
+            const bool blocks = POOL && t < t_window;
+            const int key0 = blocks ? (t - t_begin) * WA_KT : t * WA_KT, lo = blocks ? 0 : lo_key, hi = blocks ? seen - 1 : last_pos, rows = blocks ? p.blocks : p.cap;
+            const int slot0 = key0 < rows ? key0 : key0 % rows;
+            const bool whole = key0 >= lo && key0 + WA_KT - 1 <= hi && slot0 + WA_KT <= rows; // in one piece
+            int offs[C::COPIES];
 #pragma unroll
-            for (int st = 0; st < C::KSTEPS; st++) a[kt][st] = *reinterpret_cast<const bf16x8_t *>(Ks + (32 * kt + col) * D + ((2 * st + hf) ^ row64_swizzle(col)) * 8);
+            for (int i = 0; i < C::COPIES; i++) {
+                const int row = (wave * C::COPIES + i) * 8 + (lane >> 3), key = key0 + row;
+                offs[i] = off[i] + slot0 * ROW;
+                if (whole) continue;
+                if (slot0 + row >= rows) offs[i] -= rows * ROW; // (a cache that wraps has more rows than a tile)
+                if (key < lo || key > hi) offs[i] = NOWHERE;
+            }
+            tile_copy(blocks ? pk : ck, rows * ROW, k_lds, offs);
+            tile_copy(blocks ? pv : cv, rows * ROW, v_lds, offs);
+        };
+        if (t_begin + kg < t_end) copy(t_begin + kg, 0);
+        bf16x8_t qf[C::KSTEPS]; // the MFMA "B" operand: Q[row0 + col][16 s + 8 hf .. + 7]
+        {
+            const bf16_t *q = reinterpret_cast<const bf16_t *>(p.q) + size_t(min(row0 + col, p.n - 1)) * p.ldq + h * D;
 #pragma unroll
-        for (int kt = 0; kt < 2; kt++)
+            for (int s = 0; s < C::KSTEPS; s++) {
+                lm_u32x4 v = *reinterpret_cast<const lm_u32x4 *>(q + 16 * s + 8 * hf);
+                if (scale < 0.0f) v ^= 0x80008000u; // (as in window_attn_kernel)
+                qf[s] = __builtin_bit_cast(bf16x8_t, v);
+            }
+        }
+        int voff[2][C::DT]; // where this lane points the transposing loads: keys 4 hf + (lane % 16) / 4 (+ 8), columns 32 dt + 16 ((lane / 16) % 2) + 4 (lane % 4)
 #pragma unroll
-            for (int v = 0; v < 16; v++) s[kt][v] = 0.0f;
+        for (int j = 0; j < 2; j++)
 #pragma unroll
-        for (int st = 0; st < C::KSTEPS; st++)
+            for (int dt = 0; dt < C::DT; dt++) {
+                const int key = 8 * j + 4 * hf + ((lane & 15) >> 2), c = 32 * dt + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+                voff[j][dt] = key * D + ((c >> 3 ^ row64_swizzle(key)) << 3 | (c & 7));
+            }
+        __builtin_amdgcn_s_waitcnt(0xf70); // vmcnt(0): the query rows have arrived (else the compiler waits for them, and every copy, in each round)
+        const int mine0 = POOL ? blocks_seen(pos, p.window, p.pool) - 1 - 4 * hf : 0; // the last block that this lane's row sees, from its first one
+        m_run = -INFINITY;
+        l_run = 0.0f;
 #pragma unroll
-            for (int kt = 0; kt < 2; kt++) s[kt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[kt][st], qf[st], s[kt], 0, 0, 0);
-        // s[kt][v]: key key0 + 32 kt + 8 (v / 4) + 4 hf + v % 4 against this lane's query
-        if (blocks || key0 + WA_KT - 1 > first_pos || (p.window && key0 <= first_pos + WA_Q - 1 - p.window)) { // some row does not see the whole tile
-            const int age0 = blocks ? mine0 - (t - t_begin) * WA_KT : pos - key0 - 4 * hf; // how far back this lane's first key (block) is
-            const unsigned ages = !blocks && p.window ? (unsigned)p.window : 0x7fffffffu;
+        for (int dt = 0; dt < C::DT; dt++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) o[dt][v] = 0.0f;
+        for (int left = (t_end - t_begin + C::GROUPS - 1) / C::GROUPS, stage = 0, t = t_begin + kg; left > 0; left--, t += C::GROUPS, stage ^= 1) {
+            const int key0 = t * WA_KT;
+            tile_landed<0>(); // this wavefront's part of the tile; behind the barrier everybody's, and the tile before has been read by all
+            asm volatile("s_barrier" ::: "memory");
+            if (t + C::GROUPS < t_end) copy(t + C::GROUPS, stage ^ 1);
+            if (t >= t_end) continue;
+            const bool blocks = POOL && t < t_window;
+            if (!blocks && (key0 > first_pos + WA_Q - 1 || (p.window && key0 + WA_KT <= first_pos - p.window + 1))) continue; // no row sees any of it
+            const bf16_t *Ks = wa_lds + (kg * C::STAGES + stage) * 2 * C::TILE, *Vs = Ks + C::TILE;
+            float16_t s[2];
+            bf16x8_t a[2][C::KSTEPS];
 #pragma unroll
             for (int kt = 0; kt < 2; kt++)
 #pragma unroll
-                for (int v = 0; v < 16; v++) // (a key ahead of the query wraps to a large age)
-                    s[kt][v] = (unsigned)(age0 - (32 * kt + 8 * (v >> 2) + (v & 3))) < ages ? s[kt][v] : -INFINITY;
-        }
-        asm volatile("" : "+v"(s[0]), "+v"(s[1])); // (in these registers on both paths: left alone, the scores are copied on each)
-        float mx = -INFINITY;
+                for (int st = 0; st < C::KSTEPS; st++) a[kt][st] = *reinterpret_cast<const bf16x8_t *>(Ks + (32 * kt + col) * D + ((2 * st + hf) ^ row64_swizzle(col)) * 8);
 #pragma unroll
-        for (int kt = 0; kt < 2; kt++)
+            for (int kt = 0; kt < 2; kt++)
 #pragma unroll
-            for (int v = 0; v < 16; v++) mx = fmaxf(mx, s[kt][v]);
-        mx = half_max(mx);
-        const float m_new = fmaxf(m_run, mx * c2), m_use = m_new == -INFINITY ? 0.0f : m_new;
-        float alpha = 1.0f;
-        if (__any(m_new != m_run)) {
-            alpha = __builtin_amdgcn_exp2f(m_run - m_use);
-            m_run = m_new;
+                for (int v = 0; v < 16; v++) s[kt][v] = 0.0f;
 #pragma unroll
-            for (int dt = 0; dt < C::DT; dt++)
+            for (int st = 0; st < C::KSTEPS; st++)
 #pragma unroll
-                for (int v = 0; v < 16; v++) o[dt][v] *= alpha;
-        }
-        float psum = 0.0f;
+                for (int kt = 0; kt < 2; kt++) s[kt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[kt][st], qf[st], s[kt], 0, 0, 0);
+            // s[kt][v]: key key0 + 32 kt + 8 (v / 4) + 4 hf + v % 4 against this lane's query
+            if (blocks || key0 + WA_KT - 1 > first_pos || (p.window && key0 <= first_pos + WA_Q - 1 - p.window)) { // some row does not see the whole tile
+                const int age0 = blocks ? mine0 - (t - t_begin) * WA_KT : pos - key0 - 4 * hf; // how far back this lane's first key (block) is
+                const unsigned ages = !blocks && p.window ? (unsigned)p.window : 0x7fffffffu;
 #pragma unroll
-        for (int kt = 0; kt < 2; kt++)
+                for (int kt = 0; kt < 2; kt++)
 #pragma unroll
-            for (int v = 0; v < 16; v++) {
-                const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(s[kt][v], c2, -m_use));
-                s[kt][v] = e;
-                psum += e;
+                    for (int v = 0; v < 16; v++) // (a key ahead of the query wraps to a large age)
+                        s[kt][v] = (unsigned)(age0 - (32 * kt + 8 * (v >> 2) + (v & 3))) < ages ? s[kt][v] : -INFINITY;
             }
-        l_run = l_run * alpha + psum;
-        // contraction step (kt, sp) uses the keys a lane holds in s[kt][8 sp .. 8 sp + 7], as in window_attn_kernel
+            asm volatile("" : "+v"(s[0]), "+v"(s[1])); // (in these registers on both paths: left alone, the scores are copied on each)
+            float mx = -INFINITY;
 #pragma unroll
-        for (int kt = 0; kt < 2; kt++)
+            for (int kt = 0; kt < 2; kt++)
 #pragma unroll
-            for (int sp = 0; sp < 2; sp++) {
-                lm_u32x4 hi_bits, lo_bits;
+                for (int v = 0; v < 16; v++) mx = fmaxf(mx, s[kt][v]);
+            mx = half_max(mx);
+            const float m_new = fmaxf(m_run, mx * c2), m_use = m_new == -INFINITY ? 0.0f : m_new;
+            float alpha = 1.0f;
+            if (__any(m_new != m_run)) {
+                alpha = __builtin_amdgcn_exp2f(m_run - m_use);
+                m_run = m_new;
 #pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    const uint2 pair = split_pair(s[kt][8 * sp + 2 * e], s[kt][8 * sp + 2 * e + 1]);
-                    hi_bits[e] = pair.x;
-                    lo_bits[e] = pair.y;
-                }
-                const bf16x8_t hi = __builtin_bit_cast(bf16x8_t, hi_bits), lo = __builtin_bit_cast(bf16x8_t, lo_bits);
-                bf16x8_t v[C::DT];
+                for (int dt = 0; dt < C::DT; dt++)
 #pragma unroll
-                for (int dt = 0; dt < C::DT; dt++) {
-                    const wa_short4_t a0 = wa_read_tr(Vs + voff[0][dt] + (32 * kt + 16 * sp) * D), a1 = wa_read_tr(Vs + voff[1][dt] + (32 * kt + 16 * sp) * D);
-                    v[dt] = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7));
-                }
-#pragma unroll
-                for (int dt = 0; dt < C::DT; dt++) o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v[dt], lo, o[dt], 0, 0, 0);
-#pragma unroll
-                for (int dt = 0; dt < C::DT; dt++) o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v[dt], hi, o[dt], 0, 0, 0);
+                    for (int v = 0; v < 16; v++) o[dt][v] *= alpha;
             }
-    }
+            float psum = 0.0f;
+#pragma unroll
+            for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) {
+                    const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(s[kt][v], c2, -m_use));
+                    s[kt][v] = e;
+                    psum += e;
+                }
+            l_run = l_run * alpha + psum;
+            // contraction step (kt, sp) uses the keys a lane holds in s[kt][8 sp .. 8 sp + 7], as in window_attn_kernel
+#pragma unroll
+            for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+                for (int sp = 0; sp < 2; sp++) {
+                    lm_u32x4 hi_bits, lo_bits;
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        const uint2 pair = split_pair(s[kt][8 * sp + 2 * e], s[kt][8 * sp + 2 * e + 1]);
+                        hi_bits[e] = pair.x;
+                        lo_bits[e] = pair.y;
+                    }
+                    const bf16x8_t hi = __builtin_bit_cast(bf16x8_t, hi_bits), lo = __builtin_bit_cast(bf16x8_t, lo_bits);
+                    bf16x8_t v[C::DT];
+#pragma unroll
+                    for (int dt = 0; dt < C::DT; dt++) {
+                        const wa_short4_t a0 = wa_read_tr(Vs + voff[0][dt] + (32 * kt + 16 * sp) * D), a1 = wa_read_tr(Vs + voff[1][dt] + (32 * kt + 16 * sp) * D);
+                        v[dt] = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7));
+                    }
+                    if (STRICT) {
+                        const int from = (blocks ? 0 : lo_mine - key0) - 4 * hf; // the first value that the 32 rows read, counted from this lane's first
+                        const int count = blocks ? max(0, seen_mine - (t - t_begin) * WA_KT) : first_pos + WA_Q - lo_mine; // and how many there are
+                        lm_u32x4 read;
+#pragma unroll
+                        for (int e = 0; e < 4; e++) {
+                            const int key = 32 * kt + 16 * sp + 8 * (e >> 1) + 2 * (e & 1) - from;
+                            read[e] = ((unsigned)key < (unsigned)count ? 0xffffu : 0u) | ((unsigned)(key + 1) < (unsigned)count ? 0xffff0000u : 0u);
+                        }
+#pragma unroll
+                        for (int dt = 0; dt < C::DT; dt++) v[dt] = __builtin_bit_cast(bf16x8_t, __builtin_bit_cast(lm_u32x4, v[dt]) & read);
+                    }
+#pragma unroll
+                    for (int dt = 0; dt < C::DT; dt++) o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v[dt], lo, o[dt], 0, 0, 0);
+#pragma unroll
+                    for (int dt = 0; dt < C::DT; dt++) o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v[dt], hi, o[dt], 0, 0, 0);
+                }
+        }
+    };
+    walk(std::false_type(), tid & 63);
+    const int lane = lane_again(), col = lane & 31, hf = lane >> 5;
 
     // o[dt][4 j + e] is element 32 dt + 8 j + 4 hf + e of this lane's row.  The second group hands its result over, [wave][register][lane].
     float *so = reinterpret_cast<float *>(wa_lds) + wave * (C::DT * 16 + 2) * 64 + lane;
@@ -541,19 +571,40 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void w
     // what the results still need, requested before the merge: this lane's gate granules 4 dt + 2 i + hf, cos and sin of two pairs each
     const int row = row0 + col, at_row = min(row, p.n - 1);
     const bf16_t *gate = p.gate ? reinterpret_cast<const bf16_t *>(p.gate) + size_t(at_row) * p.ldq + h * D : nullptr;
-    bf16x8_t gz[C::DT][2] = {};
-    if (kg == 0 && gate)
+    bf16x8_t gz[C::DT][2];
+    float4_t turn[4][2];
+    auto request = [&] {
 #pragma unroll
         for (int dt = 0; dt < C::DT; dt++)
 #pragma unroll
-            for (int i = 0; i < 2; i++) gz[dt][i] = *reinterpret_cast<const bf16x8_t *>(gate + (4 * dt + 2 * i + hf) * 8);
-    float4_t turn[4][2];
-    if (kg == 0 && p.rotv) // (over all of the head: the other one of a pair is 32 elements away)
+            for (int i = 0; i < 2; i++) gz[dt][i] = kg == 0 && gate ? *reinterpret_cast<const bf16x8_t *>(gate + (4 * dt + 2 * i + hf) * 8) : bf16x8_t{};
+        if (kg == 0 && p.rotv) // (over all of the head: the other one of a pair is 32 elements away)
 #pragma unroll
-        for (int j = 0; j < 4; j++)
+            for (int j = 0; j < 4; j++)
 #pragma unroll
-            for (int e = 0; e < 2; e++) turn[j][e] = reinterpret_cast<const float4_t *>(p.rotv + size_t(p.pos0 + at_row) * (D / 2))[4 * j + 2 * hf + e];
+                for (int e = 0; e < 2; e++) turn[j][e] = reinterpret_cast<const float4_t *>(p.rotv + size_t(p.pos0 + at_row) * (D / 2))[4 * j + 2 * hf + e];
+    };
+    request();
+    // Where wavefronts have different rows and a result is not finite, once more: it may be a value that only the others read.  (Zeros put in place of
+    // such values in every tile that may have some, by a choice per step, took 10 to 27 % more; this check 0 to 0.4 us: 32 heads with keys of their own,
+    // window 1024, 768 rows 19.9 -> 20.3 us, 1920 rows 38.4 -> 37.9.)
+    int *redo = reinterpret_cast<int *>(reinterpret_cast<char *>(wa_lds) + C::TILE_BYTES);
+    if (APART) {
+        float zero[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int dt = 0; dt < C::DT; dt++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) zero[v & 3] = __builtin_fmaf(o[dt][v], 0.0f, zero[v & 3]);
+        const bool again = __any((zero[0] + zero[1]) + (zero[2] + zero[3]) != 0.0f);
+        if (lane == 0) redo[kg * WA_WAVES + wave] = again;
+    }
     __syncthreads(); // every wavefront is done with the tiles
+    if (APART && __builtin_expect(__any(redo[lane % (C::GROUPS * WA_WAVES)]), 0)) { // (its code behind everything else: in between it costs 1 us of instruction fetches)
+        walk(std::true_type(), lane_again()); // (nothing of the first walk is kept for this one)
+        l_run += __shfl_xor(l_run, 32);
+        request();
+        __syncthreads();
+    }
     if (kg == 1) {
 #pragma unroll
         for (int dt = 0; dt < C::DT; dt++)
@@ -692,9 +743,11 @@ template <class Kernel> int launch_as(moon_ctx *ctx, const WindowAttn &p, Kernel
 template <int P, bool POOL> int launch_mfma_as(moon_ctx *ctx, const WindowAttn &p) {
     if constexpr (P == 64)
         if (shares_tiles(ctx, p)) {
-            static std::atomic<bool> attr_set[64];
+            static std::atomic<bool> attr_set[64], attr_apart[64];
             const int per = p.H / p.G, rows = ws_rows(per);
-            MOON_TRY(launch_as(ctx, p, window_attn_shared_kernel<POOL>, attr_set, WsCfg::LDS_BYTES, (p.n + rows - 1) / rows * (p.H / ws_heads(per)), 512));
+            const int workgroups = (p.n + rows - 1) / rows * (p.H / ws_heads(per));
+            if (rows > WA_Q) MOON_TRY(launch_as(ctx, p, window_attn_shared_kernel<POOL, true>, attr_apart, WsCfg::LDS_BYTES, workgroups, 512));
+            else MOON_TRY(launch_as(ctx, p, window_attn_shared_kernel<POOL, false>, attr_set, WsCfg::LDS_BYTES, workgroups, 512));
             MOON_NOTE_KERNEL(ctx, "window_attn_shared_kernel %d rows of %d heads", rows, ws_heads(per));
             return MOON_OK;
         }

@@ -515,6 +515,31 @@ def test_attention_over_shared_tiles(moon, ctx, kv_heads, window, pool, calls):
     assert_close(got["bfloat16"], got["float32"], "bfloat16")
 
 
+@pytest.mark.parametrize("kv_heads", [16, 32, 64])
+@pytest.mark.parametrize("window,pool", [(30, 16), (30, 1), (100, 5)])
+def test_a_row_that_is_not_finite_reaches_no_block_of_rows_before_it(moon, ctx, tmp_path, kv_heads, window, pool):
+    """Heads that share key tiles, windows shorter than a workgroup's rows, so that its last rows see blocks of its first ones: a token of NaN leaves the
+    bits of all blocks of 32 rows before it (the delta rule's state carries it to every row behind it)."""
+    rows, spoiled = 500, 127
+    cfg = config(128, 64, [parallel(softmax_mixer(64, kv_heads, 64, 64, window, 0.25, pool), delta(1, 1, 64, 64, 2))])
+    w, ids = weights(cfg, 3), tokens(rows, 127)
+    w["embed"][spoiled] = np.nan
+    m = opened(moon, ctx, write_folder(tmp_path / "run", cfg, w), "bfloat16", 2048)
+
+    def stream(at):
+        m.reset()
+        m.forward(np.where(np.arange(rows) == at, spoiled, ids).astype(np.uint32))
+        return m.hidden_f32(rows)
+
+    clean = stream(-1)
+    assert np.isfinite(clean).all()
+    for at in (38, 100, 230, 300, 460, 499):
+        got, before = stream(at), at // 32 * 32
+        assert np.isnan(got[at]).all()
+        assert np.array_equal(got[:before], clean[:before]), (at, np.flatnonzero(~(got == clean).all(1)[:before]))
+    m.close()
+
+
 @pytest.mark.parametrize("dim,rows", [(64, 1), (64, 112), (64, 113), (64, 128), (64, 129), (64, 300), (128, 63), (128, 65), (128, 144), (256, 32), (256, 33), (256, 50), (512, 16),
                                       (512, 17), (512, 50)])
 def test_chunks_around_the_delta_rules_rounds(moon, ctx, tmp_path, dim, rows):

@@ -480,6 +480,32 @@ def test_attention_over_shared_tiles(moon, ctx, kv_heads, window, calls):
     compare_streams(moon, ctx, cfg, calls, sum(calls) + 5)
 
 
+@pytest.mark.parametrize("kv_heads", [16, 32, 64])
+@pytest.mark.parametrize("window", [100, 1000])
+def test_a_row_that_is_not_finite_reaches_only_blocks_of_rows_that_read_it(moon, ctx, tmp_path, kv_heads, window):
+    """Heads that share key tiles: a token of NaN, at places of a tile that rows around it share.  Of blocks of 32 rows without it among their
+    keys (from their first row's window to their last row) the residual stream keeps its bits."""
+    rows, spoiled = 500, 127
+    cfg = config(128, 64, [layer(attention(64, kv_heads, 64, 64, window, 0.25, True))])
+    w, ids = weights(cfg, 3), tokens(rows, 127)
+    w["embed"][spoiled] = np.nan
+    m = opened(moon, ctx, write_folder(tmp_path / "run", cfg, w), "bfloat16", 2048)
+
+    def stream(at):
+        m.reset()
+        m.forward(np.where(np.arange(rows) == at, spoiled, ids).astype(np.uint32))
+        return m.hidden_f32(rows)
+
+    clean, first = stream(-1), np.arange(rows) // 32 * 32
+    assert np.isfinite(clean).all()
+    for at in (70, 100, 230, 460, 499):
+        reads = (first - window < at) & (at <= first + 31)
+        got = stream(at)
+        assert np.isnan(got[at]).all()
+        assert np.array_equal(got[~reads], clean[~reads]), (at, np.flatnonzero(~(got == clean).all(1) & ~reads))
+    m.close()
+
+
 @pytest.mark.parametrize("experts,top", [(1, 1), (63, 5), (64, 8), (64, 64), (65, 8), (130, 70)])
 def test_choice_of_experts_where_scores_tie(moon, ctx, tmp_path, experts, top):
     """Up to 64 experts are a lane's each, more are walked.  Router weights of zero: every score is 1/2, corrections that repeat decide, and the lower
