@@ -1,0 +1,45 @@
+"""Waits in the built code of the attention kernels that copy tiles to LDS while they work on others (compiled here, no device needed)."""
+import os
+import re
+import subprocess
+
+import pytest
+from conftest import ROOT
+
+CSRC = os.path.join(ROOT, "moondream-zig_amd", "csrc")
+
+
+@pytest.fixture(scope="module")
+def copying_loops(tmp_path_factory):
+    """(file, kernel) -> the first loop of the kernel that copies tiles to LDS, as lines of assembly"""
+    flags = subprocess.run(["make", "-s", "-C", CSRC, "--eval", "flags: ; @echo $(HIPCC) $(HIPFLAGS)", "flags"], check=True, capture_output=True, text=True).stdout.split()
+    out = {}
+    for name in ("attn_prefill", "attn_window"):
+        path = tmp_path_factory.mktemp(name) / "out.s"
+        subprocess.run([*flags, "-w", "--offload-device-only", "-S", f"{name}.hip", "-o", str(path)], check=True, cwd=CSRC, capture_output=True)
+        for kernel, body in re.findall(r"^(_Z\w+):(.*?)^\.Lfunc_end", path.read_text(), re.S | re.M):
+            blocks = re.split(r"^(?=\.LBB\w+:|; %bb\.\d+:)", body, flags=re.M)
+            headers = [re.match(r"\.L(BB\w+):", b).group(1) for b in blocks if re.match(r"\.LBB\w+:.*Loop Header", b)]
+            for header in headers:
+                loop = "".join(b for b in blocks if b.startswith(f".L{header}:") or re.match(rf".*in Loop: Header={header}\b", b))
+                if re.search(r"buffer_load_dwordx4 .* lds$", loop, re.M):
+                    out[name, kernel] = loop.splitlines()
+                    break
+    return out
+
+
+def test_the_kernels_are_there(copying_loops):
+    names = " ".join(kernel for _, kernel in copying_loops)
+    assert len(re.findall(r"window_attn_shared_kernel", names)) == 4 and len(re.findall(r"flash_attn64_kernelILi(?:64|72)", names)) == 3
+
+
+def test_no_wait_for_copies_but_those_in_the_source(copying_loops):
+    """A copy is under way while the tile before it is worked on.  The compiler does not see what the source waits for: loads that it still counts as under way
+    ahead of the loop become a wait in the loop, and with it for the copies issued last."""
+    for kernel, loop in copying_loops.items():
+        inside, found = False, []
+        for line in loop:
+            inside = inside and "#ASMEND" not in line or "#ASMSTART" in line
+            if not inside and re.search(r"s_waitcnt.*vmcnt", line):
+                found.append(line.strip())
+        assert not found, (kernel, found)
