@@ -741,7 +741,7 @@ __device__ __forceinline__ void flash_rows96(const FaArgs &p) {
         }
     }
     // (as in flash_rows64; without it every round waited for the tile just asked for: back to back, with K and V in the L2, 1 % or nothing, inside
-    // the encoder a picture's 3.41 -> 3.37 ms)
+    // the encoder 1458 rows 24.5 -> 23.6 us)
     __builtin_amdgcn_s_waitcnt(0xf70);
     float16_t o[C::DT];
 #pragma unroll
@@ -752,8 +752,7 @@ __device__ __forceinline__ void flash_rows96(const FaArgs &p) {
     const float c2 = p.scale * 1.4426950408889634f; // > 0: the maximum of the scaled scores is the scaled maximum
 
     for (int left = (n_tiles + FA_WAVES - 1) / FA_WAVES, stage = 0; left > 0; left--, t += FA_WAVES, stage ^= 1) {
-        tile_landed<0>(); // this wavefront's part of the tile; behind the barrier everybody's, and the tile before has been read by all
-        asm volatile("s_barrier" ::: "memory");
+        tile_handed_over();
         if (t + FA_WAVES < n_tiles) copy(t + FA_WAVES, stage ^ 1);
         if (t >= n_tiles) continue;
         const half_t *Ks = smem + (group * C::STAGES + stage) * 2 * C::TILE, *Vs = Ks + C::TILE;

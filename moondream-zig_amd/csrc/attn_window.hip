@@ -466,8 +466,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void w
             for (int v = 0; v < 16; v++) o[dt][v] = 0.0f;
         for (int left = (t_end - t_begin + C::GROUPS - 1) / C::GROUPS, stage = 0, t = t_begin + kg; left > 0; left--, t += C::GROUPS, stage ^= 1) {
             const int key0 = t * WA_KT;
-            tile_landed<0>(); // this wavefront's part of the tile; behind the barrier everybody's, and the tile before has been read by all
-            asm volatile("s_barrier" ::: "memory");
+            tile_handed_over();
             if (t + C::GROUPS < t_end) copy(t + C::GROUPS, stage ^ 1);
             if (t >= t_end) continue;
             const bool blocks = POOL && t < t_window;
@@ -586,8 +585,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void w
     };
     request();
     // Where wavefronts have different rows and a result is not finite, once more: it may be a value that only the others read.  (Zeros put in place of
-    // such values in every tile that may have some, by a choice per step, took 10 to 27 % more; this check 0 to 0.4 us: 32 heads with keys of their own,
-    // window 1024, 768 rows 19.9 -> 20.3 us, 1920 rows 38.4 -> 37.9.)
+    // such values in every tile that may have some, by a choice per step, took 10 to 27 % more; this check takes up to 1 us: 32 heads with keys of their own,
+    // window 1024, 768 rows 19.9 -> 20.4 us, 1301 rows 28.1 -> 28.8, 1920 rows 37.8 -> 38.9.)
     int *redo = reinterpret_cast<int *>(reinterpret_cast<char *>(wa_lds) + C::TILE_BYTES);
     if (APART) {
         float zero[4] = {0.0f, 0.0f, 0.0f, 0.0f};

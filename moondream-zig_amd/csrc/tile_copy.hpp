@@ -1,4 +1,4 @@
-// Copies of whole tiles from memory to LDS that take no registers on the way, for the attention kernels with 64 query rows.
+// Copies of whole tiles from memory to LDS that take no registers on the way, for the attention kernels whose tiles serve more than 32 query rows.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -32,5 +32,8 @@ __device__ __forceinline__ void tile_copy(const void *rows, int left, unsigned l
 }
 #pragma clang diagnostic pop
 template <int NEWER> __device__ __forceinline__ void tile_landed() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NEWER) : "memory"); }
+// For tiles that wavefronts share: behind this the tile that all of them copied is whole, and the one before has been read by all, since their reads
+// of it have returned (the compiler's own waits for them stand where it needs the values, which may be behind the barrier).
+__device__ __forceinline__ void tile_handed_over() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 } // namespace

@@ -43,3 +43,13 @@ def test_no_wait_for_copies_but_those_in_the_source(copying_loops):
             if not inside and re.search(r"s_waitcnt.*vmcnt", line):
                 found.append(line.strip())
         assert not found, (kernel, found)
+
+
+def test_tiles_are_handed_over_behind_waits_of_the_source(copying_loops):
+    """Behind a shared tile's barrier others copy over the tile before: reads of it must have returned, whatever the compiler puts between them and the barrier."""
+    shared = {kernel: [i for i, line in enumerate(loop) if "s_barrier" in line] for kernel, loop in copying_loops.items()}
+    assert sum(map(bool, shared.values())) == 5
+    for kernel, barriers in shared.items():
+        for i in barriers:
+            lines = [line.split(";")[0].split() for line in copying_loops[kernel][:i] if line.split(";")[0].strip()]
+            assert lines[-1] == ["s_waitcnt", "vmcnt(0)", "lgkmcnt(0)"], (kernel, lines[-1])
