@@ -2,7 +2,7 @@
 // attention.multiMaskedSDPA with the mask of createAttentionMask, attention.zig:256-281, 416-541) and the
 // non-causal 729-token vision attention (16 heads x 72, attention.multiMasklessSDPA, attention.zig:125-234).
 //
-// One 256-thread workgroup owns 32 query rows of one head (64 in flash_attn64_kernel, for large calls).  Its four wavefronts split the key range in tiles
+// One 256-thread workgroup owns 32 query rows of one head (64 in flash_attn64_kernel and 96 in flash_attn96_kernel, for large calls).  Its four wavefronts split the key range in tiles
 // of 64 keys (wave w takes tiles w, w+4, ...), each running an online-softmax pass of its own over private LDS
 // staging, so the main loop has no workgroup barrier; the four partial results (m, l, O) are merged through
 // LDS at the end.  Per tile a wave computes, with v_mfma_f32_32x32x16_f16 and f32 accumulation,
@@ -408,7 +408,7 @@ template <int D> __device__ __forceinline__ int fb_slot(int key) { return D == 7
 template <int D> __device__ __forceinline__ int fb_swizzle(int key) { return D == 72 ? 0 : row64_swizzle(key); }
 
 template <int D>
-__device__ __forceinline__ void flash_rows64(const FaArgs &p) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void flash_attn64_kernel(FaArgs p) {
     using C = FbCfg<D>;
     constexpr int QS = C::QS;
     extern __shared__ __attribute__((aligned(16))) half_t smem[];
@@ -669,11 +669,12 @@ __device__ __forceinline__ void flash_rows64(const FaArgs &p) {
 // The same for calls of which 96 rows of a head per workgroup still fit one round, one workgroup to a compute unit (heads of 72): three
 // blocks of 32 rows, each walked by four wavefronts as in flash_attn_kernel, twelve in all; the three with the same tiles share them.  With 64
 // rows per workgroup such a call puts two workgroups on some units and one on others (16 heads, 1458 rows: 368 on 256), and
-// the units with two decide.  Here every SIMD has three wavefronts of six tiles each.  A tile (three wavefronts a SIMD) takes 2.9 us, about the
-// sum of what the vector unit (1.2), the matrix core (1.0) and LDS (1.0) need for it: the barrier per tile keeps the wavefronts in step, so
-// the three hardly overlap.  Calls back to back, 64 rows -> 96: 16 heads, 1100 rows 19.9 -> 15.0 us, 1250 20.6 -> 16.0, 1458 23.2 -> 19.4 (28.7 -> 24.0
-// inside the encoder); 32 heads, 600 rows 14.6 -> 11.1, 729 15.1 -> 12.1; 8 heads, 2916 rows 40.8 -> 33.3.  In two rounds it loses (16 x 2000: 33.0 against 44.4) or
-// gains little (32 x 1250: 32.6 and 30.9), and where 32 rows per workgroup fit one round they are better (16 x 1024: 12.9 and 13.3).
+// the units with two decide.  Here every SIMD has three wavefronts of six tiles each.  A tile of each (256 keys) takes 2.2 us, launch, first tiles and
+// merge 5.7 (256 to 1,536 keys, 256 workgroups).  Inside the encoder the vector unit has 48 % of a unit's busy cycles, the matrix core 28, LDS 18;
+// a wavefront waits for 48 % of its own, among others for its LDS operands, which are read one step at a time.
+// Calls back to back, 64 rows -> 96: 16 heads, 1100 rows 19.8 -> 15.0 us, 1250 20.6 -> 15.8, 1458 23.0 -> 18.6 (28.7 -> 23.6
+// inside the encoder); 32 heads, 600 rows 14.5 -> 11.0, 729 15.1 -> 11.8; 8 heads, 2916 rows 39.8 -> 32.0.  In two rounds it loses (16 x 2000: 31.9 against 43.3, 32 x 1000: 19.0
+// against 25.8) or gains little (32 x 1250: 31.8 and 30.7), and where 32 rows per workgroup fit one round they are better (16 x 1024: 12.5 and 13.4, 32 x 512: 8.7 and 9.3).
 // Tried and slower: three blocks per wavefront, the accumulators in both halves of the registers (42.5 us at 1458 rows).
 // Each row goes through the same operations in the same order as above: the same bits (tested).
 constexpr int FC_BLOCKS = 3, FC_THREADS = 64 * FC_BLOCKS * FA_WAVES;
@@ -693,7 +694,7 @@ struct FcCfg {
 };
 
 template <int D>
-__device__ __forceinline__ void flash_rows96(const FaArgs &p) {
+__global__ __launch_bounds__(FC_THREADS) __attribute__((amdgpu_waves_per_eu(3))) void flash_attn96_kernel(FaArgs p) {
     using C = FcCfg<D>;
     extern __shared__ __attribute__((aligned(16))) half_t smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), block = wave % C::BLOCKS, group = wave / C::BLOCKS;
@@ -704,7 +705,7 @@ __device__ __forceinline__ void flash_rows96(const FaArgs &p) {
     if (n_items % 8 == 0) item = (item % 8) * (n_items / 8) + item / 8;
     const int h = item / (int)gridDim.x, q0 = item % (int)gridDim.x * C::Q;
     const unsigned lds0 = __builtin_amdgcn_readfirstlane((unsigned)reinterpret_cast<unsigned long>((__attribute__((address_space(3))) const half_t *)smem));
-    int voff[2][C::DT]; // where this lane points the transposing loads, as in flash_rows64
+    int voff[2][C::DT]; // where this lane points the transposing loads, as in flash_attn64_kernel
 #pragma unroll
     for (int j = 0; j < 2; j++)
 #pragma unroll
@@ -740,7 +741,7 @@ __device__ __forceinline__ void flash_rows96(const FaArgs &p) {
             if (d < D) qf[s] = *reinterpret_cast<const half8_t *>(qp + d);
         }
     }
-    // (as in flash_rows64; without it every round waited for the tile just asked for: back to back, with K and V in the L2, 1 % or nothing, inside
+    // (as in flash_attn64_kernel; without it every round waited for the tile just asked for: back to back, with K and V in the L2, 1 % or nothing, inside
     // the encoder 1458 rows 24.5 -> 23.6 us)
     __builtin_amdgcn_s_waitcnt(0xf70);
     float16_t o[C::DT];
@@ -772,7 +773,7 @@ __device__ __forceinline__ void flash_rows96(const FaArgs &p) {
                 s[kt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8_t, a), qf[st], s[kt], 0, 0, 0);
             }
         }
-        // s[kt][v] = score of key key0 + 32*kt + 8*(v/4) + 4*hf + v%4; from here on as in flash_rows64
+        // s[kt][v] = score of key key0 + 32*kt + 8*(v/4) + 4*hf + v%4; from here on as in flash_attn64_kernel
         if (key0 + FA_KT > p.Lkv) {
             const int seen = p.Lkv - 1 - key0 - 4 * hf; // keys past this one of the tile are masked
 #pragma unroll
@@ -825,7 +826,7 @@ __device__ __forceinline__ void flash_rows96(const FaArgs &p) {
             }
     }
 
-    // merge the four groups' results, as in flash_rows64
+    // merge the four groups' results, as in flash_attn64_kernel
     float *so = reinterpret_cast<float *>(smem);                                          // [group][q][SD]
     float *sm = reinterpret_cast<float *>(reinterpret_cast<char *>(smem) + C::ML_OFFSET); // [group][q]
     float *sl = sm + FA_WAVES * C::Q;                                                     // [group][q]
@@ -871,12 +872,6 @@ __device__ __forceinline__ void flash_rows96(const FaArgs &p) {
     }
 }
 
-template <int D, bool SHARED>
-__global__ __launch_bounds__(SHARED ? FC_THREADS : 256) __attribute__((amdgpu_waves_per_eu(SHARED ? 3 : 2))) void flash_attn64_kernel(FaArgs p) {
-    if constexpr (SHARED) flash_rows96<D>(p);
-    else flash_rows64<D>(p);
-}
-
 template <int D>
 int launch_flash(moon_ctx *ctx, const FaArgs &p) {
     // Two workgroups fit a compute unit.  Sixty-four rows from where 32 rows would take a second round (rows of all heads > 64 per unit),
@@ -906,8 +901,8 @@ int launch_flash(moon_ctx *ctx, const FaArgs &p) {
     static std::atomic<bool> set32[64], set64[64], set96[64];
     if constexpr (D == 72)
         if (two && p.causal_pos < 0 && size_t(p.Lq + 95) / 96 * p.H <= cus)
-            return go(flash_attn64_kernel<D, true>, set96, FcCfg<D>::Q, FC_THREADS, FcCfg<D>::LDS_BYTES, "flash_attn64_kernel<72, shared>");
-    if (two) return go(flash_attn64_kernel<D, false>, set64, FbCfg<D>::Q, 256, FbCfg<D>::LDS_BYTES, D == 64 ? "flash_attn64_kernel<64>" : "flash_attn64_kernel<72>");
+            return go(flash_attn96_kernel<D>, set96, FcCfg<D>::Q, FC_THREADS, FcCfg<D>::LDS_BYTES, "flash_attn96_kernel<72>");
+    if (two) return go(flash_attn64_kernel<D>, set64, FbCfg<D>::Q, 256, FbCfg<D>::LDS_BYTES, D == 64 ? "flash_attn64_kernel<64>" : "flash_attn64_kernel<72>");
     return go(flash_attn_kernel<D>, set32, FA_Q, 256, FaCfg<D>::LDS_BYTES, D == 64 ? "flash_attn_kernel<64>" : "flash_attn_kernel<72>");
 }
 

@@ -162,11 +162,21 @@ def test_matrix_core_attention_over_seeded_random_shapes(moon, O, ctx):
     print(f"\nworst rel-Frobenius over 48 shapes: {worst:.2e}")
 
 
+def form(H, rows, D, causal):
+    """The kernel that a call of many rows takes."""
+    cus = compute_units()
+    if not (H * rows >= 112 * cus if causal else H * rows > (96 if D == 64 else 64) * cus):
+        return f"flash_attn_kernel<{D}>"
+    return f"flash_attn{96 if D == 72 and not causal and H * -(-rows // 96) <= cus else 64}_kernel<{D}>"
+
+
 # 64 rows per workgroup where all heads together have more than 64 rows for each compute unit (heads of 64: 96; causal: at least 112),
-# 32 below (on 256 units 32 heads cross the line behind 512, 768 and 895 rows); the last block of 64 with 1, 32, 33 and 64 rows
+# 32 below (on 256 units 32 heads cross the line behind 512, 768 and 895 rows); the last block of 64 with 1, 32, 33 and 64 rows.
+# Heads of 72 take 96 rows as long as there is a compute unit for every 96 (32 heads: up to 768 rows).
 @pytest.mark.parametrize("S,D,pos", [(511, 72, None), (512, 72, None), (513, 72, None), (544, 64, None), (545, 72, None), (767, 64, 62), (768, 64, 0),
                                      (769, 64, 62), (800, 64, 1), (801, 64, 62), (544, 72, None), (576, 72, None), (768, 64, None), (769, 64, None), (800, 64, None),
-                                     (832, 64, None), (895, 64, 62), (896, 64, 0), (897, 64, 62), (928, 64, 1), (929, 64, 62), (960, 64, 0)])
+                                     (832, 64, None), (895, 64, 62), (896, 64, 0), (897, 64, 62), (928, 64, 1), (929, 64, 62), (960, 64, 0),
+                                     (768, 72, None), (769, 72, None), (800, 72, None), (801, 72, None), (832, 72, None)])
 def test_both_row_blocks_of_the_matrix_core_attention(moon, O, ctx, S, D, pos):
     """Scores that grow along the keys, from far below one to tens: every tile raises the maximum of its rows."""
     H, L = 32, S + (pos or 0)
@@ -178,9 +188,7 @@ def test_both_row_blocks_of_the_matrix_core_attention(moon, O, ctx, S, D, pos):
         mask = moon.attention.create_attention_mask(pos, S)
         out, want = moon.attention.multi_masked_sdpa(q, k, v, mask, H, D, ctx=ctx), O.sdpa_multi(q, k, v, mask)
     assert O.rel_frobenius(out, want) <= TOL
-    cus = compute_units()
-    sixty_four = H * S >= 112 * cus if pos is not None else H * S > (96 if D == 64 else 64) * cus
-    assert ctx.last_kernel().startswith("flash_attn64_kernel" if sixty_four else "flash_attn_kernel")
+    assert ctx.last_kernel().split(" ")[0] == form(H, S, D, pos is not None)
 
 
 @pytest.mark.parametrize("D,causal", [(64, False), (64, True), (72, False)])
@@ -198,7 +206,7 @@ def test_values_that_are_not_finite_meet_the_same_rows_in_both_row_blocks(moon, 
         return moon.attention.multi_masked_sdpa(*cut, moon.attention.create_attention_mask(lo, hi - lo), H, D, ctx=ctx)
 
     whole = rows(0, L)
-    assert "flash_attn64" in ctx.last_kernel()
+    assert ctx.last_kernel().split(" ")[0] == f"flash_attn64_kernel<{D}>"
     parts = []
     for lo in range(0, L, 64):
         parts.append(rows(lo, min(lo + 64, L)))
@@ -220,7 +228,7 @@ def test_row_blocks_that_share_tiles_give_the_same_bits(moon, ctx, H, Lq, Lkv):
     q[0, 17], v[1, Lkv // 2, 3], v[2, Lkv - 1, 5] = np.nan, np.inf, np.nan
     whole = moon.attention.multi_maskless_sdpa(H, 72, q, k, v, ctx=ctx)
     if compute_units() == 256:
-        assert ctx.last_kernel().startswith("flash_attn64_kernel<72, shared>")
+        assert ctx.last_kernel().startswith("flash_attn96_kernel<72> ")
     parts = []
     for lo in range(0, Lq, 64):
         lo = min(lo, Lq - 16)  # (fewer rows take another kernel)
@@ -238,12 +246,12 @@ def test_the_last_tile_reads_nothing_that_an_earlier_call_left(moon, O, ctx, D):
     bad = np.full_like(v, np.nan)
     moon.attention.multi_maskless_sdpa(H, D, q, bad, bad, ctx=ctx)
     out = moon.attention.multi_maskless_sdpa(H, D, q, k, v, ctx=ctx)
-    assert "flash_attn64" in ctx.last_kernel()
+    assert ctx.last_kernel().split(" ")[0] == f"flash_attn64_kernel<{D}>"
     assert O.rel_frobenius(out, O.sdpa_multi(q, k, v, None)) <= TOL
 
 
 @pytest.mark.parametrize("D", [64, 72])
-@pytest.mark.parametrize("rows", [64, 16384])  # 32 rows per workgroup, 64
+@pytest.mark.parametrize("rows", [64, 16384, 16416, 24608])  # on 256 units 32 rows per workgroup up to 16,384, then heads of 72 take 96, and behind 24,576 rows all take 64
 @pytest.mark.parametrize("units", [1.45, 0.49])  # a probability, in steps of f16 below its normal range: rounded, it would count as one of them or none
 def test_matrix_core_attention_sums_probabilities_in_f32(moon, ctx, rows, D, units):
     """One key whose value is 1 and many faint ones of value 0: the result is the reciprocal of the softmax denominator, 1 + keys x p.
@@ -257,6 +265,7 @@ def test_matrix_core_attention_sums_probabilities_in_f32(moon, ctx, rows, D, uni
     k[:, 1:, 0] = faint
     v[:, 0] = 1.0
     out = moon.attention.multi_maskless_sdpa(1, D, q, k, v, ctx=ctx)
+    assert ctx.last_kernel().split(" ")[0] == form(1, rows, D, False)
     want = 1.0 / (1.0 + (keys - 1) * p)
     assert np.abs(out.astype(np.float64) - want).max() <= 2.0**-12 + 0.01 * (1.0 - want)
 

@@ -30,7 +30,7 @@ def copying_loops(tmp_path_factory):
 
 def test_the_kernels_are_there(copying_loops):
     names = " ".join(kernel for _, kernel in copying_loops)
-    assert len(re.findall(r"window_attn_shared_kernel", names)) == 4 and len(re.findall(r"flash_attn64_kernelILi(?:64|72)", names)) == 3
+    assert len(re.findall(r"window_attn_shared_kernel", names)) == 4 and len(re.findall(r"flash_attn(?:64|96)_kernel", names)) == 3
 
 
 def test_no_wait_for_copies_but_those_in_the_source(copying_loops):
