@@ -96,6 +96,8 @@ int moon_set_gemm_kernel(moon_ctx *ctx, const char *name);
  * matrix product, matrix-vector product or attention call on this context dispatched; "" before the first.  The text lives in
  * the context and changes with the next such call. */
 const char *moon_last_kernel(const moon_ctx *ctx);
+/* The same for the latest attention alone: in a session's call products follow it. */
+const char *moon_last_attention(const moon_ctx *ctx);
 int moon_sync(moon_ctx *ctx);
 /* Releases workspaces. Replaces attention.cleanupThreadPool() (attention.zig:814-818): the
  * reference frees its persistent worker pool there; here it drops cached device buffers. */

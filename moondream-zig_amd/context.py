@@ -119,6 +119,10 @@ class Context:
         """What the latest product / attention call dispatched (kernel name, grid, k split)."""
         return self.lib.moon_last_kernel(self.handle).decode()
 
+    def last_attention(self) -> str:
+        """What the latest attention dispatched, also inside a session's call."""
+        return self.lib.moon_last_attention(self.handle).decode()
+
     # ---- resident weights
     def register_weight(self, w: np.ndarray):
         self.check(self.lib.moon_weight_register(self.handle, ptr(w), w.size))

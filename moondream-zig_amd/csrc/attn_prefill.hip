@@ -895,7 +895,7 @@ int launch_flash(moon_ctx *ctx, const FaArgs &p) {
         }
         hipLaunchKernelGGL(kernel, dim3(blocks, (unsigned)p.H), dim3(threads), lds, ctx->stream, p);
         MOON_HIP(ctx, hipGetLastError());
-        MOON_NOTE_KERNEL(ctx, "%s %d workgroups", name, (int)blocks * p.H);
+        MOON_NOTE_ATTENTION(ctx, "%s %d workgroups", name, (int)blocks * p.H);
         return MOON_OK;
     };
     static std::atomic<bool> set32[64], set64[64], set96[64];

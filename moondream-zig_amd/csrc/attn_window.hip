@@ -747,12 +747,12 @@ template <int P, bool POOL> int launch_mfma_as(moon_ctx *ctx, const WindowAttn &
             const int workgroups = (p.n + rows - 1) / rows * (p.H / ws_heads(per));
             if (rows > WA_Q) MOON_TRY(launch_as(ctx, p, window_attn_shared_kernel<POOL, true>, attr_apart, WsCfg::LDS_BYTES, workgroups, 512));
             else MOON_TRY(launch_as(ctx, p, window_attn_shared_kernel<POOL, false>, attr_set, WsCfg::LDS_BYTES, workgroups, 512));
-            MOON_NOTE_KERNEL(ctx, "window_attn_shared_kernel %d rows of %d heads", rows, ws_heads(per));
+            MOON_NOTE_ATTENTION(ctx, "window_attn_shared_kernel %d rows of %d heads%s", rows, ws_heads(per), POOL ? ", blocks" : "");
             return MOON_OK;
         }
     static std::atomic<bool> attr_set[64];
     MOON_TRY(launch_as(ctx, p, window_attn_kernel<P, POOL>, attr_set, WaCfg<P>::LDS_BYTES, (p.n + WA_Q - 1) / WA_Q * p.H, 256));
-    MOON_NOTE_KERNEL(ctx, "window_attn_kernel<%d>", P);
+    MOON_NOTE_ATTENTION(ctx, "window_attn_kernel<%d>", P);
     return MOON_OK;
 }
 // (a call before whose window no block lies yet takes the kernel without them)
@@ -780,6 +780,6 @@ int launch_window_attention(moon_ctx *ctx, int dtype, const WindowAttn &p) {
     if (dtype == MOON_DTYPE_BF16) hipLaunchKernelGGL(window_attn_rows_kernel<bf16_t>, grid, dim3(256), 0, ctx->stream, p);
     else hipLaunchKernelGGL(window_attn_rows_kernel<float>, grid, dim3(256), 0, ctx->stream, p);
     MOON_HIP(ctx, hipGetLastError());
-    MOON_NOTE_KERNEL(ctx, "window_attn_rows_kernel");
+    MOON_NOTE_ATTENTION(ctx, "window_attn_rows_kernel");
     return MOON_OK;
 }

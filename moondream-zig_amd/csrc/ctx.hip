@@ -127,6 +127,7 @@ extern "C" int moon_set_gemm_kernel(moon_ctx *ctx, const char *name) {
 }
 
 extern "C" const char *moon_last_kernel(const moon_ctx *ctx) { return ctx ? ctx->last_kernel : ""; }
+extern "C" const char *moon_last_attention(const moon_ctx *ctx) { return ctx ? ctx->last_attention : ""; }
 
 extern "C" const char *moon_last_error(const moon_ctx *ctx) { return ctx ? ctx->err.c_str() : g_create_error.c_str(); }
 

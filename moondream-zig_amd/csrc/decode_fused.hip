@@ -1308,7 +1308,7 @@ int launch_decode_attention_merged(moon_ctx *ctx, const half_t *qkv, half_t *cac
         hipLaunchKernelGGL((decode_attn_merged_kernel<64, 10>), dim3((unsigned)(H * DEC_SPLITS)), dim3(256), 0, ctx->stream, qkv, cache_k, cache_v, table,
                            partial, out, head_count, count_target, (int)H, (int)rot_dim, (int)max_seq, (int)pos, pos_dev, (int)head_stride);
     MOON_HIP(ctx, hipGetLastError());
-    MOON_NOTE_KERNEL(ctx, "decode_attn_merged_kernel<64> %d workgroups", (int)(H * DEC_SPLITS));
+    MOON_NOTE_ATTENTION(ctx, "decode_attn_merged_kernel<64> %d workgroups", (int)(H * DEC_SPLITS));
     return MOON_OK;
 }
 

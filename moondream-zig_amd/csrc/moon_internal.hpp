@@ -6,6 +6,7 @@
 #include <cstdarg>
 #include <cstdint>
 #include <cstdio>
+#include <cstring>
 #include <map>
 #include <mutex>
 #include <string>
@@ -36,6 +37,7 @@ struct moon_ctx {
     std::string err;
     int cu_count = 0;
     char last_kernel[96] = ""; // moon_last_kernel: what the latest product / attention launch dispatched (set by the launchers)
+    char last_attention[96] = ""; // moon_last_attention: the latest attention launch
     char gemm_kernel[8] = ""; // moon_set_gemm_kernel / MOON_GEMM_KERNEL: a product kernel to take where the shape allows it ("": by shape)
     // staging for host-pointer ops: a, b, c, bias/aux, mask
     GrowBuf stage[6];
@@ -63,6 +65,7 @@ struct moon_ctx {
 int moon_fail(moon_ctx *ctx, int code, const char *fmt, ...);
 // Notes what a launcher dispatched, for moon_last_kernel (a few dozen nanoseconds per call).
 #define MOON_NOTE_KERNEL(ctx, ...) snprintf((ctx)->last_kernel, sizeof (ctx)->last_kernel, __VA_ARGS__)
+#define MOON_NOTE_ATTENTION(ctx, ...) (MOON_NOTE_KERNEL(ctx, __VA_ARGS__), memcpy((ctx)->last_attention, (ctx)->last_kernel, sizeof (ctx)->last_kernel))
 int moon_grow(moon_ctx *ctx, GrowBuf &b, size_t bytes);
 
 #define MOON_HIP(ctx, expr)                                                                          \

@@ -8,6 +8,7 @@ import sys
 import generax_oracle as G
 import numpy as np
 import pytest
+from conftest import compute_units
 from decoder_checks import feed, opened, row_errors, rows_close, run, streams_of_both_types
 from generax_models import MODELS, ODD, attention, beacon_weights, config, delta, parallel, plain, rotation, softmax_mixer, weights
 from rikanex_models import tokens, write_folder
@@ -496,14 +497,25 @@ def test_tile_heights_of_a_joined_layer(moon, ctx, rows, ff, height):
     assert_close(got, want, "bfloat16")
 
 
+# what 64 heads take by their key heads
+SHARED = {16: "window_attn_shared_kernel 32 rows of 4 heads", 32: "window_attn_shared_kernel 64 rows of 2 heads", 64: "window_attn_shared_kernel 128 rows of 1 heads"}
+
+
 @pytest.mark.parametrize("kv_heads", [16, 32, 64])
 @pytest.mark.parametrize("window,pool,calls", [(1000, 16, [256]), (64, 5, [333]), (65, 64, [321]), (100, 1, [300, 257]), (30, 16, [2048, 500]), (1, 3, [190])], ids=str)
 def test_attention_over_shared_tiles(moon, ctx, kv_heads, window, pool, calls):
     """64 heads in groups of four, two and one, whose calls of some hundred rows share key tiles: blocks ahead of the window (up to 300 of them,
-    none in the first case), and heads that turn back.  bf16 against f32, whose attention is a plain loop per row."""
+    none in the first case), and heads that turn back.  bf16 against f32, whose attention is a plain loop per row.  (A second call with a block per row
+    before its window has more tiles than its rows pay for: there the first call shares.)"""
     mixer = attention(64, kv_heads, 64, 64, window, 0.25, rotation(64, 1e4))
     cfg = config(128, 64, [parallel(softmax_mixer(64, kv_heads, 64, 64, window, 0.25, pool), delta(1, 1, 64, 64, 2)), plain(mixer), plain(dict(mixer, kv_from=1))], softcap=30.0)
     ids, got = tokens(sum(calls), 128), {}
+    if compute_units() == 256:
+        for layers in (1, 3):  # (the note is that of a call's last attention)
+            m = moon.text_model.TextModel.open_synthetic(dict(cfg, layers=cfg["layers"][:layers]), "bfloat16", sum(calls) + 5, seed=5, std=0.05, ctx=ctx)
+            m.forward(ids[:calls[0]])
+            assert ctx.last_attention() == SHARED[kv_heads] + (", blocks" if layers == 1 and calls[0] - window >= pool else "")
+            m.close()
     for dtype in DTYPES:
         m = moon.text_model.TextModel.open_synthetic(cfg, dtype, sum(calls) + 5, seed=5, std=0.05, ctx=ctx)
         at = 0
@@ -532,6 +544,8 @@ def test_a_row_that_is_not_finite_reaches_no_block_of_rows_before_it(moon, ctx, 
         return m.hidden_f32(rows)
 
     clean = stream(-1)
+    if compute_units() == 256:
+        assert ctx.last_attention() == SHARED[kv_heads] + ", blocks"
     assert np.isfinite(clean).all()
     for at in (38, 100, 230, 300, 460, 499):
         got, before = stream(at), at // 32 * 32

@@ -457,8 +457,9 @@ def test_heads_that_fill_a_compute_units_memory(moon, ctx, tmp_path, dtype):
     assert_close(run(moon, ctx, tmp_path, cfg, w, ids, dtype, [1]), R.forward(cfg, w, ids)[0], dtype)
 
 
-def compare_streams(moon, ctx, cfg, calls, max_seq):
-    """Residual streams of the last call's rows, bf16 against f32 (whose attention is a plain loop per row)."""
+def compare_streams(moon, ctx, cfg, calls, max_seq, note):
+    """Residual streams of the last call's rows, bf16 against f32 (whose attention is a plain loop per row); note: what the bf16 session's attention must
+    have been in every call, as dispatched on 256 compute units."""
     ids, got = tokens(sum(calls), cfg["vocab"]), {}
     for dtype in DTYPES:
         m = moon.text_model.TextModel.open_synthetic(cfg, dtype, max_seq, seed=5, std=0.05, ctx=ctx)
@@ -466,9 +467,15 @@ def compare_streams(moon, ctx, cfg, calls, max_seq):
         for n in calls:
             m.forward(ids[at:at + n])
             at += n
+            if dtype == "bfloat16" and compute_units() == 256:
+                assert ctx.last_attention() == note
         got[dtype] = m.hidden_f32(calls[-1])
         m.close()
     assert_close(got["bfloat16"], got["float32"], "bfloat16")
+
+
+# what 64 heads take by their key heads
+SHARED = {16: "window_attn_shared_kernel 32 rows of 4 heads", 32: "window_attn_shared_kernel 64 rows of 2 heads", 64: "window_attn_shared_kernel 128 rows of 1 heads"}
 
 
 @pytest.mark.parametrize("kv_heads", [16, 32, 64])
@@ -477,7 +484,14 @@ def test_attention_over_shared_tiles(moon, ctx, kv_heads, window, calls):
     """64 heads in groups of four, two and one, whose calls of some hundred rows share key tiles: whole and ragged blocks of rows and tiles, windows
     at their edges, rows behind others, and (2048 + 500) a cache whose rows are used again.  Scores with a spread of about 2."""
     cfg = config(128, 64, [layer(attention(64, kv_heads, 64, 64, window, 0.25, True)), layer(attention(64, kv_heads, 64, 64, window, -0.25, True))], embed_scale=2.0)
-    compare_streams(moon, ctx, cfg, calls, sum(calls) + 5)
+    compare_streams(moon, ctx, cfg, calls, sum(calls) + 5, SHARED[kv_heads])
+
+
+@pytest.mark.parametrize("rows,note", [(95, "window_attn_kernel<64>"), (96, "window_attn_shared_kernel 32 rows of 4 heads")])
+def test_where_heads_begin_to_share_tiles(moon, ctx, rows, note):
+    """64 heads, two tiles of keys: from 24 rows for every compute unit on."""
+    cfg = config(128, 64, [layer(attention(64, 16, 64, 64, 1000, 0.25, True))], embed_scale=2.0)
+    compare_streams(moon, ctx, cfg, [rows], rows, note)
 
 
 @pytest.mark.parametrize("kv_heads", [16, 32, 64])
@@ -497,6 +511,8 @@ def test_a_row_that_is_not_finite_reaches_only_blocks_of_rows_that_read_it(moon,
         return m.hidden_f32(rows)
 
     clean, first = stream(-1), np.arange(rows) // 32 * 32
+    if compute_units() == 256:
+        assert ctx.last_attention() == SHARED[kv_heads]
     assert np.isfinite(clean).all()
     for at in (70, 100, 230, 460, 499):
         reads = (first - window < at) & (at <= first + 31)
