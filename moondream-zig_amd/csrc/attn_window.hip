@@ -718,15 +718,28 @@ __global__ __launch_bounds__(256) void window_attn_rows_kernel(WindowAttn p) {
     }
 }
 
-// Where the shared tiles pay.  The kernel with merged wavefronts spreads any call over the device, its time goes with the rows times their
-// tiles; the other's goes with the longest walk, T tiles, and a start and an end.  On 256 units, merged -> shared (us): 32 heads, window 1024,
-// 600 rows (75 per unit, T = 10) 16.7 -> 17.0, 768 (96, 12) 19.2 -> 19.3 (with blocks 18.9 -> 17.4, rotated 18.7 -> 17.4), 960 (120, 15) 22.9 -> 22.9
-// (21.9 -> 20.8, 22.4 -> 21.5), 1100 (138, 18) 28.4 -> 26.4, 1920 (240, 18) 49.7 -> 36.8; 16 heads, window 512 (T = 10), 960 rows (60) 12.5 -> 16.7,
-// 1200 (75) 17.6 -> 17.2, 1920 (120) 23.2 -> 19.3; window 1000 (T = 17), 1500 (94) 25.0 -> 26.0, 1920 (120) 28.1 -> 27.4.
+// Where the shared tiles pay.  The kernel with merged wavefronts spreads any call over the device: its time goes with the tiles that all rows walk
+// (x: rows times tiles, per unit) and with the rounds of 64 rows per unit.  The other's goes with the longest walk, T tiles of about 1 us, behind a start
+// and an end of 6 us, 9 with a gate.  On 256 units, merged -> shared (us), r rows per unit:
+//   gate, 32 heads     window 1024  600 rows (r 75, T 10, x 390) 17.9 -> 18.4, 768 (96, 12, 624) 20.6 -> 21.2, 960 (120, 15, 960) 23.8 -> 24.4, 1024 (128, 16, 1088) 24.1 -> 24.6,
+//                      1100 (138, 18, 1250) 28.9 -> 26.7, 1920 52.2 -> 38.2; window 512  600 (75, 10, 387) 18.0 -> 18.6, 768 (96, 9, 576) 21.0 -> 19.2; window 256  600 (75, 6, 295) 16.5 -> 15.1
+//   gate, other heads  16, window 256  900 (56, 6, 241) 13.2 -> 14.2; 16, window 512  1100 (69, 10, 475) 17.8 -> 18.5, 1300 (81, 10, 587) 20.7 -> 18.8; 16, window 1024  1400 (88, 17, 944)
+//                      24.6 -> 26.0, 1700 (106, 17, 1262) 26.7 -> 26.8; 64, 256 rows (64, 4, 160) 9.3 -> 12.7, 300 (75, 5, 215) 15.1 -> 14.3
+//   none, rotated      64, 256 rows (64, 4, 160) 8.6 -> 9.8; 16, window 256  900 (56, 6, 241) 12.9 -> 11.8; 32, window 1024  768 (96, 12, 624) 18.8 -> 17.5, 960 22.7 -> 21.5, 1920 51 -> 36
 bool shares_tiles(moon_ctx *ctx, const WindowAttn &p) {
-    const int last = p.pos0 + p.n - 1, lo = p.window ? std::max(0, last - (WA_Q - 1) - p.window + 1) : 0, seen = p.pool ? std::max(0, last - p.window + 1) / p.pool : 0;
-    const size_t tiles = last / WA_KT - lo / WA_KT + 1 + (seen + WA_KT - 1) / WA_KT, cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
-    return p.dimp == WsCfg::D && p.vdimp == WsCfg::D && (!p.rotv || p.vdim == WsCfg::D) && size_t(p.n) * p.H >= (7 * tiles + 10) * cus;
+    if (p.dimp != WsCfg::D || p.vdimp != WsCfg::D || (p.rotv && p.vdim != WsCfg::D)) return false;
+    const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
+    auto walk = [&](int first, int last) { // tiles of the block of rows that has these positions
+        const int lo = p.window ? std::max(0, first - p.window + 1) : 0, seen = p.pool ? std::max(0, last - p.window + 1) / p.pool : 0;
+        return last / WA_KT - lo / WA_KT + 1 + (seen + WA_KT - 1) / WA_KT;
+    };
+    const int end = p.pos0 + p.n, longest = walk(std::max(0, end - WA_Q), end - 1);
+    if ((long long)p.n * p.H < (7 * longest + 10) * (long long)cus) return false;
+    const long long rows = (long long)p.n * p.H;
+    if (p.gate && (rows <= 64LL * cus || rows > 128LL * cus)) return rows > 64LL * cus;
+    long long walked = 0;
+    for (int first = p.pos0; first < end; first += WA_Q) walked += std::min(WA_Q, end - first) * walk(first, std::min(first + WA_Q, end) - 1);
+    return walked * p.H >= (p.gate ? 93 * longest - 381 : 30 * longest + 50) * (long long)cus;
 }
 
 template <class Kernel> int launch_as(moon_ctx *ctx, const WindowAttn &p, Kernel kernel, std::atomic<bool> (&attr_set)[64], size_t lds, int workgroups, int threads) {

@@ -497,18 +497,18 @@ def test_tile_heights_of_a_joined_layer(moon, ctx, rows, ff, height):
     assert_close(got, want, "bfloat16")
 
 
-# what 64 heads take by their key heads
-SHARED = {16: "window_attn_shared_kernel 32 rows of 4 heads", 32: "window_attn_shared_kernel 64 rows of 2 heads", 64: "window_attn_shared_kernel 128 rows of 1 heads"}
+# what 128 heads take by their key heads
+SHARED = {32: "window_attn_shared_kernel 32 rows of 4 heads", 64: "window_attn_shared_kernel 64 rows of 2 heads", 128: "window_attn_shared_kernel 128 rows of 1 heads"}
 
 
-@pytest.mark.parametrize("kv_heads", [16, 32, 64])
+@pytest.mark.parametrize("kv_heads", [32, 64, 128])
 @pytest.mark.parametrize("window,pool,calls", [(1000, 16, [256]), (64, 5, [333]), (65, 64, [321]), (100, 1, [300, 257]), (30, 16, [2048, 500]), (1, 3, [190])], ids=str)
 def test_attention_over_shared_tiles(moon, ctx, kv_heads, window, pool, calls):
-    """64 heads in groups of four, two and one, whose calls of some hundred rows share key tiles: blocks ahead of the window (up to 300 of them,
+    """128 heads in groups of four, two and one, whose calls of some hundred rows share key tiles: blocks ahead of the window (up to 300 of them,
     none in the first case), and heads that turn back.  bf16 against f32, whose attention is a plain loop per row.  (A second call with a block per row
     before its window has more tiles than its rows pay for: there the first call shares.)"""
-    mixer = attention(64, kv_heads, 64, 64, window, 0.25, rotation(64, 1e4))
-    cfg = config(128, 64, [parallel(softmax_mixer(64, kv_heads, 64, 64, window, 0.25, pool), delta(1, 1, 64, 64, 2)), plain(mixer), plain(dict(mixer, kv_from=1))], softcap=30.0)
+    mixer = attention(128, kv_heads, 64, 64, window, 0.25, rotation(64, 1e4))
+    cfg = config(128, 64, [parallel(softmax_mixer(128, kv_heads, 64, 64, window, 0.25, pool), delta(1, 1, 64, 64, 2)), plain(mixer), plain(dict(mixer, kv_from=1))], softcap=30.0)
     ids, got = tokens(sum(calls), 128), {}
     if compute_units() == 256:
         for layers in (1, 3):  # (the note is that of a call's last attention)
@@ -527,13 +527,13 @@ def test_attention_over_shared_tiles(moon, ctx, kv_heads, window, pool, calls):
     assert_close(got["bfloat16"], got["float32"], "bfloat16")
 
 
-@pytest.mark.parametrize("kv_heads", [16, 32, 64])
+@pytest.mark.parametrize("kv_heads", [32, 64, 128])
 @pytest.mark.parametrize("window,pool", [(30, 16), (30, 1), (100, 5)])
 def test_a_row_that_is_not_finite_reaches_no_block_of_rows_before_it(moon, ctx, tmp_path, kv_heads, window, pool):
     """Heads that share key tiles, windows shorter than a workgroup's rows, so that its last rows see blocks of its first ones: a token of NaN leaves the
     bits of all blocks of 32 rows before it (the delta rule's state carries it to every row behind it)."""
     rows, spoiled = 500, 127
-    cfg = config(128, 64, [parallel(softmax_mixer(64, kv_heads, 64, 64, window, 0.25, pool), delta(1, 1, 64, 64, 2))])
+    cfg = config(128, 64, [parallel(softmax_mixer(128, kv_heads, 64, 64, window, 0.25, pool), delta(1, 1, 64, 64, 2))])
     w, ids = weights(cfg, 3), tokens(rows, 127)
     w["embed"][spoiled] = np.nan
     m = opened(moon, ctx, write_folder(tmp_path / "run", cfg, w), "bfloat16", 2048)

@@ -474,33 +474,34 @@ def compare_streams(moon, ctx, cfg, calls, max_seq, note):
     assert_close(got["bfloat16"], got["float32"], "bfloat16")
 
 
-# what 64 heads take by their key heads
-SHARED = {16: "window_attn_shared_kernel 32 rows of 4 heads", 32: "window_attn_shared_kernel 64 rows of 2 heads", 64: "window_attn_shared_kernel 128 rows of 1 heads"}
+# what 128 heads take by their key heads
+SHARED = {32: "window_attn_shared_kernel 32 rows of 4 heads", 64: "window_attn_shared_kernel 64 rows of 2 heads", 128: "window_attn_shared_kernel 128 rows of 1 heads"}
 
 
-@pytest.mark.parametrize("kv_heads", [16, 32, 64])
+@pytest.mark.parametrize("kv_heads", [32, 64, 128])
 @pytest.mark.parametrize("window,calls", [(1000, [256]), (1000, [333]), (64, [161]), (65, [321]), (100, [300, 257]), (100, [2048, 500]), (1, [190])], ids=str)
 def test_attention_over_shared_tiles(moon, ctx, kv_heads, window, calls):
-    """64 heads in groups of four, two and one, whose calls of some hundred rows share key tiles: whole and ragged blocks of rows and tiles, windows
+    """128 heads in groups of four, two and one, whose calls of some hundred rows share key tiles: whole and ragged blocks of rows and tiles, windows
     at their edges, rows behind others, and (2048 + 500) a cache whose rows are used again.  Scores with a spread of about 2."""
-    cfg = config(128, 64, [layer(attention(64, kv_heads, 64, 64, window, 0.25, True)), layer(attention(64, kv_heads, 64, 64, window, -0.25, True))], embed_scale=2.0)
+    cfg = config(128, 64, [layer(attention(128, kv_heads, 64, 64, window, 0.25, True)), layer(attention(128, kv_heads, 64, 64, window, -0.25, True))], embed_scale=2.0)
     compare_streams(moon, ctx, cfg, calls, sum(calls) + 5, SHARED[kv_heads])
 
 
-@pytest.mark.parametrize("rows,note", [(95, "window_attn_kernel<64>"), (96, "window_attn_shared_kernel 32 rows of 4 heads")])
-def test_where_heads_begin_to_share_tiles(moon, ctx, rows, note):
-    """64 heads, two tiles of keys: from 24 rows for every compute unit on."""
-    cfg = config(128, 64, [layer(attention(64, 16, 64, 64, 1000, 0.25, True))], embed_scale=2.0)
-    compare_streams(moon, ctx, cfg, [rows], rows, note)
+@pytest.mark.parametrize("heads,kv_heads,window,rows,shared", [(128, 32, 1000, 128, False), (128, 32, 1000, 129, True), (32, 8, 1024, 600, False), (32, 8, 1024, 1031, False), (32, 8, 1024, 1032, True),
+                                                               (16, 4, 512, 1182, False), (16, 4, 512, 1183, True)])
+def test_where_heads_begin_to_share_tiles(moon, ctx, heads, kv_heads, window, rows, shared):
+    """Gated heads: from more than 64 rows for every compute unit on, and up to 128 where all rows together walk enough tiles for the longest walk."""
+    cfg = config(128, 64, [layer(attention(heads, kv_heads, 64, 64, window, 0.25, True))], embed_scale=2.0)
+    compare_streams(moon, ctx, cfg, [rows], rows, "window_attn_shared_kernel 32 rows of 4 heads" if shared else "window_attn_kernel<64>")
 
 
-@pytest.mark.parametrize("kv_heads", [16, 32, 64])
+@pytest.mark.parametrize("kv_heads", [32, 64, 128])
 @pytest.mark.parametrize("window", [100, 1000])
 def test_a_row_that_is_not_finite_reaches_only_blocks_of_rows_that_read_it(moon, ctx, tmp_path, kv_heads, window):
     """Heads that share key tiles: a token of NaN, at places of a tile that rows around it share.  Of blocks of 32 rows without it among their
     keys (from their first row's window to their last row) the residual stream keeps its bits."""
     rows, spoiled = 500, 127
-    cfg = config(128, 64, [layer(attention(64, kv_heads, 64, 64, window, 0.25, True))])
+    cfg = config(128, 64, [layer(attention(128, kv_heads, 64, 64, window, 0.25, True))])
     w, ids = weights(cfg, 3), tokens(rows, 127)
     w["embed"][spoiled] = np.nan
     m = opened(moon, ctx, write_folder(tmp_path / "run", cfg, w), "bfloat16", 2048)
