@@ -349,7 +349,8 @@ constexpr int WS_PAIRED = 64; // workgroups of a die that are there at once: two
 // A window of 1024 is 17 tiles: the kernel above gives a wavefront four of them, and its first loads, scores' masks and merge cost as much
 // as the tiles.  What bounds this one is the vector unit (of about 1,370 cycles a tile and wavefront, exponentials 510, the weights' second
 // term 380) and, in calls of one workgroup per unit, latency: start and end take 7 us.
-// Times, above -> here: 32 heads, window 1024, 1920 rows 49.7 -> 36.9 us, 1301 rows 34.0 -> 27.8, with blocks 33.1 -> 26.3, rotated 36.1 -> 26.7.
+// Times, above -> here: 32 heads on 8 key heads, window 1024, 1920 rows 52.2 -> 38.2 us, 1301 rows 35.2 -> 28.2, with blocks 34.9 -> 26.6, rotated 34.7 -> 26.5; with 32
+// key heads 52.2 -> 39.8, 35.2 -> 29.4, 34.8 -> 29.0, 34.6 -> 27.4.
 // Measured and not kept: 64 rows per wavefront in the arrangement above (43.5 us at 1920 rows; better, by 15 %, only around 768); two
 // wavefronts instead of four there (46.9); remainders of the weights by two-element dot products (1 to 3 us slower); wave priorities.
 struct WsCfg {

@@ -55,7 +55,7 @@ __device__ __forceinline__ void route_wave(const float *logits, const float *cor
         idx = 0x7fffffff;
         for (; tied; tied &= tied - 1) idx = min(idx, __builtin_amdgcn_readlane(mine, __ffsll(tied) - 1));
         if (idx >= E) idx = k; // (scores that are not numbers: stay within the experts)
-        const float s = scores[idx];
+        const float s = scores[idx]; // (another lane's: LDS serves a wavefront in order)
         if (lane == (idx & 63)) choice[idx] = -INFINITY;
         if (lane == 0) {
             ids[k] = idx;

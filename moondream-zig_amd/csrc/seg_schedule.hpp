@@ -41,9 +41,9 @@ SEG_FN uint32_t seg_div(uint32_t n, const FastDiv &f) {
 // A die's run is walked in blocks of 2 x SEG_BAND tiles: the 32 tiles that a die works on at once then share 512 to 1,024 rows of either
 // operand, where whole columns of tiles (m first) read all of A again for every few columns: 117 against 123 us at 1920 x 16192 x
 // 2048 in 256-row tiles, 130 against 152 in 128-row tiles, weights from HBM.  A column of up to three tiles is a block by itself
-// (blocks would leave a single row of tiles behind: 1 to 2 % of a prompt of 300 rows).  f32 products are walked m first: multiply-adds
+// (blocks would leave a single row of tiles behind: 1 to 2 % of a prompt of 300 rows).  Plain f32 products are walked m first: multiply-adds
 // bound them and their workgroups are all in flight at once (width 512, two layers of 1301 rows: 1.35 ms in blocks, 1.32 m first).
-// A list of row tiles (grouped rows, each with weights of its own) is walked n first, see seg_find_listed.
+// A list of row tiles (grouped rows, each with weights of its own) is walked n first in both types, see seg_find_listed.
 constexpr int SEG_BAND = 8, SEG_COLUMN = 3;
 
 struct SegWalk {
@@ -125,7 +125,8 @@ SEG_FN int seg_find(const SegWalk &w, int die, int slot, int &tm, int &tn, int &
 // The same for a list of which `there` row tiles exist.  The dies share the tiles that exist, and a row tile's columns follow each other: its
 // rows stay in the die's L2 while the weights, read once, pass by.  Dealt as if the list were full, m first, a die's run held 16 % more
 // tiles than the average, and every column of tiles read all rows again: 64 experts of 704, 768 rows of width 2048 with 8 choices, first
-// product 101 -> 86 us, second 51 -> 45 (weights 369 and 184 MB, 72 and 36 us at a copy's rate).
+// product 101 -> 86 us, second 51 -> 45 (weights 369 and 184 MB, 72 and 36 us at a copy's rate); in f32 1010 -> 922 and 447 -> 447, at width 1024 508 -> 465 and
+// 268 -> 259, of 300 rows 250 -> 253 and 122 -> 124.
 SEG_FN int seg_find_listed(const SegWalk &w, int there, int die, int slot, int &tm, int &tn) {
     const int all = there * w.tiles_n, per_die = (all + SEG_DIES - 1) / SEG_DIES, at = die * per_die + slot;
     if (slot >= per_die || at >= all) return -1;
