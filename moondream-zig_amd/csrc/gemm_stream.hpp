@@ -7,8 +7,7 @@
 // 32 x 32, f32).  What bounds the loop, per k-tile at MI = 4 with every unit busy: the products alone take 0.61 us (the clock under
 // matrix load), the copies alone 0.58 (1.2 us of latency with two k-tiles, 96 KiB, in flight), the operand reads alone 0.32, all
 // together 0.85 with the operands in L2, 0.9 from HBM; MI = 2: 0.30, 0.34, 0.26 and 0.43.  Copies must be whole 128-byte lines: with
-// k-tiles of 32 (64-byte rows, four stages) a copy takes twice as long.  256 x 256 tiles in eight wavefronts that copy and multiply
-// themselves have room for two stages only, and each k-tile then pays the copies' latency (1.5 to 2.0 us for 2 x the products).
+// k-tiles of 32 (64-byte rows, four stages) a copy takes twice as long.  Tiles twice as wide are gemm_block.hpp's.
 // Stages and the barrier per k-tile are gemm_dma.hpp's, counted on over the tiles.  The epilogue has 16 KiB of LDS of its own, so it
 // runs while the loaders fill every stage.  K ranges are whole k-tiles.
 #pragma once

@@ -1,5 +1,6 @@
 // Products of the layer-list decoders: C[M, N] = A . W^T with the columns in segments (16-bit, f32, gated pairs), rows gathered
 // and grouped where a router asks for it.  bf16 runs on the matrix cores through the stream of tiles of gemm_stream.hpp; f32 is computed with f32 multiply-adds (no reduced-precision mode).
+#include "gemm_block.hpp"
 #include "gemm_stream.hpp"
 #include "layer_list.hpp"
 #include "lm_types.hpp"
@@ -36,13 +37,30 @@ __device__ __forceinline__ int seg_tile(const SegGemm &p, const SegWalk &w, bool
     return 1;
 }
 
+// Four consecutive columns of one row of a wavefront's 32-row blocks of accumulators: piece i (of eight) of lane l has row row(l, i) and
+// columns 4 column4(l, i) .. + 3; piece i < 4 holds columns below 32, piece i + 4 those 32 behind it.
+struct Pieces32 { // 32 x 32 products (gemm_stream.hpp): acc[32 columns][32 rows]
+    static __device__ __forceinline__ int row(int lane, int) { return lane & 31; }
+    static __device__ __forceinline__ int column4(int lane, int i) { return 2 * i + (lane >> 5); }
+    template <int MI> static __device__ __forceinline__ float4_t get(const float16_t (&acc)[2][MI], int mi, int i) {
+        const float16_t &a = acc[i >> 2][mi];
+        const int q = i & 3;
+        return float4_t{a[4 * q], a[4 * q + 1], a[4 * q + 2], a[4 * q + 3]};
+    }
+};
+struct Pieces16 { // 16 x 16 products (gemm_block.hpp): acc[16 columns][16 rows]
+    static __device__ __forceinline__ int row(int lane, int i) { return 16 * (i & 1) + (lane & 15); }
+    static __device__ __forceinline__ int column4(int lane, int i) { return 4 * (i >> 1) + (lane >> 4); }
+    template <int M2> static __device__ __forceinline__ float4_t get(const float4_t (&acc)[4][M2], int mi, int i) { return acc[i >> 1][2 * mi + (i & 1)]; }
+};
+
 // A multiplier wavefront's accumulators -> their segment, 32 rows at a time through its 4 KiB of LDS so that the stores are whole
 // lines: rows of 128 (gated pairs: 64) bytes, the 16-byte granules XOR-swizzled by row.
 typedef bf16_t bf16x4_t __attribute__((ext_vector_type(4)));
-template <int MI>
-__device__ __forceinline__ void seg_store(const SegGemm &p, const float16_t (&acc)[2][MI], const TilePos &t, int wm, int wn, int lane, char *scratch) {
+template <class P, int MI, class Acc>
+__device__ __forceinline__ void seg_store(const SegGemm &p, const Acc &acc, const TilePos &t, int wm, int wn, int lane, char *scratch) {
     asm volatile("" : "+v"(lane)); // (per tile: kept over the products, a lane's addresses would not fit the registers, and scratch loads held up each tile by 1 us)
-    const int n = t.n0 + wn * 64, col = lane & 31, g = lane >> 5;
+    const int n = t.n0 + wn * 64;
     if (n >= p.N) return;
     const int m_wave = t.m0 + wm * 32 * MI, row8 = lane >> 3, g8 = lane & 7;
     // the wavefront reads back what its own lanes wrote; its next writes come behind those reads, LDS serves it in order
@@ -52,14 +70,14 @@ __device__ __forceinline__ void seg_store(const SegGemm &p, const float16_t (&ac
 #pragma unroll
         for (int mi = 0; mi < MI; mi++) {
 #pragma unroll
-            for (int ni = 0; ni < 2; ni++)
+            for (int i = 0; i < 8; i++) {
+                const float4_t a = P::get(acc, mi, i);
+                const int r = P::row(lane, i), c = P::column4(lane, i);
+                bf16x4_t o;
 #pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    bf16x4_t o;
-#pragma unroll
-                    for (int e = 0; e < 4; e++) o[e] = (bf16_t)acc[ni][mi][4 * q + e];
-                    *reinterpret_cast<bf16x4_t *>(scratch + col * 128 + ((ni * 4 + q) ^ (col & 7)) * 16 + g * 8) = o;
-                }
+                for (int e = 0; e < 4; e++) o[e] = (bf16_t)a[e];
+                *reinterpret_cast<bf16x4_t *>(scratch + r * 128 + ((c >> 1) ^ (r & 7)) * 16 + (c & 1) * 8) = o;
+            }
             written();
 #pragma unroll
             for (int r = 0; r < 4; r++) {
@@ -76,10 +94,11 @@ __device__ __forceinline__ void seg_store(const SegGemm &p, const float16_t (&ac
 #pragma unroll
             for (int ni = 0; ni < 2; ni++) {
 #pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    float4_t o = {acc[ni][mi][4 * q], acc[ni][mi][4 * q + 1], acc[ni][mi][4 * q + 2], acc[ni][mi][4 * q + 3]};
+                for (int i = 4 * ni; i < 4 * ni + 4; i++) {
+                    float4_t o = P::get(acc, mi, i);
+                    const int r = P::row(lane, i), c = P::column4(lane, i) & 7;
                     if (p.softcap > 0.0f) o = float4_t{lm_softcap(o[0], p.softcap), lm_softcap(o[1], p.softcap), lm_softcap(o[2], p.softcap), lm_softcap(o[3], p.softcap)};
-                    *reinterpret_cast<float4_t *>(scratch + col * 128 + ((2 * q + g) ^ (col & 7)) * 16) = o;
+                    *reinterpret_cast<float4_t *>(scratch + r * 128 + (c ^ (r & 7)) * 16) = o;
                 }
                 written();
 #pragma unroll
@@ -95,11 +114,13 @@ __device__ __forceinline__ void seg_store(const SegGemm &p, const float16_t (&ac
 #pragma unroll
         for (int mi = 0; mi < MI; mi++) {
 #pragma unroll
-            for (int q = 0; q < 4; q++) {
+            for (int i = 0; i < 4; i++) {
+                const float4_t gate = P::get(acc, mi, i), up = P::get(acc, mi, i + 4);
+                const int r = P::row(lane, i), c = P::column4(lane, i);
                 bf16x4_t o;
 #pragma unroll
-                for (int e = 0; e < 4; e++) o[e] = (bf16_t)(lm_silu(acc[0][mi][4 * q + e]) * acc[1][mi][4 * q + e]);
-                *reinterpret_cast<bf16x4_t *>(scratch + col * 64 + (q ^ ((col >> 1) & 3)) * 16 + g * 8) = o;
+                for (int e = 0; e < 4; e++) o[e] = (bf16_t)(lm_silu(gate[e]) * up[e]);
+                *reinterpret_cast<bf16x4_t *>(scratch + r * 64 + ((c >> 1) ^ ((r >> 1) & 3)) * 16 + (c & 1) * 8) = o;
             }
             written();
 #pragma unroll
@@ -151,7 +172,34 @@ __global__ __launch_bounds__(DMA_THREADS) void seg_gemm_bf16_kernel(SegGemm p, S
     const int wm = role_wave & 1, wn = role_wave >> 1;
     char *scratch = reinterpret_cast<char *>(lds_stream) + S::STAGES * S::STAGE_BYTES + role_wave * STREAM_SCRATCH_BYTES;
     stream_multiply<MfmaBf16, MI, TilePos>(wm, wn, lane, next, [&](const TilePos &t) { return (p.kb[t.split + 1] - p.kb[t.split]) / BK; },
-                                           [&](const TilePos &t, const float16_t (&acc)[2][MI]) { seg_store<MI>(p, acc, t, wm, wn, lane, scratch); });
+                                           [&](const TilePos &t, const float16_t (&acc)[2][MI]) { seg_store<Pieces32, MI>(p, acc, t, wm, wn, lane, scratch); });
+}
+
+// The same in tiles of 64 MI x 256 (gemm_block.hpp); no gathered rows and no list.
+template <int MI>
+__global__ __launch_bounds__(DMA_THREADS) void seg_gemm_bf16_block_kernel(SegGemm p, SegWalk w) {
+    extern __shared__ __attribute__((aligned(16))) half_t lds_stream[];
+    using S = Block<MI>;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    auto next = [&](TilePos &t, int &round) {
+        for (;;) {
+            const int r = seg_tile(p, w, false, blockIdx.x % SEG_DIES, seg_slot(w.longest_first, blockIdx.x / SEG_DIES, gridDim.x / SEG_DIES, round++), S::ROWS, S::COLUMNS, t);
+            if (r != 0) return r > 0;
+        }
+    };
+    auto ktiles = [&](const TilePos &t) { return (p.kb[t.split + 1] - p.kb[t.split]) / BK; };
+    auto buffer = [](const void *from, int first, int n, int pitch) { // n rows (the launcher has checked that both operands fit a descriptor)
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(reinterpret_cast<const char *>(from)) + size_t(first) * pitch, 0, n * pitch, 0x00020000);
+    };
+    auto open = [&](const TilePos &t, BlockSource &s) {
+        s.a = buffer(p.A, t.m0, t.m_end - t.m0, p.lda * 2);
+        s.w = buffer(p.W, t.n0, min(p.N - t.n0, S::COLUMNS), p.K * 2);
+        s.k = p.kb[t.split] * 2;
+        s.n_ktiles = ktiles(t);
+    };
+    char *scratch = reinterpret_cast<char *>(lds_stream) + 2 * S::STAGE_BYTES + wave * S::SCRATCH_BYTES;
+    block_stream<BlockBf16, MI, TilePos>(lds_stream, wave, lane, p.lda * 2, p.K * 2, next, open, ktiles,
+                                         [&](const TilePos &t, int wm, int wn, const float4_t (&acc)[4][2 * MI]) { seg_store<Pieces16, MI>(p, acc, t, wm, wn, lane, scratch); });
 }
 
 // f32: 64 x 64 tile, a thread owns rows ty, ty + 16, .. and columns tx, tx + 16, tx + 32, tx + 48 (so a gate column and its up
@@ -199,7 +247,9 @@ __global__ __launch_bounds__(256) void seg_gemm_f32_kernel(SegGemm p, SegWalk w)
 
 } // namespace
 
-// the tile height (in 64 rows) for a product whose ranges are set
+// The tile for a product whose ranges are set: its height in 64 rows, + SEG_BLOCK where it is 256 columns wide.  Plain f32 results keep the
+// narrow tiles: wide ones need more ranges of k to fill the chip, and each range's sums cost a slab (1920 x 2048 x 7552: 58 us in two ranges of 256 x 128, 57 in
+// three of 192 x 256, whose third slab costs 3 us in row_finish; 768 rows 31 in four ranges, 32 in eight).
 static int seg_choose(moon_ctx *ctx, const SegGemm &p) {
     const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
     int best = 2;
@@ -208,6 +258,12 @@ static int seg_choose(moon_ctx *ctx, const SegGemm &p) {
         if (const double e = seg_estimate(cus, mi, p.M, p.N, p.kb, p.splits, p.longest_first); e < t) {
             t = e;
             best = mi;
+        }
+    if (p.splits > 1 || p.tile_group || p.rows || (!p.n16 && p.n32 == p.N)) return best;
+    for (int mi = 3; mi <= 4; mi++)
+        if (const double e = seg_block_estimate(cus, mi, p.M, p.N, p.K); e < t) {
+            t = e;
+            best = SEG_BLOCK + mi;
         }
     return best;
 }
@@ -253,12 +309,14 @@ int launch_seg_gemm(moon_ctx *ctx, int dtype, SegGemm p) {
     for (int s = 0; s < p.splits; s++)
         if (p.kb[0] || p.kb[s] >= p.kb[s + 1] || p.kb[s + 1] % BK || p.kb[p.splits] != p.K)
             return moon_fail(ctx, MOON_EINVAL, "segmented product: %d k splits leave one empty", p.splits);
-    int rows = 64;
+    int rows = 64, columns = 64;
     if (dtype == MOON_DTYPE_BF16) {
         const size_t lim = (size_t(1) << 31) - 4096;
         if (size_t(p.a_rows) * p.lda * 2 >= lim || size_t(p.N) * p.K * 2 >= lim)
             return moon_fail(ctx, MOON_EINVAL_DIM, "segmented product: an operand of 2 GiB or more");
-        const int mi = p.tile_group ? 2 : seg_choose(ctx, p);
+        const int tile = p.tile_group ? 2 : p.tile ? p.tile : seg_choose(ctx, p), mi = tile % SEG_BLOCK;
+        if (mi < (tile > SEG_BLOCK ? 3 : 2) || mi > 4 || tile > SEG_BLOCK + 4 || (tile > SEG_BLOCK && p.rows)) return moon_fail(ctx, MOON_EINVAL, "segmented product: tile form %d", tile);
+        columns = tile > SEG_BLOCK ? 256 : BN;
         rows = 64 * mi;
         auto go = [&](auto kern, size_t lds, std::atomic<bool> (&attr_set)[64]) -> int {
             const int dev = ctx->device >= 0 && ctx->device < 64 ? ctx->device : -1;
@@ -267,13 +325,15 @@ int launch_seg_gemm(moon_ctx *ctx, int dtype, SegGemm p) {
                 if (dev >= 0) attr_set[dev].store(true);
             }
             const int cus = std::max(SEG_DIES, (ctx->cu_count > 0 ? ctx->cu_count : 256) / SEG_DIES * SEG_DIES);
-            const int tiles_n = (p.N + BN - 1) / BN;
+            const int tiles_n = (p.N + columns - 1) / columns;
             const SegWalk w = p.tile_group ? seg_walk_listed(p.max_tiles, tiles_n) : seg_walk((p.M + rows - 1) / rows, tiles_n, false, p.kb, p.splits, p.longest_first);
             hipLaunchKernelGGL(kern, dim3((unsigned)seg_workgroups(w, cus)), dim3(DMA_THREADS), lds, ctx->stream, p, w);
             return MOON_OK;
         };
-        static std::atomic<bool> set_listed[64], set2[64], set3[64], set4[64];
+        static std::atomic<bool> set_listed[64], set2[64], set3[64], set4[64], wide3[64], wide4[64];
         if (p.tile_group) MOON_TRY(go(seg_gemm_bf16_kernel<2, true>, Stream<2>::LDS_BYTES, set_listed));
+        else if (tile == SEG_BLOCK + 4) MOON_TRY(go(seg_gemm_bf16_block_kernel<4>, Block<4>::LDS_BYTES, wide4));
+        else if (tile == SEG_BLOCK + 3) MOON_TRY(go(seg_gemm_bf16_block_kernel<3>, Block<3>::LDS_BYTES, wide3));
         else if (mi == 4) MOON_TRY(go(seg_gemm_bf16_kernel<4, false>, Stream<4>::LDS_BYTES, set4));
         else if (mi == 3) MOON_TRY(go(seg_gemm_bf16_kernel<3, false>, Stream<3>::LDS_BYTES, set3));
         else MOON_TRY(go(seg_gemm_bf16_kernel<2, false>, Stream<2>::LDS_BYTES, set2));
@@ -282,6 +342,6 @@ int launch_seg_gemm(moon_ctx *ctx, int dtype, SegGemm p) {
         hipLaunchKernelGGL(seg_gemm_f32_kernel, dim3((unsigned)(SEG_DIES * w.slots)), dim3(256), 0, ctx->stream, p, w);
     }
     MOON_HIP(ctx, hipGetLastError());
-    MOON_NOTE_KERNEL(ctx, "%s %d rows a tile, k split %d", dtype == MOON_DTYPE_BF16 ? "seg_gemm_bf16_kernel" : "seg_gemm_f32_kernel", rows, p.splits);
+    MOON_NOTE_KERNEL(ctx, "%s %d rows a tile, k split %d", dtype != MOON_DTYPE_BF16 ? "seg_gemm_f32_kernel" : columns == BN ? "seg_gemm_bf16_kernel" : "seg_gemm_bf16_block_kernel", rows, p.splits);
     return MOON_OK;
 }

@@ -166,4 +166,19 @@ inline double seg_estimate(int cus, int mi, int M, int N, const int *kb, int spl
     return longest;
 }
 
+// The same for tiles of 64 mi x 256 (gemm_block.hpp).  A round's k-tiles take the longer the more units are busy (clock and L2): fitted to 70 products, 200 to
+// 2048 rows by 5000 to 16832 columns by 1024 or 2048, of which these choose the faster kernel for 69 (the other one 1 % off); 15 to 20 % faster than narrow tiles alone where they
+// choose wide ones.
+struct SegBlockTime {
+    double k_tile, busy, rest; // us: k-tile of a lone unit, what is added with all busy, a tile's rest
+};
+inline SegBlockTime seg_block_time(int mi) { return mi == 3 ? SegBlockTime{0.55, 0.75, 4.0} : SegBlockTime{1.08, 0.42, 4.5}; }
+inline double seg_block_estimate(int cus, int mi, int M, int N, int K) {
+    const SegBlockTime t = seg_block_time(mi);
+    const int tiles = (M + 64 * mi - 1) / (64 * mi) * ((N + 255) / 256), n = cus / SEG_DIES < 1 ? 1 : cus / SEG_DIES;
+    double us = 0;
+    for (int left = (tiles + SEG_DIES - 1) / SEG_DIES; left > 0; left -= n) us += t.rest + K / SEG_K_TILE * (t.k_tile + t.busy * (left < n ? left : n) / n);
+    return us;
+}
+
 } // namespace
