@@ -35,5 +35,14 @@ template <class T> __device__ __forceinline__ float dot_piece(const lm_u32x4 &w,
 
 // library exponentials: the gates and weights are wanted to f32 accuracy
 __device__ __forceinline__ float lm_sigmoid(float z) { return 1.0f / (1.0f + expf(-z)); }
-__device__ __forceinline__ float lm_silu(float z) { return z / (1.0f + expf(-z)); }
+// z / (1 + exp(-z)): exp(-z) = 2^r 2^f with |f| <= 1/2 and f to twice f32's digits, the hardware's 2^f and 1 / d (of a quarter of d: above 2^126 its reciprocal is no
+// normal number), one correction of the quotient.  The same bits as z / (1.0f + expf(-z)) (tested) in a quarter fewer instruction cycles: the library's ranges and scalings serve
+// arguments that do not occur here.  A gated product's epilogue is these: 1920 x 16128 x 2048 120 -> 115 us, 768 rows 54.8 -> 53.1.
+__device__ __forceinline__ float lm_silu(float z) {
+    constexpr float hi = -1.44269502e+00f, lo = -1.92596299e-08f; // -1 / ln 2
+    const float x = __builtin_amdgcn_fmed3f(z, -200.0f, 200.0f), t = x * hi, r = __builtin_rintf(t);
+    const float f = (t - r) + __builtin_fmaf(x, lo, __builtin_fmaf(x, hi, -t)), d = 1.0f + __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f(f), (int)r);
+    const float i = __builtin_amdgcn_rcpf(d * 0.25f) * 0.25f, q = z * i;
+    return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-q, d, z), i, q), d, z); // (infinities and NaN as a division gives them)
+}
 __device__ __forceinline__ float lm_softcap(float z, float cap) { return cap * tanhf(z / cap); }
