@@ -16,11 +16,13 @@
 // workspace; resident model weights are transposed once at load time instead.
 // Small grids (tiles < CUs) split K across workgroups: f32 partials to a workspace, then a fixed-order
 // reduction applies the epilogue (deterministic, no atomics).
+#include <algorithm>
 #include <atomic>
 #include <cstring>
 
-#include "gemm_dma.hpp"
+#include "gemm_block.hpp"
 #include "gemm_wide.hpp"
+#include "seg_schedule.hpp"
 
 namespace {
 
@@ -282,58 +284,6 @@ __device__ __forceinline__ void gemm_tile_out(const GemmArgs &p, int m0, int n0,
     }
 }
 
-// gemm_tile_out for a qkv projection, with what qkv_rope_cache_vec_kernel does to the finished rows folded in (the same
-// values, roundings and rotations: the results are the same bits), so that the projection never goes to memory unrotated.
-// The tile's 128 columns are two whole heads of q, k or v (heads are 64 wide, tiles start at multiples of 128).  A thread
-// finishes eight consecutive columns of a row; where those are rotated it also forms the eight partner values, rot_dim / 2
-// further on or back in the same head, from the parked tile and their bias.
-template <int ROWS>
-__device__ __forceinline__ void gemm_tile_out_rope(const GemmArgs &p, int m0, int n0, int t, const half_t *scratch) {
-    const int nl = (t & 15) * 8, n = n0 + nl, d0 = nl & 63; // d0: first of the eight columns within its head
-    if (n >= p.N) return;
-    const int hd = p.rope_H * 64;
-    const int region = n / hd, head = (n - region * hd) >> 6; // 0: q, 1: k, 2: v
-    const int half = p.rope_dim >> 1;
-    const bool rotated = region < 2 && d0 < p.rope_dim, low = d0 < half;
-    const int shift = low ? half : -half; // to the partner's columns (where rotated)
-    const half8_t bias = *reinterpret_cast<const half8_t *>(p.bias + n);
-    half8_t biasp = bias;
-    if (rotated) biasp = *reinterpret_cast<const half8_t *>(p.bias + n + shift);
-    half_t *dst0 = (region == 0 ? p.rope_q + size_t(head) * p.M * 64 : (region == 1 ? p.rope_ck : p.rope_cv) + (size_t(head) * p.rope_max_seq + p.rope_pos0) * 64) + d0;
-#pragma unroll
-    for (int r = 0; r < ROWS / 32; r++) {
-        const int ml = r * 32 + (t >> 4), m = m0 + ml;
-        if (m >= p.M) continue;
-        const half8_t v = *reinterpret_cast<const half8_t *>(scratch + ml * TILE_PITCH + nl);
-        half8_t o;
-#pragma unroll
-        for (int e = 0; e < 8; e++) o[e] = apply_epilogue_v<MOON_EPI_BIAS>((float)v[e], bias[e]);
-        if (rotated) {
-            const half8_t vp = *reinterpret_cast<const half8_t *>(scratch + ml * TILE_PITCH + nl + shift);
-            const float4 *tab = reinterpret_cast<const float4 *>(p.rope_table + ((size_t)(p.rope_pos0 + m) * half + (low ? d0 : d0 - half)) * 2);
-#pragma unroll
-            for (int e4 = 0; e4 < 4; e4++) {
-                const float4 cs = tab[e4]; // (cos, sin) of two consecutive d
-#pragma unroll
-                for (int j = 0; j < 2; j++) {
-                    const int e = 2 * e4 + j;
-                    const float c = j ? cs.z : cs.x, sn = j ? cs.w : cs.y;
-                    const half_t mine = o[e], other = apply_epilogue_v<MOON_EPI_BIAS>((float)vp[e], biasp[e]);
-                    half_t a, b;
-                    if (low) {
-                        rotate_pair((float)mine, (float)other, c, sn, a, b);
-                        o[e] = a;
-                    } else {
-                        rotate_pair((float)other, (float)mine, c, sn, a, b);
-                        o[e] = b;
-                    }
-                }
-            }
-        }
-        *reinterpret_cast<half8_t *>(dst0 + size_t(m) * 64) = o;
-    }
-}
-
 // The wavefront-specialised kernel (gemm_dma.hpp) on a 128 x 128 tile.  BKN: the second operand is [K, N].
 template <int EPI, bool BKN = false>
 __global__ __launch_bounds__(DMA_THREADS) void gemm_nt_dma_kernel(GemmArgs p) {
@@ -416,15 +366,13 @@ template <int MI> struct Dma2 {
 
 // PARTIAL: the workgroup multiplies k-tiles [kt0, kt0 + n_ktiles) of tile `wg` only and leaves the f32 sums in slab `split` of
 // p.partial (no epilogue); otherwise the whole of K, and wg is taken from the workgroup index.
-// ROPE: the epilogue of a qkv projection that writes the rotated q and the cache rows (gemm_tile_out_rope) instead of C.
 // BKN: the second operand is [K, N], read in place as in gemm_nt_dma_kernel<EPI, true>.
-template <int EPI, int MI, bool PARTIAL = false, bool ROPE = false, bool BKN = false>
+template <int EPI, int MI, bool PARTIAL = false, bool BKN = false>
 __device__ __forceinline__ void gemm_nt_dma2_body(const GemmArgs &p, int wg_arg = 0, int kt0 = 0, int n_ktiles_arg = 0, int split = 0) {
     static_assert(MI == 3 || MI == 4, "192- or 256-row tiles");
     static_assert(!PARTIAL || EPI == MOON_EPI_NONE, "partial sums take no epilogue");
-    static_assert(!ROPE || (EPI == MOON_EPI_BIAS && !PARTIAL), "the rotating epilogue follows a bias");
     constexpr int BM2 = Dma2<MI>::BM2, STAGE2_HALFS = Dma2<MI>::STAGE2_HALFS, A_LOADS = Dma2<MI>::A_LOADS;
-    constexpr bool SHARED_EPILOGUE = (EPI == MOON_EPI_BIAS_GELU || ROPE) && !PARTIAL; // all eight wavefronts finish the tile
+    constexpr bool SHARED_EPILOGUE = EPI == MOON_EPI_BIAS_GELU && !PARTIAL; // all eight wavefronts finish the tile
     static_assert(size_t(BM2) * TILE_PITCH <= size_t(DMA2_STAGES) * STAGE2_HALFS, "the parked tile fits the staging area");
     extern __shared__ __attribute__((aligned(16))) half_t lds2[]; // [stage][act: 256 rows | weight: 128 rows][64 halfs]
 
@@ -496,8 +444,7 @@ __device__ __forceinline__ void gemm_nt_dma2_body(const GemmArgs &p, int wg_arg 
         if constexpr (SHARED_EPILOGUE) { // the loaders take their half of the epilogue (see the multipliers' end)
             lds_barrier();               // the multipliers have read the last k-tile
             lds_barrier();               // ... and parked the tile
-            if constexpr (ROPE) gemm_tile_out_rope<BM2>(p, m0, n0, t, lds2);
-            else gemm_tile_out<EPI, BM2>(p, m0, n0, t, lds2);
+            gemm_tile_out<EPI, BM2>(p, m0, n0, t, lds2);
         }
         return;
     }
@@ -630,8 +577,7 @@ __device__ __forceinline__ void gemm_nt_dma2_body(const GemmArgs &p, int wg_arg 
                     *reinterpret_cast<half4_t *>(lds2 + (wm * 32 * MI + mi * 32 + frag_row) * TILE_PITCH + wn * 64 + ni * 32 + 8 * q + 4 * frag_g) = o;
                 }
         lds_barrier();
-        if constexpr (ROPE) gemm_tile_out_rope<BM2>(p, m0, n0, t, lds2);
-        else gemm_tile_out<EPI, BM2>(p, m0, n0, t, lds2);
+        gemm_tile_out<EPI, BM2>(p, m0, n0, t, lds2);
         return;
     }
     if constexpr (PARTIAL) {
@@ -689,19 +635,141 @@ __device__ __forceinline__ void gemm_nt_dma2_body(const GemmArgs &p, int wg_arg 
 // (the two tile heights as kernels of their own with one template parameter, like the other kernels of this file)
 template <int EPI, bool BKN = false>
 __global__ __launch_bounds__(DMA_THREADS) void gemm_nt_dma256_kernel(GemmArgs p) {
-    gemm_nt_dma2_body<EPI, 4, false, false, BKN>(p);
+    gemm_nt_dma2_body<EPI, 4, false, BKN>(p);
 }
 template <int EPI, bool BKN = false>
 __global__ __launch_bounds__(DMA_THREADS) void gemm_nt_dma192_kernel(GemmArgs p) {
-    gemm_nt_dma2_body<EPI, 3, false, false, BKN>(p);
+    gemm_nt_dma2_body<EPI, 3, false, BKN>(p);
 }
 
-// A decoder block's qkv projection with the rotation and the cache update in its epilogue (one kernel per tile height)
-__global__ __launch_bounds__(DMA_THREADS) void gemm_nt_dma256_rope_kernel(GemmArgs p) {
-    gemm_nt_dma2_body<MOON_EPI_BIAS, 4, false, true>(p);
+// Tiles of 64 MI x 256 in a stream (gemm_block.hpp), one product or two of the same rows side by side: columns of tiles [0, columns0) are p[0]'s.
+struct GemmBlockArgs {
+    GemmArgs p[2];
+    int columns0;
+    SegWalk walk;
+};
+// A wavefront's accumulators, 32 rows at a time through its 4 KiB of LDS: rounded to f16 and parked as rows of 128 bytes (16-byte granules XOR-swizzled by row),
+// then eight columns of a row per lane are finished and stored.  The wavefront's 64 columns are one head of a qkv projection: the partners that a rotated
+// column needs lie in the same parked row; what is written are the values, roundings and rotations of qkv_rope_cache_vec_kernel on the finished rows.
+constexpr int EPI_ROPE = 4;
+template <int EPI, int MI>
+__device__ __forceinline__ void gemm_block_out(const GemmArgs &p, const float4_t (&acc)[4][2 * MI], int m_wave, int n0, int lane, char *scratch) {
+    asm volatile("" : "+v"(lane)); // (per tile, see seg_store)
+    if (n0 >= p.N) return;
+    const int row8 = lane >> 3, g8 = lane & 7, n = n0 + g8 * 8, d0 = g8 * 8;
+    const bool inside = n < p.N;
+    half8_t bias = {0, 0, 0, 0, 0, 0, 0, 0}, biasp = bias;
+    if (EPI != MOON_EPI_NONE && inside) bias = *reinterpret_cast<const half8_t *>(p.bias + n);
+    half_t *out = p.C;
+    int ld = p.N, col = n, partner = 0;
+    bool rotated = false, low = false;
+    const int half = p.rope_dim >> 1;
+    if (EPI == EPI_ROPE) {
+        const int hd = p.rope_H * 64, region = n0 / hd, head = (n0 - region * hd) >> 6; // 0: q, 1: k, 2: v
+        rotated = region < 2 && d0 < p.rope_dim;
+        low = d0 < half;
+        partner = low ? half : -half;
+        if (rotated) biasp = *reinterpret_cast<const half8_t *>(p.bias + n + partner);
+        out = region == 0 ? p.rope_q + size_t(head) * p.M * 64 : (region == 1 ? p.rope_ck : p.rope_cv) + (size_t(head) * p.rope_max_seq + p.rope_pos0) * 64;
+        ld = 64;
+        col = d0;
+    }
+#pragma unroll
+    for (int mi = 0; mi < MI; mi++) {
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const int r = 16 * h + (lane & 15), g = 2 * i + (lane >> 5);
+                half4_t o;
+#pragma unroll
+                for (int e = 0; e < 4; e++) o[e] = (half_t)acc[i][2 * mi + h][e];
+                *reinterpret_cast<half4_t *>(scratch + r * 128 + (g ^ (r & 7)) * 16 + (lane >> 4 & 1) * 8) = o;
+            }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // (the wavefront reads what its own lanes wrote)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int ml = r * 8 + row8, m = m_wave + mi * 32 + ml;
+            if (m >= p.M || !inside) continue;
+            const half8_t v = *reinterpret_cast<const half8_t *>(scratch + ml * 128 + (g8 ^ (ml & 7)) * 16);
+            half8_t res = {0, 0, 0, 0, 0, 0, 0, 0}, o;
+            if (EPI == MOON_EPI_BIAS_RESID) res = *reinterpret_cast<const half8_t *>(p.resid + size_t(m) * p.N + n);
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                half_t x = apply_epilogue_v<EPI == EPI_ROPE ? MOON_EPI_BIAS : EPI>((float)v[e], bias[e]);
+                if (EPI == MOON_EPI_BIAS_RESID) x = (half_t)((float)res[e] + (float)x);
+                o[e] = x;
+            }
+            if (EPI == EPI_ROPE && rotated) {
+                const half8_t vp = *reinterpret_cast<const half8_t *>(scratch + ml * 128 + ((g8 + (partner >> 3)) ^ (ml & 7)) * 16);
+                const float4 *tab = reinterpret_cast<const float4 *>(p.rope_table + ((size_t)(p.rope_pos0 + m) * half + (low ? d0 : d0 - half)) * 2);
+#pragma unroll
+                for (int e4 = 0; e4 < 4; e4++) {
+                    const float4 cs = tab[e4]; // (cos, sin) of two consecutive d
+#pragma unroll
+                    for (int j = 0; j < 2; j++) {
+                        const int e = 2 * e4 + j;
+                        const float c = j ? cs.z : cs.x, sn = j ? cs.w : cs.y;
+                        const half_t mine = o[e], other = apply_epilogue_v<MOON_EPI_BIAS>((float)vp[e], biasp[e]);
+                        half_t a, b;
+                        if (low) {
+                            rotate_pair((float)mine, (float)other, c, sn, a, b);
+                            o[e] = a;
+                        } else {
+                            rotate_pair((float)other, (float)mine, c, sn, a, b);
+                            o[e] = b;
+                        }
+                    }
+                }
+            }
+            *reinterpret_cast<half8_t *>(out + size_t(m) * ld + col) = o;
+        }
+        asm volatile("" ::: "memory");
+    }
+    // (used on every path: a load that may still be under way at the head of the next tile's loop would be waited for, with all copies, in each of its rounds)
+    asm volatile("" ::"v"(bias), "v"(biasp));
 }
-__global__ __launch_bounds__(DMA_THREADS) void gemm_nt_dma192_rope_kernel(GemmArgs p) {
-    gemm_nt_dma2_body<MOON_EPI_BIAS, 3, false, true>(p);
+struct GemmBlockTile {
+    int m0, n0, second;
+};
+template <int EPI, int EPI2, int MI>
+__global__ __launch_bounds__(DMA_THREADS) void gemm_nt_block_kernel(GemmBlockArgs a) {
+    extern __shared__ __attribute__((aligned(16))) half_t lds_block[]; // (the tile product addresses LDS from 0)
+    using S = Block<MI>;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    auto next = [&](GemmBlockTile &t, int &round) {
+        int tm, tn, range;
+        for (;;) {
+            const int r = seg_find(a.walk, blockIdx.x % SEG_DIES, seg_slot(0, blockIdx.x / SEG_DIES, gridDim.x / SEG_DIES, round++), tm, tn, range);
+            if (r < 0) return false;
+            if (r > 0) break;
+        }
+        t.second = EPI2 >= 0 && tn >= a.columns0;
+        t.m0 = tm * S::ROWS;
+        t.n0 = (t.second ? tn - a.columns0 : tn) * S::COLUMNS;
+        return true;
+    };
+    const int pitch = a.p[0].K * 2;
+    auto buffer = [&](const half_t *from, int first, int n) {
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(reinterpret_cast<const char *>(from)) + size_t(first) * pitch, 0, n * pitch, 0x00020000);
+    };
+    auto open = [&](const GemmBlockTile &t, BlockSource &s) {
+        const GemmArgs &p = EPI2 >= 0 && t.second ? a.p[1] : a.p[0];
+        s.a = buffer(p.A, t.m0, min(p.M - t.m0, S::ROWS));
+        s.w = buffer(p.Bt, t.n0, min(p.N - t.n0, S::COLUMNS));
+        s.k = 0;
+        s.n_ktiles = p.K / BK;
+    };
+    char *scratch = reinterpret_cast<char *>(lds_block) + 2 * S::STAGE_BYTES + wave * S::SCRATCH_BYTES;
+    block_stream<BlockF16, MI, GemmBlockTile>(
+        lds_block, wave, lane, pitch, pitch, next, open, [&](const GemmBlockTile &) { return a.p[0].K / BK; },
+        [&](const GemmBlockTile &t, int wm, int wn, const float4_t (&acc)[4][2 * MI]) {
+            const int m = t.m0 + wm * 32 * MI, n = t.n0 + wn * 64;
+            if constexpr (EPI2 >= 0) {
+                if (t.second) return gemm_block_out<EPI2, MI>(a.p[1], acc, m, n, lane, scratch);
+            }
+            gemm_block_out<EPI, MI>(a.p[0], acc, m, n, lane, scratch);
+        });
 }
 
 // TWO products with the same [M, N] result shape in one launch, each with its own split of K, f32 partial sums only (the
@@ -881,6 +949,55 @@ __global__ __launch_bounds__(256) void transpose_kernel(const half_t *__restrict
     }
 }
 
+// What products take, us, launch included, with weights from HBM, kt k-tiles: fitted to 54 products of 200 to 1920 rows by 3072 to 14336 columns by 1024 or 2048.
+// Tiles of 64 mi x 256 in rounds over the units; f: part of the units that a round keeps busy.
+double block_us(int cus, int mi, size_t M, size_t columns, size_t kt) {
+    const size_t tiles = (M + 64 * mi - 1) / (64 * mi) * columns;
+    double us = mi == 3 ? 10.5 : 11;
+    for (size_t left = tiles; left > 0; left -= std::min(left, (size_t)cus)) {
+        const double f = (double)std::min(left, (size_t)cus) / cus;
+        us += (left < tiles ? 6 : 0) + kt * (mi == 3 ? 0.78 + 0.42 * f : 1.03 + 0.5 * f);
+    }
+    return us;
+}
+int block_height(int cus, size_t M, size_t columns, size_t kt, double *us) {
+    const double three = block_us(cus, 3, M, columns, kt), four = block_us(cus, 4, M, columns, kt);
+    *us = std::min(three, four);
+    return three <= four ? 3 : 4;
+}
+// The narrow kernels as run_gemm takes them: 128 x 128 tiles, split in k where they are few (the reduction 6 us), otherwise a workgroup per tile of 192 or 256 rows.
+double narrow_us(int cus, size_t M, size_t N, size_t kt) {
+    const size_t columns = (N + BN - 1) / BN, t128 = (M + 127) / 128 * columns, t192 = (M + 191) / 192 * columns, t256 = (M + 255) / 256 * columns;
+    if (t128 * 2 <= (size_t)cus) return 10 + 0.47 * kt / std::max<size_t>(1, std::min({(size_t)cus / t128, kt / 8, (size_t)8}));
+    if (t128 <= (size_t)cus) return 4 + 0.47 * kt;
+    if (t192 <= (size_t)cus && t192 > t256) return 7 + kt * (0.45 + 0.28 * t192 / cus);
+    double us = 7.5;
+    for (size_t left = t256; left > 0; left -= std::min(left, (size_t)cus)) us += (left < t256 ? 6 : 0) + kt * std::max(0.6, 0.28 + 0.62 * std::min(left, (size_t)cus) / cus);
+    return us;
+}
+
+// a.p and a.columns0 are set
+template <int EPI, int EPI2>
+int launch_block(moon_ctx *ctx, GemmBlockArgs &a, int mi) {
+    const int cus = std::max(SEG_DIES, (ctx->cu_count > 0 ? ctx->cu_count : 256) / SEG_DIES * SEG_DIES), rows = 64 * mi;
+    const int kb[2] = {0, a.p[0].K}, columns = a.columns0 + (EPI2 >= 0 ? (a.p[1].N + 255) / 256 : 0);
+    a.walk = seg_walk((a.p[0].M + rows - 1) / rows, columns, false, kb, 1, 0);
+    static std::atomic<bool> attr_set[2][64];
+    const int dev = ctx->device >= 0 && ctx->device < 64 ? ctx->device : -1;
+    auto go = [&](auto kern, size_t lds, std::atomic<bool> *set) -> int {
+        if (dev < 0 || !set[dev].load()) { // this much dynamic LDS needs the opt-in once per device and instantiation
+            MOON_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+            if (dev >= 0) set[dev].store(true);
+        }
+        hipLaunchKernelGGL(kern, dim3((unsigned)seg_workgroups(a.walk, cus)), dim3(DMA_THREADS), lds, ctx->stream, a);
+        MOON_HIP(ctx, hipGetLastError());
+        return MOON_OK;
+    };
+    MOON_TRY(mi == 3 ? go(gemm_nt_block_kernel<EPI, EPI2, 3>, Block<3>::LDS_BYTES, attr_set[0]) : go(gemm_nt_block_kernel<EPI, EPI2, 4>, Block<4>::LDS_BYTES, attr_set[1]));
+    MOON_NOTE_KERNEL(ctx, "gemm_nt_block_kernel %d rows a tile, %d tiles", rows, a.walk.all);
+    return MOON_OK;
+}
+
 // ln: optional LayerNorm of the finished rows of C into ln->out.  *ln_done says whether it was fused (into the split-K
 // reduction); if not, the caller runs it as a launch of its own.  With ln->add set only the fused form can apply the
 // epilogue: where the product does not take it, nothing is launched and GEMM_NOT_FUSED comes back.
@@ -1016,6 +1133,22 @@ int run_gemm(moon_ctx *ctx, const half_t *A, const half_t *B, const half_t *bias
             MOON_HIP(ctx, hipGetLastError());
         }
         return MOON_OK;
+    }
+    // Wide tiles (gemm_block.hpp) where the narrow ones come to more than one per unit and are estimated to take longer: 1025 x 8192 x 2048 58 -> 43 us, 1301 x 6144 x
+    // 2048 53 -> 40, 1536 x 8192 x 8192 218 -> 165; 768 x 8192 x 2048 keeps one round of 192 x 128 (31 against 41).  MOON_GEMM_KERNEL=b192|b256 names them.
+    if (buffers_ok && K % BK == 0 && N % 8 == 0 && p.lds_epilogue && !must_fuse && !native_kn) {
+        double us;
+        int mi = force ? !strcmp(force, "b192") ? 3 : !strcmp(force, "b256") ? 4 : 0 : 0;
+        if (!force && tiles > cus) {
+            mi = block_height(cus, M, (N + 255) / 256, K / BK, &us);
+            if (us >= narrow_us(cus, M, N, K / BK)) mi = 0;
+        }
+        if (mi) {
+            GemmBlockArgs a{};
+            a.p[0] = p;
+            a.columns0 = (N + 255) / 256;
+            return launch_block<EPI, -1>(ctx, a, mi);
+        }
     }
     // More 128 x 128 tiles than CUs: the 256 x 128 kernel (MOON_GEMM_KERNEL=regs|dma keeps the 128 x 128 ones).
     if (tiles > cus && buffers_ok && K % BK == 0 && N % 8 == 0 && p.lds_epilogue && !(force && (!strcmp(force, "regs") || !strcmp(force, "dma")))) {
@@ -1181,39 +1314,34 @@ int launch_gemm_partials(moon_ctx *ctx, const half_t *A, const half_t *B, size_t
     return rc;
 }
 
-int launch_gemm_qkv_rope(moon_ctx *ctx, const half_t *A, const half_t *W, const half_t *bias, size_t M, size_t K, half_t *q_out, half_t *cache_k,
-                         half_t *cache_v, const float *table, size_t H, size_t D, size_t rot_dim, size_t max_seq, size_t pos0, bool *done) {
+int launch_gemm_front(moon_ctx *ctx, const half_t *A, const half_t *W, const half_t *bias, const half_t *W1, const half_t *bias1, half_t *out1, size_t N1, size_t M,
+                      size_t K, half_t *q_out, half_t *cache_k, half_t *cache_v, const float *table, size_t H, size_t D, size_t rot_dim, size_t max_seq, size_t pos0,
+                      bool *done) {
     *done = false;
     const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
     const size_t N = 3 * H * D, buf_max = (size_t(1) << 31) - 4096;
     const auto al16 = [](const void *q) { return reinterpret_cast<uintptr_t>(q) % 16 == 0; };
     if (ctx->gemm_kernel[0] || getenv("MOON_GEMM_NO_ROPE")) return MOON_OK; // (a kernel was named for measurements, or the fusion switched off)
     if (D != 64 || !H || rot_dim % 16 || rot_dim > D || !M || M > 0x3fffffff || K % BK || !K || pos0 + M > max_seq || max_seq > 0x3fffffff) return MOON_OK;
-    if (M * K * 2 >= buf_max || N * K * 2 >= buf_max) return MOON_OK;
-    if (!al16(A) || !al16(W) || !al16(bias) || !al16(q_out) || !al16(cache_k) || !al16(cache_v) || !al16(table)) return MOON_OK;
-    // the shapes that launch_gemm gives to the 256- and 192-row kernels: more 128 x 128 tiles than compute units
-    const int tiles_n = (int)((N + BN - 1) / BN);
-    if (size_t((M + BM - 1) / BM) * tiles_n <= size_t(cus)) return MOON_OK;
-    const int t256 = (int)((M + 255) / 256) * tiles_n, t192 = (int)((M + 191) / 192) * tiles_n;
-    const bool use192 = t192 <= cus && t192 > t256 && ((M + 191) / 192) * 192 <= ((M + 255) / 256) * 256;
-    GemmArgs p;
-    p.A = A;
-    p.Bt = W;
-    p.bias = bias;
-    p.resid = nullptr;
-    p.C = nullptr;
-    p.partial = nullptr;
-    p.M = (int)M;
-    p.N = (int)N;
-    p.K = (int)K;
-    p.tiles_m = (int)(use192 ? (M + 191) / 192 : (M + 255) / 256);
-    p.tiles_n = tiles_n;
-    p.splits = 1;
-    p.k_per_split = (int)K;
-    p.a_bytes = (int)(M * K * 2);
-    p.bt_bytes = (int)(N * K * 2);
-    p.lds_epilogue = 1;
-    p.super_m = p.super_n = 1;
+    if (!N1 || N1 % 8 || N1 > 0x3fffffff || M * K * 2 >= buf_max || N * K * 2 >= buf_max || N1 * K * 2 >= buf_max) return MOON_OK;
+    if (!al16(A) || !al16(W) || !al16(bias) || !al16(W1) || !al16(bias1) || !al16(out1) || !al16(q_out) || !al16(cache_k) || !al16(cache_v) || !al16(table)) return MOON_OK;
+    // apart: two products and, 4.5 us, the rotation
+    double us;
+    const int columns0 = (int)((N + 255) / 256), mi = block_height(cus, M, columns0 + (N1 + 255) / 256, K / BK, &us);
+    if (us >= narrow_us(cus, M, N, K / BK) + narrow_us(cus, M, N1, K / BK) + 4.5) return MOON_OK;
+    GemmBlockArgs a{};
+    a.columns0 = columns0;
+    for (int i = 0; i < 2; i++) {
+        GemmArgs &p = a.p[i];
+        p.A = A;
+        p.Bt = i ? W1 : W;
+        p.bias = i ? bias1 : bias;
+        p.C = i ? out1 : nullptr;
+        p.M = (int)M;
+        p.N = (int)(i ? N1 : N);
+        p.K = (int)K;
+    }
+    GemmArgs &p = a.p[0];
     p.rope_q = q_out;
     p.rope_ck = cache_k;
     p.rope_cv = cache_v;
@@ -1222,20 +1350,7 @@ int launch_gemm_qkv_rope(moon_ctx *ctx, const half_t *A, const half_t *W, const 
     p.rope_dim = (int)rot_dim;
     p.rope_max_seq = (int)max_seq;
     p.rope_pos0 = (int)pos0;
-    const int total = p.tiles_m * p.tiles_n;
-    const size_t lds_bytes = use192 ? Dma2<3>::LDS_BYTES : Dma2<4>::LDS_BYTES;
-    static std::atomic<bool> attr_set[2][64];
-    const int dev = ctx->device >= 0 && ctx->device < 64 ? ctx->device : -1;
-    if (dev < 0 || !attr_set[use192 ? 1 : 0][dev].load()) {
-        const void *kern = use192 ? reinterpret_cast<const void *>(gemm_nt_dma192_rope_kernel) : reinterpret_cast<const void *>(gemm_nt_dma256_rope_kernel);
-        MOON_HIP(ctx, hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes));
-        if (dev >= 0) attr_set[use192 ? 1 : 0][dev].store(true);
-    }
-    const dim3 grid(((total + 7) / 8) * 8);
-    if (use192) hipLaunchKernelGGL(gemm_nt_dma192_rope_kernel, grid, dim3(DMA_THREADS), lds_bytes, ctx->stream, p);
-    else hipLaunchKernelGGL(gemm_nt_dma256_rope_kernel, grid, dim3(DMA_THREADS), lds_bytes, ctx->stream, p);
-    MOON_NOTE_KERNEL(ctx, "%s %d workgroups", use192 ? "gemm_nt_dma192_rope_kernel" : "gemm_nt_dma256_rope_kernel", total);
-    MOON_HIP(ctx, hipGetLastError());
+    MOON_TRY((launch_block<EPI_ROPE, MOON_EPI_BIAS_GELU>(ctx, a, mi)));
     *done = true;
     return MOON_OK;
 }

@@ -33,6 +33,9 @@ struct BlockBf16 {
         return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
     }
 };
+struct BlockF16 {
+    static __device__ __forceinline__ float4_t mul(const half8_t &a, const half8_t &b, const float4_t &c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
+};
 struct BlockSource {
     __amdgpu_buffer_rsrc_t a, w;
     int k, n_ktiles; // bytes of the next k-tile, how many are left

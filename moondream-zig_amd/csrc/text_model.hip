@@ -395,9 +395,9 @@ int layer_forward(moon_text_model *m, size_t layer, size_t n, size_t pos, bool p
         MOON_TRY(launch_gemv_nt(ctx, m->ln_in, fc1_w, fc1_b, m->fc1, z.ffn, z.d, MOON_EPI_BIAS_GELU));
         MOON_TRY(launch_gemv_nt(ctx, m->fc1, fc2_w, fc2_b, m->mlp, z.d, z.ffn, MOON_EPI_BIAS));
     } else {
-        bool roped = false; // the projection with the rotation and the cache update in its epilogue, where the shape has that form
-        MOON_TRY(launch_gemm_qkv_rope(ctx, m->ln_in, qkv_w, qkv_b, n, z.d, m->q_rot, ck, cv, m->freqs, z.H, z.D, m->cfg.rot_dim, z.S, pos, &roped));
-        if (!roped) {
+        bool front = false; // the projection, with the rotation and the cache update in its epilogue, and fc1 in one launch, where the shape has that form
+        MOON_TRY(launch_gemm_front(ctx, m->ln_in, qkv_w, qkv_b, fc1_w, fc1_b, m->fc1, z.ffn, n, z.d, m->q_rot, ck, cv, m->freqs, z.H, z.D, m->cfg.rot_dim, z.S, pos, &front));
+        if (!front) {
             MOON_TRY(launch_gemm(ctx, m->ln_in, qkv_w, qkv_b, m->qkv, n, 3 * z.d, z.d, MOON_B_NK, MOON_EPI_BIAS));
             MOON_TRY(launch_qkv_rope_cache(ctx, m->qkv, m->q_rot, ck, cv, m->freqs, n, z.H, z.D, m->cfg.rot_dim, z.S, pos));
         }
@@ -407,7 +407,7 @@ int layer_forward(moon_text_model *m, size_t layer, size_t n, size_t pos, bool p
             // out_proj and fc2 as one launch (each alone leaves a quarter of the device idle at 768 rows), finished together
             // with the LayerNorm that comes next: the next block's, or after the last block the model's final one (which the
             // LM head applies to the one row it needs by itself; here it only keeps the last block on the same launches)
-            MOON_TRY(launch_gemm(ctx, m->ln_in, fc1_w, fc1_b, m->fc1, n, z.ffn, z.d, MOON_B_NK, MOON_EPI_BIAS_GELU));
+            if (!front) MOON_TRY(launch_gemm(ctx, m->ln_in, fc1_w, fc1_b, m->fc1, n, z.ffn, z.d, MOON_B_NK, MOON_EPI_BIAS_GELU));
             const bool last = layer + 1 == z.L;
             GemmLayerNorm next{last ? m->lno_w : m->ln_w + (layer + 1) * z.d, last ? m->lno_b : m->ln_b + (layer + 1) * z.d, m->ln_in, m->cfg.ln_eps};
             next.add = m->attn_proj;
@@ -428,7 +428,7 @@ int layer_forward(moon_text_model *m, size_t layer, size_t n, size_t pos, bool p
             return launch_gemm(ctx, m->fc1, fc2_w, fc2_b, m->hidden, n, z.d, z.ffn, MOON_B_NK, 3 /* bias, then += into hidden */, m->hidden, &next);
         }
         MOON_TRY(launch_gemm(ctx, m->attn, out_w, out_b, m->attn_proj, n, z.d, z.d, MOON_B_NK, MOON_EPI_BIAS));
-        MOON_TRY(launch_gemm(ctx, m->ln_in, fc1_w, fc1_b, m->fc1, n, z.ffn, z.d, MOON_B_NK, MOON_EPI_BIAS_GELU));
+        if (!front) MOON_TRY(launch_gemm(ctx, m->ln_in, fc1_w, fc1_b, m->fc1, n, z.ffn, z.d, MOON_B_NK, MOON_EPI_BIAS_GELU));
         MOON_TRY(launch_gemm(ctx, m->fc1, fc2_w, fc2_b, m->mlp, n, z.d, z.ffn, MOON_B_NK, MOON_EPI_BIAS));
     }
     return launch_residual2(ctx, m->hidden, m->attn_proj, m->mlp, n * z.d);
