@@ -649,31 +649,16 @@ struct GemmBlockArgs {
     SegWalk walk;
 };
 // A wavefront's accumulators, 32 rows at a time through its 4 KiB of LDS: rounded to f16 and parked as rows of 128 bytes (16-byte granules XOR-swizzled by row),
-// then eight columns of a row per lane are finished and stored.  The wavefront's 64 columns are one head of a qkv projection: the partners that a rotated
-// column needs lie in the same parked row; what is written are the values, roundings and rotations of qkv_rope_cache_vec_kernel on the finished rows.
+// then eight columns of a row per lane are finished and stored.
 constexpr int EPI_ROPE = 4;
 template <int EPI, int MI>
 __device__ __forceinline__ void gemm_block_out(const GemmArgs &p, const float4_t (&acc)[4][2 * MI], int m_wave, int n0, int lane, char *scratch) {
     asm volatile("" : "+v"(lane)); // (per tile, see seg_store)
     if (n0 >= p.N) return;
-    const int row8 = lane >> 3, g8 = lane & 7, n = n0 + g8 * 8, d0 = g8 * 8;
+    const int row8 = lane >> 3, g8 = lane & 7, n = n0 + g8 * 8;
     const bool inside = n < p.N;
-    half8_t bias = {0, 0, 0, 0, 0, 0, 0, 0}, biasp = bias;
+    half8_t bias = {0, 0, 0, 0, 0, 0, 0, 0};
     if (EPI != MOON_EPI_NONE && inside) bias = *reinterpret_cast<const half8_t *>(p.bias + n);
-    half_t *out = p.C;
-    int ld = p.N, col = n, partner = 0;
-    bool rotated = false, low = false;
-    const int half = p.rope_dim >> 1;
-    if (EPI == EPI_ROPE) {
-        const int hd = p.rope_H * 64, region = n0 / hd, head = (n0 - region * hd) >> 6; // 0: q, 1: k, 2: v
-        rotated = region < 2 && d0 < p.rope_dim;
-        low = d0 < half;
-        partner = low ? half : -half;
-        if (rotated) biasp = *reinterpret_cast<const half8_t *>(p.bias + n + partner);
-        out = region == 0 ? p.rope_q + size_t(head) * p.M * 64 : (region == 1 ? p.rope_ck : p.rope_cv) + (size_t(head) * p.rope_max_seq + p.rope_pos0) * 64;
-        ld = 64;
-        col = d0;
-    }
 #pragma unroll
     for (int mi = 0; mi < MI; mi++) {
 #pragma unroll
@@ -696,38 +681,80 @@ __device__ __forceinline__ void gemm_block_out(const GemmArgs &p, const float4_t
             if (EPI == MOON_EPI_BIAS_RESID) res = *reinterpret_cast<const half8_t *>(p.resid + size_t(m) * p.N + n);
 #pragma unroll
             for (int e = 0; e < 8; e++) {
-                half_t x = apply_epilogue_v<EPI == EPI_ROPE ? MOON_EPI_BIAS : EPI>((float)v[e], bias[e]);
+                half_t x = apply_epilogue_v<EPI>((float)v[e], bias[e]);
                 if (EPI == MOON_EPI_BIAS_RESID) x = (half_t)((float)res[e] + (float)x);
                 o[e] = x;
             }
-            if (EPI == EPI_ROPE && rotated) {
-                const half8_t vp = *reinterpret_cast<const half8_t *>(scratch + ml * 128 + ((g8 + (partner >> 3)) ^ (ml & 7)) * 16);
-                const float4 *tab = reinterpret_cast<const float4 *>(p.rope_table + ((size_t)(p.rope_pos0 + m) * half + (low ? d0 : d0 - half)) * 2);
-#pragma unroll
-                for (int e4 = 0; e4 < 4; e4++) {
-                    const float4 cs = tab[e4]; // (cos, sin) of two consecutive d
-#pragma unroll
-                    for (int j = 0; j < 2; j++) {
-                        const int e = 2 * e4 + j;
-                        const float c = j ? cs.z : cs.x, sn = j ? cs.w : cs.y;
-                        const half_t mine = o[e], other = apply_epilogue_v<MOON_EPI_BIAS>((float)vp[e], biasp[e]);
-                        half_t a, b;
-                        if (low) {
-                            rotate_pair((float)mine, (float)other, c, sn, a, b);
-                            o[e] = a;
-                        } else {
-                            rotate_pair((float)other, (float)mine, c, sn, a, b);
-                            o[e] = b;
-                        }
-                    }
-                }
-            }
-            *reinterpret_cast<half8_t *>(out + size_t(m) * ld + col) = o;
+            *reinterpret_cast<half8_t *>(p.C + size_t(m) * p.N + n) = o;
         }
         asm volatile("" ::: "memory");
     }
     // (used on every path: a load that may still be under way at the head of the next tile's loop would be waited for, with all copies, in each of its rounds)
-    asm volatile("" ::"v"(bias), "v"(biasp));
+    asm volatile("" ::"v"(bias));
+}
+// The same for a qkv projection whose heads' first 32 dimensions of 64 are rotated: the wavefront's 64 columns are one head of q, k or v, a column and its partner 16
+// further on are in one lane, and what is written are the values, roundings and rotations of qkv_rope_cache_vec_kernel on the finished rows.  Rotated where they
+// lie, before they are parked, with the angles of the next 32 rows on their way: from the parked rows, a row's angles after another, every 8 rows of
+// the tile waited for the table (900 rows of width 2048: 70 us with fc1, 57 so).
+template <int MI>
+__device__ __forceinline__ void gemm_block_out_rope(const GemmArgs &p, const float4_t (&acc)[4][2 * MI], int m_wave, int n0, int lane, char *scratch) {
+    asm volatile("" : "+v"(lane));
+    if (n0 >= p.N) return;
+    const int row8 = lane >> 3, g8 = lane & 7, col = lane & 15, quad = lane >> 4;
+    const int hd = p.rope_H * 64, region = n0 / hd, head = (n0 - region * hd) >> 6; // 0: q, 1: k, 2: v
+    half_t *out = region == 0 ? p.rope_q + size_t(head) * p.M * 64 : (region == 1 ? p.rope_ck : p.rope_cv) + (size_t(head) * p.rope_max_seq + p.rope_pos0) * 64;
+    half4_t bias[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) bias[i] = *reinterpret_cast<const half4_t *>(p.bias + n0 + 16 * i + 4 * quad);
+    float4 angle[2][2], next[2][2]; // [16 rows]: (cos, sin) of two columns, of the two behind them
+    auto fetch = [&](int mi, float4 (&t)[2][2]) {
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int m = min(m_wave + mi * 32 + h * 16 + col, p.M - 1);
+            const float4 *from = reinterpret_cast<const float4 *>(p.rope_table + ((size_t)(p.rope_pos0 + m) * 16 + 4 * quad) * 2);
+            t[h][0] = from[0];
+            t[h][1] = from[1];
+        }
+    };
+    fetch(0, next);
+#pragma unroll
+    for (int mi = 0; mi < MI; mi++) {
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+            for (int j = 0; j < 2; j++) angle[h][j] = next[h][j];
+        if (mi + 1 < MI) fetch(mi + 1, next);
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            half4_t o[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) o[i][e] = apply_epilogue_v<MOON_EPI_BIAS>(acc[i][2 * mi + h][e], bias[i][e]);
+            if (region < 2) {
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const float4 cs = angle[h][e >> 1];
+                    half_t a, b;
+                    rotate_pair((float)o[0][e], (float)o[1][e], e & 1 ? cs.z : cs.x, e & 1 ? cs.w : cs.y, a, b);
+                    o[0][e] = a;
+                    o[1][e] = b;
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int r = 16 * h + col, g = 2 * i + (quad >> 1);
+                *reinterpret_cast<half4_t *>(scratch + r * 128 + (g ^ (r & 7)) * 16 + (quad & 1) * 8) = o[i];
+            }
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int ml = r * 8 + row8, m = m_wave + mi * 32 + ml;
+            if (m < p.M) *reinterpret_cast<half8_t *>(out + size_t(m) * 64 + g8 * 8) = *reinterpret_cast<const half8_t *>(scratch + ml * 128 + (g8 ^ (ml & 7)) * 16);
+        }
+        asm volatile("" ::: "memory");
+    }
 }
 struct GemmBlockTile {
     int m0, n0, second;
@@ -768,7 +795,8 @@ __global__ __launch_bounds__(DMA_THREADS) void gemm_nt_block_kernel(GemmBlockArg
             if constexpr (EPI2 >= 0) {
                 if (t.second) return gemm_block_out<EPI2, MI>(a.p[1], acc, m, n, lane, scratch);
             }
-            gemm_block_out<EPI, MI>(a.p[0], acc, m, n, lane, scratch);
+            if constexpr (EPI == EPI_ROPE) gemm_block_out_rope<MI>(a.p[0], acc, m, n, lane, scratch);
+            else gemm_block_out<EPI, MI>(a.p[0], acc, m, n, lane, scratch);
         });
 }
 
@@ -1322,13 +1350,13 @@ int launch_gemm_front(moon_ctx *ctx, const half_t *A, const half_t *W, const hal
     const size_t N = 3 * H * D, buf_max = (size_t(1) << 31) - 4096;
     const auto al16 = [](const void *q) { return reinterpret_cast<uintptr_t>(q) % 16 == 0; };
     if (ctx->gemm_kernel[0] || getenv("MOON_GEMM_NO_ROPE")) return MOON_OK; // (a kernel was named for measurements, or the fusion switched off)
-    if (D != 64 || !H || rot_dim % 16 || rot_dim > D || !M || M > 0x3fffffff || K % BK || !K || pos0 + M > max_seq || max_seq > 0x3fffffff) return MOON_OK;
+    if (D != 64 || !H || rot_dim != 32 || !M || M > 0x3fffffff || K % BK || !K || pos0 + M > max_seq || max_seq > 0x3fffffff) return MOON_OK;
     if (!N1 || N1 % 8 || N1 > 0x3fffffff || M * K * 2 >= buf_max || N * K * 2 >= buf_max || N1 * K * 2 >= buf_max) return MOON_OK;
     if (!al16(A) || !al16(W) || !al16(bias) || !al16(W1) || !al16(bias1) || !al16(out1) || !al16(q_out) || !al16(cache_k) || !al16(cache_v) || !al16(table)) return MOON_OK;
-    // apart: two products and, 4.5 us, the rotation
+    // apart: two products, the GELU of one (2.5 us) and the rotation (4.5)
     double us;
     const int columns0 = (int)((N + 255) / 256), mi = block_height(cus, M, columns0 + (N1 + 255) / 256, K / BK, &us);
-    if (us >= narrow_us(cus, M, N, K / BK) + narrow_us(cus, M, N1, K / BK) + 4.5) return MOON_OK;
+    if (us >= narrow_us(cus, M, N, K / BK) + narrow_us(cus, M, N1, K / BK) + 7.0) return MOON_OK;
     GemmBlockArgs a{};
     a.columns0 = columns0;
     for (int i = 0; i < 2; i++) {
@@ -1347,7 +1375,6 @@ int launch_gemm_front(moon_ctx *ctx, const half_t *A, const half_t *W, const hal
     p.rope_cv = cache_v;
     p.rope_table = table;
     p.rope_H = (int)H;
-    p.rope_dim = (int)rot_dim;
     p.rope_max_seq = (int)max_seq;
     p.rope_pos0 = (int)pos0;
     MOON_TRY((launch_block<EPI_ROPE, MOON_EPI_BIAS_GELU>(ctx, a, mi)));

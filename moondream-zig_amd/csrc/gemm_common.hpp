@@ -26,8 +26,8 @@ struct GemmArgs {
     // a product whose epilogue is EPI_ROPE only: it is a decoder block's qkv projection [M, 3 * H * 64]; instead of C they write the
     // rotated q [H][M][64] and the cache rows [H][max_seq][64] of k (rotated) and v at positions pos0 .. pos0 + M - 1
     half_t *rope_q, *rope_ck, *rope_cv;
-    const float *rope_table; // [max_seq][rot_dim / 2][2] (cos, sin)
-    int rope_H, rope_dim, rope_max_seq, rope_pos0;
+    const float *rope_table; // [max_seq][16][2] (cos, sin): 32 of a head's dimensions are rotated
+    int rope_H, rope_max_seq, rope_pos0;
 };
 
 template <int N>
