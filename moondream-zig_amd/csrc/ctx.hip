@@ -116,7 +116,7 @@ extern "C" void moon_ctx_destroy(moon_ctx *ctx) {
 extern "C" int moon_set_gemm_kernel(moon_ctx *ctx, const char *name) {
     if (!ctx) return MOON_EINVAL;
     std::lock_guard<std::mutex> lock(ctx->mu);
-    static const char *const known[] = {"", "regs", "dma", "dma256", "b192", "b256", "w114", "w212", "w221"};
+    static const char *const known[] = {"", "regs", "dma", "dma256", "b192", "b256", "thin", "w114", "w212", "w221"};
     if (!name) name = "";
     for (const char *k : known)
         if (!strcmp(name, k)) {

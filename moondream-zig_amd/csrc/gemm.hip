@@ -21,6 +21,7 @@
 #include <cstring>
 
 #include "gemm_block.hpp"
+#include "gemm_thin.hpp"
 #include "gemm_wide.hpp"
 #include "seg_schedule.hpp"
 
@@ -759,31 +760,33 @@ __device__ __forceinline__ void gemm_block_out_rope(const GemmArgs &p, const flo
 struct GemmBlockTile {
     int m0, n0, second;
 };
+template <class S, bool TWO>
+__device__ __forceinline__ bool gemm_block_next(const GemmBlockArgs &a, GemmBlockTile &t, int &round) {
+    int tm, tn, range;
+    for (;;) {
+        const int r = seg_find(a.walk, blockIdx.x % SEG_DIES, seg_slot(0, blockIdx.x / SEG_DIES, gridDim.x / SEG_DIES, round++), tm, tn, range);
+        if (r < 0) return false;
+        if (r > 0) break;
+    }
+    t.second = TWO && tn >= a.columns0;
+    t.m0 = tm * S::ROWS;
+    t.n0 = (t.second ? tn - a.columns0 : tn) * S::COLUMNS;
+    return true;
+}
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t gemm_rows(const half_t *from, int first, int n, int pitch) { // rows first .. first + n - 1
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(reinterpret_cast<const char *>(from)) + size_t(first) * pitch, 0, n * pitch, 0x00020000);
+}
 template <int EPI, int EPI2, int MI>
 __global__ __launch_bounds__(DMA_THREADS) void gemm_nt_block_kernel(GemmBlockArgs a) {
     extern __shared__ __attribute__((aligned(16))) half_t lds_block[]; // (the tile product addresses LDS from 0)
     using S = Block<MI>;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    auto next = [&](GemmBlockTile &t, int &round) {
-        int tm, tn, range;
-        for (;;) {
-            const int r = seg_find(a.walk, blockIdx.x % SEG_DIES, seg_slot(0, blockIdx.x / SEG_DIES, gridDim.x / SEG_DIES, round++), tm, tn, range);
-            if (r < 0) return false;
-            if (r > 0) break;
-        }
-        t.second = EPI2 >= 0 && tn >= a.columns0;
-        t.m0 = tm * S::ROWS;
-        t.n0 = (t.second ? tn - a.columns0 : tn) * S::COLUMNS;
-        return true;
-    };
+    auto next = [&](GemmBlockTile &t, int &round) { return gemm_block_next<S, EPI2 >= 0>(a, t, round); };
     const int pitch = a.p[0].K * 2;
-    auto buffer = [&](const half_t *from, int first, int n) {
-        return __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(reinterpret_cast<const char *>(from)) + size_t(first) * pitch, 0, n * pitch, 0x00020000);
-    };
     auto open = [&](const GemmBlockTile &t, BlockSource &s) {
         const GemmArgs &p = EPI2 >= 0 && t.second ? a.p[1] : a.p[0];
-        s.a = buffer(p.A, t.m0, min(p.M - t.m0, S::ROWS));
-        s.w = buffer(p.Bt, t.n0, min(p.N - t.n0, S::COLUMNS));
+        s.a = gemm_rows(p.A, t.m0, min(p.M - t.m0, S::ROWS), pitch);
+        s.w = gemm_rows(p.Bt, t.n0, min(p.N - t.n0, S::COLUMNS), pitch);
         s.k = 0;
         s.n_ktiles = p.K / BK;
     };
@@ -797,6 +800,37 @@ __global__ __launch_bounds__(DMA_THREADS) void gemm_nt_block_kernel(GemmBlockArg
             }
             if constexpr (EPI == EPI_ROPE) gemm_block_out_rope<MI>(a.p[0], acc, m, n, lane, scratch);
             else gemm_block_out<EPI, MI>(a.p[0], acc, m, n, lane, scratch);
+        });
+}
+
+// The same for few rows in tiles of 128 x 64 (gemm_thin.hpp).
+template <int EPI, int EPI2>
+__global__ __launch_bounds__(DMA_THREADS) void gemm_nt_thin_kernel(GemmBlockArgs a) {
+    extern __shared__ __attribute__((aligned(16))) half_t lds_thin[];
+    const int lane = threadIdx.x & 63, role_wave = __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) & 3);
+    int round = 0;
+    auto next = [&](GemmBlockTile &t) { return gemm_block_next<Thin, EPI2 >= 0>(a, t, round); };
+    if (threadIdx.x >= 256) {
+        thin_load<GemmBlockTile>(lds_thin, role_wave, lane, next, [&](const GemmBlockTile &t, BlockSource &s, int &pitch_a, int &pitch_w) {
+            const GemmArgs &p = EPI2 >= 0 && t.second ? a.p[1] : a.p[0];
+            pitch_a = pitch_w = p.K * 2;
+            s.a = gemm_rows(p.A, t.m0, min(p.M - t.m0, Thin::ROWS), pitch_a);
+            s.w = gemm_rows(p.Bt, t.n0, min(p.N - t.n0, Thin::COLUMNS), pitch_w);
+            s.k = 0;
+            s.n_ktiles = p.K / BK;
+        });
+        return;
+    }
+    char *scratch = reinterpret_cast<char *>(lds_thin) + Thin::STAGES * Thin::STAGE_BYTES + role_wave * Thin::SCRATCH_BYTES;
+    thin_multiply<BlockF16, GemmBlockTile>(
+        role_wave, lane, next, [&](const GemmBlockTile &) { return a.p[0].K / BK; },
+        [&](const GemmBlockTile &t, const float4_t (&acc)[4][2]) {
+            const int m = t.m0 + 32 * role_wave;
+            if constexpr (EPI2 >= 0) {
+                if (t.second) return gemm_block_out<EPI2, 1>(a.p[1], acc, m, t.n0, lane, scratch);
+            }
+            if constexpr (EPI == EPI_ROPE) gemm_block_out_rope<1>(a.p[0], acc, m, t.n0, lane, scratch);
+            else gemm_block_out<EPI, 1>(a.p[0], acc, m, t.n0, lane, scratch);
         });
 }
 
@@ -820,6 +854,77 @@ __global__ __launch_bounds__(DMA_THREADS) void gemm_nt_dma192_pair_kernel(GemmPa
     const int k_begin = split * p.k_per_split, k_end = min(p.K, k_begin + p.k_per_split);
     if (k_end <= k_begin) return;
     gemm_nt_dma2_body<MOON_EPI_NONE, 3, true>(p, tile, k_begin / BK, (k_end - k_begin) / BK, split);
+}
+
+// A wavefront's sums as they are, to slab `split`: 32 rows by 32 columns at a time through its LDS, so that the stores are whole lines.
+template <int MI>
+__device__ __forceinline__ void gemm_block_partial(const GemmArgs &p, const float4_t (&acc)[4][2 * MI], int m_wave, int n0, int split, int lane, char *scratch) {
+    asm volatile("" : "+v"(lane));
+    const int row8 = lane >> 3, g8 = lane & 7;
+#pragma unroll
+    for (int mi = 0; mi < MI; mi++)
+#pragma unroll
+        for (int ni = 0; ni < 2; ni++) {
+            const int n = n0 + 32 * ni + 4 * g8;
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    const int r = 16 * h + (lane & 15), g = 4 * i + (lane >> 4);
+                    *reinterpret_cast<float4_t *>(scratch + r * 128 + (g ^ (r & 7)) * 16) = acc[2 * ni + i][2 * mi + h];
+                }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int ml = r * 8 + row8, m = m_wave + mi * 32 + ml;
+                const float4_t v = *reinterpret_cast<const float4_t *>(scratch + ml * 128 + (g8 ^ (ml & 7)) * 16);
+                if (m < p.M && n < p.N) *reinterpret_cast<float4_t *>(p.partial + (size_t(split) * p.M + m) * p.N + n) = v;
+            }
+            asm volatile("" ::: "memory");
+        }
+}
+// The same two products for few rows: tiles of 128 x 64 times the ranges of k.
+struct GemmThinUnit {
+    int m0, n0, second, split;
+};
+__global__ __launch_bounds__(DMA_THREADS) void gemm_nt_thin_pair_kernel(GemmPairArgs a) {
+    extern __shared__ __attribute__((aligned(16))) half_t lds_thin[];
+    const int lane = threadIdx.x & 63, role_wave = __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) & 3);
+    const int per_xcd = (a.units_total + 7) / 8, unit = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
+    if (unit >= a.units_total || (int)blockIdx.x / 8 >= per_xcd) return;
+    bool taken = false;
+    auto next = [&](GemmThinUnit &t) { // one unit per workgroup
+        if (taken) return false;
+        taken = true;
+        t.second = unit >= a.units0;
+        const GemmArgs &p = t.second ? a.p[1] : a.p[0];
+        const int u = t.second ? unit - a.units0 : unit, tiles = p.tiles_m * p.tiles_n, tile = u % tiles;
+        t.split = u / tiles;
+        t.m0 = tile % p.tiles_m * Thin::ROWS;
+        t.n0 = tile / p.tiles_m * Thin::COLUMNS;
+        return true;
+    };
+    auto range = [&](const GemmThinUnit &t, int &k0) {
+        const GemmArgs &p = t.second ? a.p[1] : a.p[0];
+        k0 = t.split * p.k_per_split;
+        return (min(p.K, k0 + p.k_per_split) - k0) / BK;
+    };
+    if (threadIdx.x >= 256) {
+        thin_load<GemmThinUnit>(lds_thin, role_wave, lane, next, [&](const GemmThinUnit &t, BlockSource &s, int &pitch_a, int &pitch_w) {
+            const GemmArgs &p = t.second ? a.p[1] : a.p[0];
+            pitch_a = pitch_w = p.K * 2;
+            s.a = gemm_rows(p.A, t.m0, min(p.M - t.m0, Thin::ROWS), pitch_a);
+            s.w = gemm_rows(p.Bt, t.n0, min(p.N - t.n0, Thin::COLUMNS), pitch_w);
+            int k0;
+            s.n_ktiles = range(t, k0);
+            s.k = k0 * 2;
+        });
+        return;
+    }
+    char *scratch = reinterpret_cast<char *>(lds_thin) + Thin::STAGES * Thin::STAGE_BYTES + role_wave * Thin::SCRATCH_BYTES;
+    thin_multiply<BlockF16, GemmThinUnit>(
+        role_wave, lane, next, [&](const GemmThinUnit &t) { int k0; return range(t, k0); },
+        [&](const GemmThinUnit &t, const float4_t (&acc)[4][2]) { gemm_block_partial<1>(t.second ? a.p[1] : a.p[0], acc, t.m0 + 32 * role_wave, t.n0, t.split, lane, scratch); });
 }
 
 template <int EPI>
@@ -977,6 +1082,24 @@ __global__ __launch_bounds__(256) void transpose_kernel(const half_t *__restrict
     }
 }
 
+template <int EPI, int EPI2>
+int launch_thin(moon_ctx *ctx, GemmBlockArgs &a) {
+    const int cus = std::max(SEG_DIES, (ctx->cu_count > 0 ? ctx->cu_count : 256) / SEG_DIES * SEG_DIES);
+    const int kb[2] = {0, a.p[0].K}, columns = a.columns0 + (EPI2 >= 0 ? (a.p[1].N + Thin::COLUMNS - 1) / Thin::COLUMNS : 0);
+    a.walk = seg_walk((a.p[0].M + Thin::ROWS - 1) / Thin::ROWS, columns, false, kb, 1, 0);
+    static std::atomic<bool> attr_set[64];
+    const int dev = ctx->device >= 0 && ctx->device < 64 ? ctx->device : -1;
+    const auto kern = gemm_nt_thin_kernel<EPI, EPI2>;
+    if (dev < 0 || !attr_set[dev].load()) { // this much dynamic LDS needs the opt-in once per device and instantiation
+        MOON_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)Thin::LDS_BYTES));
+        if (dev >= 0) attr_set[dev].store(true);
+    }
+    hipLaunchKernelGGL(kern, dim3((unsigned)seg_workgroups(a.walk, cus)), dim3(DMA_THREADS), Thin::LDS_BYTES, ctx->stream, a);
+    MOON_HIP(ctx, hipGetLastError());
+    MOON_NOTE_KERNEL(ctx, "gemm_nt_thin_kernel %d tiles", a.walk.all);
+    return MOON_OK;
+}
+
 // What products take, us, launch included, with weights from HBM, kt k-tiles: fitted to 54 products of 200 to 1920 rows by 3072 to 14336 columns by 1024 or 2048.
 // Tiles of 64 mi x 256 in rounds over the units; f: part of the units that a round keeps busy.
 double block_us(int cus, int mi, size_t M, size_t columns, size_t kt) {
@@ -992,6 +1115,11 @@ int block_height(int cus, size_t M, size_t columns, size_t kt, double *us) {
     const double three = block_us(cus, 3, M, columns, kt), four = block_us(cus, 4, M, columns, kt);
     *us = std::min(three, four);
     return three <= four ? 3 : 4;
+}
+// Tiles of 128 x 64 (gemm_thin.hpp), at most one per unit; otherwise never.
+double thin_us(int cus, size_t M, size_t N, size_t kt) {
+    const size_t tiles = (M + Thin::ROWS - 1) / Thin::ROWS * ((N + Thin::COLUMNS - 1) / Thin::COLUMNS);
+    return tiles > (size_t)cus ? 1e30 : 5.5 + kt * (0.24 + 0.1 * tiles / cus + 0.0008 * std::min(M, (size_t)Thin::ROWS));
 }
 // The narrow kernels as run_gemm takes them: 128 x 128 tiles, split in k where they are few (the reduction 6 us), otherwise a workgroup per tile of 192 or 256 rows.
 double narrow_us(int cus, size_t M, size_t N, size_t kt) {
@@ -1161,6 +1289,14 @@ int run_gemm(moon_ctx *ctx, const half_t *A, const half_t *B, const half_t *bias
             MOON_HIP(ctx, hipGetLastError());
         }
         return MOON_OK;
+    }
+    // Tiles of 128 x 64 (gemm_thin.hpp) are taken where they are named (MOON_GEMM_KERNEL=thin): by themselves they would beat ranges of k at some shapes (160 x 8192 x
+    // 2048 21.6 -> 14.9 us), but a [K, N] operand and its [N, K] copy have to give the same bits, and there is no such kernel for the former.
+    if (force && !strcmp(force, "thin") && buffers_ok && K % BK == 0 && N % 8 == 0 && p.lds_epilogue && !must_fuse) {
+        GemmBlockArgs a{};
+        a.p[0] = p;
+        a.columns0 = (N + Thin::COLUMNS - 1) / Thin::COLUMNS;
+        return launch_thin<EPI, -1>(ctx, a);
     }
     // Wide tiles (gemm_block.hpp) where the narrow ones come to more than one per unit and are estimated to take longer: 1025 x 8192 x 2048 58 -> 43 us, 1301 x 6144 x
     // 2048 53 -> 40, 1536 x 8192 x 8192 218 -> 165; 768 x 8192 x 2048 keeps one round of 192 x 128 (31 against 41).  MOON_GEMM_KERNEL=b192|b256 names them.
@@ -1356,9 +1492,10 @@ int launch_gemm_front(moon_ctx *ctx, const half_t *A, const half_t *W, const hal
     // apart: two products, the GELU of one (2.5 us) and the rotation (4.5)
     double us;
     const int columns0 = (int)((N + 255) / 256), mi = block_height(cus, M, columns0 + (N1 + 255) / 256, K / BK, &us);
-    if (us >= narrow_us(cus, M, N, K / BK) + narrow_us(cus, M, N1, K / BK) + 7.0) return MOON_OK;
+    const double thin = N % Thin::COLUMNS ? 1e30 : thin_us(cus, M, N + N1, K / BK);
+    if (std::min(us, thin) >= narrow_us(cus, M, N, K / BK) + narrow_us(cus, M, N1, K / BK) + 7.0) return MOON_OK;
     GemmBlockArgs a{};
-    a.columns0 = columns0;
+    a.columns0 = thin < us ? (int)(N / Thin::COLUMNS) : columns0;
     for (int i = 0; i < 2; i++) {
         GemmArgs &p = a.p[i];
         p.A = A;
@@ -1377,7 +1514,8 @@ int launch_gemm_front(moon_ctx *ctx, const half_t *A, const half_t *W, const hal
     p.rope_H = (int)H;
     p.rope_max_seq = (int)max_seq;
     p.rope_pos0 = (int)pos0;
-    MOON_TRY((launch_block<EPI_ROPE, MOON_EPI_BIAS_GELU>(ctx, a, mi)));
+    if (thin < us) MOON_TRY((launch_thin<EPI_ROPE, MOON_EPI_BIAS_GELU>(ctx, a)));
+    else MOON_TRY((launch_block<EPI_ROPE, MOON_EPI_BIAS_GELU>(ctx, a, mi)));
     *done = true;
     return MOON_OK;
 }
@@ -1389,12 +1527,14 @@ int launch_gemm_pair_ln(moon_ctx *ctx, const half_t *A_add, const half_t *B_add,
     const size_t buf_max = (size_t(1) << 31) - 4096;
     const auto al16 = [](const void *q) { return reinterpret_cast<uintptr_t>(q) % 16 == 0; };
     if (ctx->gemm_kernel[0] || getenv("MOON_GEMM_NO_PAIR")) return MOON_OK; // (a kernel was named for measurements: the products run one by one)
-    if (M < 192 || M > 0x3fffffff || N % 8 || N > (size_t)LN_FUSE_MAX_N || K % BK || K_add % BK || !K || !K_add) return MOON_OK;
+    if (M < 2 || M > 0x3fffffff || N % 8 || N > (size_t)LN_FUSE_MAX_N || K % BK || K_add % BK || !K || !K_add) return MOON_OK;
     if (M * K * 2 >= buf_max || N * K * 2 >= buf_max || M * K_add * 2 >= buf_max || N * K_add * 2 >= buf_max) return MOON_OK;
     if (!al16(A) || !al16(B) || !al16(A_add) || !al16(B_add) || !al16(bias) || !al16(bias_add) || !al16(resid) || !al16(C) || !al16(ln.gamma) ||
         !al16(ln.beta) || !al16(ln.out) || !ln.add || !al16(ln.add))
         return MOON_OK;
-    const int tiles_m = (int)((M + 191) / 192), tiles_n = (int)((N + BN - 1) / BN), tiles = tiles_m * tiles_n;
+    // below 192 rows tiles of 128 x 64 (gemm_thin.hpp): 37 rows of width 2048, apart 8.3 and 15.9 us
+    const bool thin = M < 192;
+    const int tile_m = thin ? Thin::ROWS : 192, tile_n = thin ? Thin::COLUMNS : BN, tiles_m = (int)((M + tile_m - 1) / tile_m), tiles_n = (int)((N + tile_n - 1) / tile_n), tiles = tiles_m * tiles_n;
     if (tiles * 2 > cus) return MOON_OK;
     // splits (s_add, s): all workgroups in one round, the longest run of k-tiles as short as it gets
     const int kt_add = (int)(K_add / BK), kt = (int)(K / BK);
@@ -1437,15 +1577,16 @@ int launch_gemm_pair_ln(moon_ctx *ctx, const half_t *A_add, const half_t *B_add,
     MOON_TRY(fill(a.p[1], A, B, K, best_s, ctx->work[0]));
     a.units0 = tiles * a.p[0].splits;
     a.units_total = a.units0 + tiles * a.p[1].splits;
-    static std::atomic<bool> attr_set[64];
+    static std::atomic<bool> attr_set[2][64];
     const int dev = ctx->device >= 0 && ctx->device < 64 ? ctx->device : -1;
-    if (dev < 0 || !attr_set[dev].load()) {
-        MOON_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_nt_dma192_pair_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                          (int)Dma2<3>::LDS_BYTES));
-        if (dev >= 0) attr_set[dev].store(true);
+    const auto kern = thin ? gemm_nt_thin_pair_kernel : gemm_nt_dma192_pair_kernel;
+    const size_t lds_bytes = thin ? Thin::LDS_BYTES : Dma2<3>::LDS_BYTES;
+    if (dev < 0 || !attr_set[thin][dev].load()) {
+        MOON_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes));
+        if (dev >= 0) attr_set[thin][dev].store(true);
     }
-    hipLaunchKernelGGL(gemm_nt_dma192_pair_kernel, dim3(((a.units_total + 7) / 8) * 8), dim3(DMA_THREADS), Dma2<3>::LDS_BYTES, ctx->stream, a);
-    MOON_NOTE_KERNEL(ctx, "gemm_nt_dma192_pair_kernel %d + %d workgroups, k splits %d and %d + splitk_reduce_ln_kernel", a.units0, a.units_total - a.units0,
+    hipLaunchKernelGGL(kern, dim3(((a.units_total + 7) / 8) * 8), dim3(DMA_THREADS), lds_bytes, ctx->stream, a);
+    MOON_NOTE_KERNEL(ctx, "%s %d + %d workgroups, k splits %d and %d + splitk_reduce_ln_kernel", thin ? "gemm_nt_thin_pair_kernel" : "gemm_nt_dma192_pair_kernel", a.units0, a.units_total - a.units0,
                      a.p[0].splits, a.p[1].splits);
     MOON_HIP(ctx, hipGetLastError());
     hipLaunchKernelGGL(splitk_reduce_ln_kernel<MOON_EPI_BIAS_RESID>, dim3((unsigned)M), dim3(256), 0, ctx->stream, a.p[1].partial, bias, resid, ln.add,

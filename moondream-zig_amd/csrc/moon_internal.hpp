@@ -145,7 +145,7 @@ int launch_gemm_front(moon_ctx *ctx, const half_t *A, const half_t *W, const hal
 // Two products with the same [M, N] result in ONE launch, then the launch that finishes both, as launch_gemm does with
 // ln->add_partial set: C = f16(resid + f16(add + t)), add = f16(f16(A_add . B_add^T) + bias_add), t = f16(f16(A . B^T) + bias),
 // and the LayerNorm of the finished rows into ln.out (ln.add must name M x N halfs all the same).  Both B operands are [N, K].
-// Only for shapes where that fills the device in one round (M >= 192, N <= 2048, K's multiples of 64, 16-byte aligned
+// Only for shapes where that fits the device in one round (M >= 2, N <= 2048, K's multiples of 64, 16-byte aligned
 // operands); *done says whether anything was launched, and if not the caller runs the products one by one.
 int launch_gemm_pair_ln(moon_ctx *ctx, const half_t *A_add, const half_t *B_add, const half_t *bias_add, size_t K_add, const half_t *A, const half_t *B,
                         const half_t *bias, size_t K, const half_t *resid, half_t *C, size_t M, size_t N, const GemmLayerNorm &ln, bool *done);
