@@ -1116,10 +1116,13 @@ int block_height(int cus, size_t M, size_t columns, size_t kt, double *us) {
     *us = std::min(three, four);
     return three <= four ? 3 : 4;
 }
-// Tiles of 128 x 64 (gemm_thin.hpp), at most one per unit; otherwise never.
+// Tiles of 128 x 64 (gemm_thin.hpp); later rounds find their first k-tiles on their way.
 double thin_us(int cus, size_t M, size_t N, size_t kt) {
-    const size_t tiles = (M + Thin::ROWS - 1) / Thin::ROWS * ((N + Thin::COLUMNS - 1) / Thin::COLUMNS);
-    return tiles > (size_t)cus ? 1e30 : 5.5 + kt * (0.24 + 0.1 * tiles / cus + 0.0008 * std::min(M, (size_t)Thin::ROWS));
+    const size_t rows = (M + Thin::ROWS - 1) / Thin::ROWS, tiles = rows * ((N + Thin::COLUMNS - 1) / Thin::COLUMNS);
+    double us = 5.5;
+    for (size_t left = tiles; left > 0; left -= std::min(left, (size_t)cus))
+        us += (left < tiles ? 0.85 : 1.0) * kt * (0.24 + 0.1 * std::min(left, (size_t)cus) / cus + 0.0008 * M / rows);
+    return us;
 }
 // The narrow kernels as run_gemm takes them: 128 x 128 tiles, split in k where they are few (the reduction 6 us), otherwise a workgroup per tile of 192 or 256 rows.
 double narrow_us(int cus, size_t M, size_t N, size_t kt) {

@@ -116,9 +116,9 @@ struct SegGemm {
     int longest_first;        // the tiles of the longest k-range start first, on every die (where the ranges differ); otherwise no range may be longer than the first
     int c32_rows;             // splits > 1: rows that c32 has room for, all slabs together
     float softcap;            // > 0: on the f32 segment
-    int tile;                 // bf16, no list: 2, 3, 4: tiles of so many 64 rows and 128 columns, SEG_BLOCK + 3, + 4: and 256 columns; 0: by shape
+    int tile;                 // bf16, no list: 2, 3, 4: tiles of so many 64 rows and 128 columns, SEG_BLOCK + 3, + 4: and 256 columns, SEG_THIN + 2: and 64; 0: by shape
 };
-constexpr int SEG_BLOCK = 16;
+constexpr int SEG_BLOCK = 16, SEG_THIN = 32;
 constexpr int SEG_TILE_ROWS = 128; // rows of a tile (both element types walk tile lists of this height)
 int launch_seg_gemm(moon_ctx *ctx, int dtype, SegGemm p);
 // k splits worth taking for an all-f32 product of this shape; together their slabs have at most max_rows rows

@@ -2,6 +2,7 @@
 // and grouped where a router asks for it.  bf16 runs on the matrix cores through the stream of tiles of gemm_stream.hpp; f32 is computed with f32 multiply-adds (no reduced-precision mode).
 #include "gemm_block.hpp"
 #include "gemm_stream.hpp"
+#include "gemm_thin.hpp"
 #include "layer_list.hpp"
 #include "lm_types.hpp"
 #include "seg_schedule.hpp"
@@ -175,6 +176,10 @@ __global__ __launch_bounds__(DMA_THREADS) void seg_gemm_bf16_kernel(SegGemm p, S
                                            [&](const TilePos &t, const float16_t (&acc)[2][MI]) { seg_store<Pieces32, MI>(p, acc, t, wm, wn, lane, scratch); });
 }
 
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t seg_rows(const void *from, int first, int n, int pitch) { // n rows (the launcher has checked that both operands fit a descriptor)
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(reinterpret_cast<const char *>(from)) + size_t(first) * pitch, 0, n * pitch, 0x00020000);
+}
+
 // The same in tiles of 64 MI x 256 (gemm_block.hpp); no gathered rows and no list.
 template <int MI>
 __global__ __launch_bounds__(DMA_THREADS) void seg_gemm_bf16_block_kernel(SegGemm p, SegWalk w) {
@@ -188,18 +193,43 @@ __global__ __launch_bounds__(DMA_THREADS) void seg_gemm_bf16_block_kernel(SegGem
         }
     };
     auto ktiles = [&](const TilePos &t) { return (p.kb[t.split + 1] - p.kb[t.split]) / BK; };
-    auto buffer = [](const void *from, int first, int n, int pitch) { // n rows (the launcher has checked that both operands fit a descriptor)
-        return __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(reinterpret_cast<const char *>(from)) + size_t(first) * pitch, 0, n * pitch, 0x00020000);
-    };
     auto open = [&](const TilePos &t, BlockSource &s) {
-        s.a = buffer(p.A, t.m0, t.m_end - t.m0, p.lda * 2);
-        s.w = buffer(p.W, t.n0, min(p.N - t.n0, S::COLUMNS), p.K * 2);
+        s.a = seg_rows(p.A, t.m0, t.m_end - t.m0, p.lda * 2);
+        s.w = seg_rows(p.W, t.n0, min(p.N - t.n0, S::COLUMNS), p.K * 2);
         s.k = p.kb[t.split] * 2;
         s.n_ktiles = ktiles(t);
     };
     char *scratch = reinterpret_cast<char *>(lds_stream) + 2 * S::STAGE_BYTES + wave * S::SCRATCH_BYTES;
     block_stream<BlockBf16, MI, TilePos>(lds_stream, wave, lane, p.lda * 2, p.K * 2, next, open, ktiles,
                                          [&](const TilePos &t, int wm, int wn, const float4_t (&acc)[4][2 * MI]) { seg_store<Pieces16, MI>(p, acc, t, wm, wn, lane, scratch); });
+}
+
+// The same for few rows in tiles of 128 x 64 (gemm_thin.hpp); no gathered rows and no list.
+__global__ __launch_bounds__(DMA_THREADS) void seg_gemm_bf16_thin_kernel(SegGemm p, SegWalk w) {
+    extern __shared__ __attribute__((aligned(16))) half_t lds_stream[];
+    using S = Thin;
+    const int lane = threadIdx.x & 63, role_wave = __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) & 3);
+    int round = 0;
+    auto next = [&](TilePos &t) {
+        for (;;) {
+            const int r = seg_tile(p, w, false, blockIdx.x % SEG_DIES, seg_slot(w.longest_first, blockIdx.x / SEG_DIES, gridDim.x / SEG_DIES, round++), S::ROWS, S::COLUMNS, t);
+            if (r != 0) return r > 0;
+        }
+    };
+    auto ktiles = [&](const TilePos &t) { return (p.kb[t.split + 1] - p.kb[t.split]) / BK; };
+    if (threadIdx.x >= 256) {
+        thin_load<TilePos>(lds_stream, role_wave, lane, next, [&](const TilePos &t, BlockSource &s, int &pitch_a, int &pitch_w) {
+            pitch_a = p.lda * 2;
+            pitch_w = p.K * 2;
+            s.a = seg_rows(p.A, t.m0, t.m_end - t.m0, pitch_a);
+            s.w = seg_rows(p.W, t.n0, min(p.N - t.n0, S::COLUMNS), pitch_w);
+            s.k = p.kb[t.split] * 2;
+            s.n_ktiles = ktiles(t);
+        });
+        return;
+    }
+    char *scratch = reinterpret_cast<char *>(lds_stream) + S::STAGES * S::STAGE_BYTES + role_wave * S::SCRATCH_BYTES;
+    thin_multiply<BlockBf16, TilePos>(role_wave, lane, next, ktiles, [&](const TilePos &t, const float4_t (&acc)[4][2]) { seg_store<Pieces16, 1>(p, acc, t, role_wave, 0, lane, scratch); });
 }
 
 // f32: 64 x 64 tile, a thread owns rows ty, ty + 16, .. and columns tx, tx + 16, tx + 32, tx + 48 (so a gate column and its up
@@ -247,7 +277,7 @@ __global__ __launch_bounds__(256) void seg_gemm_f32_kernel(SegGemm p, SegWalk w)
 
 } // namespace
 
-// The tile for a product whose ranges are set: its height in 64 rows, + SEG_BLOCK where it is 256 columns wide.  Plain f32 results keep the
+// The tile for a product whose ranges are set: its height in 64 rows, + SEG_BLOCK where it is 256 columns wide, + SEG_THIN where it is 64.  Plain f32 results keep the
 // narrow tiles: wide ones need more ranges of k to fill the chip, and each range's sums cost a slab (1920 x 2048 x 7552: 58 us in two ranges of 256 x 128, 57 in
 // three of 192 x 256, whose third slab costs 3 us in row_finish; 768 rows 31 in four ranges, 32 in eight).
 static int seg_choose(moon_ctx *ctx, const SegGemm &p) {
@@ -259,7 +289,12 @@ static int seg_choose(moon_ctx *ctx, const SegGemm &p) {
             t = e;
             best = mi;
         }
-    if (p.splits > 1 || p.tile_group || p.rows || (!p.n16 && p.n32 == p.N)) return best;
+    if (p.tile_group || p.rows) return best;
+    if (const double e = seg_thin_estimate(cus, p.M, p.N, p.kb, p.splits); e < t) {
+        t = e;
+        best = SEG_THIN + 2;
+    }
+    if (p.splits > 1 || (!p.n16 && p.n32 == p.N)) return best;
     for (int mi = 3; mi <= 4; mi++)
         if (const double e = seg_block_estimate(cus, mi, p.M, p.N, p.K); e < t) {
             t = e;
@@ -293,6 +328,10 @@ int seg_gemm_splits(moon_ctx *ctx, int dtype, size_t M, size_t N, size_t K, size
                 t = e;
                 best = splits;
             }
+        if (const double e = seg_thin_estimate(cus, (int)M, (int)N, kb, splits) + (splits - 1) * slab; e < t) {
+            t = e;
+            best = splits;
+        }
     }
     return best;
 }
@@ -315,8 +354,9 @@ int launch_seg_gemm(moon_ctx *ctx, int dtype, SegGemm p) {
         if (size_t(p.a_rows) * p.lda * 2 >= lim || size_t(p.N) * p.K * 2 >= lim)
             return moon_fail(ctx, MOON_EINVAL_DIM, "segmented product: an operand of 2 GiB or more");
         const int tile = p.tile_group ? 2 : p.tile ? p.tile : seg_choose(ctx, p), mi = tile % SEG_BLOCK;
-        if (mi < (tile > SEG_BLOCK ? 3 : 2) || mi > 4 || tile > SEG_BLOCK + 4 || (tile > SEG_BLOCK && p.rows)) return moon_fail(ctx, MOON_EINVAL, "segmented product: tile form %d", tile);
-        columns = tile > SEG_BLOCK ? 256 : BN;
+        if (tile != SEG_THIN + 2 && (mi < (tile > SEG_BLOCK ? 3 : 2) || mi > 4 || tile > SEG_BLOCK + 4)) return moon_fail(ctx, MOON_EINVAL, "segmented product: tile form %d", tile);
+        if (tile > 4 && p.rows) return moon_fail(ctx, MOON_EINVAL, "segmented product: tile form %d", tile);
+        columns = tile > SEG_THIN ? Thin::COLUMNS : tile > SEG_BLOCK ? 256 : BN;
         rows = 64 * mi;
         auto go = [&](auto kern, size_t lds, std::atomic<bool> (&attr_set)[64]) -> int {
             const int dev = ctx->device >= 0 && ctx->device < 64 ? ctx->device : -1;
@@ -330,8 +370,9 @@ int launch_seg_gemm(moon_ctx *ctx, int dtype, SegGemm p) {
             hipLaunchKernelGGL(kern, dim3((unsigned)seg_workgroups(w, cus)), dim3(DMA_THREADS), lds, ctx->stream, p, w);
             return MOON_OK;
         };
-        static std::atomic<bool> set_listed[64], set2[64], set3[64], set4[64], wide3[64], wide4[64];
+        static std::atomic<bool> set_listed[64], set2[64], set3[64], set4[64], wide3[64], wide4[64], thin2[64];
         if (p.tile_group) MOON_TRY(go(seg_gemm_bf16_kernel<2, true>, Stream<2>::LDS_BYTES, set_listed));
+        else if (tile == SEG_THIN + 2) MOON_TRY(go(seg_gemm_bf16_thin_kernel, Thin::LDS_BYTES, thin2));
         else if (tile == SEG_BLOCK + 4) MOON_TRY(go(seg_gemm_bf16_block_kernel<4>, Block<4>::LDS_BYTES, wide4));
         else if (tile == SEG_BLOCK + 3) MOON_TRY(go(seg_gemm_bf16_block_kernel<3>, Block<3>::LDS_BYTES, wide3));
         else if (mi == 4) MOON_TRY(go(seg_gemm_bf16_kernel<4, false>, Stream<4>::LDS_BYTES, set4));
@@ -342,6 +383,6 @@ int launch_seg_gemm(moon_ctx *ctx, int dtype, SegGemm p) {
         hipLaunchKernelGGL(seg_gemm_f32_kernel, dim3((unsigned)(SEG_DIES * w.slots)), dim3(256), 0, ctx->stream, p, w);
     }
     MOON_HIP(ctx, hipGetLastError());
-    MOON_NOTE_KERNEL(ctx, "%s %d rows a tile, k split %d", dtype != MOON_DTYPE_BF16 ? "seg_gemm_f32_kernel" : columns == BN ? "seg_gemm_bf16_kernel" : "seg_gemm_bf16_block_kernel", rows, p.splits);
+    MOON_NOTE_KERNEL(ctx, "%s %d rows a tile, k split %d", dtype != MOON_DTYPE_BF16 ? "seg_gemm_f32_kernel" : columns == BN ? "seg_gemm_bf16_kernel" : columns > BN ? "seg_gemm_bf16_block_kernel" : "seg_gemm_bf16_thin_kernel", rows, p.splits);
     return MOON_OK;
 }

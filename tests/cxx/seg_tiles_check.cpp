@@ -75,7 +75,7 @@ int main() {
         if (hipMemcpy(da, a.data(), a.size() * 2, hipMemcpyHostToDevice) || hipMemcpy(dw, w.data(), w.size() * 2, hipMemcpyHostToDevice)) return printf("copy\n"), 2;
         std::vector<uint16_t> first16, first_g, c16(n16), cg(ng);
         std::vector<uint32_t> first32, c32(n32);
-        for (int tile : {2, 3, 4, SEG_BLOCK + 3, SEG_BLOCK + 4}) {
+        for (int tile : {2, 3, 4, SEG_BLOCK + 3, SEG_BLOCK + 4, SEG_THIN + 2}) {
             printf("%d x %d x %d, segments %d %d, %d ranges, tile %d\n", s.M, s.N, s.K, s.n16, s.n32, s.splits, tile);
             fflush(stdout);
             (void)hipMemset(d16, 0x5a, n16 * 2);
