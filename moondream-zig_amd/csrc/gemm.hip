@@ -883,6 +883,38 @@ __device__ __forceinline__ void gemm_block_partial(const GemmArgs &p, const floa
             asm volatile("" ::: "memory");
         }
 }
+// The same two products in tiles of 192 x 256 (gemm_block.hpp) times the ranges of k, one unit per workgroup.
+struct GemmUnit {
+    int m0, n0, split;
+};
+__global__ __launch_bounds__(DMA_THREADS) void gemm_nt_block_pair_kernel(GemmPairArgs a) {
+    extern __shared__ __attribute__((aligned(16))) half_t lds_block[];
+    using S = Block<3>;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int per_xcd = (a.units_total + 7) / 8, unit = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
+    if (unit >= a.units_total) return;
+    const bool second = unit >= a.units0;
+    const GemmArgs &p = second ? a.p[1] : a.p[0];
+    const int u = second ? unit - a.units0 : unit, tiles = p.tiles_m * p.tiles_n, split = u / tiles, tile = u % tiles;
+    const int k0 = split * p.k_per_split, n_ktiles = (min(p.K, k0 + p.k_per_split) - k0) / BK, pitch = p.K * 2;
+    if (n_ktiles <= 0) return;
+    auto next = [&](GemmUnit &t, int &round) {
+        if (round++) return false;
+        t = {tile % p.tiles_m * S::ROWS, tile / p.tiles_m * S::COLUMNS, split};
+        return true;
+    };
+    char *scratch = reinterpret_cast<char *>(lds_block) + 2 * S::STAGE_BYTES + wave * S::SCRATCH_BYTES;
+    block_stream<BlockF16, 3, GemmUnit>(
+        lds_block, wave, lane, pitch, pitch, next,
+        [&](const GemmUnit &t, BlockSource &s) {
+            s.a = gemm_rows(p.A, t.m0, min(p.M - t.m0, S::ROWS), pitch);
+            s.w = gemm_rows(p.Bt, t.n0, min(p.N - t.n0, S::COLUMNS), pitch);
+            s.k = k0 * 2;
+            s.n_ktiles = n_ktiles;
+        },
+        [&](const GemmUnit &) { return n_ktiles; },
+        [&](const GemmUnit &t, int wm, int wn, const float4_t (&acc)[4][6]) { gemm_block_partial<3>(p, acc, t.m0 + wm * 96, t.n0 + wn * 64, t.split, lane, scratch); });
+}
 // The same two products for few rows: tiles of 128 x 64 times the ranges of k.
 struct GemmThinUnit {
     int m0, n0, second, split;
@@ -1535,24 +1567,44 @@ int launch_gemm_pair_ln(moon_ctx *ctx, const half_t *A_add, const half_t *B_add,
     if (!al16(A) || !al16(B) || !al16(A_add) || !al16(B_add) || !al16(bias) || !al16(bias_add) || !al16(resid) || !al16(C) || !al16(ln.gamma) ||
         !al16(ln.beta) || !al16(ln.out) || !ln.add || !al16(ln.add))
         return MOON_OK;
-    // below 192 rows tiles of 128 x 64 (gemm_thin.hpp): 37 rows of width 2048, apart 8.3 and 15.9 us
-    const bool thin = M < 192;
-    const int tile_m = thin ? Thin::ROWS : 192, tile_n = thin ? Thin::COLUMNS : BN, tiles_m = (int)((M + tile_m - 1) / tile_m), tiles_n = (int)((N + tile_n - 1) / tile_n), tiles = tiles_m * tiles_n;
-    if (tiles * 2 > cus) return MOON_OK;
-    // splits (s_add, s): all workgroups in one round, the longest run of k-tiles as short as it gets
+    // Splits (s_add, s): all workgroups in one round, the longest run of k-tiles as short as it gets, us at `fixed` for a launch and `one` + `all` * busy units for a k-tile,
+    // and for every range its sums, written and read (8 TB/s: they stay in the memory-side cache).
     const int kt_add = (int)(K_add / BK), kt = (int)(K / BK);
-    int best_a = 0, best_s = 0, best_len = 1 << 30;
-    for (int sa = 1; sa <= 8 && sa <= kt_add; sa++)
-        for (int s = 1; s <= 8 && s <= kt; s++) {
-            if (tiles * (sa + s) > cus) continue;
-            const int len = std::max((kt_add + sa - 1) / sa, (kt + s - 1) / s);
-            if (len < best_len || (len == best_len && sa + s < best_a + best_s)) {
-                best_len = len;
-                best_a = sa;
-                best_s = s;
+    struct Plan {
+        int tiles_m = 0, tiles_n = 0, a = 0, s = 0;
+        double us = 1e30;
+    };
+    const auto plan = [&](int tile_m, int tile_n, double fixed, double one, double all) {
+        Plan p;
+        p.tiles_m = (int)((M + tile_m - 1) / tile_m);
+        p.tiles_n = (int)((N + tile_n - 1) / tile_n);
+        const int tiles = p.tiles_m * p.tiles_n;
+        int best_len = 1 << 30;
+        for (int sa = 1; sa <= 8 && sa <= kt_add; sa++)
+            for (int s = 1; s <= 8 && s <= kt; s++) {
+                if (tiles * (sa + s) > cus) continue;
+                const int len = std::max((kt_add + sa - 1) / sa, (kt + s - 1) / s);
+                if (len < best_len || (len == best_len && sa + s < p.a + p.s)) {
+                    best_len = len;
+                    p.a = sa;
+                    p.s = s;
+                }
             }
+        if (p.a) p.us = fixed + best_len * (one + all * tiles * (p.a + p.s) / cus) + (p.a + p.s) * (double)M * N * 8 / 8e6;
+        return p;
+    };
+    // Below 192 rows tiles of 128 x 64 (gemm_thin.hpp): 37 rows of width 2048, apart 8.3 and 15.9 us.  From there on 192 x 128, or 192 x 256 (gemm_block.hpp) where those leave few ranges of
+    // k: a layer of width 2048 at 850 rows 139 -> 128 us, 1025 192 -> 161, 1536 230 -> 198; at 768 rows 192 x 128 is 2 % faster, at width 1024 up to 9.
+    const bool thin = M < 192;
+    Plan best = thin ? plan(Thin::ROWS, Thin::COLUMNS, 0, 1, 0) : plan(192, BN, 7, 0.45, 0.28);
+    bool wide = false;
+    if (!thin)
+        if (const Plan w = plan(192, 256, 10, 0.78, 0.42); w.us < best.us) {
+            best = w;
+            wide = true;
         }
-    if (!best_a) return MOON_OK;
+    if (!best.a) return MOON_OK;
+    const int tiles_m = best.tiles_m, tiles_n = best.tiles_n, tiles = tiles_m * tiles_n, best_a = best.a, best_s = best.s;
     GemmPairArgs a;
     const auto fill = [&](GemmArgs &p, const half_t *Ap, const half_t *Bp, size_t Kp, int splits, GrowBuf &ws) -> int {
         p.A = Ap;
@@ -1580,16 +1632,16 @@ int launch_gemm_pair_ln(moon_ctx *ctx, const half_t *A_add, const half_t *B_add,
     MOON_TRY(fill(a.p[1], A, B, K, best_s, ctx->work[0]));
     a.units0 = tiles * a.p[0].splits;
     a.units_total = a.units0 + tiles * a.p[1].splits;
-    static std::atomic<bool> attr_set[2][64];
-    const int dev = ctx->device >= 0 && ctx->device < 64 ? ctx->device : -1;
-    const auto kern = thin ? gemm_nt_thin_pair_kernel : gemm_nt_dma192_pair_kernel;
-    const size_t lds_bytes = thin ? Thin::LDS_BYTES : Dma2<3>::LDS_BYTES;
-    if (dev < 0 || !attr_set[thin][dev].load()) {
+    static std::atomic<bool> attr_set[3][64];
+    const int dev = ctx->device >= 0 && ctx->device < 64 ? ctx->device : -1, which = thin ? 1 : wide ? 2 : 0;
+    const auto kern = thin ? gemm_nt_thin_pair_kernel : wide ? gemm_nt_block_pair_kernel : gemm_nt_dma192_pair_kernel;
+    const size_t lds_bytes = thin ? Thin::LDS_BYTES : wide ? Block<3>::LDS_BYTES : Dma2<3>::LDS_BYTES;
+    if (dev < 0 || !attr_set[which][dev].load()) {
         MOON_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes));
-        if (dev >= 0) attr_set[thin][dev].store(true);
+        if (dev >= 0) attr_set[which][dev].store(true);
     }
     hipLaunchKernelGGL(kern, dim3(((a.units_total + 7) / 8) * 8), dim3(DMA_THREADS), lds_bytes, ctx->stream, a);
-    MOON_NOTE_KERNEL(ctx, "%s %d + %d workgroups, k splits %d and %d + splitk_reduce_ln_kernel", thin ? "gemm_nt_thin_pair_kernel" : "gemm_nt_dma192_pair_kernel", a.units0, a.units_total - a.units0,
+    MOON_NOTE_KERNEL(ctx, "%s %d + %d workgroups, k splits %d and %d + splitk_reduce_ln_kernel", thin ? "gemm_nt_thin_pair_kernel" : wide ? "gemm_nt_block_pair_kernel" : "gemm_nt_dma192_pair_kernel", a.units0, a.units_total - a.units0,
                      a.p[0].splits, a.p[1].splits);
     MOON_HIP(ctx, hipGetLastError());
     hipLaunchKernelGGL(splitk_reduce_ln_kernel<MOON_EPI_BIAS_RESID>, dim3((unsigned)M), dim3(256), 0, ctx->stream, a.p[1].partial, bias, resid, ln.add,
