@@ -35,7 +35,8 @@ template <int MI> struct StreamSource {
 };
 __device__ __forceinline__ int stream_row_a(int mi, int role_wave, int j, int lane) { return 16 * mi * role_wave + 8 * j + (lane >> 3); }
 
-template <int MI, class Tile, class Next, class Open>
+// ONCE: the weights are read by one tile, or a few, and are not to push the activations out of the L2 (non-temporal copies).
+template <int MI, bool ONCE, class Tile, class Next, class Open>
 __device__ __forceinline__ void stream_load(half_t *lds, int role_wave, Next next, Open open) {
     using S = Stream<MI>;
     Tile t;
@@ -50,7 +51,7 @@ __device__ __forceinline__ void stream_load(half_t *lds, int role_wave, Next nex
             __builtin_amdgcn_raw_ptr_buffer_load_lds(s.a, (__attribute__((address_space(3))) void *)(dst + (16 * MI * role_wave + 8 * j) * BK), 16, s.off_a[j], s.k, 0, 0);
 #pragma unroll
         for (int j = 0; j < 4; j++)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(s.w, (__attribute__((address_space(3))) void *)(dst + S::ROWS * BK + (32 * role_wave + 8 * j) * BK), 16, s.off_w[j], s.k, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(s.w, (__attribute__((address_space(3))) void *)(dst + S::ROWS * BK + (32 * role_wave + 8 * j) * BK), 16, s.off_w[j], s.k, 0, ONCE ? 2 : 0);
         stage = stage + 1 == S::STAGES ? 0 : stage + 1;
         issued++;
         s.k += BK * 2;

@@ -137,7 +137,7 @@ __device__ __forceinline__ void seg_store(const SegGemm &p, const Acc &acc, cons
 
 // LISTED: row tiles from a list.  A kernel of its own: with both ways to a tile in one, the plain products of a prompt of 768 rows lost
 // 0.4 to 0.8 us each.
-template <int MI, bool LISTED>
+template <int MI, bool LISTED, bool ONCE = false>
 __global__ __launch_bounds__(DMA_THREADS) void seg_gemm_bf16_kernel(SegGemm p, SegWalk w) {
     extern __shared__ __attribute__((aligned(16))) half_t lds_stream[]; // (the tile product addresses LDS from 0: nothing static beside it)
     using S = Stream<MI>;
@@ -150,7 +150,7 @@ __global__ __launch_bounds__(DMA_THREADS) void seg_gemm_bf16_kernel(SegGemm p, S
         }
     };
     if (threadIdx.x >= 256) {
-        stream_load<MI, TilePos>(lds_stream, role_wave, next, [&](const TilePos &t, StreamSource<MI> &s) {
+        stream_load<MI, ONCE, TilePos>(lds_stream, role_wave, next, [&](const TilePos &t, StreamSource<MI> &s) {
             // (the launcher has checked that both operands fit a descriptor)
             const bf16_t *weights = reinterpret_cast<const bf16_t *>(p.W) + size_t(t.group) * p.w_group;
             s.a = __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p.A), 0, p.a_rows * p.lda * 2, 0x00020000);
@@ -370,8 +370,11 @@ int launch_seg_gemm(moon_ctx *ctx, int dtype, SegGemm p) {
             hipLaunchKernelGGL(kern, dim3((unsigned)seg_workgroups(w, cus)), dim3(DMA_THREADS), lds, ctx->stream, p, w);
             return MOON_OK;
         };
-        static std::atomic<bool> set_listed[64], set2[64], set3[64], set4[64], wide3[64], wide4[64], thin2[64];
-        if (p.tile_group) MOON_TRY(go(seg_gemm_bf16_kernel<2, true>, Stream<2>::LDS_BYTES, set_listed));
+        static std::atomic<bool> set_listed[64], set_once[64], set2[64], set3[64], set4[64], wide3[64], wide4[64], thin2[64];
+        // Groups of up to a row tile each read their weights once, non-temporally: 12 layers of width 2048, 64 experts of 704, 8 a row, 61 rows 170 -> 159 us a layer, 768 rows 229 -> 220.  With two
+        // row tiles in a group the second one finds them in the L2 otherwise: 1025 rows 284 and 301, 1301 320 and 362; as fast either way at 950 rows, 119 a group.
+        if (p.tile_group && p.M <= SEG_ONCE_ROWS * (p.max_tiles - p.M / SEG_TILE_ROWS)) MOON_TRY(go(seg_gemm_bf16_kernel<2, true, true>, Stream<2>::LDS_BYTES, set_once));
+        else if (p.tile_group) MOON_TRY(go(seg_gemm_bf16_kernel<2, true>, Stream<2>::LDS_BYTES, set_listed));
         else if (tile == SEG_THIN + 2) MOON_TRY(go(seg_gemm_bf16_thin_kernel, Thin::LDS_BYTES, thin2));
         else if (tile == SEG_BLOCK + 4) MOON_TRY(go(seg_gemm_bf16_block_kernel<4>, Block<4>::LDS_BYTES, wide4));
         else if (tile == SEG_BLOCK + 3) MOON_TRY(go(seg_gemm_bf16_block_kernel<3>, Block<3>::LDS_BYTES, wide3));
