@@ -89,8 +89,8 @@ void moon_ctx_destroy(moon_ctx *ctx);
 const char *moon_last_error(const moon_ctx *ctx);
 /* Measurement and test knob without a counterpart in the reference: names the matrix-product kernel that moon_hgemm,
  * moon_hgemm_trans, moon_linear and the sessions of this context take wherever the shape allows it ("regs", "dma",
- * "dma256", "w114", "w212", "w221"; "" or NULL: chosen by shape, the default).  Every kernel computes the same product to
- * the same rounding points; only the time changes.  The context starts with the value of MOON_GEMM_KERNEL. */
+ * "dma256", "b192", "b256", "thin", "w114", "w212", "w221"; "" or NULL: chosen by shape, the default).  Every kernel computes
+ * the same product to the same rounding points; only the time changes, and with it whether f32 sums are added in ranges of k.  The context starts with the value of MOON_GEMM_KERNEL. */
 int moon_set_gemm_kernel(moon_ctx *ctx, const char *name);
 /* Measurement aid without a counterpart in the reference: the name (with its grid and k split) of the kernel that the latest
  * matrix product, matrix-vector product or attention call on this context dispatched; "" before the first.  The text lives in
@@ -459,7 +459,7 @@ int moon_bin_vision_io_weights(const moon_bin *bin, const moon_vision_config *cf
  *   MOON_LAYER_QKV_WGS=n           decode mode 0: workgroups that take qkv rows (default: the attention and output workgroups)
  *   MOON_LAYER_FC1_OUT_ROWS=n      decode mode 0: fc1 rows per output wavefront (default: about a third of an fc1-only wavefront's
  *                                  share, at least one; 0 is allowed)
- *   MOON_GEMM_KERNEL=regs|dma|dma256|w114|w212|w221  forces one of the MFMA product kernels where the shape allows it (default: by shape)
+ *   MOON_GEMM_KERNEL=regs|dma|dma256|b192|b256|thin|w114|w212|w221  forces one of the MFMA product kernels where the shape allows it (default: by shape)
  *   MOON_GEMM_EPILOGUE=direct      the product kernels store their tile without the pass through LDS (default: through LDS)
  *   MOON_SAMPLE_SEPARATE=1         sampled loops with top_k <= 3: the LM-head launch leaves every token to sample_kernel instead of
  *                                  deciding it where it provably can (read at every call, so a test can compare the two in one process)
@@ -468,8 +468,9 @@ int moon_bin_vision_io_weights(const moon_bin *bin, const moon_vision_config *cf
  *                                  f16 roundings, differ
  *   MOON_GEMM_KN_TRANSPOSE=1       products with a [K, N] second operand always run over a transposed copy instead of reading the operand
  *                                  in place where the shape allows (read at every call; the same bits either way)
- *   MOON_GEMM_NO_ROPE=1            text prefill: the qkv projection and the rotation + cache update run as two launches instead of
- *                                  one (read at every call; the same bits either way)
+ *   MOON_GEMM_NO_ROPE=1            text prefill: the qkv projection, the rotation + cache update and fc1 run as three launches instead
+ *                                  of one (read at every call; the same bits where neither product alone is taken in ranges of k,
+ *                                  otherwise, at few rows, f32 sums in another order)
  * Every other setting gives the same results, bit for bit; only the time changes. */
 
 #ifdef __cplusplus

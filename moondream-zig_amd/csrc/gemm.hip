@@ -7,7 +7,8 @@
 // (row>>1)&7 so the 128-bit operand reads of 32 consecutive rows and the 128-bit staging writes are bank-conflict
 // free), several k-tiles deep, with one barrier per k-tile.  Three kernels share this: two specialised by wavefront
 // (loaders that copy global -> LDS directly, multipliers that only read LDS and issue MFMAs) and a register-staged one
-// (256 threads, two workgroups per CU) for whatever those do not take.
+// (256 threads, two workgroups per CU) for whatever those do not take.  Grids of several rounds and a decoder's prompts take other
+// tiles: 192 and 256 x 256 (gemm_block.hpp, all eight wavefronts copy and multiply) and 128 x 64 (gemm_thin.hpp, short prompts).
 // The weight rows feed the MFMA "A" operand and the activation rows the "B" operand, so every lane ends up
 // holding 4 consecutive n for one m.  f32 accumulation over the whole K, one rounding to f16 (then the bias / GELU
 // roundings) exactly as the reference does.

@@ -1,0 +1,61 @@
+"""GPU parity of the wide (192 / 256 x 256) and thin (128 x 64) f16 product tiles against the CPU oracle: by themselves where they are
+named, and where a decoder's prompt takes them (q, k, v with their rotation beside fc1; out_proj beside fc2)."""
+import numpy as np
+import pytest
+
+from conftest import TOL
+
+pytestmark = pytest.mark.gpu
+
+
+# The tiles' edges in rows and columns (a lone row and the last of a tile, one more), columns that are no whole pieces of 64 or 256, and
+# one to seven k-tiles (the thin kernel's ring holds six).  TOL is the bar of every f16 product here: one rounding of f32 sums.
+@pytest.mark.parametrize("kernel", ["b192", "b256", "thin"])
+@pytest.mark.parametrize("M,N,K,epi", [(2, 8, 64, "none"), (63, 64, 128, "bias"), (127, 72, 448, "bias_gelu"), (128, 256, 384, "bias"), (129, 264, 64, "bias_gelu"),
+                                       (191, 248, 192, "none"), (192, 520, 320, "bias"), (193, 512, 128, "bias_gelu"), (255, 200, 192, "bias"),
+                                       (256, 256, 256, "none"), (257, 328, 64, "bias"), (385, 1032, 448, "bias_gelu"), (513, 136, 128, "none")])
+def test_named_tiles_at_their_edges(moon, O, ctx, kernel, M, N, K, epi):
+    L = moon._lib
+    a = O.fill_normal_f16((M, K), 0, 0, 1.0)
+    w = O.fill_normal_f16((N, K), 0, 1, 0.05)
+    b = O.fill_normal_f16((N,), 0, 2, 0.1)
+    code = {"none": L.EPI_NONE, "bias": L.EPI_BIAS, "bias_gelu": L.EPI_BIAS_GELU}[epi]
+    got = np.empty((M, N), dtype=np.float16)
+    ctx.set_gemm_kernel(kernel)
+    try:
+        ctx.check(ctx.lib.moon_linear(ctx.handle, a.ctypes.data, M, K, w.ctypes.data, N, L.B_NK, b.ctypes.data if epi != "none" else None, code, got.ctypes.data))
+        took = ctx.last_kernel()
+    finally:
+        ctx.set_gemm_kernel("")
+    assert ("thin" if kernel == "thin" else "block") in took
+    ref = O.hgemm_trans(a, w)
+    if epi != "none":
+        ref = O.bias_add(ref, b)
+    if epi == "bias_gelu":
+        ref = O.gelu(ref)
+    assert O.rel_frobenius(got, ref) <= TOL
+    # No row or column drowns in the norm of all: sums in another order move each of at most three roundings (product, bias, GELU, whose
+    # slope stays below 1.13) by one step of f16 at the largest value, 2^-10 of it.
+    far = np.abs(got.astype(np.float32) - ref.astype(np.float32)).max()
+    assert far <= 4 * 2.0**-10 * np.abs(ref.astype(np.float32)).max()
+
+
+# Prompts in pieces, each behind the ones before it, at the tiles' edges: two rows, a row short of a thin tile, a whole one, one and two
+# rows more, the last size of thin pairs (191) and the first of tall ones, a feed-forward whose width is no whole k-tile (its product
+# is not paired, and its last columns are no whole tile), and at width 2048 the pair in 192 x 256 tiles.
+@pytest.mark.parametrize("dim,hidden,heads,pieces", [(512, 2048, 8, (2, 127, 128, 129, 65)), (512, 2048, 8, (191, 192, 193, 257)), (192, 776, 3, (130, 37, 385)),
+                                                     (192, 832, 3, (64, 129, 513)), (2048, 8192, 32, (1025, 37))])
+def test_prompts_at_the_edges_of_the_tiles(moon, O, ctx, dim, hidden, heads, pieces):
+    cfg = dict(O.TEXT_CFG, vocab=1024, dim=dim, hidden_dim=hidden, n_layers=2, n_heads=heads, head_dim=64, rot_dim=32, max_seq=1088)
+    weights = O.synth_text_weights(cfg, 9)
+    ref = O.TextModel(weights, cfg)
+    mcfg = moon.text_model.make_config(vocab=cfg["vocab"], dim=dim, hidden_dim=hidden, n_layers=2, n_heads=heads, max_seq=cfg["max_seq"])
+    dev = moon.text_model.TextModel(mcfg, weights=weights, ctx=ctx)
+    cache = ref.new_cache()
+    for i, rows in enumerate(pieces):
+        ids = O.fill_uniform_u32(rows, i, 57, cfg["vocab"])
+        h_ref = ref.text_decoder(ref.text_encoder(ids), cache)
+        dev.forward(ids)
+        assert O.rel_frobenius(dev.hidden(rows), h_ref) <= TOL, (i, rows)
+        assert O.rel_frobenius(dev.logits().reshape(1, -1), ref.lm_head(h_ref).reshape(1, -1)) <= TOL, (i, rows)
+    dev.close()
