@@ -341,28 +341,21 @@ __global__ __launch_bounds__(256) void decode_lm_head_topk_kernel(LmHeadArgs a) 
         const half_t v = have ? s_logit[wave][lane] : __builtin_bit_cast(half_t, (unsigned short)0xfc00);
         const unsigned hb = __builtin_bit_cast(unsigned short, v);
         q.bad = __ballot(have && (hb & 0x7c00u) == 0x7c00u && hb != 0xfc00u) ? 1u : 0u;
-        unsigned long long key = have ? quick_key(v, a0 + lane) : 0ull;
+        unsigned key = have ? ((unsigned)(quick_key(v, 0) >> 32) << 16) | (63 - lane) : 0u; // (the order of quick_key: the wavefront's indexes rise with the lane)
 #pragma unroll
         for (int r = 0; r < QUICK_KEYS; r++) { // the largest key left, QUICK_KEYS times
-            unsigned long long best = key;
-#pragma unroll
-            for (int off = 32; off >= 1; off >>= 1) {
-                const unsigned lo = __shfl_xor((unsigned)best, off, 64), hi = __shfl_xor((unsigned)(best >> 32), off, 64);
-                const unsigned long long o = ((unsigned long long)hi << 32) | lo;
-                best = o > best ? o : best;
-            }
-            q.key[r] = best;
+            const unsigned best = wave_max(key);
+            q.key[r] = best ? ((unsigned long long)(best >> 16) << 32) | (unsigned)~(unsigned)(a0 + 63 - (int)(best & 63u)) : 0ull;
             if (key == best) key = 0;
         }
         if (q.key[0]) {
             const float mx = (float)quick_key_logit(q.key[0]), f = (float)v;
-            float e = have && f > -INFINITY && mx > -INFINITY ? __expf((f - mx) * inv_t) : 0.f;
-#pragma unroll
-            for (int off = 32; off >= 1; off >>= 1) e += __shfl_xor(e, off, 64);
             q.mx = mx;
-            q.sum = e;
+            q.sum = wave_sum(have && f > -INFINITY && mx > -INFINITY ? __expf((f - mx) * inv_t) : 0.f);
         }
     }
+    // The exchange and the merges are the tail of every launch.  Maxima move over the wavefront without a trip through LDS, and the four wavefronts' sixteen keys are
+    // ranked by a lane each against all of them, where shuffles and one thread's merges had taken 4.5 us more: 51200 rows of width 1024 29.9 -> 25.4 us.
     auto publish = [&]() __attribute__((always_inline)) { // this wavefront's q -> LDS (inlined: q stays in registers)
         if (lane == 0) {
 #pragma unroll
@@ -372,21 +365,34 @@ __global__ __launch_bounds__(256) void decode_lm_head_topk_kernel(LmHeadArgs a) 
             s_bad[wave] = q.bad;
         }
     };
-    auto gather = [&]() __attribute__((always_inline)) { // thread 0: the other three wavefronts' q merged into its own
-        for (int w = 1; w < 4; w++) {
-            QuickTop o;
+    auto gather = [&]() __attribute__((always_inline)) { // the first wavefront: all four's q merged, the same in every lane
+        const int i = lane & 15;
+        const unsigned long long mine = s_keys[i / QUICK_KEYS][i % QUICK_KEYS];
+        int rank = 0;
 #pragma unroll
-            for (int j = 0; j < QUICK_KEYS; j++) o.key[j] = s_keys[w][j];
-            o.mx = s_mx[w];
-            o.sum = s_sum[w];
-            o.bad = s_bad[w];
-            quick_merge(q, o, inv_t);
+        for (int j = 0; j < 4 * QUICK_KEYS; j++) {
+            const unsigned long long o = s_keys[j / QUICK_KEYS][j % QUICK_KEYS];
+            rank += o > mine || (o == mine && j < i) ? 1 : 0;
+        }
+        const unsigned lo = (unsigned)mine, hi = (unsigned)(mine >> 32);
+#pragma unroll
+        for (int j = 0; j < QUICK_KEYS; j++) {
+            const int at = __builtin_ctzll(__ballot(rank == j)); // (every rank is some lane's)
+            q.key[j] = ((unsigned long long)(unsigned)__builtin_amdgcn_readlane(hi, at) << 32) | (unsigned)__builtin_amdgcn_readlane(lo, at);
+        }
+        q.mx = fmaxf(fmaxf(s_mx[0], s_mx[1]), fmaxf(s_mx[2], s_mx[3]));
+        q.sum = 0.f;
+        q.bad = 0;
+#pragma unroll
+        for (int w = 0; w < 4; w++) {
+            q.sum += s_sum[w] > 0.f ? s_sum[w] * __expf((s_mx[w] - q.mx) * inv_t) : 0.f;
+            q.bad |= s_bad[w] | (s_sum[w] != s_sum[w] ? 1u : 0u);
         }
     };
     publish();
     lds_barrier();
+    if (wave == 0) gather();
     if (tid == 0) {
-        gather();
         unsigned long long *mine = a.partials + size_t(blockIdx.x) * QUICK_WORDS;
 #pragma unroll
         for (int j = 0; j < QUICK_KEYS; j++) __hip_atomic_store(mine + j, q.key[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -429,26 +435,30 @@ __global__ __launch_bounds__(256) void decode_lm_head_topk_kernel(LmHeadArgs a) 
             quick_merge(q, o, inv_t);
         }
     }
-    // over the wavefront: a butterfly in which both partners merge the other's q into their own (the keys are distinct
-    // except for the empty key 0, and merging is symmetric: both end with the same q)
+    // over the wavefront: the largest of the lanes' first keys, QUICK_KEYS times (by its upper half, then by the lower of those that share it)
+    unsigned long long top[QUICK_KEYS];
 #pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-        QuickTop o;
+    for (int r = 0; r < QUICK_KEYS; r++) {
+        const unsigned hi = (unsigned)(q.key[0] >> 32), lo = (unsigned)q.key[0], best_hi = wave_max(hi), best_lo = wave_max(hi == best_hi ? lo : 0u);
+        top[r] = ((unsigned long long)best_hi << 32) | best_lo;
+        if (q.key[0] == top[r]) {
 #pragma unroll
-        for (int j = 0; j < QUICK_KEYS; j++) {
-            const unsigned lo = __shfl_xor((unsigned)q.key[j], off, 64), hi = __shfl_xor((unsigned)(q.key[j] >> 32), off, 64);
-            o.key[j] = ((unsigned long long)hi << 32) | lo;
+            for (int j = 0; j + 1 < QUICK_KEYS; j++) q.key[j] = q.key[j + 1];
+            q.key[QUICK_KEYS - 1] = 0;
         }
-        o.mx = __shfl_xor(q.mx, off, 64);
-        o.sum = __shfl_xor(q.sum, off, 64);
-        o.bad = __shfl_xor(q.bad, off, 64);
-        quick_merge(q, o, inv_t);
     }
-    lds_barrier();
+    const float mx = wave_max(q.mx);
+    const unsigned bad = __ballot(q.bad || q.sum != q.sum) ? 1u : 0u;
+    q.sum = wave_sum(q.sum > 0.f ? q.sum * __expf((q.mx - mx) * inv_t) : 0.f);
+    q.mx = mx;
+    q.bad = bad;
+#pragma unroll
+    for (int j = 0; j < QUICK_KEYS; j++) q.key[j] = top[j];
     publish();
     lds_barrier();
+    if (wave != 0) return;
+    gather();
     if (tid == 0) {
-        gather();
         uint32_t tok = 0;
         const float u = a.u_dev[a.state[1]];
         const bool ok = quick_top_k(q, a.top_k, a.temperature, a.scale, u, &tok);

@@ -116,3 +116,12 @@ __device__ __forceinline__ float wave_max(float v) {
     v = fmaxf(v, dpp_move<DPP_ROW_MIRROR>(v));
     return fmaxf(fmaxf(read_lane(v, 0), read_lane(v, 16)), fmaxf(read_lane(v, 32), read_lane(v, 48)));
 }
+template <int CTRL> __device__ __forceinline__ unsigned dpp_move(unsigned v) { return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, true); }
+__device__ __forceinline__ unsigned wave_max(unsigned v) {
+    v = max(v, dpp_move<DPP_QUAD_XOR1>(v));
+    v = max(v, dpp_move<DPP_QUAD_XOR2>(v));
+    v = max(v, dpp_move<DPP_ROW_HALF_MIRROR>(v));
+    v = max(v, dpp_move<DPP_ROW_MIRROR>(v));
+    const unsigned r0 = __builtin_amdgcn_readlane(v, 0), r1 = __builtin_amdgcn_readlane(v, 16), r2 = __builtin_amdgcn_readlane(v, 32), r3 = __builtin_amdgcn_readlane(v, 48);
+    return max(max(r0, r1), max(r2, r3));
+}

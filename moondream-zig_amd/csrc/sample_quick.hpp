@@ -69,17 +69,6 @@ __device__ __forceinline__ half_t quick_key_logit(unsigned long long key) {
     const unsigned hb = (ord & 0x8000u) ? (ord & 0x7fffu) : (~ord & 0xffffu);
     return __builtin_bit_cast(half_t, (unsigned short)hb);
 }
-__device__ __forceinline__ void quick_insert(QuickTop &q, unsigned long long x) {
-    if (x > q.key[QUICK_KEYS - 1]) {
-        q.key[QUICK_KEYS - 1] = x;
-#pragma unroll
-        for (int j = QUICK_KEYS - 1; j > 0; j--) {
-            const unsigned long long a = q.key[j - 1], b = q.key[j];
-            q.key[j - 1] = a > b ? a : b;
-            q.key[j] = a > b ? b : a;
-        }
-    }
-}
 // the rough sum: exp by the hardware, any order (top_k's result does not depend on it beyond what quick_top_k allows for)
 __device__ __forceinline__ void quick_add_sum(QuickTop &q, float mx, float sum, float inv_t) {
     if (!(sum > 0.f)) return;
@@ -89,16 +78,21 @@ __device__ __forceinline__ void quick_add_sum(QuickTop &q, float mx, float sum, 
     } else
         q.sum += sum * __expf((mx - q.mx) * inv_t);
 }
-__device__ __forceinline__ void quick_add(QuickTop &q, half_t v, int index, float inv_t) {
-    const unsigned hb = __builtin_bit_cast(unsigned short, v);
-    if ((hb & 0x7c00u) == 0x7c00u && hb != 0xfc00u) q.bad = 1; // NaN or +inf
-    quick_insert(q, quick_key(v, index));
-    const float f = (float)v;
-    if (f > -INFINITY) quick_add_sum(q, f, 1.f, inv_t);
-}
+// The larger of the one's j-th and the other's j-th last key are the QUICK_KEYS largest of both (distinct but for the empty 0), rising and then falling: two
+// exchanges sort them, where inserting four keys one by one is a chain of sixteen.
 __device__ __forceinline__ void quick_merge(QuickTop &q, const QuickTop &o, float inv_t) {
+    static_assert(QUICK_KEYS == 4, "two exchanges sort four keys");
 #pragma unroll
-    for (int j = 0; j < QUICK_KEYS; j++) quick_insert(q, o.key[j]);
+    for (int j = 0; j < QUICK_KEYS; j++) q.key[j] = q.key[j] > o.key[QUICK_KEYS - 1 - j] ? q.key[j] : o.key[QUICK_KEYS - 1 - j];
+#pragma unroll
+    for (int step = 2; step >= 1; step >>= 1)
+#pragma unroll
+        for (int j = 0; j < QUICK_KEYS; j++)
+            if (!(j & step)) {
+                const unsigned long long a = q.key[j], b = q.key[j + step];
+                q.key[j] = a > b ? a : b;
+                q.key[j + step] = a > b ? b : a;
+            }
     quick_add_sum(q, o.mx, o.sum, inv_t);
     q.bad |= o.bad;
 }
