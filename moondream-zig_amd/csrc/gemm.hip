@@ -1242,16 +1242,17 @@ int run_gemm(moon_ctx *ctx, const half_t *A, const half_t *B, const half_t *bias
     // The kernels with 128 x 128 accumulators per wavefront (gemm_wide.hpp)
     const bool wide_ok = buffers_ok && K % 16 == 0 && N % 8 == 0 && p.lds_epilogue;
     int wide = 0; // 114: 128 x 128 tiles, 212: 256 x 128, 221: 256 x 256
-    // Default: 256 x 256 tiles where they fill every CU at least once (measured 5 % faster than the 256 x 128 kernel at
-    // 4096^3); the other two arrangements measured equal to or slower than the wavefront-specialised kernels on every shape
-    // of the two models (their sum over the four wavefronts costs what their k-loop saves) and are only taken when named.
-    if (wide_ok && !force && size_t((M + 255) / 256) * ((N + 255) / 256) >= size_t(cus) && !must_fuse) wide = 221;
+    // 256 x 256 tiles where they fill every CU at least once: those of gemm_block.hpp (4096^3 119 -> 100 us, 2048 x 8192 x 8192 220 -> 191, 4096 x 4096 x 1024 36 -> 31; the same bits),
+    // and for a K that has no whole k-tiles of them the ones of gemm_wide.hpp, 5 % faster there than the 256 x 128 kernel.  The other two arrangements measured equal to or slower
+    // than the wavefront-specialised kernels on every shape of the two models (their sum over the four wavefronts costs what their k-loop saves) and are only taken when named.
+    const bool large = wide_ok && !force && size_t((M + 255) / 256) * ((N + 255) / 256) >= size_t(cus) && !must_fuse;
+    if (large && K % BK) wide = 221;
     if (wide_ok && force && !strcmp(force, "w114")) wide = 114;
     if (wide_ok && force && !strcmp(force, "w212")) wide = 212;
     if (wide_ok && force && !strcmp(force, "w221")) wide = 221;
     // A [K, N] operand is read as it lies by the wavefront-specialised kernels (the 128 x 128 one up to one tile per compute
     // unit, the 192- / 256-row ones beyond); the other kernels get a transposed copy first.  MOON_GEMM_KN_TRANSPOSE: always the copy.
-    const bool native_kn = b_layout == MOON_B_KN && N % 8 == 0 && K % 16 == 0 && buffers_ok && !force && !wide && !getenv("MOON_GEMM_KN_TRANSPOSE") &&
+    const bool native_kn = b_layout == MOON_B_KN && N % 8 == 0 && K % 16 == 0 && buffers_ok && !force && !large && !getenv("MOON_GEMM_KN_TRANSPOSE") &&
                            (tiles <= cus || (K % BK == 0 && p.lds_epilogue));
     if (b_layout == MOON_B_KN && !native_kn) {
         MOON_TRY(moon_grow(ctx, ctx->work[2], size_t(N) * K * sizeof(half_t)));
@@ -1341,7 +1342,7 @@ int run_gemm(moon_ctx *ctx, const half_t *A, const half_t *B, const half_t *bias
         int mi = force ? !strcmp(force, "b192") ? 3 : !strcmp(force, "b256") ? 4 : 0 : 0;
         if (!force && tiles > cus) {
             mi = block_height(cus, M, (N + 255) / 256, K / BK, &us);
-            if (us >= narrow_us(cus, M, N, K / BK)) mi = 0;
+            if (!large && us >= narrow_us(cus, M, N, K / BK)) mi = 0;
         }
         if (mi) {
             GemmBlockArgs a{};

@@ -59,3 +59,18 @@ def test_prompts_at_the_edges_of_the_tiles(moon, O, ctx, dim, hidden, heads, pie
         assert O.rel_frobenius(dev.hidden(rows), h_ref) <= TOL, (i, rows)
         assert O.rel_frobenius(dev.logits().reshape(1, -1), ref.lm_head(h_ref).reshape(1, -1)) <= TOL, (i, rows)
     dev.close()
+
+
+# 256 x 256 tiles enough for every compute unit: whole k-tiles take the wide tiles, a K without them (80) the kernel with 128 x 128 accumulators
+# a wavefront; the [K, N] operand and its [N, K] copy give the same bits.
+@pytest.mark.parametrize("M,N,K,kernel", [(4097, 4088, 64, "gemm_nt_block_kernel"), (3841, 4104, 192, "gemm_nt_block_kernel"), (4000, 4096, 80, "gemm_nt_wide_kernel")])
+def test_products_of_many_wide_tiles(moon, O, ctx, M, N, K, kernel):
+    a = O.fill_normal_f16((M, K), 0, 0, 1.0)
+    w = O.fill_normal_f16((N, K), 0, 1, 0.05)
+    got = moon.hgemm_trans.matmul(a, w, ctx=ctx)
+    assert kernel in ctx.last_kernel()
+    assert np.array_equal(moon.hgemm.matmul(a, np.ascontiguousarray(w.T), ctx=ctx), got)
+    assert kernel in ctx.last_kernel()
+    ref = O.hgemm_trans(a, w)
+    assert O.rel_frobenius(got, ref) <= TOL
+    assert np.abs(got.astype(np.float32) - ref.astype(np.float32)).max() <= 2 * 2.0**-10 * np.abs(ref.astype(np.float32)).max()
