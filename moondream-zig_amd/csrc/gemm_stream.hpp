@@ -32,10 +32,10 @@ template <int MI> struct StreamSource {
     __amdgpu_buffer_rsrc_t a, w;
     int off_a[2 * MI], off_w[4]; // bytes at k = 0
     int k, n_ktiles;             // bytes of the first k-tile, their number (>= 1)
+    bool once;                   // (with ONCE) no other row tile reads these weights: they are not to push the activations out of the L2 (non-temporal copies)
 };
 __device__ __forceinline__ int stream_row_a(int mi, int role_wave, int j, int lane) { return 16 * mi * role_wave + 8 * j + (lane >> 3); }
 
-// ONCE: the weights are read by one tile, or a few, and are not to push the activations out of the L2 (non-temporal copies).
 template <int MI, bool ONCE, class Tile, class Next, class Open>
 __device__ __forceinline__ void stream_load(half_t *lds, int role_wave, Next next, Open open) {
     using S = Stream<MI>;
@@ -49,9 +49,15 @@ __device__ __forceinline__ void stream_load(half_t *lds, int role_wave, Next nex
 #pragma unroll
         for (int j = 0; j < 2 * MI; j++)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(s.a, (__attribute__((address_space(3))) void *)(dst + (16 * MI * role_wave + 8 * j) * BK), 16, s.off_a[j], s.k, 0, 0);
+        if (ONCE && s.once) {
 #pragma unroll
-        for (int j = 0; j < 4; j++)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(s.w, (__attribute__((address_space(3))) void *)(dst + S::ROWS * BK + (32 * role_wave + 8 * j) * BK), 16, s.off_w[j], s.k, 0, ONCE ? 2 : 0);
+            for (int j = 0; j < 4; j++)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(s.w, (__attribute__((address_space(3))) void *)(dst + S::ROWS * BK + (32 * role_wave + 8 * j) * BK), 16, s.off_w[j], s.k, 0, 2);
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(s.w, (__attribute__((address_space(3))) void *)(dst + S::ROWS * BK + (32 * role_wave + 8 * j) * BK), 16, s.off_w[j], s.k, 0, 0);
+        }
         stage = stage + 1 == S::STAGES ? 0 : stage + 1;
         issued++;
         s.k += BK * 2;

@@ -119,7 +119,6 @@ struct SegGemm {
     int tile;                 // bf16, no list: 2, 3, 4: tiles of so many 64 rows and 128 columns, SEG_BLOCK + 3, + 4: and 256 columns, SEG_THIN + 2: and 64; 0: by shape
 };
 constexpr int SEG_BLOCK = 16, SEG_THIN = 32;
-constexpr int SEG_ONCE_ROWS = 112; // rows of a group on average up to which a group is taken to be one row tile
 constexpr int SEG_TILE_ROWS = 128; // rows of a tile (both element types walk tile lists of this height)
 int launch_seg_gemm(moon_ctx *ctx, int dtype, SegGemm p);
 // k splits worth taking for an all-f32 product of this shape; together their slabs have at most max_rows rows

@@ -16,6 +16,7 @@ static_assert(SEG_K_TILE == BK && SEG_TILE_COLUMNS == BN && SEG_MAX_SPLITS <= SE
 
 struct TilePos {
     int m0, m_end, n0, group, split;
+    bool lone; // of a list: the group has no other row tile
 };
 // A die's slot (seg_schedule.hpp) -> its tile; returns what seg_find does.
 __device__ __forceinline__ int seg_tile(const SegGemm &p, const SegWalk &w, bool listed, int die, int slot, int tile_m, int tile_n, TilePos &t) {
@@ -27,7 +28,9 @@ __device__ __forceinline__ int seg_tile(const SegGemm &p, const SegWalk &w, bool
         t.split = 0;
         t.group = entry(p.tile_group, tm);
         t.m0 = entry(p.tile_row, tm);
-        t.m_end = min(t.m0 + tile_m, entry(p.tile_end, tm));
+        const int end = entry(p.tile_end, tm);
+        t.m_end = min(t.m0 + tile_m, end);
+        t.lone = end <= t.m0 + tile_m && (tm == 0 || entry(p.tile_group, tm - 1) != t.group);
     } else {
         if (const int r = seg_find(w, die, slot, tm, tn, t.split); r <= 0) return r;
         t.group = 0;
@@ -137,7 +140,7 @@ __device__ __forceinline__ void seg_store(const SegGemm &p, const Acc &acc, cons
 
 // LISTED: row tiles from a list.  A kernel of its own: with both ways to a tile in one, the plain products of a prompt of 768 rows lost
 // 0.4 to 0.8 us each.
-template <int MI, bool LISTED, bool ONCE = false>
+template <int MI, bool LISTED>
 __global__ __launch_bounds__(DMA_THREADS) void seg_gemm_bf16_kernel(SegGemm p, SegWalk w) {
     extern __shared__ __attribute__((aligned(16))) half_t lds_stream[]; // (the tile product addresses LDS from 0: nothing static beside it)
     using S = Stream<MI>;
@@ -150,7 +153,7 @@ __global__ __launch_bounds__(DMA_THREADS) void seg_gemm_bf16_kernel(SegGemm p, S
         }
     };
     if (threadIdx.x >= 256) {
-        stream_load<MI, ONCE, TilePos>(lds_stream, role_wave, next, [&](const TilePos &t, StreamSource<MI> &s) {
+        stream_load<MI, LISTED, TilePos>(lds_stream, role_wave, next, [&](const TilePos &t, StreamSource<MI> &s) {
             // (the launcher has checked that both operands fit a descriptor)
             const bf16_t *weights = reinterpret_cast<const bf16_t *>(p.W) + size_t(t.group) * p.w_group;
             s.a = __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p.A), 0, p.a_rows * p.lda * 2, 0x00020000);
@@ -167,6 +170,9 @@ __global__ __launch_bounds__(DMA_THREADS) void seg_gemm_bf16_kernel(SegGemm p, S
             }
             s.k = p.kb[t.split] * 2;
             s.n_ktiles = (p.kb[t.split + 1] - p.kb[t.split]) / BK;
+            // A group's only row tile: 64 experts of 704, 8 a row, width 2048, us a layer with all copies ordinary, all non-temporal, and by this rule: 61 rows 158, 143, 143, 768 rows 234, 248, 225,
+            // 1025 rows 270, not tried, 261 with random choices; 768 rows over the experts evenly 229, 218, 218.  A second row tile finds what the first one left in the L2.
+            s.once = LISTED && t.lone;
         });
         return;
     }
@@ -370,11 +376,8 @@ int launch_seg_gemm(moon_ctx *ctx, int dtype, SegGemm p) {
             hipLaunchKernelGGL(kern, dim3((unsigned)seg_workgroups(w, cus)), dim3(DMA_THREADS), lds, ctx->stream, p, w);
             return MOON_OK;
         };
-        static std::atomic<bool> set_listed[64], set_once[64], set2[64], set3[64], set4[64], wide3[64], wide4[64], thin2[64];
-        // Groups of up to a row tile each read their weights once, non-temporally: 12 layers of width 2048, 64 experts of 704, 8 a row, 61 rows 170 -> 159 us a layer, 768 rows 229 -> 220.  With two
-        // row tiles in a group the second one finds them in the L2 otherwise: 1025 rows 284 and 301, 1301 320 and 362; as fast either way at 950 rows, 119 a group.
-        if (p.tile_group && p.M <= SEG_ONCE_ROWS * (p.max_tiles - p.M / SEG_TILE_ROWS)) MOON_TRY(go(seg_gemm_bf16_kernel<2, true, true>, Stream<2>::LDS_BYTES, set_once));
-        else if (p.tile_group) MOON_TRY(go(seg_gemm_bf16_kernel<2, true>, Stream<2>::LDS_BYTES, set_listed));
+        static std::atomic<bool> set_listed[64], set2[64], set3[64], set4[64], wide3[64], wide4[64], thin2[64];
+        if (p.tile_group) MOON_TRY(go(seg_gemm_bf16_kernel<2, true>, Stream<2>::LDS_BYTES, set_listed));
         else if (tile == SEG_THIN + 2) MOON_TRY(go(seg_gemm_bf16_thin_kernel, Thin::LDS_BYTES, thin2));
         else if (tile == SEG_BLOCK + 4) MOON_TRY(go(seg_gemm_bf16_block_kernel<4>, Block<4>::LDS_BYTES, wide4));
         else if (tile == SEG_BLOCK + 3) MOON_TRY(go(seg_gemm_bf16_block_kernel<3>, Block<3>::LDS_BYTES, wide3));
