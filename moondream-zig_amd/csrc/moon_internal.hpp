@@ -137,10 +137,10 @@ int launch_gemm(moon_ctx *ctx, const half_t *A, const half_t *B, const half_t *b
                 size_t M, size_t N, size_t K, int b_layout, int epilogue, const half_t *resid = nullptr, const GemmLayerNorm *ln = nullptr);
 // A decoder block's two products of the same rows in ONE launch: out1 [M][N1] = gelu(A . W1^T + bias1), and the qkv projection [M, K] . [3 * H * D, K]^T + bias
 // with launch_qkv_rope_cache folded into its epilogue: the rotated q goes to q_out [H][M][D], the rotated k and v to rows pos0 .. pos0 + M - 1 of the cache
-// [H][max_seq][D]; the projection itself is not written anywhere.  The same bits as the launches one by one where those take no ranges of k.  Only for D = 64, rot_dim = 32, K % 64 == 0 and where that is
-// estimated to be shorter; *done says whether anything was launched.
+// [H][max_seq][D]; the projection itself is written nowhere for D = 64 and rot_dim = 32, otherwise to qkv, which a launch of launch_qkv_rope_cache then reads.  The same bits as the
+// launches one by one where those take no ranges of k.  Only for K % 64 == 0 and where that is estimated to be shorter; *done says whether anything was launched.
 int launch_gemm_front(moon_ctx *ctx, const half_t *A, const half_t *W, const half_t *bias, const half_t *W1, const half_t *bias1, half_t *out1, size_t N1, size_t M,
-                      size_t K, half_t *q_out, half_t *cache_k, half_t *cache_v, const float *table, size_t H, size_t D, size_t rot_dim, size_t max_seq, size_t pos0,
+                      size_t K, half_t *qkv, half_t *q_out, half_t *cache_k, half_t *cache_v, const float *table, size_t H, size_t D, size_t rot_dim, size_t max_seq, size_t pos0,
                       bool *done);
 // Two products with the same [M, N] result in ONE launch, then the launch that finishes both, as launch_gemm does with
 // ln->add_partial set: C = f16(resid + f16(add + t)), add = f16(f16(A_add . B_add^T) + bias_add), t = f16(f16(A . B^T) + bias),

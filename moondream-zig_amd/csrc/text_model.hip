@@ -396,7 +396,7 @@ int layer_forward(moon_text_model *m, size_t layer, size_t n, size_t pos, bool p
         MOON_TRY(launch_gemv_nt(ctx, m->fc1, fc2_w, fc2_b, m->mlp, z.d, z.ffn, MOON_EPI_BIAS));
     } else {
         bool front = false; // the projection, with the rotation and the cache update in its epilogue, and fc1 in one launch, where the shape has that form
-        MOON_TRY(launch_gemm_front(ctx, m->ln_in, qkv_w, qkv_b, fc1_w, fc1_b, m->fc1, z.ffn, n, z.d, m->q_rot, ck, cv, m->freqs, z.H, z.D, m->cfg.rot_dim, z.S, pos, &front));
+        MOON_TRY(launch_gemm_front(ctx, m->ln_in, qkv_w, qkv_b, fc1_w, fc1_b, m->fc1, z.ffn, n, z.d, m->qkv, m->q_rot, ck, cv, m->freqs, z.H, z.D, m->cfg.rot_dim, z.S, pos, &front));
         if (!front) {
             MOON_TRY(launch_gemm(ctx, m->ln_in, qkv_w, qkv_b, m->qkv, n, 3 * z.d, z.d, MOON_B_NK, MOON_EPI_BIAS));
             MOON_TRY(launch_qkv_rope_cache(ctx, m->qkv, m->q_rot, ck, cv, m->freqs, n, z.H, z.D, m->cfg.rot_dim, z.S, pos));

@@ -42,14 +42,16 @@ def test_named_tiles_at_their_edges(moon, O, ctx, kernel, M, N, K, epi):
 
 # Prompts in pieces, each behind the ones before it, at the tiles' edges: two rows, a row short of a thin tile, a whole one, one and two
 # rows more, the last size of thin pairs (191) and the first of tall ones, a feed-forward whose width is no whole k-tile (its product
-# is not paired, and its last columns are no whole tile), and at width 2048 the pair in 192 x 256 tiles.
-@pytest.mark.parametrize("dim,hidden,heads,pieces", [(512, 2048, 8, (2, 127, 128, 129, 65)), (512, 2048, 8, (191, 192, 193, 257)), (192, 776, 3, (130, 37, 385)),
-                                                     (192, 832, 3, (64, 129, 513)), (2048, 8192, 32, (1025, 37))])
-def test_prompts_at_the_edges_of_the_tiles(moon, O, ctx, dim, hidden, heads, pieces):
-    cfg = dict(O.TEXT_CFG, vocab=1024, dim=dim, hidden_dim=hidden, n_layers=2, n_heads=heads, head_dim=64, rot_dim=32, max_seq=1088)
+# is not paired, and its last columns are no whole tile), at width 2048 the pair in 192 x 256 tiles, and heads of which other parts than the
+# first half turn (the projection is written, the rotation a launch of its own).
+@pytest.mark.parametrize("dim,hidden,heads,rot,pieces", [(512, 2048, 8, 32, (2, 127, 128, 129, 65)), (512, 2048, 8, 32, (191, 192, 193, 257)), (192, 776, 3, 32, (130, 37, 385)),
+                                                         (192, 832, 3, 32, (64, 129, 513)), (2048, 8192, 32, 32, (1025, 37)), (512, 2048, 8, 64, (37, 128, 700)),
+                                                         (192, 776, 3, 6, (129, 193)), (2048, 8192, 32, 16, (769,))])
+def test_prompts_at_the_edges_of_the_tiles(moon, O, ctx, dim, hidden, heads, rot, pieces):
+    cfg = dict(O.TEXT_CFG, vocab=1024, dim=dim, hidden_dim=hidden, n_layers=2, n_heads=heads, head_dim=64, rot_dim=rot, max_seq=1088)
     weights = O.synth_text_weights(cfg, 9)
     ref = O.TextModel(weights, cfg)
-    mcfg = moon.text_model.make_config(vocab=cfg["vocab"], dim=dim, hidden_dim=hidden, n_layers=2, n_heads=heads, max_seq=cfg["max_seq"])
+    mcfg = moon.text_model.make_config(vocab=cfg["vocab"], dim=dim, hidden_dim=hidden, n_layers=2, n_heads=heads, rot_dim=rot, max_seq=cfg["max_seq"])
     dev = moon.text_model.TextModel(mcfg, weights=weights, ctx=ctx)
     cache = ref.new_cache()
     for i, rows in enumerate(pieces):
