@@ -61,6 +61,7 @@ __device__ __forceinline__ void block_stream(half_t *lds, int wave, int lane, in
     BlockSource s;
     int issue_round = 0;
     if (!next(t, issue_round)) return;
+    int read_round = issue_round; // (a first slot may be empty: the first tile need not be the first round's)
     ahead = t;
     open(ahead, s);
     unsigned to = 0; // stage of the k-tile being copied
@@ -132,7 +133,6 @@ __device__ __forceinline__ void block_stream(half_t *lds, int wave, int lane, in
     lds_barrier();
 #pragma unroll
     for (int i = 0; i < 2; i++) { read_w0(i, 0); read_w0(i, 1); read_a0(i); }
-    int read_round = 1;
     for (bool more = true; more;) {
 #pragma unroll
         for (int i = 0; i < 4; i++)

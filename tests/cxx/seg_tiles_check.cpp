@@ -35,9 +35,10 @@ int main() {
     if (hipSetDevice(0) != hipSuccess || hipStreamCreate(&ctx.stream) != hipSuccess) return printf("no device\n"), 2;
     ctx.cu_count = 256;
     struct Shape {
-        int M, n16, n32, N, K, lda, splits, kb[4], longest_first;
+        int M, n16, n32, N, K, lda, splits, kb[SEG_MAX_SPLITS + 1], longest_first;
     };
-    // edges of a tile's rows and columns, segments that meet inside a tile, one k-tile, two, an odd number; more tiles than compute units; ranges of k
+    // edges of a tile's rows and columns, segments that meet inside a tile, one k-tile, two, an odd number; more tiles than compute units; ranges of k, with 38 wide
+    // tiles each so that a die's last slots are empty and some workgroups' first tile is in their second round
     const Shape shapes[] = {
         {1, 64, 64, 64, 64, 64, 1, {}, 0},
         {63, 0, 0, 64, 128, 136, 1, {}, 0},
@@ -51,6 +52,7 @@ int main() {
         {2000, 3072, 3136, 12352, 192, 192, 1, {}, 0},
         {300, 0, 640, 640, 704, 712, 3, {0, 128, 256, 704}, 1},
         {450, 0, 2048, 2048, 640, 640, 3, {0, 256, 512, 640}, 0},
+        {300, 0, 4864, 4864, 640, 640, 8, {0, 128, 192, 320, 384, 448, 512, 576, 640}, 1},
     };
     int failures = 0, checked = 0;
     std::mt19937_64 rng(1);
