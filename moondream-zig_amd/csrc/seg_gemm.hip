@@ -296,7 +296,7 @@ static int seg_choose(moon_ctx *ctx, const SegGemm &p) {
             best = mi;
         }
     if (p.tile_group || p.rows) return best;
-    if (const double e = seg_thin_estimate(cus, p.M, p.N, p.kb, p.splits); e < t) {
+    if (const double e = seg_thin_estimate(cus, p.M, p.N, p.kb, p.splits, p.longest_first); e < t) {
         t = e;
         best = SEG_THIN + 2;
     }
@@ -334,7 +334,7 @@ int seg_gemm_splits(moon_ctx *ctx, int dtype, size_t M, size_t N, size_t K, size
                 t = e;
                 best = splits;
             }
-        if (const double e = seg_thin_estimate(cus, (int)M, (int)N, kb, splits) + (splits - 1) * slab; e < t) {
+        if (const double e = seg_thin_estimate(cus, (int)M, (int)N, kb, splits, false) + (splits - 1) * slab; e < t) {
             t = e;
             best = splits;
         }

@@ -184,9 +184,10 @@ inline double seg_block_estimate(int cus, int mi, int M, int N, int K) {
 // The same for tiles of 128 x 64 (gemm_thin.hpp) and ranges of k, at most a tile per unit, up to three rows of them: 8 to 128 rows x 16128 x 2048 narrow 20.6 to 25.6, thin 17.7 to 20.1 us;
 // 61 x 2048 x 7552 in eight ranges 12.6 and 10.0, 61 x 4992 x 1024 10.1 and 7.7.  In more rounds they lose: 61 x 16832 x 2048, 263 thin tiles, 23.0 and 27.7.
 constexpr int SEG_THIN_ROWS = 128;
-inline double seg_thin_estimate(int cus, int M, int N, const int *kb, int splits) {
-    const int rows = (M + SEG_THIN_ROWS - 1) / SEG_THIN_ROWS, tiles = rows * ((N + 63) / 64) * splits;
-    if (rows > 3 || tiles > cus) return 1e30;
+inline double seg_thin_estimate(int cus, int M, int N, const int *kb, int splits, bool longest_first) {
+    const int rows = (M + SEG_THIN_ROWS - 1) / SEG_THIN_ROWS, range = rows * ((N + 63) / 64), tiles = range * splits;
+    const int slots = longest_first ? (range + SEG_DIES - 1) / SEG_DIES * splits : (tiles + SEG_DIES - 1) / SEG_DIES, n = cus / SEG_DIES < 1 ? 1 : cus / SEG_DIES;
+    if (rows > 3 || slots > n) return 1e30; // (a die's slots: with ranges dealt longest first it has the same share of each, rounded up)
     int longest = 0;
     for (int s = 0; s < splits; s++) longest = kb[s + 1] - kb[s] > longest ? kb[s + 1] - kb[s] : longest;
     return 1.0 + longest / SEG_K_TILE * (0.24 + 0.1 * tiles / cus + 0.0008 * M / rows);

@@ -1,6 +1,6 @@
 // Host check of the schedule of the segmented products (moondream-zig_amd/csrc/seg_schedule.hpp): division by multiplication against
 // the division, every tile of every range taken exactly once whatever the shape and the number of workgroups, the estimate against the
-// sums along every workgroup's walk, and the walk against a first-free-takes-the-next one where the ranges of k differ in length.
+// sums along every workgroup's walk (thin tiles: none has two), and the walk against a first-free-takes-the-next one where the ranges of k differ in length.
 #include "seg_schedule.hpp"
 
 #include <algorithm>
@@ -80,6 +80,23 @@ int main() {
         expect(std::all_of(seen.begin(), seen.end(), [](int n) { return n == 1; }), "every tile once", M, N, splits, cus);
         const double longest = *std::max_element(us.begin(), us.end()), said = seg_estimate(cus, mi, M, N, kb, splits, longest_first);
         expect(std::fabs(said - longest) <= 1e-9 * longest, "estimate of the walk", M, N, splits, cus);
+    }
+
+    // few rows in tiles of 128 x 64: where they are priced, no workgroup has to take two
+    for (int i = 0; i < 4000; i++) {
+        const int M = (int)in(1, 400), N = 64 * (int)in(1, 260), splits = (int)in(1, 8), longest_first = (int)in(0, 1), cus = (int)(i % 4 ? 256 : in(8, 320));
+        int kb[9] = {0};
+        for (int s = 0; s < splits; s++) kb[s + 1] = kb[s] + 64 * (int)(longest_first ? in(1, 40) : 8);
+        if (seg_thin_estimate(cus, M, N, kb, splits, longest_first) >= 1e30) continue;
+        const SegWalk w = seg_walk((M + SEG_THIN_ROWS - 1) / SEG_THIN_ROWS, (N + 63) / 64, false, kb, splits, longest_first);
+        const int grid = seg_workgroups(w, cus / SEG_DIES * SEG_DIES);
+        int most = 0;
+        for (int b = 0; b < grid; b++) {
+            int taken = 0;
+            for (int round = 0, r, tm, tn, range; (r = seg_find(w, b % SEG_DIES, seg_slot(longest_first, b / SEG_DIES, grid / SEG_DIES, round), tm, tn, range)) >= 0; round++) taken += r;
+            most = std::max(most, taken);
+        }
+        expect(most <= 1, "a thin tile per workgroup", M, N, splits, cus);
     }
 
     // listed row tiles: those that exist once each, and no die with more than an eighth of them, rounded up
