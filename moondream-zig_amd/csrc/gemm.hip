@@ -22,6 +22,7 @@
 #include <cstring>
 
 #include "gemm_block.hpp"
+#include "gemm_choice.hpp"
 #include "gemm_thin.hpp"
 #include "gemm_wide.hpp"
 #include "seg_schedule.hpp"
@@ -1133,40 +1134,8 @@ int launch_thin(moon_ctx *ctx, GemmBlockArgs &a) {
     return MOON_OK;
 }
 
-// What products take, us, launch included, with weights from HBM, kt k-tiles: fitted to 54 products of 200 to 1920 rows by 3072 to 14336 columns by 1024 or 2048.
-// Tiles of 64 mi x 256 in rounds over the units; f: part of the units that a round keeps busy.
-double block_us(int cus, int mi, size_t M, size_t columns, size_t kt) {
-    const size_t tiles = (M + 64 * mi - 1) / (64 * mi) * columns;
-    double us = mi == 3 ? 10.5 : 11;
-    for (size_t left = tiles; left > 0; left -= std::min(left, (size_t)cus)) {
-        const double f = (double)std::min(left, (size_t)cus) / cus;
-        us += (left < tiles ? 6 : 0) + kt * (mi == 3 ? 0.78 + 0.42 * f : 1.03 + 0.5 * f);
-    }
-    return us;
-}
-int block_height(int cus, size_t M, size_t columns, size_t kt, double *us) {
-    const double three = block_us(cus, 3, M, columns, kt), four = block_us(cus, 4, M, columns, kt);
-    *us = std::min(three, four);
-    return three <= four ? 3 : 4;
-}
-// Tiles of 128 x 64 (gemm_thin.hpp); later rounds find their first k-tiles on their way.
-double thin_us(int cus, size_t M, size_t N, size_t kt) {
-    const size_t rows = (M + Thin::ROWS - 1) / Thin::ROWS, tiles = rows * ((N + Thin::COLUMNS - 1) / Thin::COLUMNS);
-    double us = 5.5;
-    for (size_t left = tiles; left > 0; left -= std::min(left, (size_t)cus))
-        us += (left < tiles ? 0.85 : 1.0) * kt * (0.24 + 0.1 * std::min(left, (size_t)cus) / cus + 0.0008 * M / rows);
-    return us;
-}
-// The narrow kernels as run_gemm takes them: 128 x 128 tiles, split in k where they are few (the reduction 6 us), otherwise a workgroup per tile of 192 or 256 rows.
-double narrow_us(int cus, size_t M, size_t N, size_t kt) {
-    const size_t columns = (N + BN - 1) / BN, t128 = (M + 127) / 128 * columns, t192 = (M + 191) / 192 * columns, t256 = (M + 255) / 256 * columns;
-    if (t128 * 2 <= (size_t)cus) return 10 + 0.47 * kt / std::max<size_t>(1, std::min({(size_t)cus / t128, kt / 8, (size_t)8}));
-    if (t128 <= (size_t)cus) return 4 + 0.47 * kt;
-    if (t192 <= (size_t)cus && t192 > t256) return 7 + kt * (0.45 + 0.28 * t192 / cus);
-    double us = 7.5;
-    for (size_t left = t256; left > 0; left -= std::min(left, (size_t)cus)) us += (left < t256 ? 6 : 0) + kt * std::max(0.6, 0.28 + 0.62 * std::min(left, (size_t)cus) / cus);
-    return us;
-}
+static_assert(CHOICE_K_TILE == BK && CHOICE_COLUMNS == BN && CHOICE_THIN_ROWS == Thin::ROWS && CHOICE_THIN_COLUMNS == Thin::COLUMNS && CHOICE_WIDE_COLUMNS == Block<3>::COLUMNS,
+              "the tiles that gemm_choice.hpp prices");
 
 // a.p and a.columns0 are set
 template <int EPI, int EPI2>
@@ -1528,14 +1497,11 @@ int launch_gemm_front(moon_ctx *ctx, const half_t *A, const half_t *W, const hal
     if (!al16(A) || !al16(W) || !al16(bias) || !al16(W1) || !al16(bias1) || !al16(out1) || !al16(qkv) || !al16(q_out) || !al16(cache_k) || !al16(cache_v) || !al16(table)) return MOON_OK;
     // Heads of 64 of which the first 32 turn are rotated where the product leaves them; otherwise the projection is written and rotated by a launch of its own
     // (width 2048, 64 turning: 37 rows 73 -> 53 us a layer, 900 rows 153 -> 140, 1301 rows 261 -> 197; width 1024 at 900 rows as before).
-    // Apart: two products, the GELU of one (2.5 us) and the rotation (4.5).
     const bool fused = D == 64 && rot_dim == 32;
-    double us;
-    const int columns0 = (int)((N + 255) / 256), mi = block_height(cus, M, columns0 + (N1 + 255) / 256, K / BK, &us);
-    const double thin = thin_us(cus, M, N + N1, K / BK);
-    if (std::min(us, thin) >= narrow_us(cus, M, N, K / BK) + narrow_us(cus, M, N1, K / BK) + (fused ? 7.0 : 2.5)) return MOON_OK;
+    const FrontForm form = front_form(cus, M, N, N1, K / BK, fused);
+    if (!form.thin && !form.mi) return MOON_OK;
     GemmBlockArgs a{};
-    a.columns0 = thin < us ? (int)((N + Thin::COLUMNS - 1) / Thin::COLUMNS) : columns0;
+    a.columns0 = (int)(form.thin ? (N + Thin::COLUMNS - 1) / Thin::COLUMNS : (N + 255) / 256);
     for (int i = 0; i < 2; i++) {
         GemmArgs &p = a.p[i];
         p.A = A;
@@ -1548,8 +1514,8 @@ int launch_gemm_front(moon_ctx *ctx, const half_t *A, const half_t *W, const hal
     }
     *done = true;
     if (!fused) {
-        if (thin < us) MOON_TRY((launch_thin<MOON_EPI_BIAS, MOON_EPI_BIAS_GELU>(ctx, a)));
-        else MOON_TRY((launch_block<MOON_EPI_BIAS, MOON_EPI_BIAS_GELU>(ctx, a, mi)));
+        if (form.thin) MOON_TRY((launch_thin<MOON_EPI_BIAS, MOON_EPI_BIAS_GELU>(ctx, a)));
+        else MOON_TRY((launch_block<MOON_EPI_BIAS, MOON_EPI_BIAS_GELU>(ctx, a, form.mi)));
         return launch_qkv_rope_cache(ctx, qkv, q_out, cache_k, cache_v, table, M, H, D, rot_dim, max_seq, pos0);
     }
     GemmArgs &p = a.p[0];
@@ -1560,7 +1526,7 @@ int launch_gemm_front(moon_ctx *ctx, const half_t *A, const half_t *W, const hal
     p.rope_H = (int)H;
     p.rope_max_seq = (int)max_seq;
     p.rope_pos0 = (int)pos0;
-    return thin < us ? launch_thin<EPI_ROPE, MOON_EPI_BIAS_GELU>(ctx, a) : launch_block<EPI_ROPE, MOON_EPI_BIAS_GELU>(ctx, a, mi);
+    return form.thin ? launch_thin<EPI_ROPE, MOON_EPI_BIAS_GELU>(ctx, a) : launch_block<EPI_ROPE, MOON_EPI_BIAS_GELU>(ctx, a, form.mi);
 }
 
 int launch_gemm_pair_ln(moon_ctx *ctx, const half_t *A_add, const half_t *B_add, const half_t *bias_add, size_t K_add, const half_t *A, const half_t *B,
@@ -1575,44 +1541,10 @@ int launch_gemm_pair_ln(moon_ctx *ctx, const half_t *A_add, const half_t *B_add,
     if (!al16(A) || !al16(B) || !al16(A_add) || !al16(B_add) || !al16(bias) || !al16(bias_add) || !al16(resid) || !al16(C) || !al16(ln.gamma) ||
         !al16(ln.beta) || !al16(ln.out) || !ln.add || !al16(ln.add))
         return MOON_OK;
-    // Splits (s_add, s): all workgroups in one round, the longest run of k-tiles as short as it gets, us at `fixed` for a launch and `one` + `all` * busy units for a k-tile,
-    // and for every range its sums, written and read (8 TB/s: they stay in the memory-side cache).
-    const int kt_add = (int)(K_add / BK), kt = (int)(K / BK);
-    struct Plan {
-        int tiles_m = 0, tiles_n = 0, a = 0, s = 0;
-        double us = 1e30;
-    };
-    const auto plan = [&](int tile_m, int tile_n, double fixed, double one, double all) {
-        Plan p;
-        p.tiles_m = (int)((M + tile_m - 1) / tile_m);
-        p.tiles_n = (int)((N + tile_n - 1) / tile_n);
-        const int tiles = p.tiles_m * p.tiles_n;
-        int best_len = 1 << 30;
-        for (int sa = 1; sa <= 8 && sa <= kt_add; sa++)
-            for (int s = 1; s <= 8 && s <= kt; s++) {
-                if (tiles * (sa + s) > cus) continue;
-                const int len = std::max((kt_add + sa - 1) / sa, (kt + s - 1) / s);
-                if (len < best_len || (len == best_len && sa + s < p.a + p.s)) {
-                    best_len = len;
-                    p.a = sa;
-                    p.s = s;
-                }
-            }
-        if (p.a) p.us = fixed + best_len * (one + all * tiles * (p.a + p.s) / cus) + (p.a + p.s) * (double)M * N * 8 / 8e6;
-        return p;
-    };
-    // Below 192 rows tiles of 128 x 64 (gemm_thin.hpp): 37 rows of width 2048, apart 8.3 and 15.9 us.  From there on 192 x 128, or 192 x 256 (gemm_block.hpp) where those leave few ranges of
-    // k: a layer of width 2048 at 850 rows 139 -> 128 us, 1025 192 -> 161, 1536 230 -> 198; at 768 rows 192 x 128 is 2 % faster, at width 1024 up to 9.
-    const bool thin = M < 192;
-    Plan best = thin ? plan(Thin::ROWS, Thin::COLUMNS, 0, 1, 0) : plan(192, BN, 7, 0.45, 0.28);
-    bool wide = false;
-    if (!thin)
-        if (const Plan w = plan(192, 256, 10, 0.78, 0.42); w.us < best.us) {
-            best = w;
-            wide = true;
-        }
-    if (!best.a) return MOON_OK;
-    const int tiles_m = best.tiles_m, tiles_n = best.tiles_n, tiles = tiles_m * tiles_n, best_a = best.a, best_s = best.s;
+    const PairForm form = pair_form(cus, M, N, (int)(K_add / BK), (int)(K / BK));
+    if (!form.a) return MOON_OK;
+    const bool thin = form.tile == PAIR_THIN, wide = form.tile == PAIR_WIDE;
+    const int tiles_m = form.tiles_m, tiles_n = form.tiles_n, tiles = tiles_m * tiles_n;
     GemmPairArgs a;
     const auto fill = [&](GemmArgs &p, const half_t *Ap, const half_t *Bp, size_t Kp, int splits, GrowBuf &ws) -> int {
         p.A = Ap;
@@ -1636,8 +1568,8 @@ int launch_gemm_pair_ln(moon_ctx *ctx, const half_t *A_add, const half_t *B_add,
         p.partial = (float *)ws.ptr;
         return MOON_OK;
     };
-    MOON_TRY(fill(a.p[0], A_add, B_add, K_add, best_a, ctx->work[3]));
-    MOON_TRY(fill(a.p[1], A, B, K, best_s, ctx->work[0]));
+    MOON_TRY(fill(a.p[0], A_add, B_add, K_add, form.a, ctx->work[3]));
+    MOON_TRY(fill(a.p[1], A, B, K, form.s, ctx->work[0]));
     a.units0 = tiles * a.p[0].splits;
     a.units_total = a.units0 + tiles * a.p[1].splits;
     static std::atomic<bool> attr_set[3][64];

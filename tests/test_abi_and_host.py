@@ -111,6 +111,11 @@ def test_schedule_of_the_segmented_products():
     _host_check("seg_schedule")
 
 
+def test_choice_of_the_product_tiles():
+    """csrc/gemm_choice.hpp on the host: the prompts of the GPU tests take the tiles that those tests are about."""
+    _host_check("gemm_choice")
+
+
 def test_places_of_waiting_workgroups():
     """csrc/wait_places.hpp on the host: the decode calls that may be in flight on a device at once, from several contexts and threads."""
     _host_check("wait_places")

@@ -293,8 +293,8 @@ def test_decode_modes_agree_on_the_narrow_layer(moon, O, ctx, cached):
 
 
 def test_prefill_with_out_proj_and_fc2_in_one_launch(moon, O, ctx, monkeypatch):
-    """At 192 rows and more the prefill runs a block's out_proj and fc2 as ONE launch (their partial sums are finished
-    together); MOON_GEMM_NO_PAIR keeps them apart.  Same arithmetic but other splits of K.  Three layers of the real width
+    """The prefill runs a block's out_proj and fc2 as ONE launch where the device holds it in one round (their partial sums are
+    finished together); MOON_GEMM_NO_PAIR keeps them apart.  Same arithmetic but other splits of K.  Three layers of the real width
     (the first two take the joint launch) on a ragged prompt (333 rows: the last row block of the 192-row tiles is partial):
     both forms match the oracle, agree with each other, and are not the same bits (which they would be if the joint launch
     had not been taken)."""
@@ -332,11 +332,10 @@ def test_prefill_of_other_widths_through_the_joint_launch(moon, O, ctx, dim, hid
 
 
 def test_prefill_with_the_rotation_in_the_qkv_product(moon, O, ctx, monkeypatch):
-    """Where the qkv projection takes the 192- / 256-row kernels (more 128 x 128 tiles than compute units: from 641 rows on at
-    this width) its epilogue rotates q and k and writes the cache rows itself; MOON_GEMM_NO_ROPE runs the projection and the
-    rotation as two launches.  The same values, roundings and rotations: hidden states, logits and the ids decoded from the
-    cache are the same bits, for a ragged first chunk at position 0 (700 rows: 192-row tiles, the last one partial) and a
-    second chunk that starts at position 700 (1000 rows: 256-row tiles)."""
+    """The prefill's qkv projection rotates q and k in its epilogue, writes the cache rows itself and runs beside fc1;
+    MOON_GEMM_NO_ROPE runs the projection, the rotation and fc1 as three launches.  The same values, roundings and rotations:
+    hidden states, logits and the ids decoded from the cache are the same bits, for a ragged first chunk at position 0 (700
+    rows: 192 x 256 tiles, the last ones partial) and a second chunk that starts at position 700 (1000 rows: 256 x 256 tiles)."""
     cfg = dict(O.TEXT_CFG, n_layers=2, vocab=2048)
     ref, dev = _text_pair(moon, O, ctx, cfg, seed=5)
     a, b = O.fill_uniform_u32(700, 0, 52, cfg["vocab"]), O.fill_uniform_u32(1000, 0, 53, cfg["vocab"])

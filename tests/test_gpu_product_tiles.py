@@ -63,6 +63,33 @@ def test_prompts_at_the_edges_of_the_tiles(moon, O, ctx, dim, hidden, heads, rot
     dev.close()
 
 
+# The same prompts with the projection, its rotation and fc1 in one launch and in three: of widths below 1024 neither product alone is taken in ranges
+# of k, so the bits are the same, in thin tiles (width 512) and wide ones of both heights (960; the first piece is thin there too), behind other pieces, and where
+# the rotation is a launch of its own either way (64 turning).  Which form a piece takes is asked of the choice itself (tests/cxx/gemm_choice_check.cpp); that out_proj and fc2 shared
+# a launch, and its tiles, of the last launch.
+@pytest.mark.parametrize("dim,hidden,heads,rot,pieces", [(512, 2048, 8, 32, (37, 129, 191, 385)), (512, 2048, 8, 64, (37, 129, 191, 385)), (960, 3840, 15, 32, (129, 897)),
+                                                         (960, 3840, 15, 32, (130, 1729))])
+def test_one_launch_gives_the_bits_of_three(moon, O, ctx, monkeypatch, dim, hidden, heads, rot, pieces):
+    cfg = moon.text_model.make_config(vocab=1024, dim=dim, hidden_dim=hidden, n_layers=2, n_heads=heads, rot_dim=rot, max_seq=2048)
+    dev = moon.text_model.TextModel(cfg, seed=6, std=0.03, ctx=ctx)
+    out = []
+    for apart in (False, True):
+        if apart:
+            monkeypatch.setenv("MOON_GEMM_NO_ROPE", "1")
+        dev.reset()
+        got = []
+        for i, rows in enumerate(pieces):
+            dev.forward(O.fill_uniform_u32(rows, i, 58, 1024))
+            assert ctx.last_kernel().startswith("gemm_nt_thin_pair_kernel" if rows < 192 else "gemm_nt_dma192_pair_kernel"), rows
+            got += [dev.hidden(rows).copy(), dev.logits().copy()]
+        got.append(np.asarray(dev.greedy(5)).astype(np.uint32).view(np.uint16))
+        out.append(got)
+    monkeypatch.delenv("MOON_GEMM_NO_ROPE")
+    dev.close()
+    for x, y in zip(*out):
+        assert np.array_equal(x.view(np.uint16), y.view(np.uint16))
+
+
 # 256 x 256 tiles enough for every compute unit: whole k-tiles take the wide tiles, a K without them (80) the kernel with 128 x 128 accumulators
 # a wavefront; the [K, N] operand and its [N, K] copy give the same bits.
 @pytest.mark.parametrize("M,N,K,kernel", [(4097, 4088, 64, "gemm_nt_block_kernel"), (3841, 4104, 192, "gemm_nt_block_kernel"), (4000, 4096, 80, "gemm_nt_wide_kernel")])
