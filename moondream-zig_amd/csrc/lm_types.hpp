@@ -35,11 +35,13 @@ template <class T> __device__ __forceinline__ float dot_piece(const lm_u32x4 &w,
 
 // library exponentials: the gates and weights are wanted to f32 accuracy
 __device__ __forceinline__ float lm_sigmoid(float z) { return 1.0f / (1.0f + expf(-z)); }
-// z / (1 + exp(-z)): exp(-z) = 2^r 2^f with |f| <= 1/2 and f to twice f32's digits, the hardware's 2^f and 1 / d (of a quarter of d: above 2^126 its reciprocal is no
-// normal number), one correction of the quotient.  The same bits as z / (1.0f + expf(-z)) (tested) in a quarter fewer instruction cycles: the library's ranges and scalings serve
-// arguments that do not occur here.  A gated product's epilogue is these: 1920 x 16128 x 2048 120 -> 115 us, 768 rows 54.8 -> 53.1.
+// z / (1 + exp(-z)).  exp(-z) = 2^r 2^f, r whole and |f| <= 1/2: the product with -1 / ln 2 in two pieces (Dekker's, with fused multiply-adds for the exact rest), so f has twice f32's
+// digits, the hardware's 2^f, and a division by the hardware's 1 / d (of a quarter of d: above 2^126 its reciprocal is no normal number) with one Newton correction of the
+// quotient.  These are the steps of the compiler's own expf for gfx950 without its ranges and scalings, which serve arguments that do not occur here, and its second piece of 1 / ln 2 (one unit
+// below the nearest float, with which 15 results differ): the same bits as z / (1.0f + expf(-z)), for every f32 value (tested), in a quarter fewer instruction
+// cycles.  A gated product's epilogue is these: 1920 x 16128 x 2048 120 -> 115 us, 768 rows 54.8 -> 53.1.
 __device__ __forceinline__ float lm_silu(float z) {
-    constexpr float hi = -1.44269502e+00f, lo = -1.92596299e-08f; // -1 / ln 2
+    constexpr float hi = -1.44269502e+00f, lo = -1.92596286e-08f; // -1 / ln 2
     const float x = __builtin_amdgcn_fmed3f(z, -200.0f, 200.0f), t = x * hi, r = __builtin_rintf(t);
     const float f = (t - r) + __builtin_fmaf(x, lo, __builtin_fmaf(x, hi, -t)), d = 1.0f + __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f(f), (int)r);
     const float i = __builtin_amdgcn_rcpf(d * 0.25f) * 0.25f, q = z * i;
