@@ -459,7 +459,8 @@ int moon_bin_vision_io_weights(const moon_bin *bin, const moon_vision_config *cf
  *   MOON_LAYER_QKV_WGS=n           decode mode 0: workgroups that take qkv rows (default: the attention and output workgroups)
  *   MOON_LAYER_FC1_OUT_ROWS=n      decode mode 0: fc1 rows per output wavefront (default: about a third of an fc1-only wavefront's
  *                                  share, at least one; 0 is allowed)
- *   MOON_GEMM_KERNEL=regs|dma|dma256|b192|b256|thin|w114|w212|w221  forces one of the MFMA product kernels where the shape allows it (default: by shape)
+ *   MOON_GEMM_KERNEL=regs|dma|dma256|b192|b256|thin|w114|w212|w221  forces one of the MFMA product kernels where the shape allows it (default: by shape); f32 sums
+ *                                  may be added in another order than the default's, in a prefill too, which then takes no joint launches
  *   MOON_GEMM_EPILOGUE=direct      the product kernels store their tile without the pass through LDS (default: through LDS)
  *   MOON_SAMPLE_SEPARATE=1         sampled loops with top_k <= 3: the LM-head launch leaves every token to sample_kernel instead of
  *                                  deciding it where it provably can (read at every call, so a test can compare the two in one process)
@@ -469,9 +470,9 @@ int moon_bin_vision_io_weights(const moon_bin *bin, const moon_vision_config *cf
  *   MOON_GEMM_KN_TRANSPOSE=1       products with a [K, N] second operand always run over a transposed copy instead of reading the operand
  *                                  in place where the shape allows (read at every call; the same bits either way)
  *   MOON_GEMM_NO_ROPE=1            text prefill: the qkv projection, the rotation + cache update and fc1 run as three launches instead
- *                                  of one (read at every call; the same bits where neither product alone is taken in ranges of k,
- *                                  otherwise, at few rows, f32 sums in another order)
- * Every other setting gives the same results, bit for bit; only the time changes. */
+ *                                  of one, or of two where heads turn in another part than their first 32 dimensions (read at every call; the
+ *                                  same bits where neither product alone is taken in ranges of k, otherwise, at few rows, f32 sums in another order)
+ * Every setting but MOON_GEMM_KERNEL, MOON_GEMM_NO_PAIR and MOON_GEMM_NO_ROPE gives the same results, bit for bit; only the time changes. */
 
 #ifdef __cplusplus
 }

@@ -698,7 +698,7 @@ __device__ __forceinline__ void gemm_block_out(const GemmArgs &p, const float4_t
 // The same for a qkv projection whose heads' first 32 dimensions of 64 are rotated: the wavefront's 64 columns are one head of q, k or v, a column and its partner 16
 // further on are in one lane, and what is written are the values, roundings and rotations of qkv_rope_cache_vec_kernel on the finished rows.  Rotated where they
 // lie, before they are parked, with the angles of the next 32 rows on their way: from the parked rows, a row's angles after another, every 8 rows of
-// the tile waited for the table (900 rows of width 2048: 70 us with fc1, 57 so).
+// the tile waited for the table (900 rows of width 2048 with fc1: 70 us, 64 so, 57 without a rotation).
 template <int MI>
 __device__ __forceinline__ void gemm_block_out_rope(const GemmArgs &p, const float4_t (&acc)[4][2 * MI], int m_wave, int n0, int lane, char *scratch) {
     asm volatile("" : "+v"(lane));
@@ -1212,7 +1212,8 @@ int run_gemm(moon_ctx *ctx, const half_t *A, const half_t *B, const half_t *bias
     const bool wide_ok = buffers_ok && K % 16 == 0 && N % 8 == 0 && p.lds_epilogue;
     int wide = 0; // 114: 128 x 128 tiles, 212: 256 x 128, 221: 256 x 256
     // 256 x 256 tiles where they fill every CU at least once: those of gemm_block.hpp (4096^3 119 -> 100 us, 2048 x 8192 x 8192 220 -> 191, 4096 x 4096 x 1024 36 -> 31; the same bits),
-    // and for a K that has no whole k-tiles of them the ones of gemm_wide.hpp, 5 % faster there than the 256 x 128 kernel.  The other two arrangements measured equal to or slower
+    // and for a K that has no whole k-tiles of them the ones of gemm_wide.hpp, where the alternative is the register-staged 128 x 128 kernel (4096 x 4096 x 1008 55 us, 43 so; x 4080 205, 130; 8192 x 8192 x 1008 219, 163;
+    // 4096 x 16384 x 528 128, 107; at K = 80 equal, 8192 x 8192 49, 51).  The other two arrangements of gemm_wide.hpp measured equal to or slower
     // than the wavefront-specialised kernels on every shape of the two models (their sum over the four wavefronts costs what their k-loop saves) and are only taken when named.
     const bool large = wide_ok && !force && size_t((M + 255) / 256) * ((N + 255) / 256) >= size_t(cus) && !must_fuse;
     if (large && K % BK) wide = 221;

@@ -1,10 +1,11 @@
 // The tile product as a stream of tiles (gemm_stream.hpp) in tiles of 64 MI (m) x 256 (n) x 64 (k), MI = 3 or 4: eight wavefronts, two per
 // SIMD, that all copy and all multiply, 32 MI (m) x 64 (n) each.
-// A tile twice as wide as gemm_stream.hpp's needs three quarters (MI = 4) of its copies and operand bytes per product, and what one
-// wavefront of a SIMD waits for the other one covers.  A k-tile at MI = 4 takes 1.37 us (1.53 PFLOP/s) where two of gemm_stream.hpp's take 1.59; its copies alone 0.9,
-// without copies 1.13.  What bounds it is power: on random operands a loop of nothing but 32 x 32 x 16 products reaches 1.69 PFLOP/s and one of 16 x 16 x 32
-// products 1.92 (both 2.4 and more on zeros; sums are read and written half as often, and come out with the same bits): hence these.
-//   1920 x 16128 x 2048 (gated, bf16, weights from HBM): 129 -> 112 us; 768 rows 61 -> 51; 1301 x 16832 x 2048 103 -> 88.
+// A tile twice as wide as gemm_stream.hpp's needs two thirds (MI = 4) of its copies per product, 512 rows a k-tile where two of those copy 768, and as many operand reads from LDS; what one
+// wavefront of a SIMD waits for the other one covers.  A k-tile at MI = 4 takes 1.37 us with every unit busy (1.57 PFLOP/s) where two of gemm_stream.hpp's take 1.59; its copies alone 0.9,
+// without copies 1.13.  What bounds it: the products, at the clock that they leave (1.7 to 1.8 of 2.4 GHz), and cycles without one; the matrix cores are busy in 78 % of the cycles at 4096^3 and in 70 % at
+// 1920 x 16128 x 2048.  On random operands nothing but 16 x 16 x 32 products reaches 1.99 PFLOP/s in f16 and 2.08 in bf16 (a k-tile in 1.03 to 1.08 us), of 32 x 32 x 16 ones 1.72 and 1.87 (both 2.4 and
+// more on zeros; sums are read and written half as often, and come out with the same bits): hence these.
+//   1920 x 16128 x 2048 (gated, bf16) among a model's launches, weights from HBM: 136 us in narrow tiles, 117 so (113 with lm_silu's shorter form); 768 rows 58, 51 (47); 1301 x 16832 x 2048 by itself 103 -> 88.
 // LDS holds two k-tiles, 56 or 64 KiB each, and 4 KiB of each wavefront for its epilogue.  Two whole stages would leave one k-tile's time for a copy (1.2 us at this load); so
 // a wavefront's products go by quarters, first half of its rows with the first half of its columns, then first x second, second x second,
 // second x first, an operand half stays in registers for the two quarters that it has, and its place in LDS is free for the k-tile after

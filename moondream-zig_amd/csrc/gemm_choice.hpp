@@ -12,6 +12,10 @@ constexpr int CHOICE_THIN_ROWS = 128, CHOICE_THIN_COLUMNS = 64;        // gemm_t
 constexpr int CHOICE_WIDE_COLUMNS = 256;                               // gemm_block.hpp, by 64 mi rows
 
 // What products take, us, launch included, with weights from HBM, kt k-tiles: fitted to 54 products of 200 to 1920 rows by 3072 to 14336 columns by 1024 or 2048.
+// Over 42 weights (3072 to 24576 columns by 512 to 4096) at 8 to 1920 rows the wide and thin tiles' say 0.8 to 1.5 times what was measured (1.0 to 1.3 at the median of each K), the narrow kernels' 0.6 to 2.2 (0.9 to
+// 1.2), so a choice errs towards launches apart.  432 prompts of 12 models (width 512 to 2560, 2 to 1900 rows) against those launches: 1.27 times as fast in the mean, none slower but width 2560 at 100 to 160 rows, 2.5 %
+// (its rows lie 5,120 bytes apart, and a thin k-tile of 100 of them takes 1.3 times as long as of 37).
+// seg_schedule.hpp prices the same loops for bf16 products, without a launch and beside other narrow kernels: each set of constants was fitted to its own measurements.
 // Tiles of 64 mi x 256 in rounds over the units; f: part of the units that a round keeps busy.
 inline double block_us(int cus, int mi, size_t M, size_t columns, size_t kt) {
     const size_t tiles = (M + 64 * mi - 1) / (64 * mi) * columns;
@@ -91,6 +95,8 @@ inline PairForm pair_plan(int cus, size_t M, size_t N, int kt_add, int kt, PairT
 }
 // Below 192 rows tiles of 128 x 64 (gemm_thin.hpp): 37 rows of width 2048, apart 8.3 and 15.9 us.  From there on 192 x 128, or 192 x 256 (gemm_block.hpp) where those leave few ranges of
 // k: a layer of width 2048 at 850 rows 139 -> 128 us, 1025 192 -> 161, 1536 230 -> 198; at 768 rows 192 x 128 is 2 % faster, at width 1024 up to 9.
+// The line at 192 rows: a layer of width 1024 and 2048 takes 32.6 and 62.4 us at 170 rows, 36.0 and 64.1 in 192 x 128.  Thin tiles go on to win up to 256 rows (230: 33.3 and 68.0, 192 x 128 36.8 and 72.8) and
+// lose behind them at width 2048 (260: 91.6 and 79.9; at width 1024 40.3 and 43.1), which this line does not use.
 inline PairForm pair_form(int cus, size_t M, size_t N, int kt_add, int kt) {
     if (M < 192) return pair_plan(cus, M, N, kt_add, kt, PAIR_THIN, CHOICE_THIN_ROWS, CHOICE_THIN_COLUMNS, 0, 1, 0);
     const PairForm narrow = pair_plan(cus, M, N, kt_add, kt, PAIR_NARROW, 192, CHOICE_COLUMNS, 7, 0.45, 0.28), wide = pair_plan(cus, M, N, kt_add, kt, PAIR_WIDE, 192, CHOICE_WIDE_COLUMNS, 10, 0.78, 0.42);

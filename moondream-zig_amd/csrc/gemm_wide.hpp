@@ -9,7 +9,8 @@
 //   each k-tile between them (16-wide steps wk*KS .. wk*KS+KS-1), their accumulators being summed through LDS once, after
 //   the k-loop, in a fixed order.
 //   1 x 1 x 4 (k-tile 64): 128 x 128 per workgroup, for shapes with about as many such tiles as CUs,
-//   2 x 1 x 2 (k-tile 64): 256 x 128,   2 x 2 x 1 (k-tile 32): 256 x 256, for large shapes.
+//   2 x 1 x 2 (k-tile 64): 256 x 128,   2 x 2 x 1 (k-tile 32): 256 x 256, for large shapes whose K is
+//   no multiple of 64 (those that are take gemm_block.hpp's tiles).
 // There are no loader wavefronts: every wavefront copies its share of the next k-tiles global -> LDS with
 // buffer_load_dwordx4 ... lds (no staging registers), STAGES k-tiles deep, one barrier per k-tile.  With a single
 // wavefront per SIMD nothing else fills the matrix core while that wavefront issues other instructions, so the operand

@@ -39,7 +39,7 @@ __device__ __forceinline__ float lm_sigmoid(float z) { return 1.0f / (1.0f + exp
 // digits, the hardware's 2^f, and a division by the hardware's 1 / d (of a quarter of d: above 2^126 its reciprocal is no normal number) with one Newton correction of the
 // quotient.  These are the steps of the compiler's own expf for gfx950 without its ranges and scalings, which serve arguments that do not occur here, and its second piece of 1 / ln 2 (one unit
 // below the nearest float, with which 15 results differ): the same bits as z / (1.0f + expf(-z)), for every f32 value (tested), in a quarter fewer instruction
-// cycles.  A gated product's epilogue is these: 1920 x 16128 x 2048 120 -> 115 us, 768 rows 54.8 -> 53.1.
+// cycles.  A gated product's epilogue is these: 1920 x 16128 x 2048 among a model's launches 117.3 -> 112.7 us, 768 rows 50.8 -> 47.2.
 __device__ __forceinline__ float lm_silu(float z) {
     constexpr float hi = -1.44269502e+00f, lo = -1.92596286e-08f; // -1 / ln 2
     const float x = __builtin_amdgcn_fmed3f(z, -200.0f, 200.0f), t = x * hi, r = __builtin_rintf(t);
