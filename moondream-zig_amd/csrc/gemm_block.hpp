@@ -5,7 +5,7 @@
 // without copies 1.13.  What bounds it: the products, at the clock that they leave (1.7 to 1.8 of 2.4 GHz), and cycles without one; the matrix cores are busy in 78 % of the cycles at 4096^3 and in 70 % at
 // 1920 x 16128 x 2048.  On random operands nothing but 16 x 16 x 32 products reaches 1.99 PFLOP/s in f16 and 2.08 in bf16 (a k-tile in 1.03 to 1.08 us), of 32 x 32 x 16 ones 1.72 and 1.87 (both 2.4 and
 // more on zeros; sums are read and written half as often, and come out with the same bits): hence these.
-//   1920 x 16128 x 2048 (gated, bf16) among a model's launches, weights from HBM: 136 us in narrow tiles, 117 so (113 with lm_silu's shorter form); 768 rows 58, 51 (47); 1301 x 16832 x 2048 by itself 103 -> 88.
+//   1920 x 16128 x 2048 (gated, bf16) among a model's launches, weights from HBM: 136 us in narrow tiles, 117 so (113 with lm_silu's shorter form; other boxes to 107); 768 rows 58, 51 (47); 1301 x 16832 x 2048 by itself 103 -> 88.
 // LDS holds two k-tiles, 56 or 64 KiB each, and 4 KiB of each wavefront for its epilogue.  Two whole stages would leave one k-tile's time for a copy (1.2 us at this load); so
 // a wavefront's products go by quarters, first half of its rows with the first half of its columns, then first x second, second x second,
 // second x first, an operand half stays in registers for the two quarters that it has, and its place in LDS is free for the k-tile after
