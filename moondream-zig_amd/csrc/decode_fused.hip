@@ -9,6 +9,7 @@
 #include "attn_decode.hpp"
 #include "norm.hpp"
 #include "sample_quick.hpp"
+#include "launch_waits.hpp"
 #include "wait_places.hpp"
 #include <algorithm>
 #include <cmath>
@@ -496,7 +497,6 @@ struct FrontArgs {
     const uint32_t *pos_dev;
 };
 
-constexpr long long FRONT_TIMEOUT_TICKS = 100000000LL; // 1 s of the 100 MHz wall clock
 constexpr int FRONT_COUNTER_STRIDE = 32;               // uint32 slots per 128-byte line: one line per head
 
 template <int CH, int PF>
@@ -628,50 +628,13 @@ struct LayerArgs {
 // front of a dependent access of this compute unit, the sooner it is served; 2 and 1 measured 3 and 12 % slower, 8 and 16 slower too)
 constexpr int LAYER_OUT_CHUNK = 4;
 constexpr int LAYER_PIECE_SLEEP = 6; // units of 64 cycles between two piece requests (see RowGroups::load_pieces)
-constexpr int LAYER_LINE = 32;                       // uint32 per 128-byte line
 constexpr int LAYER_SYNC_FC1_LEAF = 0;               // lines 0..31: fc1 workgroups reported, 32 leaves
 constexpr int LAYER_FC1_LEAVES = 32;
 constexpr int LAYER_SYNC_QKV = LAYER_FC1_LEAVES;     // then one line per head: q, k, v rows written; then one per head: q rows written
-// The two counters that all the output workgroups wait for ("fc1 leaves complete", "heads merged") exist in LAYER_COPIES copies
-// each: whoever completes a leaf or merges a head adds to every copy (one atomic instruction, a lane per copy), and an output
-// workgroup polls the copy of its index.  512 workgroups polling one line keep the memory channel that holds it busy (a poll
-// is a read at the memory side), and everything else that lives in that channel, a 128th of the weight stream included,
-// waits behind them: with the polls of these two counters replaced by fixed delays (timing only) the launch was 4.7 %
-// shorter.  The copies are LAYER_COPY_STRIDE words apart (4 KiB + 256 B), which lands them in different channels whether the
-// channels interleave by 256 bytes or by pages.
-constexpr int LAYER_COPIES = 64;
-constexpr int LAYER_COPY_STRIDE = 1088;
+// The two counters that all the output workgroups wait for ("fc1 leaves complete", "heads merged") exist in LAYER_COPIES copies (launch_waits.hpp).
 constexpr int LAYER_BCAST_FC1 = 0, LAYER_BCAST_HEADS = 1; // sets of copies, behind the lines above
 __host__ __device__ inline int layer_bcast_offset(size_t H) { return (int)(LAYER_SYNC_QKV + 2 * H) * LAYER_LINE; }
 inline int layer_sync_words(size_t H) { return layer_bcast_offset(H) + 2 * LAYER_COPIES * LAYER_COPY_STRIDE; }
-
-// thread 0 of the workgroup polls *word until it reaches target; the clock and the error word are looked at once in
-// 64 polls.  Returns (to every thread) whether the wait succeeded.
-__device__ __forceinline__ bool wait_reached(uint32_t *word, uint32_t target, uint32_t *error, int *s_flag) {
-    lds_barrier();
-    if (threadIdx.x == 0) {
-        const long long t0 = wall_clock64();
-        int ok = 1;
-        for (unsigned polls = 1;; polls++) {
-            if (__hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= target) break;
-            if ((polls & 63u) == 0) {
-                if (__hip_atomic_load(error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
-                    ok = 0;
-                    break;
-                }
-                if (wall_clock64() - t0 > FRONT_TIMEOUT_TICKS) {
-                    __hip_atomic_store(error, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    ok = 0;
-                    break;
-                }
-            }
-        }
-        *s_flag = ok;
-    }
-    lds_barrier();
-    return *s_flag != 0;
-}
-
 
 // FC1_GROUP: fc1 rows a wavefront requests together.  The fewer bytes a compute unit has queued, the sooner the small
 // dependent accesses of the attention chain issued from it are served (two measured 3 % slower than one).

@@ -22,11 +22,17 @@ namespace {
 #define MOON_ARGS_8 MOON_ARGS_7 MOON_ARGS_LINE(0x1c0)
 #define MOON_ARGS_9 MOON_ARGS_8 MOON_ARGS_LINE(0x200)
 #define MOON_ARGS_10 MOON_ARGS_9 MOON_ARGS_LINE(0x240)
+#define MOON_ARGS_11 MOON_ARGS_10 MOON_ARGS_LINE(0x280)
+#define MOON_ARGS_12 MOON_ARGS_11 MOON_ARGS_LINE(0x2c0)
+#define MOON_ARGS_13 MOON_ARGS_12 MOON_ARGS_LINE(0x300)
+#define MOON_ARGS_14 MOON_ARGS_13 MOON_ARGS_LINE(0x340)
+#define MOON_ARGS_15 MOON_ARGS_14 MOON_ARGS_LINE(0x380)
+#define MOON_ARGS_16 MOON_ARGS_15 MOON_ARGS_LINE(0x3c0)
 #define MOON_ARGS_FETCH(n) if constexpr (LINES == n) asm volatile(MOON_ARGS_##n "s_waitcnt lgkmcnt(0)" : "=&s"(word), "+s"(at))
 // Args: the kernel's only parameter
 template <class Args> __device__ __forceinline__ const Args &fetch_arguments() {
     constexpr int LINES = (sizeof(Args) + 63) / 64;
-    static_assert(LINES <= 10, "more lines");
+    static_assert(LINES <= 16, "more lines");
     auto *at = __builtin_amdgcn_kernarg_segment_ptr();
     unsigned word; // (of no use itself)
     MOON_ARGS_FETCH(1);
@@ -39,6 +45,12 @@ template <class Args> __device__ __forceinline__ const Args &fetch_arguments() {
     MOON_ARGS_FETCH(8);
     MOON_ARGS_FETCH(9);
     MOON_ARGS_FETCH(10);
+    MOON_ARGS_FETCH(11);
+    MOON_ARGS_FETCH(12);
+    MOON_ARGS_FETCH(13);
+    MOON_ARGS_FETCH(14);
+    MOON_ARGS_FETCH(15);
+    MOON_ARGS_FETCH(16);
     return *(const Args *)(const __attribute__((address_space(4))) Args *)at;
 }
 

@@ -24,6 +24,11 @@ struct LayerList {
     uint32_t *grouped_rows = nullptr, *counter = nullptr, *want = nullptr;
     uint32_t *want_pinned = nullptr;
     size_t mix_partial_floats = 0, partial_rows = 0;
+    WholeCounts whole;
+    size_t counters = 0;
+    std::vector<int> whole_per_cu; // a layer's workgroups per compute unit where it runs in one launch, otherwise 0
+    WaitNeed whole_need;
+    bool any_whole = false;
     float *x1 = nullptr, *y3 = nullptr;                    // one token: the other copy of x, the parts of a joined layer's second product
     float *dt = nullptr, *delta_o = nullptr, *scratch = nullptr; // delta rule's rows: decays, outputs, chunks
     void *dgate = nullptr;
@@ -35,6 +40,8 @@ struct LayerList {
     std::vector<Table> tables;
     std::vector<void *> allocs;
 };
+
+static int plan_whole(LayerList *l);
 
 namespace {
 
@@ -424,6 +431,7 @@ int create(LayerList *l, const Design *design, const SafeTensors *file, uint64_t
     MOON_TRY(alloc_n(l, LIST_LOGIT_ROWS * l->vp, &l->logits));
     MOON_TRY(alloc_n(l, LIST_LOGIT_ROWS, &l->want));
     MOON_TRY(alloc_n(l, counters, &l->counter));
+    l->counters = counters;
     MOON_TRY(alloc_n(l, l->mix_partial_floats, &l->mix_partial));
     MOON_HIP(ctx, hipHostMalloc((void **)&l->want_pinned, LIST_LOGIT_ROWS * sizeof(uint32_t), hipHostMallocDefault));
     MOON_HIP(ctx, hipStreamSynchronize(ctx->stream));
@@ -440,7 +448,8 @@ int layer_list_create(moon_ctx *ctx, const LayerListSpec &spec, const Design *de
     l->dtype = dtype;
     l->el = dtype == MOON_DTYPE_BF16 ? 2 : 4;
     l->max_seq = max_seq;
-    const int rc = create(l, design, file, seed, std_dev);
+    int rc = create(l, design, file, seed, std_dev);
+    if (rc == MOON_OK) rc = plan_whole(l);
     if (rc != MOON_OK) {
         layer_list_destroy(l);
         return rc;
@@ -454,6 +463,7 @@ void layer_list_destroy(LayerList *l) {
     (void)hipStreamSynchronize(l->ctx->stream);
     for (void *p : l->allocs) (void)hipFree(p);
     if (l->want_pinned) (void)hipHostFree(l->want_pinned);
+    if (l->whole.error) (void)hipHostFree(l->whole.error);
     delete l;
 }
 
@@ -747,159 +757,219 @@ int layer_list_forward(LayerList *l, const uint32_t *ids_dev, size_t n_rows, siz
     return MOON_OK;
 }
 
-int layer_list_step(LayerList *l, const uint32_t *token_dev, size_t pos, const uint32_t *pos_dev) {
+// One token through a layer: the arguments of its launches.
+struct TokenArgs {
+    DecodeProj p{};
+    DecodeMix x{};
+    DecodeOut o{};
+};
+struct TokenAt { // on the way through the layers
+    const LayerDev *joined = nullptr; // the layer before, if x waits for its parts
+    float *x_now, *x_next;
+    // Behind a joined layer the next first product completes x and moves it to the other copy; it ends up in l->x.
+    explicit TokenAt(const LayerList *l) : x_now(l->x), x_next(l->x1) {
+        for (size_t i = 0; i + 1 < l->layers.size(); i++)
+            if (l->layers[i].out_l) std::swap(x_now, x_next);
+    }
+};
+static TokenArgs token_args(const LayerList *l, size_t i, TokenAt &at, const uint32_t *token_dev, size_t pos, const uint32_t *pos_dev) {
+    const int dp = (int)l->dp;
+    TokenArgs t;
+    const LayerDev &d = l->layers[i];
+    const MixerSpec &mx = d.spec.mixer;
+    const FeedForwardSpec &ff = d.spec.ff;
+    const DeltaSpec &de = d.spec.delta;
+    const bool experts = ff.kind == FeedForwardSpec::EXPERTS;
+    DecodeProj &p = t.p;
+    p.x = at.x_now;
+    if (at.joined) {
+        p.y = l->y3;
+        p.out_l = at.joined->out_l;
+        p.out_r = at.joined->out_r;
+        p.x_new = at.x_next;
+        std::swap(at.x_now, at.x_next);
+    }
+    at.joined = d.out_l ? &d : nullptr;
+    p.token = i == 0 ? token_dev : nullptr;
+    p.embed = l->embed;
+    p.embed_scale = l->spec.embed_scale;
+    p.gamma = d.gamma;
+    p.beta = d.beta;
+    p.eps = l->spec.eps;
+    p.width = (int)l->spec.width;
+    p.dp = dp;
+    p.w1 = d.w1;
+    p.n16 = d.n16;
+    p.n32 = d.n32;
+    p.nall = d.nall;
+    p.n16_used = de.heads ? d.od + (int)(de.rank_a + de.rank_g) : d.og + (mx.gate ? (int)mx.heads * d.vdimp : 0);
+    p.n32_used = (int)(de.heads ? de.heads : ff.experts);
+    p.ff = ff.kind == FeedForwardSpec::DENSE ? (int)ff.ff : 0;
+    p.proj = l->proj;
+    p.logits = l->router;
+    p.glu = (char *)l->a2 + size_t(d.ka + d.kr) * l->el;
+    p.h = experts ? l->h : nullptr;
+    DecodeMix &x = t.x;
+    x.proj = l->proj;
+    x.H = (int)mx.heads;
+    x.G = (int)mx.kv_heads;
+    x.dim = (int)mx.dim;
+    x.vdim = (int)mx.vdim;
+    x.dimp = d.dimp;
+    x.vdimp = d.vdimp;
+    x.ok = d.ok;
+    x.ov = d.ov;
+    x.og = d.og;
+    x.qk_rms = mx.qk_rms;
+    x.gate = mx.gate;
+    x.mixes = d.mixes;
+    x.window = (int)mx.window;
+    x.cap = d.cap;
+    x.eps = l->spec.eps;
+    x.lambda = d.lambda;
+    x.scale = mx.scale;
+    x.sink = d.sink;
+    x.ck = d.ck;
+    x.cv = d.cv;
+    x.v_first = first_values(l, d, &x.cap_first);
+    x.pos = pos;
+    x.pos_dev = pos_dev;
+    x.partial = l->mix_partial;
+    x.partial_floats = l->mix_partial_floats;
+    x.counter = l->counter;
+    x.out = l->a2;
+    x.whole = mx.qk_whole_norm;
+    x.rot_dims = (int)mx.rot_dims;
+    x.pool = (int)mx.pool;
+    x.blocks = d.blocks;
+    x.borrowed = mx.kv_from >= 0;
+    x.qn = d.qn;
+    x.kn = d.kn;
+    x.temp = d.temp;
+    x.rot = d.rot;
+    x.rotv = d.rotv;
+    x.pk = d.pk;
+    x.pv = d.pv;
+    if (de.heads) {
+        x.dH = (int)de.heads;
+        x.dG = (int)de.kv_heads;
+        x.ddim = (int)de.dim;
+        x.dvdim = (int)de.vdim;
+        x.ddimp = d.ddimp;
+        x.dvdimp = d.dvdimp;
+        x.taps = (int)de.conv;
+        x.oc = d.oc;
+        x.channels = d.channels;
+        x.od = d.od;
+        x.rank_a = (int)de.rank_a;
+        x.rank_g = (int)de.rank_g;
+        x.kd = d.kd;
+        x.lr16 = d.lr16;
+        x.beta = l->router;
+        x.conv = d.conv;
+        x.a_log = d.a_log;
+        x.dt_bias = d.dt_bias;
+        x.dnorm = d.dnorm;
+        x.wlr = d.wlr;
+        x.state = d.state;
+        x.ring = d.ring;
+        x.dout = (char *)l->a2 + size_t(d.ka) * l->el;
+    }
+    DecodeOut &o = t.o;
+    if (experts) {
+        x.logits = l->router;
+        x.correction = d.correction;
+        x.E = (int)ff.experts;
+        x.top = (int)ff.top;
+        x.ff = (int)ff.ff;
+        x.ffp = d.ffp;
+        x.h = l->h;
+        x.wgu = d.wgu;
+        x.act = l->act;
+        x.ids = l->ids;
+        x.weight = l->weight;
+        o.top = x.top;
+        o.ffp = d.ffp;
+        o.wd = d.wd;
+        o.act = l->act;
+        o.ids = l->ids;
+        o.weight = l->weight;
+    }
+    x.dp = dp;
+    o.x = at.x_now;
+    o.y = at.joined ? l->y3 : nullptr;
+    o.k1 = d.ka;
+    o.k2 = d.ka + d.kr;
+    o.width = (int)l->spec.width;
+    o.dp = dp;
+    o.k0 = d.k0;
+    o.w2 = d.w2;
+    o.a = l->a2;
+    o.down = o.k2 < o.k0 ? (at.joined ? l->y3 + 2 * dp : l->down) : nullptr;
+    return t;
+}
+
+// Which layers a token takes in one launch each, once everything they read has its place
+static int plan_whole(LayerList *l) {
+    moon_ctx *ctx = l->ctx;
+    TokenAt at(l);
+    const uint32_t token = 0;
+    for (size_t i = 0; i < l->layers.size(); i++) {
+        const TokenArgs t = token_args(l, i, at, &token, 0, nullptr);
+        int per_cu = 0;
+        WaitNeed need;
+        const bool can = decode_whole_supported(ctx, l->dtype, t.p, t.x, t.o, l->max_seq, &per_cu, &need);
+        l->whole_per_cu.push_back(can ? per_cu : 0);
+        if (!can) continue;
+        l->whole_need = {std::max(l->whole_need.waiting, need.waiting), l->any_whole ? std::min(l->whole_need.places, need.places) : need.places};
+        l->any_whole = true;
+    }
+    if (l->whole_need.waiting >= l->whole_need.places) l->any_whole = false;
+    if (!l->any_whole) return MOON_OK;
+    MOON_TRY(alloc_n(l, decode_whole_sync_words(), &l->whole.sync));
+    MOON_HIP(ctx, hipHostMalloc((void **)&l->whole.error, sizeof(uint32_t), hipHostMallocDefault));
+    *l->whole.error = 0;
+    MOON_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    return MOON_OK;
+}
+
+const WaitNeed *layer_list_wait_need(const LayerList *l) { return l->any_whole ? &l->whole_need : nullptr; }
+
+bool layer_list_wait_failed(LayerList *l) {
+    if (!l->any_whole || !*(volatile uint32_t *)l->whole.error) return false;
+    // workgroups that gave up have counted nothing
+    (void)launch_fill_uniform_u32(l->ctx, l->whole.sync, decode_whole_sync_words(), 0, 0, 1);
+    (void)launch_fill_uniform_u32(l->ctx, l->counter, l->counters, 0, 0, 1);
+    (void)hipStreamSynchronize(l->ctx->stream);
+    std::fill(l->whole.leaf, l->whole.leaf + 2, 0u);
+    std::fill(l->whole.reached, l->whole.reached + 3, 0u);
+    *(volatile uint32_t *)l->whole.error = 0;
+    return true;
+}
+
+int layer_list_step(LayerList *l, const uint32_t *token_dev, size_t pos, const uint32_t *pos_dev, bool whole) {
     moon_ctx *ctx = l->ctx;
     if (pos >= l->max_seq) return moon_fail(ctx, MOON_ESEQ_TOO_LONG, "layer list: position %zu", pos);
     const int dt = l->dtype, dp = (int)l->dp;
-    // Behind a joined layer the next first product completes x and moves it to the other copy; it ends up in l->x.
-    const LayerDev *joined = nullptr; // the layer before, if x waits for its parts
-    float *x_now = l->x, *x_next = l->x1;
-    for (size_t i = 0; i + 1 < l->layers.size(); i++)
-        if (l->layers[i].out_l) std::swap(x_now, x_next);
+    TokenAt at(l);
     for (size_t i = 0; i < l->layers.size(); i++) {
-        const LayerDev &d = l->layers[i];
-        const MixerSpec &mx = d.spec.mixer;
-        const FeedForwardSpec &ff = d.spec.ff;
-        const DeltaSpec &de = d.spec.delta;
-        const bool experts = ff.kind == FeedForwardSpec::EXPERTS;
-        DecodeProj p{};
-        p.x = x_now;
-        if (joined) {
-            p.y = l->y3;
-            p.out_l = joined->out_l;
-            p.out_r = joined->out_r;
-            p.x_new = x_next;
-            std::swap(x_now, x_next);
+        const TokenArgs t = token_args(l, i, at, token_dev, pos, pos_dev);
+        if (whole && l->any_whole && l->whole_per_cu[i]) {
+            MOON_TRY(launch_decode_whole(ctx, t.p, t.x, t.o, l->whole_per_cu[i], &l->whole));
+            continue;
         }
-        joined = d.out_l ? &d : nullptr;
-        p.token = i == 0 ? token_dev : nullptr;
-        p.embed = l->embed;
-        p.embed_scale = l->spec.embed_scale;
-        p.gamma = d.gamma;
-        p.beta = d.beta;
-        p.eps = l->spec.eps;
-        p.width = (int)l->spec.width;
-        p.dp = dp;
-        p.w1 = d.w1;
-        p.n16 = d.n16;
-        p.n32 = d.n32;
-        p.nall = d.nall;
-        p.n16_used = de.heads ? d.od + (int)(de.rank_a + de.rank_g) : d.og + (mx.gate ? (int)mx.heads * d.vdimp : 0);
-        p.n32_used = (int)(de.heads ? de.heads : ff.experts);
-        p.ff = ff.kind == FeedForwardSpec::DENSE ? (int)ff.ff : 0;
-        p.proj = l->proj;
-        p.logits = l->router;
-        p.glu = (char *)l->a2 + size_t(d.ka + d.kr) * l->el;
-        p.h = experts ? l->h : nullptr;
-        MOON_TRY(launch_decode_proj(ctx, dt, p));
-        DecodeMix x{};
-        x.proj = l->proj;
-        x.H = (int)mx.heads;
-        x.G = (int)mx.kv_heads;
-        x.dim = (int)mx.dim;
-        x.vdim = (int)mx.vdim;
-        x.dimp = d.dimp;
-        x.vdimp = d.vdimp;
-        x.ok = d.ok;
-        x.ov = d.ov;
-        x.og = d.og;
-        x.qk_rms = mx.qk_rms;
-        x.gate = mx.gate;
-        x.mixes = d.mixes;
-        x.window = (int)mx.window;
-        x.cap = d.cap;
-        x.eps = l->spec.eps;
-        x.lambda = d.lambda;
-        x.scale = mx.scale;
-        x.sink = d.sink;
-        x.ck = d.ck;
-        x.cv = d.cv;
-        x.v_first = first_values(l, d, &x.cap_first);
-        x.pos = pos;
-        x.pos_dev = pos_dev;
-        x.partial = l->mix_partial;
-        x.partial_floats = l->mix_partial_floats;
-        x.counter = l->counter;
-        x.out = l->a2;
-        x.whole = mx.qk_whole_norm;
-        x.rot_dims = (int)mx.rot_dims;
-        x.pool = (int)mx.pool;
-        x.blocks = d.blocks;
-        x.borrowed = mx.kv_from >= 0;
-        x.qn = d.qn;
-        x.kn = d.kn;
-        x.temp = d.temp;
-        x.rot = d.rot;
-        x.rotv = d.rotv;
-        x.pk = d.pk;
-        x.pv = d.pv;
-        if (de.heads) {
-            x.dH = (int)de.heads;
-            x.dG = (int)de.kv_heads;
-            x.ddim = (int)de.dim;
-            x.dvdim = (int)de.vdim;
-            x.ddimp = d.ddimp;
-            x.dvdimp = d.dvdimp;
-            x.taps = (int)de.conv;
-            x.oc = d.oc;
-            x.channels = d.channels;
-            x.od = d.od;
-            x.rank_a = (int)de.rank_a;
-            x.rank_g = (int)de.rank_g;
-            x.kd = d.kd;
-            x.lr16 = d.lr16;
-            x.beta = l->router;
-            x.conv = d.conv;
-            x.a_log = d.a_log;
-            x.dt_bias = d.dt_bias;
-            x.dnorm = d.dnorm;
-            x.wlr = d.wlr;
-            x.state = d.state;
-            x.ring = d.ring;
-            x.dout = (char *)l->a2 + size_t(d.ka) * l->el;
-        }
-        DecodeOut o{};
-        if (experts) {
-            x.logits = l->router;
-            x.correction = d.correction;
-            x.E = (int)ff.experts;
-            x.top = (int)ff.top;
-            x.ff = (int)ff.ff;
-            x.ffp = d.ffp;
-            x.h = l->h;
-            x.wgu = d.wgu;
-            x.act = l->act;
-            x.ids = l->ids;
-            x.weight = l->weight;
-            o.top = x.top;
-            o.ffp = d.ffp;
-            o.wd = d.wd;
-            o.act = l->act;
-            o.ids = l->ids;
-            o.weight = l->weight;
-        }
-        x.dp = dp;
-        o.x = x_now;
-        o.y = joined ? l->y3 : nullptr;
-        o.k1 = d.ka;
-        o.k2 = d.ka + d.kr;
-        o.width = (int)l->spec.width;
-        o.dp = dp;
-        o.k0 = d.k0;
-        o.w2 = d.w2;
-        o.a = l->a2;
-        o.down = o.k2 < o.k0 ? (joined ? l->y3 + 2 * dp : l->down) : nullptr;
-        MOON_TRY(launch_decode_mix(ctx, dt, x, o));
-        MOON_TRY(launch_decode_out(ctx, dt, o));
+        MOON_TRY(launch_decode_proj(ctx, dt, t.p));
+        MOON_TRY(launch_decode_mix(ctx, dt, t.x, t.o));
+        MOON_TRY(launch_decode_out(ctx, dt, t.o));
     }
-    if (!joined) return MOON_OK;
+    if (!at.joined) return MOON_OK;
     RowFinish f{};
     f.x = l->x;
     f.partial = l->y3;
     f.splits = 3;
     f.splits_l = f.splits_r = 1;
-    f.out_l = joined->out_l;
-    f.out_r = joined->out_r;
+    f.out_l = at.joined->out_l;
+    f.out_r = at.joined->out_r;
     f.eps = l->spec.eps;
     f.n = 1;
     f.width = (int)l->spec.width;

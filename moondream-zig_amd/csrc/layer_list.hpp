@@ -7,6 +7,7 @@
 #include <vector>
 
 #include "moon_internal.hpp"
+#include "wait_places.hpp"
 
 // ---- description (host)
 struct MixerSpec { // softmax attention over a KV cache; the mechanisms are independent of each other
@@ -318,6 +319,17 @@ int launch_decode_mix(moon_ctx *ctx, int dtype, const DecodeMix &p, const Decode
 
 int launch_decode_out(moon_ctx *ctx, int dtype, const DecodeOut &p);
 
+// ---- the same in one launch (layer_whole.hip), whose workgroups wait for each other
+struct WholeCounts {          // counters of a session's launches, which all use the same: what they have counted to so far
+    uint32_t *sync = nullptr; // decode_whole_sync_words
+    uint32_t *error = nullptr; // page-locked: not zero once a wait has run out of time
+    uint32_t leaf[2] = {}, reached[3] = {};
+};
+size_t decode_whole_sync_words();
+// Can this layer run so, at every position below max_seq?  per_cu: workgroups of its launch that a compute unit holds; need: the places that it takes
+bool decode_whole_supported(moon_ctx *ctx, int dtype, const DecodeProj &p, const DecodeMix &m, const DecodeOut &o, size_t max_seq, int *per_cu, WaitNeed *need);
+int launch_decode_whole(moon_ctx *ctx, const DecodeProj &p, const DecodeMix &m, const DecodeOut &o, int per_cu, WholeCounts *counts);
+
 // ---- the engine (layer_list.hip): weights, caches and buffers of one sequence's session, prompt rows and single tokens
 struct LayerList;
 struct Design;
@@ -332,8 +344,12 @@ void layer_list_destroy(LayerList *l);
 size_t layer_list_rows(const LayerList *l); // rows one forward call takes
 // n rows at positions pos .. pos + n - 1 (the cache holds everything before); x is left in rows 0 .. n - 1
 int layer_list_forward(LayerList *l, const uint32_t *ids_dev, size_t n, size_t pos);
-// one token with the decode kernels; pos_dev: the position is read on the device, pos is the largest it can be
-int layer_list_step(LayerList *l, const uint32_t *token_dev, size_t pos, const uint32_t *pos_dev);
+// one token with the decode kernels; pos_dev: the position is read on the device, pos is the largest it can be.  whole: in one launch per layer
+// where that can be, with the places of layer_list_wait_need taken
+int layer_list_step(LayerList *l, const uint32_t *token_dev, size_t pos, const uint32_t *pos_dev, bool whole);
+const WaitNeed *layer_list_wait_need(const LayerList *l); // null: no layer runs in one launch
+// behind a drained stream: has a wait run out of time?  Its counters are then ready again, the sequence's caches are not
+bool layer_list_wait_failed(LayerList *l);
 // logits of the given rows of x (host list of n <= LIST_LOGIT_ROWS) -> *logits, [n][*ld] f32 on the device
 int layer_list_logits(LayerList *l, const uint32_t *rows, size_t n, const float **logits, size_t *ld);
 const float *layer_list_hidden(const LayerList *l); // [rows][width] on the device

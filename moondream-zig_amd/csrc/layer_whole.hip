@@ -1,0 +1,341 @@
+// One token through a whole layer of a layer-list decoder in ONE launch (layer_decode.hip has the same in three).  Workgroups take roles by index:
+//   producers   h = norm(x), their rows of the first product: first q, k, v (and a delta rule's columns), counted by themselves, then the gate's and the
+//               feed-forward's silu(gate) * up
+//   attention   a split of a key head's keys each, and the delta rule's heads: ask for cache rows and states, wait for the first count, and report every
+//               merged head
+//   output      rows of the second product, two per wavefront: most of them (23 of 30 KB at width 2048, feed-forward 5504) is in registers by the time that the
+//               activation is there, the rest streams while the attention is still under way; the heads' part comes last
+// A layer of 97 MB (width 2048, 8 key heads, feed-forward 5504) took 14.6 + 11 + 4.6 us and three launches' starts, ends and gaps; the weights of its later phases stream while
+// the earlier ones run here.  695 -> 596 us a token behind 61 keys, 382 -> 327 for 12 layers behind 900; 32 key heads 381 -> 337, 4 key heads and feed-forward 2048 358 -> 292; width 1024: 504 -> 384,
+// rotated and joined 549 -> 425 (width 2048, 12 layers 421 -> 392).  What bounds it is the chain q, k, v -> attention -> merge -> output beside the stream: 4 TB/s.
+// Measured and not kept: one row per output wavefront, which leaves the producers half of the places (8 key heads 603, 32 373 of 12 layers; with 192 producers 4 key heads took
+// 1,202); gate rows ahead of the attention (615; 12 layers behind 900 keys 352); a delta rule's taps, ranks and vectors asked for ahead of the wait (no difference); the first count on 8 or 16 lines that all heads' workgroups poll, a hop less, in place of 64 copies (660, 635: 130 pollers on
+// a line hold up the stream); no pauses between the lots of an output row, longer ones, and no wave priority: 0 to 2 % either way; three workgroups a unit at width 1024 in place of two: 0 to 2 % slower.
+// Progress: producers never wait and come first in the grid, so on every die they have their places before any workgroup that waits; the
+// attention's workgroups wait for producers, the output's for both, in the grid's order (a merge also waits for the gate: producers again).  Workgroups of several launches could all the same fill the dies
+// with some that wait for another die's: calls take their places beforehand (wait_places.hpp) and run in three launches where there are
+// none.  Two launches that nobody counts together, of two processes, finish in any case: where one's producers or heads have no place on a die yet, none of its output workgroups is there, and
+// the other's waiting ones never fill a die (decode_whole_supported).  Every wait is bounded.
+// Exchanged vectors are written through to memory; the attention reads what it needs of the projections past the dies' caches, the output
+// workgroups read the two long vectors through them (no line of either is read before its count is complete).
+#include "decode_roles.hpp"
+#include "kernel_args.hpp"
+#include "launch_waits.hpp"
+
+#include <algorithm>
+
+namespace {
+
+constexpr int WHOLE_D = 64;      // padded head sizes
+constexpr int WHOLE_LEAVES = 32; // the producers' counts come together on so many lines, and then on every copy
+constexpr int WHOLE_GLU = 12;    // 1 KiB pieces of a row of the dense activation's weights
+constexpr int WHOLE_ROWS = 2;    // rows of an output wavefront
+constexpr int WHOLE_SLEEP = 6;   // units of 64 cycles between two lots of them
+enum { WHOLE_FRONT, WHOLE_ACT, WHOLE_HEADS, WHOLE_COUNTS };
+constexpr int WHOLE_COPIES_AT = 2 * WHOLE_LEAVES * LAYER_LINE; // behind the leaves of the first two
+
+struct WholeArgs {
+    DecodeProj p;
+    DecodeMix m;
+    DecodeOut o;
+    int S, keys_max, n_prod, n_attn;
+    int front16;              // rows of the 16-bit segment that the heads begin with; the gate's behind them come with the activation
+    uint32_t *sync, *error;
+    uint32_t leaf[2], reached[WHOLE_COUNTS]; // what the leaves and the copies count to
+};
+
+__device__ __forceinline__ uint32_t *whole_copy(const WholeArgs &a, int which, int i) { return a.sync + WHOLE_COPIES_AT + (which * LAYER_COPIES + i) * LAYER_COPY_STRIDE; }
+
+struct Within {
+    static constexpr bool SHARED = true;
+    const WholeArgs &a;
+    int *s_flag;
+    __device__ __forceinline__ bool wait() const {
+        return wait_reached(whole_copy(a, WHOLE_FRONT, blockIdx.x % LAYER_COPIES), a.reached[WHOLE_FRONT], a.error, s_flag);
+    }
+    __device__ __forceinline__ bool wait_gate() const {
+        return a.front16 == a.p.n16_used || wait_reached(whole_copy(a, WHOLE_ACT, blockIdx.x % LAYER_COPIES), a.reached[WHOLE_ACT], a.error, s_flag);
+    }
+    __device__ __forceinline__ void done() const {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // the heads are stored
+        lds_barrier();
+        if (threadIdx.x < LAYER_COPIES) __hip_atomic_fetch_add(whole_copy(a, WHOLE_HEADS, threadIdx.x), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+};
+
+// This producer's rows of a phase are stored: counted on its leaf, and by the leaf's last one on every copy
+__device__ __forceinline__ void whole_report(const WholeArgs &a, int phase) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    lds_barrier();
+    if (threadIdx.x >= 64) return;
+    int full = 0;
+    if (threadIdx.x == 0)
+        full = __hip_atomic_fetch_add(a.sync + (phase * WHOLE_LEAVES + blockIdx.x % WHOLE_LEAVES) * LAYER_LINE, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 == a.leaf[phase];
+    if (__builtin_amdgcn_readfirstlane(full)) __hip_atomic_fetch_add(whole_copy(a, phase, threadIdx.x), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+template <int U> __device__ __forceinline__ void whole_producer(const WholeArgs &a, char *lds, float *s_red) {
+    typedef bf16_t T;
+    const DecodeProj &p = a.p;
+    T *s_h = reinterpret_cast<T *>(lds);
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, waves = a.n_prod * 4, gw = blockIdx.x * 4 + wave;
+    const T *W = reinterpret_cast<const T *>(p.w1);
+    const int pieces = p.dp / 8;
+    const T *er = p.token ? reinterpret_cast<const T *>(p.embed) + size_t(p.token[0]) * p.dp : nullptr;
+    NormRow<T, U / 2, true, true> norm;
+    norm.request(p, er, tid);
+    // pairs of rows (segments are padded).  The first phase: what the heads begin with, and the f32 rows; the second: gate rows, then a gate/up pair each,
+    // its longer shares to the wavefronts that had the shorter ones
+    const int g16 = (a.front16 + 1) / 2, later = (p.n16_used - a.front16 + 1) / 2;
+    int g, g_end, i, i_end;
+    share(g16 + (p.n32_used + 1) / 2, waves, gw, g, g_end);
+    share(later + p.ff, waves, waves - 1 - gw, i, i_end);
+    RowDots<T, 2, U> dots;
+    const T *rows[2];
+    auto request = [&](int row, int apart) {
+        rows[0] = W + size_t(row) * p.dp;
+        rows[1] = rows[0] + size_t(apart) * p.dp;
+        dots.request(rows, 0, pieces, lane);
+    };
+    auto front = [&](int g) { request(g < g16 ? 2 * g : p.n16 + 2 * (g - g16), 1); };
+    auto second = [&](int i) { i < later ? request(a.front16 + 2 * i, 1) : request(p.n32 + pair_row(i - later, 0), 32); };
+    if (g < g_end) front(g);
+    norm.finish(p, er, blockIdx.x == 0, s_h, s_red, tid);
+    lds_barrier();
+    lm_u32x4 x[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        const int at = u * 64 + lane;
+        x[u] = lm_u32x4{0, 0, 0, 0};
+        if (at < pieces) x[u] = *reinterpret_cast<const lm_u32x4 *>(s_h + at * 8);
+    }
+    float acc[2];
+    auto sums = [&]() {
+        acc[0] = acc[1] = 0.0f;
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+            for (int j = 0; j < 2; j++) acc[j] = dot_piece<T>(dots.w[j][u], x[u], acc[j]);
+    };
+    auto store = [&](float *to) {
+        if (lane < 2) st_f<true>(to + lane, lane ? acc[1] : acc[0]);
+    };
+    for (; g < g_end; g++) {
+        sums();
+        if (g + 1 < g_end) front(g + 1);
+        acc[0] = wave_sum(acc[0]);
+        acc[1] = wave_sum(acc[1]);
+        store(g < g16 ? p.proj + 2 * g : p.logits + 2 * (g - g16));
+    }
+    whole_report(a, WHOLE_FRONT);
+    if (!(later + p.ff)) return;
+    if (i < i_end) second(i);
+    for (; i < i_end; i++) {
+        sums();
+        if (i + 1 < i_end) second(i + 1);
+        acc[0] = wave_sum(acc[0]);
+        acc[1] = wave_sum(acc[1]);
+        if (i < later) store(p.proj + a.front16 + 2 * i);
+        else if (lane == 0) st_t<true>(reinterpret_cast<T *>(p.glu) + i - later, (T)(lm_silu(acc[0]) * acc[1]));
+    }
+    whole_report(a, WHOLE_ACT);
+}
+
+// 16 bytes a lane of a stretch of `bytes`; zeros behind its end
+enum { LOAD_DIE = 1, LOAD_STREAM = 2 }; // from the die's cache on; not to be kept
+template <int HOW> __device__ __forceinline__ lm_u32x4 stretch_load(__amdgpu_buffer_rsrc_t r, int at) {
+    return __builtin_bit_cast(lm_u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, at, 0, HOW));
+}
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t stretch(const void *p, int bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, bytes, 0x00020000);
+}
+
+// W: 1 KiB pieces of a row that meet the heads, and of those that meet the delta rule's.  A wavefront owns WHOLE_ROWS rows: their parts for the
+// heads and the beginning of the first one's for the dense activation (HOLD pieces) are in registers by the time that the activation is there, the rest streams
+// while the attention is still under way.
+template <int W, bool DELTA> __device__ __forceinline__ void whole_output(const WholeArgs &a, int wg, int n_wgs, char *lds, int *s_flag) {
+    typedef bf16_t T;
+    constexpr int R = WHOLE_ROWS, HOLD = DELTA && W > 2 ? 8 : WHOLE_GLU;
+    const DecodeOut &o = a.o;
+    const int tid = threadIdx.x, lane = tid & 63, first = wg * 4 + __builtin_amdgcn_readfirstlane(tid >> 6), b = blockIdx.x % LAYER_COPIES;
+    const bool fresh = a.p.token || a.p.y; // a producer writes x in this launch
+    const int n_o = o.k1 * 2, n_d = (o.k2 - o.k1) * 2, n_f = (o.k0 - o.k2) * 2; // bytes of a row's parts
+    auto row = [&](int r) { return first + r * n_wgs * 4; };
+    auto weights = [&](int r, int column, int bytes) { return stretch(reinterpret_cast<const T *>(o.w2) + size_t(row(r)) * o.k0 + column, row(r) < o.width ? bytes : 0); };
+    lm_u32x4 wo[R][W], wd[R][DELTA ? W : 1], wf[HOLD];
+    float old[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const auto w = weights(r, 0, n_o);
+        old[r] = 0.0f;
+        if (!fresh && !o.y && row(r) < o.width) old[r] = o.x[row(r)];
+#pragma unroll
+        for (int c = 0; c < W; c++) wo[r][c] = stretch_load<LOAD_STREAM>(w, c * 1024 + lane * 16);
+    }
+    if (DELTA && n_d)
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const auto w = weights(r, o.k1, n_d);
+#pragma unroll
+            for (int c = 0; c < W; c++) wd[r][c] = stretch_load<LOAD_STREAM>(w, c * 1024 + lane * 16);
+        }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    float dot_f[R] = {};
+    if (n_f) {
+        {
+            const auto w = weights(0, o.k2, n_f);
+#pragma unroll
+            for (int c = 0; c < HOLD; c++) {
+                if (c * 1024 < n_f) wf[c] = stretch_load<LOAD_STREAM>(w, c * 1024 + lane * 16);
+                if (c % 4 == 3 && c + 1 < HOLD) {
+                    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                    __builtin_amdgcn_s_sleep(WHOLE_SLEEP);
+                }
+            }
+        }
+        if (!wait_reached(whole_copy(a, WHOLE_ACT, b), a.reached[WHOLE_ACT], a.error, s_flag)) return;
+        const auto act = stretch(reinterpret_cast<const T *>(o.a) + o.k2, n_f);
+        lm_u32x4 v[WHOLE_GLU / 4];
+#pragma unroll
+        for (int c = 0; c < WHOLE_GLU / 4; c++) v[c] = stretch_load<LOAD_DIE>(act, (c * 256 + tid) * 16);
+#pragma unroll
+        for (int c = 0; c < WHOLE_GLU / 4; c++) reinterpret_cast<lm_u32x4 *>(lds)[c * 256 + tid] = v[c];
+        lds_barrier();
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const auto w = weights(r, o.k2, n_f);
+#pragma unroll
+            for (int base = 0; base < WHOLE_GLU; base += HOLD) {
+                if (r || base)
+#pragma unroll
+                    for (int c = 0; c < HOLD; c++)
+                        if ((base + c) * 1024 < n_f && base + c < WHOLE_GLU) wf[c] = stretch_load<LOAD_STREAM>(w, (base + c) * 1024 + lane * 16);
+#pragma unroll
+                for (int c = 0; c < HOLD; c++)
+                    if ((base + c) * 1024 < n_f && base + c < WHOLE_GLU) dot_f[r] = dot_piece<T>(wf[c], reinterpret_cast<const lm_u32x4 *>(lds)[(base + c) * 64 + lane], dot_f[r]);
+            }
+            dot_f[r] = wave_sum(dot_f[r]);
+        }
+    }
+    if (!wait_reached(whole_copy(a, WHOLE_HEADS, b), a.reached[WHOLE_HEADS], a.error, s_flag)) return;
+    const auto x_o = stretch(o.a, n_o), x_d = stretch(reinterpret_cast<const T *>(o.a) + o.k1, n_d);
+    lm_u32x4 xo[W], xd[DELTA ? W : 1];
+    if (fresh && !o.y)
+#pragma unroll
+        for (int r = 0; r < R; r++)
+            if (row(r) < o.width) old[r] = ld_f<true>(o.x + row(r));
+#pragma unroll
+    for (int c = 0; c < W; c++) xo[c] = stretch_load<LOAD_DIE>(x_o, c * 1024 + lane * 16);
+    if (DELTA && n_d)
+#pragma unroll
+        for (int c = 0; c < W; c++) xd[c] = stretch_load<LOAD_DIE>(x_d, c * 1024 + lane * 16);
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const int n = row(r);
+        float dot_o = 0.0f, dot_d = 0.0f;
+#pragma unroll
+        for (int c = 0; c < W; c++) dot_o = dot_piece<T>(wo[r][c], xo[c], dot_o);
+        dot_o = wave_sum(dot_o);
+        if (DELTA && n_d) {
+#pragma unroll
+            for (int c = 0; c < W; c++) dot_d = dot_piece<T>(wd[r][c], xd[c], dot_d);
+            dot_d = wave_sum(dot_d);
+        }
+        if (lane || n >= o.width) continue;
+        if (o.y) {
+            o.y[n] = dot_o;
+            o.y[o.dp + n] = dot_d;
+            o.y[2 * o.dp + n] = dot_f[r];
+        } else o.x[n] = old[r] + (dot_o + dot_d + dot_f[r]);
+    }
+}
+
+template <int NH, int U, bool WHOLE>
+__global__ __launch_bounds__(256, NH > 4 ? 3 : 4) void decode_whole_kernel(WholeArgs) {
+    const WholeArgs &a = fetch_arguments<WholeArgs>();
+    extern __shared__ __attribute__((aligned(16))) char s_whole[];
+    __shared__ float s_red[16];
+    __shared__ int s_flag;
+    const int b = blockIdx.x, n_delta = WHOLE ? a.m.dH : 0;
+    if (b < a.n_prod) return whole_producer<U>(a, s_whole, s_red);
+    int i = b - a.n_prod;
+    if (i < a.n_attn + n_delta) {
+        __builtin_amdgcn_s_setprio(3); // the chain that the launch waits for longest
+        const Within meet{a, &s_flag};
+        float *lds = reinterpret_cast<float *>(s_whole);
+        if (i < a.n_attn) {
+            const int n_hb = mix_head_blocks(a.m.H / a.m.G);
+            return mix_attention<bf16_t, NH, WHOLE, false, WHOLE_D>(a.m, i / a.S / n_hb, i / a.S % n_hb, i % a.S, a.S, a.keys_max, lds, meet);
+        }
+        if (WHOLE) mix_delta<bf16_t, true>(a.m, i - a.n_attn, lds, meet);
+        return;
+    }
+    whole_output<U, WHOLE>(a, i - a.n_attn - n_delta, gridDim.x - a.n_prod - a.n_attn - n_delta, s_whole, &s_flag);
+}
+
+typedef void (*WholeKernel)(WholeArgs);
+template <int U, bool WHOLE> WholeKernel whole_kernel_of(int NH) {
+    return NH == 1 ? decode_whole_kernel<1, U, WHOLE> : NH == 2 ? decode_whole_kernel<2, U, WHOLE> : NH == 4 ? decode_whole_kernel<4, U, WHOLE> : decode_whole_kernel<8, U, WHOLE>;
+}
+
+struct WholePlan {
+    WholeKernel kern;
+    int S, keys_max, n_prod, n_attn, merges, grid, waiting;
+    size_t lds;
+};
+// A layer's launch with n_keys keys; false: not in one launch.  per_cu: workgroups that a compute unit holds (0: of no matter yet).
+bool whole_plan(moon_ctx *ctx, const DecodeProj &p, const DecodeMix &m, const DecodeOut &o, int n_keys, int per_cu, WholePlan *w) {
+    const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256, U = p.dp <= 1024 ? 2 : 4;
+    if (m.E || m.dimp != WHOLE_D || m.vdimp != WHOLE_D || p.width % 4 || p.dp > 2048 || (reinterpret_cast<uintptr_t>(p.x) & 15)) return false;
+    if (o.k1 > 512 * U || o.k2 - o.k1 > 512 * U || o.k0 - o.k2 > 512 * WHOLE_GLU || (o.k0 > o.k2) != (p.ff > 0)) return false;
+    if (m.dH && (m.ddimp > DELTA_ROWS * (256 / (m.dvdimp / 4)))) return false;
+    const int per = m.H / m.G, wgs = m.G * mix_head_blocks(per), nh = std::min(per, MIX_HEADS), NH = nh <= 1 ? 1 : nh <= 2 ? 2 : nh <= 4 ? 4 : 8;
+    w->S = mix_splits(n_keys, wgs, cus);
+    w->keys_max = std::max(MIX_TARGET, (n_keys + w->S - 1) / w->S); // (fewer keys: the LDS of so many all the same)
+    w->lds = std::max({size_t(p.dp) * 2, mix_lds_floats(NH, WHOLE_D, WHOLE_D, w->keys_max) * sizeof(float), size_t(p.ff ? WHOLE_GLU * 1024 : 0),
+                       m.dH ? delta_lds_floats(m.ddimp, m.dvdimp, m.kd) * sizeof(float) : 0});
+    if (w->lds > 60 * 1024 || size_t(NH) * w->S > mix_lds_floats(NH, WHOLE_D, WHOLE_D, w->keys_max) - 4 * NH - 8) return false;
+    w->kern = mix_whole(m) ? (U == 2 ? whole_kernel_of<2, true>(NH) : whole_kernel_of<4, true>(NH)) : (U == 2 ? whole_kernel_of<2, false>(NH) : whole_kernel_of<4, false>(NH));
+    w->n_attn = wgs * w->S;
+    w->merges = wgs + m.dH;
+    w->waiting = w->n_attn + m.dH + (o.width + 4 * WHOLE_ROWS - 1) / (4 * WHOLE_ROWS);
+    const int total = std::min(per_cu, U == 2 ? 2 : 4) * cus, work = std::max((p.n16_used + 1) / 2 + (p.n32_used + 1) / 2, p.ff); // (a pair of rows per wavefront at least)
+    w->n_prod = std::max(std::min(total - w->waiting, (work + 3) / 4) / WHOLE_LEAVES, 1) * WHOLE_LEAVES;
+    w->grid = w->n_prod + w->waiting;
+    return size_t(w->n_attn) * MIX_HEADS * (WHOLE_D + 2) <= m.partial_floats;
+}
+
+} // namespace
+
+size_t decode_whole_sync_words() { return WHOLE_COPIES_AT + size_t(WHOLE_COUNTS) * LAYER_COPIES * LAYER_COPY_STRIDE; }
+
+bool decode_whole_supported(moon_ctx *ctx, int dtype, const DecodeProj &p, const DecodeMix &m, const DecodeOut &o, size_t max_seq, int *per_cu, WaitNeed *need) {
+    const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
+    WholePlan w;
+    // (the splits never get fewer with more keys, and their LDS is largest with the most keys)
+    if (dtype != MOON_DTYPE_BF16 || !max_seq || !whole_plan(ctx, p, m, o, mix_keys(m, max_seq - 1), 0, &w)) return false;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, reinterpret_cast<const void *>(w.kern), 256, w.lds) != hipSuccess) return false;
+    *need = {(w.waiting + 7) / 8, *per_cu * cus / 8};
+    return need->waiting < need->places;
+}
+
+int launch_decode_whole(moon_ctx *ctx, const DecodeProj &p, const DecodeMix &m, const DecodeOut &o, int per_cu, WholeCounts *counts) {
+    MOON_TRY(check_decode_mix(ctx, m));
+    WholePlan w;
+    if (!whole_plan(ctx, p, m, o, mix_keys(m, m.pos), per_cu, &w)) return moon_fail(ctx, MOON_EINVAL, "decode: a layer that does not run in one launch");
+    counts->leaf[WHOLE_FRONT] += w.n_prod / WHOLE_LEAVES;
+    counts->reached[WHOLE_FRONT] += WHOLE_LEAVES;
+    const int front16 = m.gate && !m.dH ? m.og : p.n16_used; // (a delta rule's columns come behind the gate's)
+    if (p.ff || front16 < p.n16_used) {
+        counts->leaf[WHOLE_ACT] += w.n_prod / WHOLE_LEAVES;
+        counts->reached[WHOLE_ACT] += WHOLE_LEAVES;
+    }
+    counts->reached[WHOLE_HEADS] += w.merges;
+    WholeArgs a{p, m, o, w.S, w.keys_max, w.n_prod, w.n_attn, front16, counts->sync, counts->error, {}, {}};
+    std::copy(counts->leaf, counts->leaf + 2, a.leaf);
+    std::copy(counts->reached, counts->reached + WHOLE_COUNTS, a.reached);
+    MOON_NOTE_KERNEL(ctx, "decode_whole_kernel %d splits of the keys", w.S);
+    hipLaunchKernelGGL(w.kern, dim3(w.grid), dim3(256), w.lds, ctx->stream, a);
+    MOON_HIP(ctx, hipGetLastError());
+    return MOON_OK;
+}

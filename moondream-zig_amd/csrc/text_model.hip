@@ -308,8 +308,9 @@ struct DecodeCall {
     }
     explicit DecodeCall(moon_text_model *model) : m(model) {
         m->call_mode = m->decode_mode;
-        if (!m->fused) return;
-        if (m->whole_layer && m->call_mode == 0) need = &m->layer_wait;
+        if (m->list) need = layer_list_wait_need(m->list);
+        else if (!m->fused) return;
+        else if (m->whole_layer && m->call_mode == 0) need = &m->layer_wait;
         else if (m->front && m->call_mode != 2) need = &m->front_wait;
         if (need && !places(m->ctx->device).take(*need)) {
             need = nullptr;
@@ -452,7 +453,7 @@ int lm_head(moon_text_model *m, size_t row) {
 
 // one token through all layers; token_dev, or row 0 of m->hidden
 int step_layers(moon_text_model *m, size_t pos, bool pos_on_device, const uint32_t *token_dev) {
-    if (m->list) return layer_list_step(m->list, token_dev, pos, pos_on_device ? m->state_dev : nullptr);
+    if (m->list) return layer_list_step(m->list, token_dev, pos, pos_on_device ? m->state_dev : nullptr, m->call_mode == 0);
     for (size_t l = 0; l < m->cfg.n_layers; l++) MOON_TRY(layer_forward(m, l, 1, pos, pos_on_device, l == 0 ? token_dev : nullptr));
     return MOON_OK;
 }
@@ -588,7 +589,7 @@ extern "C" int moon_text_reset(moon_text_model *m) {
     m->cur_len = 0;
     m->last_n = 0;
     MOON_HIP(m->ctx, hipSetDevice(m->ctx->device));
-    if (m->cache_invalid) MOON_TRY(clear_sync_state(m)); // after a failed wait: counters and targets start over together
+    if (m->cache_invalid && !m->list) MOON_TRY(clear_sync_state(m)); // after a failed wait: counters and targets start over together
     m->cache_invalid = false;
     hipLaunchKernelGGL(set_state_kernel, dim3(1), dim3(1), 0, m->ctx->stream, m->state_dev, 0u, 0u);
     MOON_HIP(m->ctx, hipGetLastError());
@@ -710,14 +711,24 @@ static int wanted_logits(moon_text_model *m, size_t lo, size_t n, const size_t *
     return MOON_OK;
 }
 
+// Behind a wait that ran out of time: the cache rows of the call's tokens may be missing.
+static int lost_sequence(moon_text_model *m) {
+    m->cache_invalid = true;
+    m->last_n = 0;
+    return moon_fail(m->ctx, MOON_EHIP, "fused decode kernel: a wait between its phases timed out; the session needs moon_text_reset");
+}
+
 // A list decoder's rows: ids already in ids_pinned, at most layer_list_rows of them at a time (each part attends to the parts
 // before it through the cache, as separate calls would).
 static int forward_list_locked(moon_text_model *m, size_t n_ids, const size_t *want, size_t n_want, float *logits) {
     moon_ctx *ctx = m->ctx;
+    std::optional<DecodeCall> call;
     for (size_t done = 0; done < n_ids;) {
         const size_t n = std::min(n_ids - done, layer_list_rows(m->list));
-        if (n == 1) MOON_TRY(layer_list_step(m->list, m->ids_dev + done, m->cur_len, nullptr));
-        else MOON_TRY(layer_list_forward(m->list, m->ids_dev + done, n, m->cur_len));
+        if (n == 1) {
+            if (!call) call.emplace(m);
+            MOON_TRY(layer_list_step(m->list, m->ids_dev + done, m->cur_len, nullptr, m->call_mode == 0));
+        } else MOON_TRY(layer_list_forward(m->list, m->ids_dev + done, n, m->cur_len));
         m->cur_len += n;
         m->last_n = n;
         MOON_TRY(wanted_logits(m, done, n, want, n_want, logits));
@@ -726,6 +737,11 @@ static int forward_list_locked(moon_text_model *m, size_t n_ids, const size_t *w
     hipLaunchKernelGGL(set_state_kernel, dim3(1), dim3(1), 0, ctx->stream, m->state_dev, (uint32_t)m->cur_len, 0u);
     MOON_HIP(ctx, hipGetLastError());
     MOON_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    if (call) call->drained = true;
+    if (call && layer_list_wait_failed(m->list)) {
+        m->cur_len -= n_ids;
+        return lost_sequence(m);
+    }
     return MOON_OK;
 }
 
@@ -983,6 +999,7 @@ static int greedy_locked(moon_text_model *m, size_t n_steps, uint32_t *out_ids, 
     MOON_HIP(ctx, hipStreamSynchronize(ctx->stream));
     call.drained = true;
     if (ids_staged) memcpy(out_ids, m->stage_down, n_steps * sizeof(uint32_t));
+    if (m->list && layer_list_wait_failed(m->list)) return lost_sequence(m);
     const uint32_t front_error = words[24];
     const uint32_t final_state[4] = {words[20], words[21], words[22], words[23]};
     if (front_error != 0) {

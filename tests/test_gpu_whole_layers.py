@@ -1,0 +1,132 @@
+"""One token through a whole layer of a list decoder in one launch (layer_whole.hip): sizes at the edges of what it takes."""
+import generax_models as GM
+import generax_oracle as G
+import numpy as np
+import pytest
+import rikanex_models as RM
+import rikanex_oracle as R
+from conftest import compute_units
+from decoder_checks import feed, opened, rows_close, run
+
+pytestmark = pytest.mark.gpu
+# of the lists' other tests: an f32 sum's result rounded to bf16 (2^-9 at most, 2^-10.8 on average) some dozens of times on the way to a logit
+LIMIT = 3e-2
+ROT = GM.rotation(64, 1e4)
+
+
+def took_one_launch(ctx, splits=None):
+    if compute_units() == 256:
+        note = ctx.last_kernel()
+        assert note.startswith("decode_whole_kernel") and (splits is None or f" {splits} splits" in note), note
+
+
+def assert_close(got, want):
+    ok, text = rows_close(got, want, LIMIT)
+    assert ok, text
+
+
+# (heads of 63 and 61 are padded to 64.)  One, two, four and eight heads a workgroup, and two workgroups for a key head; widths that end inside a piece of 64 elements,
+# below and above 1024; rows that do not fill the last output workgroup; odd feed-forwards, the largest, none
+RIKANEX = {
+    "smallest": (64, 1, 1, 8, 5), "odd": (516, 6, 6, 70, 40), "pairs": (1020, 14, 7, 333, 17), "fours": (1024, 16, 4, 1728, 33), "eights": (1084, 10, 2, 1121, 64),
+    "two workgroups": (256, 12, 1, 129, 20), "no feed-forward": (320, 4, 2, None, 9),
+}
+
+
+@pytest.mark.parametrize("name", sorted(RIKANEX))
+def test_rikanex(moon, ctx, tmp_path, name):
+    width, heads, kv_heads, ff, window = RIKANEX[name]
+    mlp = RM.dense(ff) if ff else None
+    cfg = RM.config(90, width, [RM.layer(RM.attention(heads, kv_heads, 63, 61, window, 0.13, mix), mlp) for mix in (False, True, True)], embed_scale=2.0)
+    w, ids = RM.weights(cfg, 3), RM.tokens(75, 90)
+    m = opened(moon, ctx, RM.write_folder(tmp_path / "m", cfg, w), "bfloat16")
+    got = []
+    for at in range(len(ids)):
+        m.forward(ids[at:at + 1])
+        took_one_launch(ctx, min(2, -(-min(at + 1, window) // 32)))
+        got.append(m.logits_f32())
+    m.close()
+    want = R.forward(cfg, w, ids)[0]
+    assert_close(np.array(got), want)
+    assert_close(run(moon, ctx, tmp_path, cfg, w, ids, "bfloat16", [40, 1, 1, 3, 1]), want)
+
+
+@pytest.mark.parametrize("width,heads,kv_heads,ff,delta_heads", [(64, 1, 1, 8, 1), (516, 6, 3, 70, 5), (1024, 16, 4, 1728, 16), (1084, 10, 2, 321, 4), (320, 4, 1, None, 2)])
+def test_generax(moon, ctx, tmp_path, width, heads, kv_heads, ff, delta_heads):
+    """Joined layers behind each other, in front of a plain one and as the last; borrowed keys; blocks before the window."""
+    joined = GM.parallel(GM.softmax_mixer(heads, kv_heads, 64, 64, 9, 0.13, 4), GM.delta(delta_heads, 1, 64, 64, 4), ff)
+    turned = GM.attention(heads, kv_heads, 64, 64, 20, 0.13, ROT)
+    cfg = GM.config(90, width, [joined, joined, GM.plain(turned, ff), GM.plain(dict(turned, kv_from=2), ff), joined])
+    w, ids = GM.weights(cfg, 3), RM.tokens(75, 90)
+    got = run(moon, ctx, tmp_path, cfg, w, ids, "bfloat16", [1])
+    want = G.forward(cfg, w, ids)[0]
+    assert_close(got, want)
+    assert_close(run(moon, ctx, tmp_path, cfg, w, ids, "bfloat16", [40, 1, 1, 3, 1]), want)
+
+
+LARGE = [RM.config(128, 2048, [RM.layer(RM.attention(32, kv, 64, 64, window, 0.125, True), RM.dense(ff) if ff else None) for _ in range(3)], embed_scale=2.0)
+         for kv, window, ff in ((32, 1024, 6144), (8, 1024, 5504), (4, 512, 1024), (8, 64, None))]
+LARGE += [GM.config(128, width, [GM.parallel(GM.softmax_mixer(width // 64, kv, 64, 64, 512, 0.125, 16), GM.delta(width // 64, width // 64, 64, 64, 4), ff),
+                                 GM.plain(GM.attention(width // 64, kv, 64, 64, 1024, 0.125, ROT), ff)] * 2) for width, kv, ff in ((2048, 8, 5632), (2048, 32, 3712), (1024, 4, 1728))]
+
+
+@pytest.mark.parametrize("which", range(len(LARGE)))
+def test_largest_sizes_beside_f32(moon, ctx, which):
+    """Against an f32 session, which takes other kernels, behind few and many cached keys: the splits' numbers from one to the largest."""
+    out = []
+    ids = RM.tokens(1100, 128)
+    for dtype in ("bfloat16", "float32"):
+        m = moon.text_model.TextModel.open_synthetic(LARGE[which], dtype, 2048, seed=5, std=0.02, ctx=ctx)
+        rows = []
+        for prompt in (1, 31, 300, 1090):
+            m.reset()
+            rows.append(feed(m, ids[:prompt], [prompt])[-1:])
+            for i in range(3):
+                m.forward(ids[prompt + i:prompt + i + 1])
+                if dtype == "bfloat16":
+                    took_one_launch(ctx)
+                rows.append(m.logits_f32()[None])
+        out.append(np.concatenate(rows))
+        m.close()
+    assert_close(*out)
+
+
+@pytest.mark.parametrize("change", [dict(width=2112), dict(ff=6208), dict(dim=128), dict(experts=True)])
+def test_other_sizes_take_three_launches(moon, ctx, change):
+    width, dim = change.get("width", 1024), change.get("dim", 64)
+    mlp = RM.moe(64, 64, 64) if "experts" in change else RM.dense(change.get("ff", 128))
+    cfg = RM.config(128, width, [RM.layer(RM.attention(4, 2, dim, dim, 40, 0.125, True), mlp)], embed_scale=2.0)
+    out = []
+    ids = RM.tokens(40, 128)
+    for dtype in ("bfloat16", "float32"):
+        m = moon.text_model.TextModel.open_synthetic(cfg, dtype, 256, seed=5, std=0.02, ctx=ctx)
+        m.forward(ids[:30])
+        m.forward(ids[30:31])
+        assert not ctx.last_kernel().startswith("decode_whole")
+        out.append(np.concatenate([m.logits_f32()[None], feed(m, ids[31:], [1])]))
+        m.close()
+    assert_close(*out)
+
+
+def test_sessions_of_two_contexts_at_once(moon, ctx):
+    """Two threads decode: whichever call finds no places for its waiting workgroups takes three launches, with the same tokens up to rounding."""
+    import threading
+    cfg = LARGE[1]
+    ids = RM.tokens(64, 128)
+    sessions = [moon.text_model.TextModel.open_synthetic(cfg, "bfloat16", 256, seed=5, std=0.02, ctx=c) for c in (ctx, moon.Context(), moon.Context())]
+    alone = feed(sessions[0], ids, [40] + [1] * 24)
+    sessions[0].reset()
+    out = [None] * len(sessions)
+
+    def work(i):
+        out[i] = feed(sessions[i], ids, [40] + [1] * 24)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(len(sessions))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for m, got in zip(sessions, out):
+        assert got is not None
+        assert_close(got, alone)
+        m.close()
