@@ -493,31 +493,48 @@ __device__ __forceinline__ void mix_attention(const DecodeMix &p, int g, int hb,
     }
     __syncthreads();
     if (!*s_last) return;
-    // Every head's splits: this thread's elements of the first splits and all (m, l) are requested together; the weight of each
+    // Every head's splits: this thread's elements of the first splits, all (m, l) and the gate are requested together; the weight of each
     // split (a lane per split) goes through LDS.
-    constexpr int AT_ONCE = MIX_SPLITS;
+    constexpr int AT_ONCE = MIX_SPLITS, HW = (NH + 3) / 4;
     const size_t pitch = size_t(MIX_HEADS) * stride; // floats between splits
     float *s_w = lds; // [nh][S], over what the phases before have used
-    float v[AT_ONCE];
+    float v[AT_ONCE], m0[HW], l0[HW], sink[HW], gate0 = 0.0f;
+    const int i_first = min(tid, nh * vdimp - 1);
     {
-        const int i = min(tid, nh * vdimp - 1);
-        const float *ph = part + size_t(i / vdimp) * stride + i % vdimp;
+        const float *ph = part + size_t(i_first / vdimp) * stride + i_first % vdimp;
 #pragma unroll
         for (int u = 0; u < AT_ONCE; u++) v[u] = ld_f<true>(ph + min(u, S - 1) * pitch);
     }
-    if (p.gate && !meet.wait_gate()) return;
-    for (int h = wave; h < nh; h += 4) {
-        const float *ph = part + size_t(h) * stride + vdimp, sink = p.sink ? p.sink[h0 + h] : -INFINITY;
-        const float m0 = lane < S ? ld_f<true>(ph + lane * pitch) : -INFINITY, l0 = lane < S ? ld_f<true>(ph + lane * pitch + 1) : 0.0f;
-        float m = fmaxf(sink, m0), l = 0.0f;
+#pragma unroll
+    for (int i = 0; i < HW; i++) {
+        const int h = wave + 4 * i;
+        const float *ph = part + size_t(h) * stride + vdimp;
+        sink[i] = m0[i] = -INFINITY;
+        l0[i] = 0.0f;
+        if (h < nh && p.sink) sink[i] = p.sink[h0 + h];
+        if (h < nh && lane < S) {
+            m0[i] = ld_f<true>(ph + lane * pitch);
+            l0[i] = ld_f<true>(ph + lane * pitch + 1);
+        }
+    }
+    if (p.gate) {
+        if (!meet.wait_gate()) return;
+        gate0 = ld_f<COH>(p.proj + p.og + h0 * vdimp + i_first);
+    }
+#pragma unroll
+    for (int i = 0; i < HW; i++) {
+        const int h = wave + 4 * i;
+        if (h >= nh) continue;
+        const float *ph = part + size_t(h) * stride + vdimp;
+        float m = fmaxf(sink[i], m0[i]), l = 0.0f;
         for (int s = lane + 64; s < S; s += 64) m = fmaxf(m, ld_f<true>(ph + s * pitch));
         m = wave_max(m);
         for (int s = lane; s < S; s += 64) { // (an empty split: m = -inf, weight 0)
-            const float w = expf((s == lane ? m0 : ld_f<true>(ph + s * pitch)) - m);
-            l = fmaf(s == lane ? l0 : ld_f<true>(ph + s * pitch + 1), w, l);
+            const float w = expf((s == lane ? m0[i] : ld_f<true>(ph + s * pitch)) - m);
+            l = fmaf(s == lane ? l0[i] : ld_f<true>(ph + s * pitch + 1), w, l);
             s_w[h * S + s] = w;
         }
-        l = wave_sum(l) + (p.sink ? expf(sink - m) : 0.0f);
+        l = wave_sum(l) + (p.sink ? expf(sink[i] - m) : 0.0f);
         if (lane == 0) s_ml[h] = 1.0f / l;
     }
     lds_barrier();
@@ -539,7 +556,7 @@ __device__ __forceinline__ void mix_attention(const DecodeMix &p, int g, int hb,
             s_o[i] = o;
             continue;
         }
-        if (p.gate) o *= lm_sigmoid(ld_f<COH>(p.proj + p.og + (h0 + h) * vdimp + d));
+        if (p.gate) o *= lm_sigmoid(i == tid ? gate0 : ld_f<COH>(p.proj + p.og + (h0 + h) * vdimp + d));
         st_t<COH>(reinterpret_cast<T *>(p.out) + (h0 + h) * vdimp + d, (T)o);
     }
     if (!(WHOLE && p.rotv)) return meet.done();
@@ -551,7 +568,7 @@ __device__ __forceinline__ void mix_attention(const DecodeMix &p, int g, int hb,
             const float2 cs = i == tid ? back_cs : p.rotv[size_t(pos) * back + d % back];
             o = d < back ? o * cs.x + s_o[i + back] * cs.y : o * cs.x - s_o[i - back] * cs.y;
         }
-        if (p.gate) o *= lm_sigmoid(ld_f<COH>(p.proj + p.og + (h0 + h) * vdimp + d));
+        if (p.gate) o *= lm_sigmoid(i == tid ? gate0 : ld_f<COH>(p.proj + p.og + (h0 + h) * vdimp + d));
         st_t<COH>(reinterpret_cast<T *>(p.out) + (h0 + h) * vdimp + d, (T)o);
     }
     meet.done();
