@@ -2,6 +2,7 @@
 // and the persistent decode kernel.  Written for 256-thread workgroups (4 wavefronts).
 #pragma once
 #include "epilogue.hpp"
+#include "lane_fold.hpp"
 
 constexpr int DEC_SPLITS = 8;
 constexpr int DEC_MAX_KEYS = (2048 + DEC_SPLITS - 2) / (DEC_SPLITS - 1); // per split at the reference's kv limit (attention.zig:252)
@@ -107,6 +108,7 @@ __device__ __forceinline__ void decode_attn_task(const half_t *__restrict__ qkv,
     __shared__ float sscore[DEC_MAX_KEYS];
     __shared__ float sred[4][D];
     __shared__ float sstat[8];
+    __shared__ float swave[4][64];
     __shared__ int s_last;
 
     const int pos = FUSED ? pos_real : -1; // in plain mode no key is special
@@ -181,24 +183,34 @@ __device__ __forceinline__ void decode_attn_task(const half_t *__restrict__ qkv,
         score(j, j == pos ? *reinterpret_cast<const uint4 *>(&sk_new[8 * e]) : *reinterpret_cast<const uint4 *>(kbase + size_t(j) * D + 8 * e));
     lds_barrier();
 
-    // softmax statistics of this split
+    // softmax statistics of this split.  Up to 64 scores are one wavefront's: every wavefront takes them all, the same bits without two exchanges
+    // and their barriers (with the lanes' sums below, 48 tokens behind 53, width 1024, prompt included: 18.88 -> 18.42 ms; 24 tokens of width 2048 14.36 -> 14.24).
     const int nkeys = max(j1 - j0, 0);
-    float m = -INFINITY;
-    for (int i = t; i < nkeys; i += 256) m = fmaxf(m, sscore[i]);
-    m = wave_max(m);
-    if (lane == 0) sstat[wave] = m;
-    lds_barrier();
-    m = fmaxf(fmaxf(sstat[0], sstat[1]), fmaxf(sstat[2], sstat[3]));
-    float l = 0.0f;
-    for (int i = t; i < nkeys; i += 256) {
-        const float p = __expf(sscore[i] - m);
-        sscore[i] = p;
-        l += p;
+    float m = -INFINITY, l = 0.0f;
+    const float *weight = sscore;
+    if (nkeys <= 64) {
+        const float s = lane < nkeys ? sscore[lane] : -INFINITY;
+        m = wave_max(s);
+        const float p = lane < nkeys ? __expf(s - m) : 0.0f;
+        l = wave_sum(p);
+        swave[wave][lane] = p;
+        weight = swave[wave];
+    } else {
+        for (int i = t; i < nkeys; i += 256) m = fmaxf(m, sscore[i]);
+        m = wave_max(m);
+        if (lane == 0) sstat[wave] = m;
+        lds_barrier();
+        m = fmaxf(fmaxf(sstat[0], sstat[1]), fmaxf(sstat[2], sstat[3]));
+        for (int i = t; i < nkeys; i += 256) {
+            const float p = __expf(sscore[i] - m);
+            sscore[i] = p;
+            l += p;
+        }
+        l = wave_sum(l);
+        if (lane == 0) sstat[4 + wave] = l;
+        lds_barrier();
+        l = (sstat[4] + sstat[5]) + (sstat[6] + sstat[7]);
     }
-    l = wave_sum(l);
-    if (lane == 0) sstat[4 + wave] = l;
-    lds_barrier();
-    l = (sstat[4] + sstat[5]) + (sstat[6] + sstat[7]);
 
     // o = sum_j p_j v_j
     float acc[8];
@@ -206,7 +218,7 @@ __device__ __forceinline__ void decode_attn_task(const half_t *__restrict__ qkv,
     for (int i = 0; i < 8; i++) acc[i] = 0.0f;
     auto accumulate = [&](int j, const uint4 &vv) {
         const half_t *vh = reinterpret_cast<const half_t *>(&vv);
-        const float p = sscore[j - j0];
+        const float p = weight[j - j0];
 #pragma unroll
         for (int i = 0; i < 8; i++) acc[i] = fmaf(p, (float)vh[i], acc[i]);
     };
@@ -219,9 +231,7 @@ __device__ __forceinline__ void decode_attn_task(const half_t *__restrict__ qkv,
         accumulate(j, j == pos ? *reinterpret_cast<const uint4 *>(&sv_new[8 * e]) : *reinterpret_cast<const uint4 *>(vbase + size_t(j) * D + 8 * e));
 #pragma unroll
     for (int i = 0; i < 8; i++) {
-        acc[i] += __shfl_xor(acc[i], 8, 64);
-        acc[i] += __shfl_xor(acc[i], 16, 64);
-        acc[i] += __shfl_xor(acc[i], 32, 64);
+        acc[i] = add_32_away(add_16_away(add_8_away(acc[i])));
     }
     if (g == 0) {
 #pragma unroll

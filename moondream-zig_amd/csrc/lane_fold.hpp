@@ -12,6 +12,21 @@ __device__ __forceinline__ float half_max(float v) {
     return fmaxf(__builtin_bit_cast(float, r0), __builtin_bit_cast(float, r1));
 }
 
+// A lane's value plus that of the lane 8, 16 or 32 away: the additions of v + __shfl_xor(v, n) without its trip through LDS
+__device__ __forceinline__ float add_8_away(float v) { return v + dpp_move<DPP_ROW_ROR8>(v); }
+__device__ __forceinline__ float add_16_away(float v) {
+    const unsigned b = __builtin_bit_cast(unsigned, v);
+    const auto r = __builtin_amdgcn_permlane16_swap(b, b, false, false);
+    const unsigned r0 = r[0], r1 = r[1];
+    return __builtin_bit_cast(float, r0) + __builtin_bit_cast(float, r1);
+}
+__device__ __forceinline__ float add_32_away(float v) {
+    const unsigned b = __builtin_bit_cast(unsigned, v);
+    const auto r = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+    const unsigned r0 = r[0], r1 = r[1];
+    return __builtin_bit_cast(float, r0) + __builtin_bit_cast(float, r1);
+}
+
 // Sum over this lane and those below it (no trip through LDS): within rows of 16, then the last lanes of the rows before.
 __device__ __forceinline__ int lane_prefix_sum(int v) {
     v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false); // from 1, 2, 4 and 8 lanes below within the row, zero where there is none
@@ -29,8 +44,8 @@ __device__ __forceinline__ float group_sum(float v, int n) {
     if (n >= 4) v += dpp_move<DPP_QUAD_XOR2>(v);
     if (n >= 8) v += dpp_move<DPP_ROW_HALF_MIRROR>(v);
     if (n >= 16) v += dpp_move<DPP_ROW_MIRROR>(v);
-    if (n >= 32) v += __shfl_xor(v, 16);
-    if (n >= 64) v += __shfl_xor(v, 32);
+    if (n >= 32) v = add_16_away(v);
+    if (n >= 64) v = add_32_away(v);
     return v;
 }
 
