@@ -11,6 +11,9 @@
 // Measured and not kept: one row per output wavefront, which leaves the producers half of the places (8 key heads 603, 32 373 of 12 layers; with 192 producers 4 key heads took
 // 1,202); gate rows ahead of the attention (615; 12 layers behind 900 keys 352); a delta rule's taps, ranks and vectors asked for ahead of the wait (no difference); the first count on 8 or 16 lines that all heads' workgroups poll, a hop less, in place of 64 copies (660, 635: 130 pollers on
 // a line hold up the stream); no pauses between the lots of an output row, longer ones, and no wave priority: 0 to 2 % either way; three workgroups a unit at width 1024 in place of two: 0 to 2 % slower.
+// The same for routed experts (a role that waits for the router's logits, chooses and streams the gate and up rows; output workgroups that choose too and ask for the chosen down rows)
+// took 33.3 to 34.3 us a layer with 8 of 64 experts of 704 where the three launches take 32.1: the choice and the two streams behind it follow each other all the same.  Front rows spread evenly over the
+// producers, on one producer a unit, or output workgroups that start 1.3 to 5 us late: 0 to 3 % slower.
 // Progress: producers never wait and come first in the grid, so on every die they have their places before any workgroup that waits; the
 // attention's workgroups wait for producers, the output's for both, in the grid's order (a merge also waits for the gate: producers again).  Workgroups of several launches could all the same fill the dies
 // with some that wait for another die's: calls take their places beforehand (wait_places.hpp) and run in three launches where there are
