@@ -7,7 +7,7 @@
 //               activation is there, the rest streams while the attention is still under way; the heads' part comes last
 // A layer of 97 MB (width 2048, 8 key heads, feed-forward 5504) took 14.6 + 11 + 4.6 us and three launches' starts, ends and gaps; the weights of its later phases stream while
 // the earlier ones run here.  695 -> 596 us a token behind 61 keys, 382 -> 327 for 12 layers behind 900; 32 key heads 381 -> 337, 4 key heads and feed-forward 2048 358 -> 292; width 1024: 504 -> 384,
-// rotated and joined 549 -> 425 (width 2048, 12 layers 421 -> 392).  What bounds it is the chain q, k, v -> attention -> merge -> output beside the stream: 4 TB/s.
+// rotated and joined 549 -> 425 (width 2048, 12 layers 421 -> 355).  What bounds it is the chain q, k, v -> attention -> merge -> output beside the stream: 4 TB/s.
 // Measured and not kept: one row per output wavefront, which leaves the producers half of the places (8 key heads 603, 32 373 of 12 layers; with 192 producers 4 key heads took
 // 1,202); gate rows ahead of the attention (615; 12 layers behind 900 keys 352); a delta rule's taps, ranks and vectors asked for ahead of the wait (no difference); the first count on 8 or 16 lines that all heads' workgroups poll, a hop less, in place of 64 copies (660, 635: 130 pollers on
 // a line hold up the stream); no pauses between the lots of an output row, longer ones, and no wave priority: 0 to 2 % either way; three workgroups a unit at width 1024 in place of two: 0 to 2 % slower.
@@ -26,12 +26,16 @@
 #include "launch_waits.hpp"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace {
 
 constexpr int WHOLE_D = 64;      // padded head sizes
 constexpr int WHOLE_LEAVES = 32; // the producers' counts come together on so many lines, and then on every copy
-constexpr int WHOLE_GLU = 12;    // 1 KiB pieces of a row of the dense activation's weights
+// 1 KiB pieces of a row of the dense activation's weights at most (10,240 columns: the layers of a joined list whose weights are in the feed-forward have 6,464 at
+// width 2048; in three launches, as with 12 pieces, half of such a list's layers were, and a token of 12 layers took 392 us in place of 355), ..
+constexpr int WHOLE_GLU = 20;
+constexpr int WHOLE_HELD = 12;   // .. and those of an output wavefront's first row that wait in registers
 constexpr int WHOLE_ROWS = 2;    // rows of an output wavefront
 constexpr int WHOLE_SLEEP = 6;   // units of 64 cycles between two lots of them
 enum { WHOLE_FRONT, WHOLE_ACT, WHOLE_HEADS, WHOLE_COUNTS };
@@ -158,7 +162,7 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t stretch(const void *p, int byt
 // while the attention is still under way.
 template <int W, bool DELTA> __device__ __forceinline__ void whole_output(const WholeArgs &a, int wg, int n_wgs, char *lds, int *s_flag) {
     typedef bf16_t T;
-    constexpr int R = WHOLE_ROWS, HOLD = DELTA && W > 2 ? 8 : WHOLE_GLU;
+    constexpr int R = WHOLE_ROWS, HOLD = DELTA && W > 2 ? 8 : WHOLE_HELD;
     const DecodeOut &o = a.o;
     const int tid = threadIdx.x, lane = tid & 63, first = wg * 4 + __builtin_amdgcn_readfirstlane(tid >> 6), b = blockIdx.x % LAYER_COPIES;
     const bool fresh = a.p.token || a.p.y; // a producer writes x in this launch
@@ -198,24 +202,29 @@ template <int W, bool DELTA> __device__ __forceinline__ void whole_output(const 
         }
         if (!wait_reached(whole_copy(a, WHOLE_ACT, b), a.reached[WHOLE_ACT], a.error, s_flag)) return;
         const auto act = stretch(reinterpret_cast<const T *>(o.a) + o.k2, n_f);
-        lm_u32x4 v[WHOLE_GLU / 4];
+        auto copy = [&](auto from, auto to) { // 4 KiB a step, all requested before any is waited for
+            constexpr int FROM = decltype(from)::value, N = decltype(to)::value - FROM;
+            lm_u32x4 v[N];
 #pragma unroll
-        for (int c = 0; c < WHOLE_GLU / 4; c++) v[c] = stretch_load<LOAD_DIE>(act, (c * 256 + tid) * 16);
+            for (int c = 0; c < N; c++) v[c] = stretch_load<LOAD_DIE>(act, ((FROM + c) * 256 + tid) * 16);
 #pragma unroll
-        for (int c = 0; c < WHOLE_GLU / 4; c++) reinterpret_cast<lm_u32x4 *>(lds)[c * 256 + tid] = v[c];
+            for (int c = 0; c < N; c++) reinterpret_cast<lm_u32x4 *>(lds)[(FROM + c) * 256 + tid] = v[c];
+        };
+        copy(std::integral_constant<int, 0>{}, std::integral_constant<int, WHOLE_HELD / 4>{});
+        if (n_f > WHOLE_HELD * 1024) copy(std::integral_constant<int, WHOLE_HELD / 4>{}, std::integral_constant<int, WHOLE_GLU / 4>{});
         lds_barrier();
 #pragma unroll
         for (int r = 0; r < R; r++) {
             const auto w = weights(r, o.k2, n_f);
-#pragma unroll
-            for (int base = 0; base < WHOLE_GLU; base += HOLD) {
+#pragma unroll 1
+            for (int base = 0; base * 1024 < n_f; base += HOLD) {
                 if (r || base)
 #pragma unroll
                     for (int c = 0; c < HOLD; c++)
-                        if ((base + c) * 1024 < n_f && base + c < WHOLE_GLU) wf[c] = stretch_load<LOAD_STREAM>(w, (base + c) * 1024 + lane * 16);
+                        if ((base + c) * 1024 < n_f) wf[c] = stretch_load<LOAD_STREAM>(w, (base + c) * 1024 + lane * 16);
 #pragma unroll
                 for (int c = 0; c < HOLD; c++)
-                    if ((base + c) * 1024 < n_f && base + c < WHOLE_GLU) dot_f[r] = dot_piece<T>(wf[c], reinterpret_cast<const lm_u32x4 *>(lds)[(base + c) * 64 + lane], dot_f[r]);
+                    if ((base + c) * 1024 < n_f) dot_f[r] = dot_piece<T>(wf[c], reinterpret_cast<const lm_u32x4 *>(lds)[(base + c) * 64 + lane], dot_f[r]);
             }
             dot_f[r] = wave_sum(dot_f[r]);
         }
@@ -295,7 +304,7 @@ bool whole_plan(moon_ctx *ctx, const DecodeProj &p, const DecodeMix &m, const De
     const int per = m.H / m.G, wgs = m.G * mix_head_blocks(per), nh = std::min(per, MIX_HEADS), NH = nh <= 1 ? 1 : nh <= 2 ? 2 : nh <= 4 ? 4 : 8;
     w->S = mix_splits(n_keys, wgs, cus);
     w->keys_max = std::max(MIX_TARGET, (n_keys + w->S - 1) / w->S); // (fewer keys: the LDS of so many all the same)
-    w->lds = std::max({size_t(p.dp) * 2, mix_lds_floats(NH, WHOLE_D, WHOLE_D, w->keys_max) * sizeof(float), size_t(p.ff ? WHOLE_GLU * 1024 : 0),
+    w->lds = std::max({size_t(p.dp) * 2, mix_lds_floats(NH, WHOLE_D, WHOLE_D, w->keys_max) * sizeof(float), size_t(!p.ff ? 0 : o.k0 - o.k2 > 512 * WHOLE_HELD ? WHOLE_GLU * 1024 : WHOLE_HELD * 1024),
                        m.dH ? delta_lds_floats(m.ddimp, m.dvdimp, m.kd) * sizeof(float) : 0});
     if (w->lds > 60 * 1024 || size_t(NH) * w->S > mix_lds_floats(NH, WHOLE_D, WHOLE_D, w->keys_max) - 4 * NH - 8) return false;
     w->kern = mix_whole(m) ? (U == 2 ? whole_kernel_of<2, true>(NH) : whole_kernel_of<4, true>(NH)) : (U == 2 ? whole_kernel_of<2, false>(NH) : whole_kernel_of<4, false>(NH));

@@ -65,9 +65,9 @@ def test_generax(moon, ctx, tmp_path, width, heads, kv_heads, ff, delta_heads):
 
 
 LARGE = [RM.config(128, 2048, [RM.layer(RM.attention(32, kv, 64, 64, window, 0.125, True), RM.dense(ff) if ff else None) for _ in range(3)], embed_scale=2.0)
-         for kv, window, ff in ((32, 1024, 6144), (8, 1024, 5504), (4, 512, 1024), (8, 64, None))]
+         for kv, window, ff in ((32, 1024, 6144), (8, 1024, 5504), (8, 512, 6208), (1, 512, 10240), (4, 512, 1024), (8, 64, None))]
 LARGE += [GM.config(128, width, [GM.parallel(GM.softmax_mixer(width // 64, kv, 64, 64, 512, 0.125, 16), GM.delta(width // 64, width // 64, 64, 64, 4), ff),
-                                 GM.plain(GM.attention(width // 64, kv, 64, 64, 1024, 0.125, ROT), ff)] * 2) for width, kv, ff in ((2048, 8, 5632), (2048, 32, 3712), (1024, 4, 1728))]
+                                 GM.plain(GM.attention(width // 64, kv, 64, 64, 1024, 0.125, ROT), ff)] * 2) for width, kv, ff in ((2048, 8, 5632), (2048, 8, 6464), (1024, 16, 9856), (2048, 32, 3712), (1024, 4, 1728))]
 
 
 @pytest.mark.parametrize("which", range(len(LARGE)))
@@ -91,7 +91,7 @@ def test_largest_sizes_beside_f32(moon, ctx, which):
     assert_close(*out)
 
 
-@pytest.mark.parametrize("change", [dict(width=2112), dict(ff=6208), dict(dim=128), dict(experts=True)])
+@pytest.mark.parametrize("change", [dict(width=2112), dict(ff=10304), dict(dim=128), dict(experts=True)])
 def test_other_sizes_take_three_launches(moon, ctx, change):
     width, dim = change.get("width", 1024), change.get("dim", 64)
     mlp = RM.moe(64, 64, 64) if "experts" in change else RM.dense(change.get("ff", 128))
