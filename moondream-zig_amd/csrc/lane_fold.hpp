@@ -27,6 +27,20 @@ __device__ __forceinline__ float add_32_away(float v) {
     return __builtin_bit_cast(float, r0) + __builtin_bit_cast(float, r1);
 }
 
+// Of four wavefronts' values, value l of the one 2 h + w in element 2 (l / 32) + h of lane 32 w + l % 32: (wave_sum(0) + wave_sum(1)) + (wave_sum(2) + wave_sum(3)), the
+// same additions.  From the second step on lane 4 i + k has element k's sums.
+__device__ __forceinline__ float quarters_sum(const float (&v)[4], int lane) {
+    constexpr int QUAD_REVERSED = 0x1B; // and mirrored within 8: the lane 4 away
+    const bool odd = lane & 1, upper = lane & 2;
+    const float a = (odd ? v[1] : v[0]) + dpp_move<DPP_QUAD_XOR1>(odd ? v[0] : v[1]), b = (odd ? v[3] : v[2]) + dpp_move<DPP_QUAD_XOR1>(odd ? v[2] : v[3]);
+    float s = (upper ? b : a) + dpp_move<DPP_QUAD_XOR2>(upper ? a : b);
+    s += dpp_move<DPP_ROW_HALF_MIRROR>(dpp_move<QUAD_REVERSED>(s));
+    s = add_16_away(add_8_away(s));
+    s += dpp_move<DPP_QUAD_XOR2>(s);
+    s = add_32_away(s);
+    return s + dpp_move<DPP_QUAD_XOR1>(s);
+}
+
 // Sum over this lane and those below it (no trip through LDS): within rows of 16, then the last lanes of the rows before.
 __device__ __forceinline__ int lane_prefix_sum(int v) {
     v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false); // from 1, 2, 4 and 8 lanes below within the row, zero where there is none

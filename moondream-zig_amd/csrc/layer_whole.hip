@@ -32,8 +32,8 @@ namespace {
 
 constexpr int WHOLE_D = 64;      // padded head sizes
 constexpr int WHOLE_LEAVES = 32; // the producers' counts come together on so many lines, and then on every copy
-// 1 KiB pieces of a row of the dense activation's weights at most (10,240 columns: the layers of a joined list whose weights are in the feed-forward have 6,464 at
-// width 2048; in three launches, as with 12 pieces, half of such a list's layers were, and a token of 12 layers took 392 us in place of 355), ..
+// Loads of a row of the dense activation's weights at most (10,240 columns: the layers of a joined list whose weights are in the feed-forward have 6,464 at
+// width 2048; in three launches, as with 12 loads, half of such a list's layers were, and a token of 12 layers took 392 us in place of 355), ..
 constexpr int WHOLE_GLU = 20;
 constexpr int WHOLE_HELD = 12;   // .. and those of an output wavefront's first row that wait in registers
 constexpr int WHOLE_ROWS = 2;    // rows of an output wavefront
@@ -150,51 +150,70 @@ template <int U> __device__ __forceinline__ void whole_producer(const WholeArgs 
 
 // 16 bytes a lane of a stretch of `bytes`; zeros behind its end
 enum { LOAD_DIE = 1, LOAD_STREAM = 2 }; // from the die's cache on; not to be kept
-template <int HOW> __device__ __forceinline__ lm_u32x4 stretch_load(__amdgpu_buffer_rsrc_t r, int at) {
-    return __builtin_bit_cast(lm_u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, at, 0, HOW));
+template <int HOW> __device__ __forceinline__ lm_u32x4 stretch_load(__amdgpu_buffer_rsrc_t r, int at, int base) {
+    return __builtin_bit_cast(lm_u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, at, base, HOW));
 }
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t stretch(const void *p, int bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, bytes, 0x00020000);
 }
 
-// W: 1 KiB pieces of a row that meet the heads, and of those that meet the delta rule's.  A wavefront owns WHOLE_ROWS rows: their parts for the
-// heads and the beginning of the first one's for the dense activation (HOLD pieces) are in registers by the time that the activation is there, the rest streams
+// A row's sums are those of out_rows, addition for addition, so one launch and three give the same bits.  There four wavefronts take a quarter of a stretch's pieces
+// each, lane l of one its pieces l, l + 64, ..  Here one wavefront takes all four, half a wavefront a quarter: lane 32 w + j of load c has piece 32 (c / 2) + j of quarter
+// 2 (c % 2) + w, which is lane 32 (c / 2 % 2) + j there.  So a lane keeps four sums, element c % 4, and quarters_sum adds them up.
+// A token takes 1 % longer than with whole KiB in any order (24 layers of width 2048, feed-forward 5504 598 us against 590, 12 of 32 key heads 335 against 333, width
+// 1024 382 against 381).  Measured and not kept: loads of 64 pieces of one quarter (597, 340, 385), of 16 of each (599, 336, 400); whole KiB, their dots turned by
+// ds_bpermute where a quarter ends (648, 360, 435) or through LDS (596, 338, 386, and 368 in place of 360 for 12 joined layers of width 2048).
+constexpr int NOWHERE = 1 << 30; // no buffer is as long: loads zeros
+struct Quarters {
+    int pieces, mine, at; // of a quarter; this lane's first; its byte
+    __device__ __forceinline__ Quarters(int bytes, int lane) : pieces(bytes / 64), mine(lane % 32), at((lane / 32 * (bytes / 64) + lane % 32) * 16) {}
+    __device__ __forceinline__ bool any(int c) const { return c * 16 < pieces; } // (c even: loads c and c + 1)
+    __device__ __forceinline__ int offset(int c) const { return c / 2 * 512 + c % 2 * 2 * pieces * 16; }
+    __device__ __forceinline__ int piece(int c) const { return (at + offset(c)) / 16; }
+    template <int HOW> __device__ __forceinline__ lm_u32x4 load(__amdgpu_buffer_rsrc_t r, int c) const { return stretch_load<HOW>(r, c / 2 * 32 + mine < pieces ? at : NOWHERE, offset(c)); }
+};
+
+// QW: loads of a row's part for the heads, of which the delta rule's come behind the attention's.  A wavefront owns WHOLE_ROWS rows: their parts for the
+// heads and the beginning of the first one's for the dense activation (HOLD loads) are in registers by the time that the activation is there, the rest streams
 // while the attention is still under way.
-template <int W, bool DELTA> __device__ __forceinline__ void whole_output(const WholeArgs &a, int wg, int n_wgs, char *lds, int *s_flag) {
+template <int QW, bool DELTA> __device__ __forceinline__ void whole_output(const WholeArgs &a, int wg, int n_wgs, char *lds, int *s_flag) {
     typedef bf16_t T;
-    constexpr int R = WHOLE_ROWS, HOLD = DELTA && W > 2 ? 8 : WHOLE_HELD;
+    constexpr int R = WHOLE_ROWS, HOLD = QW > 4 ? 8 : WHOLE_HELD;
     const DecodeOut &o = a.o;
-    const int tid = threadIdx.x, lane = tid & 63, first = wg * 4 + __builtin_amdgcn_readfirstlane(tid >> 6), b = blockIdx.x % LAYER_COPIES;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), first = wg * 4 + wave, b = blockIdx.x % LAYER_COPIES;
     const bool fresh = a.p.token || a.p.y; // a producer writes x in this launch
-    const int n_o = o.k1 * 2, n_d = (o.k2 - o.k1) * 2, n_f = (o.k0 - o.k2) * 2; // bytes of a row's parts
+    const int n_h = o.k2 * 2, n_f = (o.k0 - o.k2) * 2; // bytes of a row's parts
+    const Quarters h(n_h, lane), f(n_f, lane);
     auto row = [&](int r) { return first + r * n_wgs * 4; };
-    auto weights = [&](int r, int column, int bytes) { return stretch(reinterpret_cast<const T *>(o.w2) + size_t(row(r)) * o.k0 + column, row(r) < o.width ? bytes : 0); };
-    lm_u32x4 wo[R][W], wd[R][DELTA ? W : 1], wf[HOLD];
+    // (rows behind the width are padding: there are dp, a multiple of 64)
+    auto weights = [&](int r, int column, int bytes) { return stretch(reinterpret_cast<const T *>(o.w2) + size_t(row(r)) * o.k0 + column, bytes); };
+    lm_u32x4 wh[R][QW], wf[HOLD];
     float old[R];
 #pragma unroll
     for (int r = 0; r < R; r++) {
-        const auto w = weights(r, 0, n_o);
+        const auto w = weights(r, 0, n_h);
         old[r] = 0.0f;
         if (!fresh && !o.y && row(r) < o.width) old[r] = o.x[row(r)];
 #pragma unroll
-        for (int c = 0; c < W; c++) wo[r][c] = stretch_load<LOAD_STREAM>(w, c * 1024 + lane * 16);
+        for (int c = 0; c < QW; c++) wh[r][c] = h.load<LOAD_STREAM>(w, c);
     }
-    if (DELTA && n_d)
-#pragma unroll
-        for (int r = 0; r < R; r++) {
-            const auto w = weights(r, o.k1, n_d);
-#pragma unroll
-            for (int c = 0; c < W; c++) wd[r][c] = stretch_load<LOAD_STREAM>(w, c * 1024 + lane * 16);
-        }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     float dot_f[R] = {};
     if (n_f) {
+        auto request = [&](__amdgpu_buffer_rsrc_t w, int base, int c) { // loads base + c .. base + c + 3
+#pragma unroll
+            for (int m = c; m < c + 4; m += 2)
+                if (f.any(base + m)) {
+                    wf[m] = f.load<LOAD_STREAM>(w, base + m);
+                    wf[m + 1] = f.load<LOAD_STREAM>(w, base + m + 1);
+                }
+        };
         {
             const auto w = weights(0, o.k2, n_f);
 #pragma unroll
-            for (int c = 0; c < HOLD; c++) {
-                if (c * 1024 < n_f) wf[c] = stretch_load<LOAD_STREAM>(w, c * 1024 + lane * 16);
-                if (c % 4 == 3 && c + 1 < HOLD) {
+            for (int c = 0; c < HOLD; c += 4) {
+                request(w, 0, c);
+                if (c + 4 < HOLD) {
                     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
                     __builtin_amdgcn_s_sleep(WHOLE_SLEEP);
                 }
@@ -202,11 +221,11 @@ template <int W, bool DELTA> __device__ __forceinline__ void whole_output(const 
         }
         if (!wait_reached(whole_copy(a, WHOLE_ACT, b), a.reached[WHOLE_ACT], a.error, s_flag)) return;
         const auto act = stretch(reinterpret_cast<const T *>(o.a) + o.k2, n_f);
-        auto copy = [&](auto from, auto to) { // 4 KiB a step, all requested before any is waited for
+        auto copy = [&](auto from, auto to) { // the vector as the lanes meet it, 4 KiB a step, all requested before any is waited for
             constexpr int FROM = decltype(from)::value, N = decltype(to)::value - FROM;
             lm_u32x4 v[N];
 #pragma unroll
-            for (int c = 0; c < N; c++) v[c] = stretch_load<LOAD_DIE>(act, ((FROM + c) * 256 + tid) * 16);
+            for (int c = 0; c < N; c++) v[c] = f.load<LOAD_DIE>(act, (FROM + c) * 4 + wave);
 #pragma unroll
             for (int c = 0; c < N; c++) reinterpret_cast<lm_u32x4 *>(lds)[(FROM + c) * 256 + tid] = v[c];
         };
@@ -216,54 +235,55 @@ template <int W, bool DELTA> __device__ __forceinline__ void whole_output(const 
 #pragma unroll
         for (int r = 0; r < R; r++) {
             const auto w = weights(r, o.k2, n_f);
+            float part[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll 1
-            for (int base = 0; base * 1024 < n_f; base += HOLD) {
-                if (r || base)
+            for (int base = 0; f.any(base); base += HOLD) {
 #pragma unroll
-                    for (int c = 0; c < HOLD; c++)
-                        if ((base + c) * 1024 < n_f) wf[c] = stretch_load<LOAD_STREAM>(w, (base + c) * 1024 + lane * 16);
+                for (int c = 0; c < HOLD; c += 4)
+                    if (r || base) request(w, base, c);
 #pragma unroll
-                for (int c = 0; c < HOLD; c++)
-                    if ((base + c) * 1024 < n_f) dot_f[r] = dot_piece<T>(wf[c], reinterpret_cast<const lm_u32x4 *>(lds)[(base + c) * 64 + lane], dot_f[r]);
+                for (int c = 0; c < HOLD; c += 2)
+                    if (f.any(base + c))
+#pragma unroll
+                        for (int m = c; m < c + 2; m++) part[m % 4] += dot_piece<T>(wf[m], reinterpret_cast<const lm_u32x4 *>(lds)[(base + m) * 64 + lane], 0.0f);
             }
-            dot_f[r] = wave_sum(dot_f[r]);
+            dot_f[r] = quarters_sum(part, lane);
         }
     }
     if (!wait_reached(whole_copy(a, WHOLE_HEADS, b), a.reached[WHOLE_HEADS], a.error, s_flag)) return;
-    const auto x_o = stretch(o.a, n_o), x_d = stretch(reinterpret_cast<const T *>(o.a) + o.k1, n_d);
-    lm_u32x4 xo[W], xd[DELTA ? W : 1];
+    const auto heads = stretch(o.a, n_h);
+    lm_u32x4 xh[QW];
     if (fresh && !o.y)
 #pragma unroll
         for (int r = 0; r < R; r++)
             if (row(r) < o.width) old[r] = ld_f<true>(o.x + row(r));
 #pragma unroll
-    for (int c = 0; c < W; c++) xo[c] = stretch_load<LOAD_DIE>(x_o, c * 1024 + lane * 16);
-    if (DELTA && n_d)
-#pragma unroll
-        for (int c = 0; c < W; c++) xd[c] = stretch_load<LOAD_DIE>(x_d, c * 1024 + lane * 16);
+    for (int c = 0; c < QW; c++) xh[c] = h.load<LOAD_DIE>(heads, c);
 #pragma unroll
     for (int r = 0; r < R; r++) {
         const int n = row(r);
-        float dot_o = 0.0f, dot_d = 0.0f;
+        float part[4] = {0.0f, 0.0f, 0.0f, 0.0f}, part_d[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int c = 0; c < W; c++) dot_o = dot_piece<T>(wo[r][c], xo[c], dot_o);
-        dot_o = wave_sum(dot_o);
-        if (DELTA && n_d) {
-#pragma unroll
-            for (int c = 0; c < W; c++) dot_d = dot_piece<T>(wd[r][c], xd[c], dot_d);
-            dot_d = wave_sum(dot_d);
+        for (int c = 0; c < QW; c++) {
+            const float d = dot_piece<T>(wh[r][c], xh[c], 0.0f);
+            const bool delta = DELTA && h.piece(c) >= o.k1 / 8; // (no layer without a delta rule has columns there)
+            part[c % 4] += delta ? 0.0f : d;
+            if (DELTA) part_d[c % 4] += delta ? d : 0.0f;
         }
+        const float dot = quarters_sum(part, lane), dot_d = DELTA ? quarters_sum(part_d, lane) : 0.0f;
         if (lane || n >= o.width) continue;
         if (o.y) {
-            o.y[n] = dot_o;
+            o.y[n] = dot;
             o.y[o.dp + n] = dot_d;
             o.y[2 * o.dp + n] = dot_f[r];
-        } else o.x[n] = old[r] + (dot_o + dot_d + dot_f[r]);
+        } else o.x[n] = old[r] + (dot + dot_f[r]);
     }
 }
 
+// Workgroups a unit: what the registers allow without scratch (wide layers with the mechanisms of WHOLE hold 64 of them for two rows' heads: 12 such layers of
+// width 2048 took 380 us a token with four a unit and up to 24 registers in scratch, 360 with three).
 template <int NH, int U, bool WHOLE>
-__global__ __launch_bounds__(256, NH > 4 ? 3 : 4) void decode_whole_kernel(WholeArgs) {
+__global__ __launch_bounds__(256, NH > 4 || (WHOLE && U > 2) ? 3 : U > 2 || WHOLE ? 4 : 5) void decode_whole_kernel(WholeArgs) {
     const WholeArgs &a = fetch_arguments<WholeArgs>();
     extern __shared__ __attribute__((aligned(16))) char s_whole[];
     __shared__ float s_red[16];
@@ -282,7 +302,7 @@ __global__ __launch_bounds__(256, NH > 4 ? 3 : 4) void decode_whole_kernel(Whole
         if (WHOLE) mix_delta<bf16_t, true>(a.m, i - a.n_attn, lds, meet);
         return;
     }
-    whole_output<U, WHOLE>(a, i - a.n_attn - n_delta, gridDim.x - a.n_prod - a.n_attn - n_delta, s_whole, &s_flag);
+    whole_output<(WHOLE ? 2 * U : U), WHOLE>(a, i - a.n_attn - n_delta, gridDim.x - a.n_prod - a.n_attn - n_delta, s_whole, &s_flag);
 }
 
 typedef void (*WholeKernel)(WholeArgs);

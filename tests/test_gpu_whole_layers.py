@@ -91,6 +91,40 @@ def test_largest_sizes_beside_f32(moon, ctx, which):
     assert_close(*out)
 
 
+# Layers without a window.  A session with room for so many keys that their splits' workgroups could fill the device takes three launches at every position.
+ROOM = {512: 170000, 1024: 84000, 2048: 40000}
+EVERYTHING = 10**6
+
+
+@pytest.mark.parametrize("width,heads,kv_heads,ff,design", [
+    (2048, 32, 32, 5504, "plain"), (2048, 32, 32, 10240, "plain"), (2048, 32, 32, None, "plain"), (1024, 16, 16, 2816, "plain"), (512, 8, 8, 192, "plain"),
+    (2048, 32, 32, 6464, "joined"), (2048, 32, 32, 320, "turned"), (1024, 16, 16, 1728, "joined"), (1024, 16, 16, 7168, "turned"), (512, 8, 8, 64, "joined")])
+def test_one_launch_and_three_give_the_same_bits(moon, ctx, width, heads, kv_heads, ff, design):
+    if design == "plain":
+        cfg = RM.config(128, width, [RM.layer(RM.attention(heads, kv_heads, 64, 64, EVERYTHING, 0.125, mix), RM.dense(ff) if ff else None) for mix in (False, True)], embed_scale=2.0)
+    elif design == "joined":
+        cfg = GM.config(128, width, [GM.parallel(GM.softmax_mixer(heads, kv_heads, 64, 64, EVERYTHING, 0.125), GM.delta(heads // 2, heads // 2, 64, 64, 4), ff)] * 2)
+    else:
+        cfg = GM.config(128, width, [GM.plain(GM.attention(heads, kv_heads, 64, 64, EVERYTHING, 0.125, ROT), ff)] * 2)
+    out, ids = [], RM.tokens(200, 128)
+    for max_seq in (256, ROOM[width]):
+        m = moon.text_model.TextModel.open_synthetic(cfg, "bfloat16", max_seq, seed=5, std=0.02, ctx=ctx)
+        rows = []
+        for prompt in (2, 31, 150): # (a prompt's products leave their own note)
+            m.reset()
+            m.forward(ids[:prompt])
+            for i in range(3):
+                m.forward(ids[prompt + i:prompt + i + 1])
+                if max_seq == 256:
+                    took_one_launch(ctx)
+                elif compute_units() == 256:
+                    assert not ctx.last_kernel().startswith("decode_whole")
+                rows.append(m.logits_f32())
+        m.close()
+        out.append(np.array(rows))
+    assert np.isfinite(out[0]).all() and np.array_equal(*(o.view(np.uint32) for o in out))
+
+
 @pytest.mark.parametrize("change", [dict(width=2112), dict(ff=10304), dict(dim=128), dict(experts=True)])
 def test_other_sizes_take_three_launches(moon, ctx, change):
     width, dim = change.get("width", 1024), change.get("dim", 64)
