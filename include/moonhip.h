@@ -352,8 +352,9 @@ int moon_text_greedy_profile(moon_text_model *m, size_t n_steps, uint32_t *out_i
  * 3 = two kernels per layer (LayerNorm + qkv + fc1 + attention; out_proj + fc2 + residual).  All modes produce the same
  * bits.  A wait that expires makes the call return MOON_EHIP.  Several contexts of one process may decode at once: a call
  * whose waiting workgroups would not leave the others' a place on the device runs as mode 2.  Other processes on the same
- * device are not counted: where several of them decode at once, ask for mode 2.  Decoders opened from a model folder have no
- * modes: they take one launch per layer or three by the same counting, and two processes' launches never hold each other up.
+ * device are not counted: where several of them decode at once, ask for mode 2.  Decoders opened from a model folder take modes
+ * 0 and 2, the same bits, where some of their layers can run as one kernel (bf16, heads of 57 to 64, no experts); the others
+ * never wait inside a kernel and refuse the call.
  * No counterpart in the reference. */
 int moon_text_set_decode_mode(moon_text_model *m, int mode);
 /* After a MOON_EHIP from moon_text_greedy / moon_text_sample caused by an expired wait inside a fused decode kernel the

@@ -17,8 +17,8 @@
 // Progress: producers never wait and come first in the grid, so on every die they have their places before any workgroup that waits; the
 // attention's workgroups wait for producers, the output's for both, in the grid's order (a merge also waits for the gate: producers again).  Workgroups of several launches could all the same fill the dies
 // with some that wait for another die's: calls take their places beforehand (wait_places.hpp) and run in three launches where there are
-// none.  Two launches that nobody counts together, of two processes, finish in any case: where one's producers or heads have no place on a die yet, none of its output workgroups is there, and
-// the other's waiting ones never fill a die (decode_whole_supported).  Every wait is bounded.
+// none.  Launches that nobody counts together, of several processes, are not kept apart so: each may hold the place that another's producers or heads need, and their
+// waits then run out.  Their sessions ask for three launches (moon_text_set_decode_mode).  Every wait is bounded.
 // Exchanged vectors are written through to memory; the attention reads what it needs of the projections past the dies' caches, the output
 // workgroups read the two long vectors through them (no line of either is read before its count is complete).
 #include "decode_roles.hpp"

@@ -84,7 +84,7 @@ struct moon_text_model {
     uint32_t *state_dev = nullptr; // [0] position (KV length), [1] tokens recorded, [2] current token, [3] stopped, [4] eos id + 1 (record_token)
     size_t cur_len = 0, last_n = 0;
     bool cache_invalid = false;    // a fused decode kernel gave up on a wait: positions may be missing from the cache until moon_text_reset
-    int decode_mode = 0;           // 0: one kernel per layer where the device holds it (default); 2: three kernels per layer; 3: two
+    int decode_mode = 0;           // 0: one kernel per layer where the device holds it (default); 2: three kernels per layer; 3: two (not of a list)
     int call_mode = 0;             // the same for the call that runs (DecodeCall)
     WaitNeed layer_wait, front_wait; // places that a call's whole-layer or front launches take
     float *attn_partial = nullptr; // [H][8][66]
@@ -308,7 +308,7 @@ struct DecodeCall {
     }
     explicit DecodeCall(moon_text_model *model) : m(model) {
         m->call_mode = m->decode_mode;
-        if (m->list) need = layer_list_wait_need(m->list);
+        if (m->list) need = m->call_mode == 0 ? layer_list_wait_need(m->list) : nullptr;
         else if (!m->fused) return;
         else if (m->whole_layer && m->call_mode == 0) need = &m->layer_wait;
         else if (m->front && m->call_mode != 2) need = &m->front_wait;
@@ -1126,7 +1126,8 @@ extern "C" int moon_text_debug_raise_wait_error(moon_text_model *m) {
 extern "C" int moon_text_set_decode_mode(moon_text_model *m, int mode) {
     if (!m) return MOON_EINVAL;
     std::lock_guard<std::mutex> lock(m->ctx->mu);
-    if (m->list) return refuse_list(m, "text_set_decode_mode");
+    if (m->list && !layer_list_wait_need(m->list)) return moon_fail(m->ctx, MOON_EINVAL, "text_set_decode_mode: no launch of this decoder waits, it has no modes");
+    if (m->list && mode != 0 && mode != 2) return moon_fail(m->ctx, MOON_EINVAL, "decode mode of a decoder opened from a model folder must be 0 (one kernel per layer) or 2 (three)");
     if (mode != 0 && mode != 2 && mode != 3)
         return moon_fail(m->ctx, MOON_EINVAL, "decode mode must be 0 (one kernel per layer), 2 (three kernels per layer) or 3 (two kernels per layer)");
     m->decode_mode = mode;

@@ -93,7 +93,8 @@ class TextModel:
 
     def set_decode_mode(self, mode: int):
         """0 (default): one fused kernel per layer; 2: three kernels per layer (no waits inside kernels); 3: two per layer.
-        Calls of several contexts at once run as 2 where the device cannot hold all that wait; several processes: ask for 2."""
+        Calls of several contexts at once run as 2 where the device cannot hold all that wait; several processes: ask for 2.
+        A decoder opened from a model folder takes 0 and 2 if any of its layers can run as one kernel (bf16, no experts), and none otherwise."""
         self.ctx.check(self.ctx.lib.moon_text_set_decode_mode(self.handle, mode))
 
     @property

@@ -91,38 +91,71 @@ def test_largest_sizes_beside_f32(moon, ctx, which):
     assert_close(*out)
 
 
-# Layers without a window.  A session with room for so many keys that their splits' workgroups could fill the device takes three launches at every position.
-ROOM = {512: 170000, 1024: 84000, 2048: 40000}
-EVERYTHING = 10**6
+def config_of(name):
+    """Configurations of the tests above and layers without a window, at every number of loads that a row takes: -> (configuration, made from weights of its own?)"""
+    if name in RIKANEX:
+        width, heads, kv_heads, ff, window = RIKANEX[name]
+        return RM.config(90, width, [RM.layer(RM.attention(heads, kv_heads, 63, 61, window, 0.13, mix), RM.dense(ff) if ff else None) for mix in (False, True, True)], embed_scale=2.0), True
+    if name.startswith("large"):
+        return LARGE[int(name[5:])], False
+    kind, width, heads, ff = name.split()
+    width, heads, ff = int(width), int(heads), int(ff) or None
+    whole = dict(window=10**6, scale=0.125)
+    if kind == "plain":
+        return RM.config(128, width, [RM.layer(RM.attention(heads, heads, 64, 64, v_mix=mix, **whole), RM.dense(ff) if ff else None) for mix in (False, True)], embed_scale=2.0), False
+    if kind == "joined":
+        return GM.config(128, width, [GM.parallel(GM.softmax_mixer(heads, heads, 64, 64, **whole), GM.delta(heads // 2, heads // 2, 64, 64, 4), ff)] * 2), False
+    if kind == "odd":
+        joined = GM.parallel(GM.softmax_mixer(heads, heads, 64, 64, 9, 0.13, 4), GM.delta(heads + 1, 1, 64, 64, 4), ff)
+        return GM.config(128, width, [joined, GM.plain(GM.attention(heads, 1, 60, 62, 20, 0.13, GM.rotation(32, 1e4)), ff), joined]), True
+    return GM.config(128, width, [GM.plain(GM.attention(heads, heads, 64, 64, rot=ROT, **whole), ff)] * 2), False
 
 
-@pytest.mark.parametrize("width,heads,kv_heads,ff,design", [
-    (2048, 32, 32, 5504, "plain"), (2048, 32, 32, 10240, "plain"), (2048, 32, 32, None, "plain"), (1024, 16, 16, 2816, "plain"), (512, 8, 8, 192, "plain"),
-    (2048, 32, 32, 6464, "joined"), (2048, 32, 32, 320, "turned"), (1024, 16, 16, 1728, "joined"), (1024, 16, 16, 7168, "turned"), (512, 8, 8, 64, "joined")])
-def test_one_launch_and_three_give_the_same_bits(moon, ctx, width, heads, kv_heads, ff, design):
-    if design == "plain":
-        cfg = RM.config(128, width, [RM.layer(RM.attention(heads, kv_heads, 64, 64, EVERYTHING, 0.125, mix), RM.dense(ff) if ff else None) for mix in (False, True)], embed_scale=2.0)
-    elif design == "joined":
-        cfg = GM.config(128, width, [GM.parallel(GM.softmax_mixer(heads, kv_heads, 64, 64, EVERYTHING, 0.125), GM.delta(heads // 2, heads // 2, 64, 64, 4), ff)] * 2)
+SAME = [*sorted(RIKANEX), *(f"large{i}" for i in range(len(LARGE))), "plain 2048 32 5504", "plain 2048 32 10240", "plain 2048 32 0", "plain 1024 16 2816", "plain 512 8 192", "joined 2048 32 6464",
+        "turned 2048 32 320", "joined 1024 16 1728", "turned 1024 16 7168", "joined 512 8 64", "odd 516 5 70", "odd 1084 9 321", "odd 320 2 0", "odd 1020 15 2050"]
+
+
+@pytest.mark.parametrize("name", SAME)
+def test_one_launch_and_three_give_the_same_bits(moon, ctx, tmp_path, name):
+    cfg, own = config_of(name)
+    if own:
+        weights = (RM if cfg["architecture"] == "Rikanex" else GM).weights(cfg, 3)
+        m = opened(moon, ctx, RM.write_folder(tmp_path / "m", cfg, weights), "bfloat16")
     else:
-        cfg = GM.config(128, width, [GM.plain(GM.attention(heads, kv_heads, 64, 64, EVERYTHING, 0.125, ROT), ff)] * 2)
-    out, ids = [], RM.tokens(200, 128)
-    for max_seq in (256, ROOM[width]):
-        m = moon.text_model.TextModel.open_synthetic(cfg, "bfloat16", max_seq, seed=5, std=0.02, ctx=ctx)
-        rows = []
-        for prompt in (2, 31, 150): # (a prompt's products leave their own note)
+        m = moon.text_model.TextModel.open_synthetic(cfg, "bfloat16", 512, seed=5, std=0.02, ctx=ctx)
+    rows, tokens, ids = {}, {}, RM.tokens(400, 90)
+    for mode in (0, 2):
+        m.set_decode_mode(mode)
+        rows[mode] = []
+        for prompt in (2, 31, 150, 390):
             m.reset()
             m.forward(ids[:prompt])
             for i in range(3):
                 m.forward(ids[prompt + i:prompt + i + 1])
-                if max_seq == 256:
+                if mode == 0:
                     took_one_launch(ctx)
-                elif compute_units() == 256:
-                    assert not ctx.last_kernel().startswith("decode_whole")
-                rows.append(m.logits_f32())
+                else:
+                    assert not ctx.last_kernel().startswith("decode_whole") # (the prompt's products have left their own note)
+                rows[mode].append(m.logits_f32())
+        tokens[mode] = m.greedy(20).tolist()
+        rows[mode].append(m.logits_f32())
+    m.close()
+    assert np.isfinite(rows[0]).all() and np.array_equal(*(np.array(rows[mode]).view(np.uint32) for mode in (0, 2)))
+    assert tokens[0] == tokens[2]
+
+
+def test_modes_of_list_decoders(moon, ctx):
+    """0 and 2 where a layer runs in one launch; none where no launch waits."""
+    dense, experts = (RM.config(128, 512, [RM.layer(RM.attention(8, 8, 64, 64, 40, 0.125), mlp)]) for mlp in (RM.dense(128), RM.moe(64, 8, 64)))
+    for cfg, dtype, modes in ((dense, "bfloat16", (0, 2)), (dense, "float32", ()), (experts, "bfloat16", ())):
+        m = moon.text_model.TextModel.open_synthetic(cfg, dtype, 64, seed=5, std=0.02, ctx=ctx)
+        for mode in range(-1, 5):
+            if mode in modes:
+                m.set_decode_mode(mode)
+            else:
+                with pytest.raises(moon.MoonError):
+                    m.set_decode_mode(mode)
         m.close()
-        out.append(np.array(rows))
-    assert np.isfinite(out[0]).all() and np.array_equal(*(o.view(np.uint32) for o in out))
 
 
 @pytest.mark.parametrize("change", [dict(width=2112), dict(ff=10304), dict(dim=128), dict(experts=True)])
