@@ -361,7 +361,7 @@ int moon_text_set_decode_mode(moon_text_model *m, int mode);
  * session refuses further forward / greedy / sample calls until moon_text_reset: workgroups that gave up may have skipped
  * the cache append of their position.  moon_text_reset then also restarts the kernels' counters.
  * moon_text_debug_raise_wait_error sets the error word those waits look at, as an expired wait does (a test hook for
- * that path; no counterpart in the reference, whose ops cannot fail this way). */
+ * that path; no counterpart in the reference, whose ops cannot fail this way; refused where no launch of the decoder waits). */
 int moon_text_debug_raise_wait_error(moon_text_model *m);
 /* current KV length */
 size_t moon_text_position(const moon_text_model *m);

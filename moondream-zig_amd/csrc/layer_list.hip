@@ -935,17 +935,20 @@ static int plan_whole(LayerList *l) {
 
 const WaitNeed *layer_list_wait_need(const LayerList *l) { return l->any_whole ? &l->whole_need : nullptr; }
 
-bool layer_list_wait_failed(LayerList *l) {
-    if (!l->any_whole || !*(volatile uint32_t *)l->whole.error) return false;
-    // workgroups that gave up have counted nothing
-    (void)launch_fill_uniform_u32(l->ctx, l->whole.sync, decode_whole_sync_words(), 0, 0, 1);
-    (void)launch_fill_uniform_u32(l->ctx, l->counter, l->counters, 0, 0, 1);
-    (void)hipStreamSynchronize(l->ctx->stream);
+bool layer_list_wait_failed(const LayerList *l) { return l->any_whole && *(volatile uint32_t *)l->whole.error; }
+
+int layer_list_clear_waits(LayerList *l) {
+    if (!l->any_whole) return MOON_OK;
+    MOON_TRY(launch_fill_uniform_u32(l->ctx, l->whole.sync, decode_whole_sync_words(), 0, 0, 1));
+    MOON_TRY(launch_fill_uniform_u32(l->ctx, l->counter, l->counters, 0, 0, 1));
+    MOON_HIP(l->ctx, hipStreamSynchronize(l->ctx->stream)); // (no launch reads the error word any more)
     std::fill(l->whole.leaf, l->whole.leaf + 2, 0u);
     std::fill(l->whole.reached, l->whole.reached + 3, 0u);
     *(volatile uint32_t *)l->whole.error = 0;
-    return true;
+    return MOON_OK;
 }
+
+void layer_list_raise_wait_error(LayerList *l) { *(volatile uint32_t *)l->whole.error = 1; }
 
 int layer_list_step(LayerList *l, const uint32_t *token_dev, size_t pos, const uint32_t *pos_dev, bool whole) {
     moon_ctx *ctx = l->ctx;

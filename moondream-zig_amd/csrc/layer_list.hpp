@@ -348,8 +348,10 @@ int layer_list_forward(LayerList *l, const uint32_t *ids_dev, size_t n, size_t p
 // where that can be, with the places of layer_list_wait_need taken
 int layer_list_step(LayerList *l, const uint32_t *token_dev, size_t pos, const uint32_t *pos_dev, bool whole);
 const WaitNeed *layer_list_wait_need(const LayerList *l); // null: no layer runs in one launch
-// behind a drained stream: has a wait run out of time?  Its counters are then ready again, the sequence's caches are not
-bool layer_list_wait_failed(LayerList *l);
+// behind a drained stream: has a wait run out of time?  Then workgroups that gave up have counted nothing and the sequence's caches may lack rows
+bool layer_list_wait_failed(const LayerList *l);
+int layer_list_clear_waits(LayerList *l); // counters, targets and the error word start over together, or on an error none of the last two
+void layer_list_raise_wait_error(LayerList *l); // as a wait that runs out (some layer runs in one launch)
 // logits of the given rows of x (host list of n <= LIST_LOGIT_ROWS) -> *logits, [n][*ld] f32 on the device
 int layer_list_logits(LayerList *l, const uint32_t *rows, size_t n, const float **logits, size_t *ld);
 const float *layer_list_hidden(const LayerList *l); // [rows][width] on the device

@@ -589,7 +589,7 @@ extern "C" int moon_text_reset(moon_text_model *m) {
     m->cur_len = 0;
     m->last_n = 0;
     MOON_HIP(m->ctx, hipSetDevice(m->ctx->device));
-    if (m->cache_invalid && !m->list) MOON_TRY(clear_sync_state(m)); // after a failed wait: counters and targets start over together
+    if (m->cache_invalid) MOON_TRY(m->list ? layer_list_clear_waits(m->list) : clear_sync_state(m)); // after a failed wait: counters and targets start over together
     m->cache_invalid = false;
     hipLaunchKernelGGL(set_state_kernel, dim3(1), dim3(1), 0, m->ctx->stream, m->state_dev, 0u, 0u);
     MOON_HIP(m->ctx, hipGetLastError());
@@ -1112,7 +1112,11 @@ extern "C" int moon_text_debug_raise_wait_error(moon_text_model *m) {
     if (!m) return MOON_EINVAL;
     moon_ctx *ctx = m->ctx;
     std::lock_guard<std::mutex> lock(ctx->mu);
-    if (m->list) return refuse_list(m, "text_debug_raise_wait_error");
+    if (m->list) {
+        if (!layer_list_wait_need(m->list)) return moon_fail(ctx, MOON_EINVAL, "text_debug_raise_wait_error: no launch of this decoder waits");
+        layer_list_raise_wait_error(m->list);
+        return MOON_OK;
+    }
     const Sizes z = sizes(m->cfg);
     MOON_HIP(ctx, hipSetDevice(ctx->device));
     // the word before each error word is unused (the tail of a counter line, or of the last counter copy): writes {0, 1} to (tail, error word)

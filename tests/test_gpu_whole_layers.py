@@ -158,6 +158,45 @@ def test_modes_of_list_decoders(moon, ctx):
         m.close()
 
 
+@pytest.mark.parametrize("name", ["plain 1024 16 2816", "joined 2048 32 6464"])
+def test_failed_wait_and_recovery(moon, ctx, name):
+    """The error word of the waits raised from the host (every kernel still runs to its end): the call fails, the position stays, work is refused until reset, and behind it
+    the session has the bits of a fresh one."""
+    cfg, _ = config_of(name)
+    ids = RM.tokens(60, 128)
+
+    def session():
+        return moon.text_model.TextModel.open_synthetic(cfg, "bfloat16", 256, seed=5, std=0.02, ctx=ctx)
+
+    def work(m):
+        m.forward(ids[:40])
+        m.forward(ids[40:41])
+        row = m.logits_f32()
+        return m.greedy(6).tolist(), row.view(np.uint32).tolist(), m.logits_f32().view(np.uint32).tolist()
+
+    m = session()
+    want = work(m)
+    m.close()
+    m = session()
+    for call in (lambda: m.forward(ids[40:41]), lambda: m.greedy(3), lambda: m.generate(9, 1), lambda: m.forward_logits(ids[40:41], [0])):
+        m.forward(ids[:40])
+        ctx.check(ctx.lib.moon_text_debug_raise_wait_error(m.handle))
+        with pytest.raises(moon.context.HipError):
+            call()
+        assert m.position == 40
+        for refused in (lambda: m.forward(ids[:1]), lambda: m.forward(ids[:5]), lambda: m.greedy(1)):
+            with pytest.raises(moon.context.HipError):
+                refused()
+        m.reset()
+        assert m.position == 0 and work(m) == want
+        m.reset()
+    m.close()
+    m = moon.text_model.TextModel.open_synthetic(cfg, "float32", 64, seed=5, std=0.02, ctx=ctx)
+    with pytest.raises(moon.MoonError):
+        ctx.check(ctx.lib.moon_text_debug_raise_wait_error(m.handle))
+    m.close()
+
+
 @pytest.mark.parametrize("change", [dict(width=2112), dict(ff=10304), dict(dim=128), dict(experts=True)])
 def test_other_sizes_take_three_launches(moon, ctx, change):
     width, dim = change.get("width", 1024), change.get("dim", 64)
