@@ -942,8 +942,7 @@ int layer_list_clear_waits(LayerList *l) {
     MOON_TRY(launch_fill_uniform_u32(l->ctx, l->whole.sync, decode_whole_sync_words(), 0, 0, 1));
     MOON_TRY(launch_fill_uniform_u32(l->ctx, l->counter, l->counters, 0, 0, 1));
     MOON_HIP(l->ctx, hipStreamSynchronize(l->ctx->stream)); // (no launch reads the error word any more)
-    std::fill(l->whole.leaf, l->whole.leaf + 2, 0u);
-    std::fill(l->whole.reached, l->whole.reached + 3, 0u);
+    l->whole.at = LaunchTargets{};
     *(volatile uint32_t *)l->whole.error = 0;
     return MOON_OK;
 }

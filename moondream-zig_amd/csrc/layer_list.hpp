@@ -6,6 +6,7 @@
 #include <string>
 #include <vector>
 
+#include "launch_counts.hpp"
 #include "moon_internal.hpp"
 #include "wait_places.hpp"
 
@@ -323,7 +324,7 @@ int launch_decode_out(moon_ctx *ctx, int dtype, const DecodeOut &p);
 struct WholeCounts {          // counters of a session's launches, which all use the same: what they have counted to so far
     uint32_t *sync = nullptr; // decode_whole_sync_words
     uint32_t *error = nullptr; // page-locked: not zero once a wait has run out of time
-    uint32_t leaf[2] = {}, reached[3] = {};
+    LaunchTargets at;
 };
 size_t decode_whole_sync_words();
 // Can this layer run so, at every position below max_seq?  per_cu: workgroups of its launch that a compute unit holds; need: the places that it takes

@@ -48,7 +48,7 @@ struct WholeArgs {
     int S, keys_max, n_prod, n_attn;
     int front16;              // rows of the 16-bit segment that the heads begin with; the gate's behind them come with the activation
     uint32_t *sync, *error;
-    uint32_t leaf[2], reached[WHOLE_COUNTS]; // what the leaves and the copies count to
+    LaunchTargets at;         // what the leaves and the copies count to
 };
 
 __device__ __forceinline__ uint32_t *whole_copy(const WholeArgs &a, int which, int i) { return a.sync + WHOLE_COPIES_AT + (which * LAYER_COPIES + i) * LAYER_COPY_STRIDE; }
@@ -58,10 +58,10 @@ struct Within {
     const WholeArgs &a;
     int *s_flag;
     __device__ __forceinline__ bool wait() const {
-        return wait_reached(whole_copy(a, WHOLE_FRONT, blockIdx.x % LAYER_COPIES), a.reached[WHOLE_FRONT], a.error, s_flag);
+        return wait_reached(whole_copy(a, WHOLE_FRONT, blockIdx.x % LAYER_COPIES), a.at.reached[WHOLE_FRONT], a.error, s_flag);
     }
     __device__ __forceinline__ bool wait_gate() const {
-        return a.front16 == a.p.n16_used || wait_reached(whole_copy(a, WHOLE_ACT, blockIdx.x % LAYER_COPIES), a.reached[WHOLE_ACT], a.error, s_flag);
+        return a.front16 == a.p.n16_used || wait_reached(whole_copy(a, WHOLE_ACT, blockIdx.x % LAYER_COPIES), a.at.reached[WHOLE_ACT], a.error, s_flag);
     }
     __device__ __forceinline__ void done() const {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // the heads are stored
@@ -77,7 +77,7 @@ __device__ __forceinline__ void whole_report(const WholeArgs &a, int phase) {
     if (threadIdx.x >= 64) return;
     int full = 0;
     if (threadIdx.x == 0)
-        full = __hip_atomic_fetch_add(a.sync + (phase * WHOLE_LEAVES + blockIdx.x % WHOLE_LEAVES) * LAYER_LINE, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 == a.leaf[phase];
+        full = __hip_atomic_fetch_add(a.sync + (phase * WHOLE_LEAVES + blockIdx.x % WHOLE_LEAVES) * LAYER_LINE, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 == a.at.leaf[phase];
     if (__builtin_amdgcn_readfirstlane(full)) __hip_atomic_fetch_add(whole_copy(a, phase, threadIdx.x), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
@@ -219,7 +219,7 @@ template <int QW, bool DELTA> __device__ __forceinline__ void whole_output(const
                 }
             }
         }
-        if (!wait_reached(whole_copy(a, WHOLE_ACT, b), a.reached[WHOLE_ACT], a.error, s_flag)) return;
+        if (!wait_reached(whole_copy(a, WHOLE_ACT, b), a.at.reached[WHOLE_ACT], a.error, s_flag)) return;
         const auto act = stretch(reinterpret_cast<const T *>(o.a) + o.k2, n_f);
         auto copy = [&](auto from, auto to) { // the vector as the lanes meet it, 4 KiB a step, all requested before any is waited for
             constexpr int FROM = decltype(from)::value, N = decltype(to)::value - FROM;
@@ -250,7 +250,7 @@ template <int QW, bool DELTA> __device__ __forceinline__ void whole_output(const
             dot_f[r] = quarters_sum(part, lane);
         }
     }
-    if (!wait_reached(whole_copy(a, WHOLE_HEADS, b), a.reached[WHOLE_HEADS], a.error, s_flag)) return;
+    if (!wait_reached(whole_copy(a, WHOLE_HEADS, b), a.at.reached[WHOLE_HEADS], a.error, s_flag)) return;
     const auto heads = stretch(o.a, n_h);
     lm_u32x4 xh[QW];
     if (fresh && !o.y)
@@ -355,19 +355,25 @@ int launch_decode_whole(moon_ctx *ctx, const DecodeProj &p, const DecodeMix &m, 
     MOON_TRY(check_decode_mix(ctx, m));
     WholePlan w;
     if (!whole_plan(ctx, p, m, o, mix_keys(m, m.pos), per_cu, &w)) return moon_fail(ctx, MOON_EINVAL, "decode: a layer that does not run in one launch");
-    counts->leaf[WHOLE_FRONT] += w.n_prod / WHOLE_LEAVES;
-    counts->reached[WHOLE_FRONT] += WHOLE_LEAVES;
     const int front16 = m.gate && !m.dH ? m.og : p.n16_used; // (a delta rule's columns come behind the gate's)
+    LaunchTargets next = counts->at;
+    next.leaf[WHOLE_FRONT] += w.n_prod / WHOLE_LEAVES;
+    next.reached[WHOLE_FRONT] += WHOLE_LEAVES;
     if (p.ff || front16 < p.n16_used) {
-        counts->leaf[WHOLE_ACT] += w.n_prod / WHOLE_LEAVES;
-        counts->reached[WHOLE_ACT] += WHOLE_LEAVES;
+        next.leaf[WHOLE_ACT] += w.n_prod / WHOLE_LEAVES;
+        next.reached[WHOLE_ACT] += WHOLE_LEAVES;
     }
-    counts->reached[WHOLE_HEADS] += w.merges;
-    WholeArgs a{p, m, o, w.S, w.keys_max, w.n_prod, w.n_attn, front16, counts->sync, counts->error, {}, {}};
-    std::copy(counts->leaf, counts->leaf + 2, a.leaf);
-    std::copy(counts->reached, counts->reached + WHOLE_COUNTS, a.reached);
+    next.reached[WHOLE_HEADS] += w.merges;
+    auto launch = [&]() -> int {
+        hipLaunchKernelGGL(w.kern, dim3(w.grid), dim3(256), w.lds, ctx->stream, WholeArgs{p, m, o, w.S, w.keys_max, w.n_prod, w.n_attn, front16, counts->sync, counts->error, next});
+        MOON_HIP(ctx, hipGetLastError());
+        return MOON_OK;
+    };
+    auto clear = [&]() -> int {
+        if (launch_fill_uniform_u32(ctx, counts->sync, decode_whole_sync_words(), 0, 0, 1) != MOON_OK) return MOON_EHIP;
+        return hipStreamSynchronize(ctx->stream) == hipSuccess ? MOON_OK : MOON_EHIP;
+    };
+    MOON_TRY(launch_counted(&counts->at, next, counts->error, launch, clear));
     MOON_NOTE_KERNEL(ctx, "decode_whole_kernel %d splits of the keys", w.S);
-    hipLaunchKernelGGL(w.kern, dim3(w.grid), dim3(256), w.lds, ctx->stream, a);
-    MOON_HIP(ctx, hipGetLastError());
     return MOON_OK;
 }

@@ -119,3 +119,8 @@ def test_choice_of_the_product_tiles():
 def test_places_of_waiting_workgroups():
     """csrc/wait_places.hpp on the host: the decode calls that may be in flight on a device at once, from several contexts and threads."""
     _host_check("wait_places")
+
+
+def test_counts_of_launches_that_wait():
+    """csrc/launch_counts.hpp on the host: counters and targets agree behind launches that ran, that did not, and that reported an earlier call's error."""
+    _host_check("launch_counts")
