@@ -162,7 +162,7 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t stretch(const void *p, int byt
 // 2 (c % 2) + w, which is lane 32 (c / 2 % 2) + j there.  So a lane keeps four sums, element c % 4, and quarters_sum adds them up.
 // A token takes 1 % longer than with whole KiB in any order (24 layers of width 2048, feed-forward 5504 598 us against 590, 12 of 32 key heads 335 against 333, width
 // 1024 382 against 381).  Measured and not kept: loads of 64 pieces of one quarter (597, 340, 385), of 16 of each (599, 336, 400); whole KiB, their dots turned by
-// ds_bpermute where a quarter ends (648, 360, 435) or through LDS (596, 338, 386, and 368 in place of 360 for 12 joined layers of width 2048).
+// ds_bpermute where a quarter ends (648, 360, 435) or through LDS (596, 338, 386).
 constexpr int NOWHERE = 1 << 30; // no buffer is as long: loads zeros
 struct Quarters {
     int pieces, mine, at; // of a quarter; this lane's first; its byte
@@ -175,7 +175,8 @@ struct Quarters {
 
 // QW: loads of a row's part for the heads, of which the delta rule's come behind the attention's.  A wavefront owns WHOLE_ROWS rows: their parts for the
 // heads and the beginning of the first one's for the dense activation (HOLD loads) are in registers by the time that the activation is there, the rest streams
-// while the attention is still under way.
+// while the attention is still under way.  Where eight loads a row are for the heads, the second row's come behind the dense activation's: with both from the start, up to 24 registers lay in scratch (12
+// layers of width 2048, joined and rotated in turn, 380 us a token in place of 358), or a unit held three workgroups in place of four (6 joined layers of 32 key heads behind 300 keys 261 in place of 207).
 template <int QW, bool DELTA> __device__ __forceinline__ void whole_output(const WholeArgs &a, int wg, int n_wgs, char *lds, int *s_flag) {
     typedef bf16_t T;
     constexpr int R = WHOLE_ROWS, HOLD = QW > 4 ? 8 : WHOLE_HELD;
@@ -189,13 +190,19 @@ template <int QW, bool DELTA> __device__ __forceinline__ void whole_output(const
     auto weights = [&](int r, int column, int bytes) { return stretch(reinterpret_cast<const T *>(o.w2) + size_t(row(r)) * o.k0 + column, bytes); };
     lm_u32x4 wh[R][QW], wf[HOLD];
     float old[R];
+    const bool more = QW > 4 && h.pieces > 64; // than four loads (6 rotated layers of width 2048, 32 key heads, 300 keys 182 -> 176 us)
+    auto heads_weights = [&](int r) {
+        const auto w = weights(r, 0, n_h);
+#pragma unroll
+        for (int c = 0; c < QW; c++)
+            if (c < 4 || more) wh[r][c] = h.load<LOAD_STREAM>(w, c);
+    };
+    constexpr int EARLY = QW > 4 ? 1 : R;
 #pragma unroll
     for (int r = 0; r < R; r++) {
-        const auto w = weights(r, 0, n_h);
         old[r] = 0.0f;
         if (!fresh && !o.y && row(r) < o.width) old[r] = o.x[row(r)];
-#pragma unroll
-        for (int c = 0; c < QW; c++) wh[r][c] = h.load<LOAD_STREAM>(w, c);
+        if (r < EARLY) heads_weights(r);
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     float dot_f[R] = {};
@@ -250,6 +257,8 @@ template <int QW, bool DELTA> __device__ __forceinline__ void whole_output(const
             dot_f[r] = quarters_sum(part, lane);
         }
     }
+#pragma unroll
+    for (int r = EARLY; r < R; r++) heads_weights(r);
     if (!wait_reached(whole_copy(a, WHOLE_HEADS, b), a.at.reached[WHOLE_HEADS], a.error, s_flag)) return;
     const auto heads = stretch(o.a, n_h);
     lm_u32x4 xh[QW];
@@ -258,18 +267,20 @@ template <int QW, bool DELTA> __device__ __forceinline__ void whole_output(const
         for (int r = 0; r < R; r++)
             if (row(r) < o.width) old[r] = ld_f<true>(o.x + row(r));
 #pragma unroll
-    for (int c = 0; c < QW; c++) xh[c] = h.load<LOAD_DIE>(heads, c);
+    for (int c = 0; c < QW; c++)
+        if (c < 4 || more) xh[c] = h.load<LOAD_DIE>(heads, c);
 #pragma unroll
     for (int r = 0; r < R; r++) {
         const int n = row(r);
         float part[4] = {0.0f, 0.0f, 0.0f, 0.0f}, part_d[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int c = 0; c < QW; c++) {
-            const float d = dot_piece<T>(wh[r][c], xh[c], 0.0f);
-            const bool delta = DELTA && h.piece(c) >= o.k1 / 8; // (no layer without a delta rule has columns there)
-            part[c % 4] += delta ? 0.0f : d;
-            if (DELTA) part_d[c % 4] += delta ? d : 0.0f;
-        }
+        for (int c = 0; c < QW; c++)
+            if (c < 4 || more) {
+                const float d = dot_piece<T>(wh[r][c], xh[c], 0.0f);
+                const bool delta = DELTA && h.piece(c) >= o.k1 / 8; // (no layer without a delta rule has columns there)
+                part[c % 4] += delta ? 0.0f : d;
+                if (DELTA) part_d[c % 4] += delta ? d : 0.0f;
+            }
         const float dot = quarters_sum(part, lane), dot_d = DELTA ? quarters_sum(part_d, lane) : 0.0f;
         if (lane || n >= o.width) continue;
         if (o.y) {
@@ -280,10 +291,8 @@ template <int QW, bool DELTA> __device__ __forceinline__ void whole_output(const
     }
 }
 
-// Workgroups a unit: what the registers allow without scratch (wide layers with the mechanisms of WHOLE hold 64 of them for two rows' heads: 12 such layers of
-// width 2048 took 380 us a token with four a unit and up to 24 registers in scratch, 360 with three).
 template <int NH, int U, bool WHOLE>
-__global__ __launch_bounds__(256, NH > 4 || (WHOLE && U > 2) ? 3 : U > 2 || WHOLE ? 4 : 5) void decode_whole_kernel(WholeArgs) {
+__global__ __launch_bounds__(256, NH > 4 ? 3 : U > 2 || WHOLE ? 4 : 5) void decode_whole_kernel(WholeArgs) {
     const WholeArgs &a = fetch_arguments<WholeArgs>();
     extern __shared__ __attribute__((aligned(16))) char s_whole[];
     __shared__ float s_red[16];
