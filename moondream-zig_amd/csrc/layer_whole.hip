@@ -259,7 +259,10 @@ template <int QW, bool DELTA> __device__ __forceinline__ void whole_output(const
     }
 #pragma unroll
     for (int r = EARLY; r < R; r++) heads_weights(r);
-    if (!wait_reached(whole_copy(a, WHOLE_HEADS, b), a.at.reached[WHOLE_HEADS], a.error, s_flag)) return;
+    // Without a feed-forward the workgroup has nothing to stream and polls from the start of the launch: with pauses 12 layers of width 1024, 4 key heads take 187 us a token in
+    // place of 299 (217 in three launches), 6 of width 2048, 8 key heads 124 in place of 239 (147), joined ones 172 in place of 280; pauses of 2 units are too short
+    // (12 joined layers 265 in place of 221), of 16 and 32 cost 1 and 3 %.
+    if (!wait_reached(whole_copy(a, WHOLE_HEADS, b), a.at.reached[WHOLE_HEADS], a.error, s_flag, !n_f)) return;
     const auto heads = stretch(o.a, n_h);
     lm_u32x4 xh[QW];
     if (fresh && !o.y)
