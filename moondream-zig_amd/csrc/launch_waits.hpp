@@ -14,19 +14,19 @@ constexpr int LAYER_LINE = 32;                       // uint32 per 128-byte line
 // channels interleave by 256 bytes or by pages.
 constexpr int LAYER_COPIES = 64;
 constexpr int LAYER_COPY_STRIDE = 1088;
-constexpr int WAIT_PAUSE = 8; // units of 64 cycles
 constexpr long long FRONT_TIMEOUT_TICKS = 100000000LL; // 1 s of the 100 MHz wall clock
 
 // thread 0 of the workgroup polls *word until it reaches target; the clock and the error word are looked at once in
-// 64 polls.  Returns (to every thread) whether the wait succeeded.  pause: WAIT_PAUSE lies between two polls.
-__device__ __forceinline__ bool wait_reached(uint32_t *word, uint32_t target, uint32_t *error, int *s_flag, bool pause = false) {
+// 64 polls.  Returns (to every thread) whether the wait succeeded.  report: for the host, written only where a wait fails.
+// error lies in the device's memory: with hundreds of workgroups that looked at a page-locked word, any wait of more than 64 polls (about 20 us) became some 10 us longer
+// (list decoders' layers in one launch: 12 without a feed-forward, width 1024 299 us a token in place of 189, 4 behind 5,000 keys 146 in place of 106).
+__device__ __forceinline__ bool wait_reached(uint32_t *word, uint32_t target, uint32_t *error, int *s_flag, uint32_t *report = nullptr) {
     lds_barrier();
     if (threadIdx.x == 0) {
         const long long t0 = wall_clock64();
         int ok = 1;
         for (unsigned polls = 1;; polls++) {
             if ((int)(__hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - target) >= 0) break; // (a count may wrap)
-            if (pause) __builtin_amdgcn_s_sleep(WAIT_PAUSE);
             if ((polls & 63u) == 0) {
                 if (__hip_atomic_load(error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
                     ok = 0;
@@ -39,6 +39,7 @@ __device__ __forceinline__ bool wait_reached(uint32_t *word, uint32_t target, ui
                 }
             }
         }
+        if (!ok && report) __hip_atomic_store(report, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         *s_flag = ok;
     }
     lds_barrier();

@@ -947,7 +947,12 @@ int layer_list_clear_waits(LayerList *l) {
     return MOON_OK;
 }
 
-void layer_list_raise_wait_error(LayerList *l) { *(volatile uint32_t *)l->whole.error = 1; }
+int layer_list_raise_wait_error(LayerList *l) {
+    *(volatile uint32_t *)l->whole.error = 1;
+    MOON_HIP(l->ctx, hipMemcpyAsync(l->whole.sync + decode_whole_sync_words() - 1, l->whole.error, sizeof(uint32_t), hipMemcpyHostToDevice, l->ctx->stream));
+    MOON_HIP(l->ctx, hipStreamSynchronize(l->ctx->stream));
+    return MOON_OK;
+}
 
 int layer_list_step(LayerList *l, const uint32_t *token_dev, size_t pos, const uint32_t *pos_dev, bool whole) {
     moon_ctx *ctx = l->ctx;

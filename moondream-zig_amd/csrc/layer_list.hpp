@@ -322,8 +322,8 @@ int launch_decode_out(moon_ctx *ctx, int dtype, const DecodeOut &p);
 
 // ---- the same in one launch (layer_whole.hip), whose workgroups wait for each other
 struct WholeCounts {          // counters of a session's launches, which all use the same: what they have counted to so far
-    uint32_t *sync = nullptr; // decode_whole_sync_words
-    uint32_t *error = nullptr; // page-locked: not zero once a wait has run out of time
+    uint32_t *sync = nullptr; // decode_whole_sync_words, the last of them not zero once a wait has run out of time: those that wait look at it
+    uint32_t *error = nullptr; // page-locked: the same for the host
     LaunchTargets at;
 };
 size_t decode_whole_sync_words();
@@ -352,7 +352,7 @@ const WaitNeed *layer_list_wait_need(const LayerList *l); // null: no layer runs
 // behind a drained stream: has a wait run out of time?  Then workgroups that gave up have counted nothing and the sequence's caches may lack rows
 bool layer_list_wait_failed(const LayerList *l);
 int layer_list_clear_waits(LayerList *l); // counters, targets and the error word start over together, or on an error none of the last two
-void layer_list_raise_wait_error(LayerList *l); // as a wait that runs out (some layer runs in one launch)
+int layer_list_raise_wait_error(LayerList *l); // as a wait that runs out (some layer runs in one launch)
 // logits of the given rows of x (host list of n <= LIST_LOGIT_ROWS) -> *logits, [n][*ld] f32 on the device
 int layer_list_logits(LayerList *l, const uint32_t *rows, size_t n, const float **logits, size_t *ld);
 const float *layer_list_hidden(const LayerList *l); // [rows][width] on the device

@@ -47,21 +47,24 @@ struct WholeArgs {
     DecodeOut o;
     int S, keys_max, n_prod, n_attn;
     int front16;              // rows of the 16-bit segment that the heads begin with; the gate's behind them come with the activation
-    uint32_t *sync, *error;
+    uint32_t *sync, *report;
     LaunchTargets at;         // what the leaves and the copies count to
 };
 
 __device__ __forceinline__ uint32_t *whole_copy(const WholeArgs &a, int which, int i) { return a.sync + WHOLE_COPIES_AT + (which * LAYER_COPIES + i) * LAYER_COPY_STRIDE; }
+
+constexpr int WHOLE_ERROR_AT = WHOLE_COPIES_AT + WHOLE_COUNTS * LAYER_COPIES * LAYER_COPY_STRIDE; // in a line of its own
+__device__ __forceinline__ uint32_t *whole_error(const WholeArgs &a) { return a.sync + WHOLE_ERROR_AT; }
 
 struct Within {
     static constexpr bool SHARED = true;
     const WholeArgs &a;
     int *s_flag;
     __device__ __forceinline__ bool wait() const {
-        return wait_reached(whole_copy(a, WHOLE_FRONT, blockIdx.x % LAYER_COPIES), a.at.reached[WHOLE_FRONT], a.error, s_flag);
+        return wait_reached(whole_copy(a, WHOLE_FRONT, blockIdx.x % LAYER_COPIES), a.at.reached[WHOLE_FRONT], whole_error(a), s_flag, a.report);
     }
     __device__ __forceinline__ bool wait_gate() const {
-        return a.front16 == a.p.n16_used || wait_reached(whole_copy(a, WHOLE_ACT, blockIdx.x % LAYER_COPIES), a.at.reached[WHOLE_ACT], a.error, s_flag);
+        return a.front16 == a.p.n16_used || wait_reached(whole_copy(a, WHOLE_ACT, blockIdx.x % LAYER_COPIES), a.at.reached[WHOLE_ACT], whole_error(a), s_flag, a.report);
     }
     __device__ __forceinline__ void done() const {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // the heads are stored
@@ -226,7 +229,7 @@ template <int QW, bool DELTA> __device__ __forceinline__ void whole_output(const
                 }
             }
         }
-        if (!wait_reached(whole_copy(a, WHOLE_ACT, b), a.at.reached[WHOLE_ACT], a.error, s_flag)) return;
+        if (!wait_reached(whole_copy(a, WHOLE_ACT, b), a.at.reached[WHOLE_ACT], whole_error(a), s_flag, a.report)) return;
         const auto act = stretch(reinterpret_cast<const T *>(o.a) + o.k2, n_f);
         auto copy = [&](auto from, auto to) { // the vector as the lanes meet it, 4 KiB a step, all requested before any is waited for
             constexpr int FROM = decltype(from)::value, N = decltype(to)::value - FROM;
@@ -259,10 +262,7 @@ template <int QW, bool DELTA> __device__ __forceinline__ void whole_output(const
     }
 #pragma unroll
     for (int r = EARLY; r < R; r++) heads_weights(r);
-    // Without a feed-forward the workgroup has nothing to stream and polls from the start of the launch: with pauses 12 layers of width 1024, 4 key heads take 187 us a token in
-    // place of 299 (217 in three launches), 6 of width 2048, 8 key heads 124 in place of 239 (147), joined ones 172 in place of 280; pauses of 2 units are too short
-    // (12 joined layers 265 in place of 221), of 16 and 32 cost 1 and 3 %.
-    if (!wait_reached(whole_copy(a, WHOLE_HEADS, b), a.at.reached[WHOLE_HEADS], a.error, s_flag, !n_f)) return;
+    if (!wait_reached(whole_copy(a, WHOLE_HEADS, b), a.at.reached[WHOLE_HEADS], whole_error(a), s_flag, a.report)) return;
     const auto heads = stretch(o.a, n_h);
     lm_u32x4 xh[QW];
     if (fresh && !o.y)
@@ -351,7 +351,7 @@ bool whole_plan(moon_ctx *ctx, const DecodeProj &p, const DecodeMix &m, const De
 
 } // namespace
 
-size_t decode_whole_sync_words() { return WHOLE_COPIES_AT + size_t(WHOLE_COUNTS) * LAYER_COPIES * LAYER_COPY_STRIDE; }
+size_t decode_whole_sync_words() { return WHOLE_ERROR_AT + 1; }
 
 bool decode_whole_supported(moon_ctx *ctx, int dtype, const DecodeProj &p, const DecodeMix &m, const DecodeOut &o, size_t max_seq, int *per_cu, WaitNeed *need) {
     const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256;

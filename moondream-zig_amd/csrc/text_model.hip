@@ -1114,8 +1114,8 @@ extern "C" int moon_text_debug_raise_wait_error(moon_text_model *m) {
     std::lock_guard<std::mutex> lock(ctx->mu);
     if (m->list) {
         if (!layer_list_wait_need(m->list)) return moon_fail(ctx, MOON_EINVAL, "text_debug_raise_wait_error: no launch of this decoder waits");
-        layer_list_raise_wait_error(m->list);
-        return MOON_OK;
+        MOON_HIP(ctx, hipSetDevice(ctx->device));
+        return layer_list_raise_wait_error(m->list);
     }
     const Sizes z = sizes(m->cfg);
     MOON_HIP(ctx, hipSetDevice(ctx->device));
