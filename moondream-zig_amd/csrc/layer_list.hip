@@ -961,10 +961,9 @@ int layer_list_step(LayerList *l, const uint32_t *token_dev, size_t pos, const u
     TokenAt at(l);
     for (size_t i = 0; i < l->layers.size(); i++) {
         const TokenArgs t = token_args(l, i, at, token_dev, pos, pos_dev);
-        if (whole && l->any_whole && l->whole_per_cu[i]) {
-            MOON_TRY(launch_decode_whole(ctx, t.p, t.x, t.o, l->whole_per_cu[i], &l->whole));
-            continue;
-        }
+        bool launched = false;
+        if (whole && l->any_whole && l->whole_per_cu[i]) MOON_TRY(launch_decode_whole(ctx, t.p, t.x, t.o, l->whole_per_cu[i], &l->whole, &launched));
+        if (launched) continue;
         MOON_TRY(launch_decode_proj(ctx, dt, t.p));
         MOON_TRY(launch_decode_mix(ctx, dt, t.x, t.o));
         MOON_TRY(launch_decode_out(ctx, dt, t.o));

@@ -329,7 +329,8 @@ struct WholeCounts {          // counters of a session's launches, which all use
 size_t decode_whole_sync_words();
 // Can this layer run so, at every position below max_seq?  per_cu: workgroups of its launch that a compute unit holds; need: the places that it takes
 bool decode_whole_supported(moon_ctx *ctx, int dtype, const DecodeProj &p, const DecodeMix &m, const DecodeOut &o, size_t max_seq, int *per_cu, WaitNeed *need);
-int launch_decode_whole(moon_ctx *ctx, const DecodeProj &p, const DecodeMix &m, const DecodeOut &o, int per_cu, WholeCounts *counts);
+// launched: false where three launches are faster at this position, and nothing is launched
+int launch_decode_whole(moon_ctx *ctx, const DecodeProj &p, const DecodeMix &m, const DecodeOut &o, int per_cu, WholeCounts *counts, bool *launched);
 
 // ---- the engine (layer_list.hip): weights, caches and buffers of one sequence's session, prompt rows and single tokens
 struct LayerList;

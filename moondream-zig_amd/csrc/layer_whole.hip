@@ -24,6 +24,7 @@
 #include "decode_roles.hpp"
 #include "kernel_args.hpp"
 #include "launch_waits.hpp"
+#include "whole_share.hpp"
 
 #include <algorithm>
 #include <type_traits>
@@ -31,7 +32,6 @@
 namespace {
 
 constexpr int WHOLE_D = 64;      // padded head sizes
-constexpr int WHOLE_LEAVES = 32; // the producers' counts come together on so many lines, and then on every copy
 // Loads of a row of the dense activation's weights at most (10,240 columns: the layers of a joined list whose weights are in the feed-forward have 6,464 at
 // width 2048; in three launches, as with 12 loads, half of such a list's layers were, and a token of 12 layers took 392 us in place of 355), ..
 constexpr int WHOLE_GLU = 20;
@@ -327,7 +327,7 @@ struct WholePlan {
     int S, keys_max, n_prod, n_attn, merges, grid, waiting;
     size_t lds;
 };
-// A layer's launch with n_keys keys; false: not in one launch.  per_cu: workgroups that a compute unit holds (0: of no matter yet).
+// A layer's launch with n_keys keys; false: not in one launch.  per_cu: workgroups that a compute unit holds (0: of no matter yet).  No producers: three launches are faster.
 bool whole_plan(moon_ctx *ctx, const DecodeProj &p, const DecodeMix &m, const DecodeOut &o, int n_keys, int per_cu, WholePlan *w) {
     const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256, U = p.dp <= 1024 ? 2 : 4;
     if (m.E || m.dimp != WHOLE_D || m.vdimp != WHOLE_D || p.width % 4 || p.dp > 2048 || (reinterpret_cast<uintptr_t>(p.x) & 15)) return false;
@@ -343,8 +343,7 @@ bool whole_plan(moon_ctx *ctx, const DecodeProj &p, const DecodeMix &m, const De
     w->n_attn = wgs * w->S;
     w->merges = wgs + m.dH;
     w->waiting = w->n_attn + m.dH + (o.width + 4 * WHOLE_ROWS - 1) / (4 * WHOLE_ROWS);
-    const int total = std::min(per_cu, U == 2 ? 2 : 4) * cus, work = std::max((p.n16_used + 1) / 2 + (p.n32_used + 1) / 2, p.ff); // (a pair of rows per wavefront at least)
-    w->n_prod = std::max(std::min(total - w->waiting, (work + 3) / 4) / WHOLE_LEAVES, 1) * WHOLE_LEAVES;
+    w->n_prod = whole_producers({(p.n16_used + 1) / 2 + (p.n32_used + 1) / 2, p.ff, U == 2, w->waiting, per_cu, cus, w->keys_max});
     w->grid = w->n_prod + w->waiting;
     return size_t(w->n_attn) * MIX_HEADS * (WHOLE_D + 2) <= m.partial_floats;
 }
@@ -363,10 +362,12 @@ bool decode_whole_supported(moon_ctx *ctx, int dtype, const DecodeProj &p, const
     return need->waiting < need->places;
 }
 
-int launch_decode_whole(moon_ctx *ctx, const DecodeProj &p, const DecodeMix &m, const DecodeOut &o, int per_cu, WholeCounts *counts) {
+int launch_decode_whole(moon_ctx *ctx, const DecodeProj &p, const DecodeMix &m, const DecodeOut &o, int per_cu, WholeCounts *counts, bool *launched) {
+    *launched = false;
     MOON_TRY(check_decode_mix(ctx, m));
     WholePlan w;
     if (!whole_plan(ctx, p, m, o, mix_keys(m, m.pos), per_cu, &w)) return moon_fail(ctx, MOON_EINVAL, "decode: a layer that does not run in one launch");
+    if (!w.n_prod) return MOON_OK;
     const int front16 = m.gate && !m.dH ? m.og : p.n16_used; // (a delta rule's columns come behind the gate's)
     LaunchTargets next = counts->at;
     next.leaf[WHOLE_FRONT] += w.n_prod / WHOLE_LEAVES;
@@ -386,6 +387,7 @@ int launch_decode_whole(moon_ctx *ctx, const DecodeProj &p, const DecodeMix &m, 
         return hipStreamSynchronize(ctx->stream) == hipSuccess ? MOON_OK : MOON_EHIP;
     };
     MOON_TRY(launch_counted(&counts->at, next, counts->error, launch, clear));
+    *launched = true;
     MOON_NOTE_KERNEL(ctx, "decode_whole_kernel %d splits of the keys", w.S);
     return MOON_OK;
 }

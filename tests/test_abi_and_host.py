@@ -124,3 +124,8 @@ def test_places_of_waiting_workgroups():
 def test_counts_of_launches_that_wait():
     """csrc/launch_counts.hpp on the host: counters and targets agree behind launches that ran, that did not, and that reported an earlier call's error."""
     _host_check("launch_counts")
+
+
+def test_producers_of_a_layers_launch():
+    """csrc/whole_share.hpp on the host: how many producers a list decoder's launch is given, and where three launches take its place."""
+    _host_check("whole_share")

@@ -144,6 +144,27 @@ def test_one_launch_and_three_give_the_same_bits(moon, ctx, tmp_path, name):
     assert tokens[0] == tokens[2]
 
 
+def test_few_producers_take_three_launches(moon, ctx):
+    """Without a window the splits' workgroups take the producers' places: behind 20,000 keys of 32 heads 128 are left, behind 22,000 64, whose wavefronts would have 56 pairs of rows each."""
+    cfg = RM.config(128, 2048, [RM.layer(RM.attention(32, 32, 64, 64, 10**6, 0.125), RM.dense(10240))], embed_scale=2.0)
+    m = moon.text_model.TextModel.open_synthetic(cfg, "bfloat16", 23000, seed=5, std=0.02, ctx=ctx)
+    ids = RM.tokens(22100, 128)
+    at = 0
+    for keys, whole in ((20000, True), (22000, False)):
+        m.forward(ids[at:keys])
+        rows = []
+        for i, mode in enumerate((0, 2)):
+            m.set_decode_mode(mode)
+            m.forward(ids[keys + 4 * i:keys + 4 * i + 3]) # (its own note)
+            m.forward(ids[keys + 4 * i + 3:keys + 4 * i + 4])
+            if compute_units() == 256:
+                assert ctx.last_kernel().startswith("decode_whole") == (whole and mode == 0)
+            rows.append(m.logits_f32())
+        at = keys + 8
+        assert np.isfinite(rows).all()
+    m.close()
+
+
 def test_modes_of_list_decoders(moon, ctx):
     """0 and 2 where a layer runs in one launch; none where no launch waits."""
     dense, experts = (RM.config(128, 512, [RM.layer(RM.attention(8, 8, 64, 64, 40, 0.125), mlp)]) for mlp in (RM.dense(128), RM.moe(64, 8, 64)))
