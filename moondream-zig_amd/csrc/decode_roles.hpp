@@ -2,6 +2,7 @@
 // a row's norm, one token's attention and one token of the gated delta rule.
 #pragma once
 #include "delta_math.hpp"
+#include "key_splits.hpp"
 #include "lane_fold.hpp"
 #include "layer_list.hpp"
 #include "lm_types.hpp"
@@ -142,9 +143,6 @@ template <class T, int NV, bool JOIN, bool COH> struct NormRow {
 };
 
 constexpr int MIX_HEADS = 8;       // query heads one workgroup serves
-constexpr int MIX_KEYS = 1024;     // keys of one split at most
-constexpr int MIX_TARGET = 32;     // keys of one split at least
-constexpr int MIX_SPLITS = 16;     // splits at most, unless MIX_KEYS asks for more: what the merge requests at once
 __host__ __device__ __forceinline__ int mix_head_blocks(int per_group) { return (per_group + MIX_HEADS - 1) / MIX_HEADS; }
 
 __device__ __forceinline__ int next_pow2(int v) { return v <= 1 ? 1 : 1 << (32 - __builtin_clz(v - 1)); }
@@ -702,10 +700,6 @@ inline bool mix_whole(const DecodeMix &p) { return p.whole || p.rot || p.rotv ||
 inline int mix_keys(const DecodeMix &p, size_t pos) {
     const int n_win = (int)(p.window ? std::min(pos + 1, (size_t)p.window) : pos + 1);
     return n_win + (p.pool ? (int)(pos + 1 - n_win) / p.pool : 0);
-}
-inline int mix_splits(int n_keys, int wgs, int cus) {
-    const int S = std::min(std::min((n_keys + MIX_TARGET - 1) / MIX_TARGET, MIX_SPLITS), std::max(1, cus / wgs));
-    return std::max(S, (n_keys + MIX_KEYS - 1) / MIX_KEYS);
 }
 inline int check_decode_mix(moon_ctx *ctx, const DecodeMix &p) {
     if (p.pool && ((p.pos + 1) / p.pool > (size_t)p.blocks || (p.pos + 1 >= (size_t)p.pool && p.pool > p.cap))) return moon_fail(ctx, MOON_EINVAL_DIM, "decode attention: %d pooled blocks kept", p.blocks);

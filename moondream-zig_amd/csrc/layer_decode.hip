@@ -367,7 +367,7 @@ int launch_decode_mix(moon_ctx *ctx, int dtype, const DecodeMix &p, const Decode
     const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256, per = p.H / p.G, wgs = p.G * mix_head_blocks(per), n_keys = mix_keys(p, p.pos), S = mix_splits(n_keys, wgs, cus);
     MOON_TRY(check_decode_mix(ctx, p));
     if (size_t(wgs) * S * MIX_HEADS * (p.vdimp + 2) > p.partial_floats) return moon_fail(ctx, MOON_ESEQ_TOO_LONG, "decode attention: %d keys", n_keys);
-    const int keys_max = (n_keys + S - 1) / S;
+    const int keys_max = mix_split_keys(n_keys, S);
     if (p.E && (p.top < 1 || p.top > p.E || p.E > ROUTER_MAX_EXPERTS)) return moon_fail(ctx, MOON_EINVAL_DIM, "router: %d of %d experts", p.top, p.E);
     const int groups = p.E ? p.top * ((p.ff + 1) / 2) : 0;
     const int n_expert = std::min((groups + 3) / 4, std::max(cus, 2 * cus - wgs * S)); // (together two workgroups per CU: more measured slower)

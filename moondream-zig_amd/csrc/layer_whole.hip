@@ -327,7 +327,8 @@ struct WholePlan {
     int S, keys_max, n_prod, n_attn, merges, grid, waiting;
     size_t lds;
 };
-// A layer's launch with n_keys keys; false: not in one launch.  per_cu: workgroups that a compute unit holds (0: of no matter yet).  No producers: three launches are faster.
+// A layer's launch with n_keys keys; false: not in one launch.  per_cu: workgroups that a compute unit holds (0: what launches with up to n_keys keys need at most).  No producers: three
+// launches are faster.
 bool whole_plan(moon_ctx *ctx, const DecodeProj &p, const DecodeMix &m, const DecodeOut &o, int n_keys, int per_cu, WholePlan *w) {
     const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256, U = p.dp <= 1024 ? 2 : 4;
     if (m.E || m.dimp != WHOLE_D || m.vdimp != WHOLE_D || p.width % 4 || p.dp > 2048 || (reinterpret_cast<uintptr_t>(p.x) & 15)) return false;
@@ -335,7 +336,7 @@ bool whole_plan(moon_ctx *ctx, const DecodeProj &p, const DecodeMix &m, const De
     if (m.dH && (m.ddimp > DELTA_ROWS * (256 / (m.dvdimp / 4)))) return false;
     const int per = m.H / m.G, wgs = m.G * mix_head_blocks(per), nh = std::min(per, MIX_HEADS), NH = nh <= 1 ? 1 : nh <= 2 ? 2 : nh <= 4 ? 4 : 8;
     w->S = mix_splits(n_keys, wgs, cus);
-    w->keys_max = std::max(MIX_TARGET, (n_keys + w->S - 1) / w->S); // (fewer keys: the LDS of so many all the same)
+    w->keys_max = std::max(MIX_TARGET, per_cu ? mix_split_keys(n_keys, w->S) : mix_most_split_keys(n_keys, wgs, cus)); // (fewer keys: the LDS of so many all the same)
     w->lds = std::max({size_t(p.dp) * 2, mix_lds_floats(NH, WHOLE_D, WHOLE_D, w->keys_max) * sizeof(float), size_t(!p.ff ? 0 : o.k0 - o.k2 > 512 * WHOLE_HELD ? WHOLE_GLU * 1024 : WHOLE_HELD * 1024),
                        m.dH ? delta_lds_floats(m.ddimp, m.dvdimp, m.kd) * sizeof(float) : 0});
     if (w->lds > 60 * 1024 || size_t(NH) * w->S > mix_lds_floats(NH, WHOLE_D, WHOLE_D, w->keys_max) - 4 * NH - 8) return false;
@@ -355,7 +356,7 @@ size_t decode_whole_sync_words() { return WHOLE_ERROR_AT + 1; }
 bool decode_whole_supported(moon_ctx *ctx, int dtype, const DecodeProj &p, const DecodeMix &m, const DecodeOut &o, size_t max_seq, int *per_cu, WaitNeed *need) {
     const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
     WholePlan w;
-    // (the splits never get fewer with more keys, and their LDS is largest with the most keys)
+    // (the splits never get fewer with more keys)
     if (dtype != MOON_DTYPE_BF16 || !max_seq || !whole_plan(ctx, p, m, o, mix_keys(m, max_seq - 1), 0, &w)) return false;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, reinterpret_cast<const void *>(w.kern), 256, w.lds) != hipSuccess) return false;
     *need = {(w.waiting + 7) / 8, *per_cu * cus / 8};

@@ -129,3 +129,8 @@ def test_counts_of_launches_that_wait():
 def test_producers_of_a_layers_launch():
     """csrc/whole_share.hpp on the host: how many producers a list decoder's launch is given, and where three launches take its place."""
     _host_check("whole_share")
+
+
+def test_splits_of_a_tokens_keys():
+    """csrc/key_splits.hpp on the host: the most keys that a split has behind up to n keys, which sizes a launch for all of a session's positions."""
+    _host_check("key_splits")
