@@ -235,6 +235,30 @@ def test_other_sizes_take_three_launches(moon, ctx, change):
     assert_close(*out)
 
 
+def test_sessions_of_two_contexts_at_once(moon, ctx):
+    """Two threads decode: whichever call finds no places for its waiting workgroups takes three launches, with the same tokens up to rounding."""
+    import threading
+    cfg = LARGE[1]
+    ids = RM.tokens(64, 128)
+    sessions = [moon.text_model.TextModel.open_synthetic(cfg, "bfloat16", 256, seed=5, std=0.02, ctx=c) for c in (ctx, moon.Context(), moon.Context())]
+    alone = feed(sessions[0], ids, [40] + [1] * 24)
+    sessions[0].reset()
+    out = [None] * len(sessions)
+
+    def work(i):
+        out[i] = feed(sessions[i], ids, [40] + [1] * 24)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(len(sessions))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for m, got in zip(sessions, out):
+        assert got is not None
+        assert_close(got, alone)
+        m.close()
+
+
 def test_sessions_of_three_contexts_at_once(moon, ctx):
     """Three threads decode with waiting workgroups that all find places (40 of 128 a die each): the bits of a session alone."""
     import threading
