@@ -3,13 +3,13 @@
 //               feed-forward's silu(gate) * up
 //   attention   a split of a key head's keys each, and the delta rule's heads: ask for cache rows and states, wait for the first count, and report every
 //               merged head
-//   output      rows of the second product, two per wavefront: most of them (23 of 30 KB at width 2048, feed-forward 5504) is in registers by the time that the
+//   output      rows of the second product, two per wavefront: most of them (19 of 30 KB at width 2048, feed-forward 5504) is in registers by the time that the
 //               activation is there, the rest streams while the attention is still under way; the heads' part comes last
 // A layer of 97 MB (width 2048, 8 key heads, feed-forward 5504) took 14.6 + 11 + 4.6 us and three launches' starts, ends and gaps; the weights of its later phases stream while
-// the earlier ones run here.  695 -> 596 us a token behind 61 keys, 382 -> 327 for 12 layers behind 900; 32 key heads 381 -> 337, 4 key heads and feed-forward 2048 358 -> 292; width 1024: 504 -> 384,
-// rotated and joined 549 -> 425 (width 2048, 12 layers 421 -> 355).  What bounds it is the chain q, k, v -> attention -> merge -> output beside the stream: 4 TB/s.
-// Measured and not kept: one row per output wavefront, which leaves the producers half of the places (8 key heads 603, 32 373 of 12 layers; with 192 producers 4 key heads took
-// 1,202); gate rows ahead of the attention (615; 12 layers behind 900 keys 352); a delta rule's taps, ranks and vectors asked for ahead of the wait (no difference); the first count on 8 or 16 lines that all heads' workgroups poll, a hop less, in place of 64 copies (660, 635: 130 pollers on
+// the earlier ones run here.  A token, LM head included, three launches a layer -> one: 24 layers behind 61 keys 724 -> 628 us, 12 behind 900 401 -> 351; 32 key heads 413 -> 370, 4 key heads and feed-forward
+// 2048 372 -> 313; width 1024, 24 layers 500 -> 393, rotated and joined 549 -> 444 (width 2048, 12 layers 440 -> 386).  What bounds it is the chain q, k, v -> attention -> merge -> output beside the stream: 4 TB/s.
+// Measured and not kept (8 key heads 592 us without the LM head, 32 335 of 12 layers at the time): one row per output wavefront, which leaves the producers half of the places (603 and 373; with 192
+// producers 4 key heads took 1,202); gate rows ahead of the attention (615; 12 layers behind 900 keys 352 against 327); a delta rule's taps, ranks and vectors asked for ahead of the wait (no difference); the first count on 8 or 16 lines that all heads' workgroups poll, a hop less, in place of 64 copies (660, 635: 130 pollers on
 // a line hold up the stream); no pauses between the lots of an output row, longer ones, and no wave priority: 0 to 2 % either way; three workgroups a unit at width 1024 in place of two: 0 to 2 % slower.
 // The same for routed experts (a role that waits for the router's logits, chooses and streams the gate and up rows; output workgroups that choose too and ask for the chosen down rows)
 // took 33.3 to 34.3 us a layer with 8 of 64 experts of 704 where the three launches take 32.1: the choice and the two streams behind it follow each other all the same.  Front rows spread evenly over the
@@ -33,7 +33,7 @@ namespace {
 
 constexpr int WHOLE_D = 64;      // padded head sizes
 // Loads of a row of the dense activation's weights at most (10,240 columns: the layers of a joined list whose weights are in the feed-forward have 6,464 at
-// width 2048; in three launches, as with 12 loads, half of such a list's layers were, and a token of 12 layers took 392 us in place of 355), ..
+// width 2048; in three launches, as with 12 loads, half of such a list's layers were, and a token of 12 layers took 392 us in place of 355 at the time), ..
 constexpr int WHOLE_GLU = 20;
 constexpr int WHOLE_HELD = 12;   // .. and those of an output wavefront's first row that wait in registers
 constexpr int WHOLE_ROWS = 2;    // rows of an output wavefront
