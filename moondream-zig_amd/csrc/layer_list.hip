@@ -921,7 +921,7 @@ static int plan_whole(LayerList *l) {
         const bool can = decode_whole_supported(ctx, l->dtype, t.p, t.x, t.o, l->max_seq, &per_cu, &need);
         l->whole_per_cu.push_back(can ? per_cu : 0);
         if (!can) continue;
-        l->whole_need = {std::max(l->whole_need.waiting, need.waiting), l->any_whole ? std::min(l->whole_need.places, need.places) : need.places};
+        l->whole_need = {std::max(l->whole_need.waiting, need.waiting), l->any_whole ? std::min(l->whole_need.places, need.places) : need.places, l->dp <= 1024 ? 2 : 1};
         l->any_whole = true;
     }
     if (l->whole_need.waiting >= l->whole_need.places) l->any_whole = false;

@@ -296,12 +296,12 @@ struct ProfScope {
 };
 
 // A call that decodes tokens one by one: the mode it runs in.  Where workgroups would wait inside launches, it holds their places on the
-// device until the stream has drained; where other contexts' calls have them, it runs in mode 2, which waits for nothing (the
-// same bits).
+// device until the stream has drained; where other contexts' calls have them (or, for lists, too many run: WaitPlaces::enter), it runs in mode 2, which
+// waits for nothing (the same bits).
 struct DecodeCall {
     moon_text_model *m;
     const WaitNeed *need = nullptr;
-    bool drained = false;
+    bool took = false, drained = false;
     static WaitPlaces &places(int device) {
         static WaitPlaces of[64];
         return of[device & 63];
@@ -312,15 +312,14 @@ struct DecodeCall {
         else if (!m->fused) return;
         else if (m->whole_layer && m->call_mode == 0) need = &m->layer_wait;
         else if (m->front && m->call_mode != 2) need = &m->front_wait;
-        if (need && !places(m->ctx->device).take(*need)) {
-            need = nullptr;
-            m->call_mode = 2;
-        }
+        if (!need) return;
+        took = places(m->ctx->device).enter(*need);
+        if (!took) m->call_mode = 2;
     }
     ~DecodeCall() {
         if (!need) return;
-        if (!drained) (void)hipStreamSynchronize(m->ctx->stream); // (an error on the way: launches may still be queued)
-        places(m->ctx->device).give(*need);
+        if (took && !drained) (void)hipStreamSynchronize(m->ctx->stream); // (an error on the way: launches may still be queued)
+        places(m->ctx->device).leave(*need, took);
     }
     DecodeCall(const DecodeCall &) = delete;
 };

@@ -35,6 +35,33 @@ int main() {
         p.give(half);
         expect(p.take(narrow) && !p.take(half), "20 beside 48: over 64");
     }
+    { // calls with a crowd count those that run without places too
+        const WaitNeed wide_list{48, 128, 1}, narrow_list{48, 128, 2};
+        for (const WaitNeed &n : {wide_list, narrow_list}) {
+            WaitPlaces p;
+            expect(p.enter(n) && p.enter(n), "two fit");
+            expect(!p.enter(n), "a third does not");
+            p.leave(n, true); // one of the first two is over and begins anew beside one with places and one without
+            const bool again = p.enter(n);
+            expect(again == (n.crowd > 1), "144 of 128 run");
+            p.leave(n, true);
+            expect(p.enter(n) == (n.crowd > 1), "the other one likewise");
+            for (int i = 0; i < 2; i++) p.leave(n, n.crowd > 1);
+            p.leave(n, false);
+            expect(p.enter(n), "none is left behind");
+        }
+        WaitPlaces p;
+        for (int i = 0; i < 5; i++) expect(p.enter(narrow_list) == (i < 2), "five, 240 of 256");
+        p.leave(narrow_list, true);
+        expect(p.enter(narrow_list), "no crowd yet");
+        expect(!p.enter(narrow_list), "a sixth");
+        p.leave(narrow_list, true);
+        expect(!p.enter(narrow_list), "288 of 256 run");
+        expect(p.enter(front) && !p.enter(wide), "without a crowd the places alone count: 32 beside 48, but not 96");
+        p.leave(narrow_list, true);
+        p.leave(front, true);
+        expect(p.enter(wide), "96 where nobody holds any");
+    }
     // threads that come and go: whatever is held at once leaves a place
     WaitPlaces p;
     std::atomic<int> waiting{0}, taken{0}, refused{0};
